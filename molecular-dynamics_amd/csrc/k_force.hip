@@ -370,23 +370,12 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_dem_fused(const CMir spos, 
     double* sw = dyn + 5 * a.wcap;
     const bool staged = win_size(W) <= a.wcap;
     if (staged) {
-        // one thread group per window row, as in stage_window
-        const int nseg = W.nseg;
-        const int gsz = max(1, (int)blockDim.x / nseg);
-        const int ngrp = (int)blockDim.x / gsz;
-        const int g = (int)threadIdx.x / gsz, l = (int)threadIdx.x - g * gsz;
-        if (g < ngrp) {
-            for (int sg = g; sg < nseg; sg += ngrp) {
-                const int off = W.seg_off[sg], beg = W.seg_beg[sg], len = W.seg_off[sg + 1] - off;
-                for (int q = l; q < len; q += gsz) {
-                    const int t = off + q, k = beg + q;
-                    const double4 p = spos[k];
-                    const double4 u = svel[k];
-                    sx[t] = p.x; sy[t] = p.y; sz[t] = p.z;
-                    su[t] = u.x; sv[t] = u.y; sw[t] = u.z;
-                }
-            }
-        }
+        double4 p[kStageInFlight], q[kStageInFlight];
+        stage_rows(W, [&](int k, int u) { p[u] = spos[k]; q[u] = svel[k]; },
+                   [&](int t, int u) {
+                       sx[t] = p[u].x; sy[t] = p[u].y; sz[t] = p[u].z;
+                       su[t] = q[u].x; sv[t] = q[u].y; sw[t] = q[u].z;
+                   });
     }
     __syncthreads();
     auto atoms = [&](auto staged_c) {

@@ -86,45 +86,43 @@ struct TileWin {
     int seg_off[kMaxSeg + 1];   // window offset of each row (prefix)
 };
 
-// Build the tile's window (whole block; barriers inside).  Row s covers
+// Build the tile's window (whole block; a barrier at the end).  Row s covers
 // cells x in [cx0-1, cx0+tx] (clipped) at y = cy0-1 + s % (ty+2),
-// z = cz0-1 + s / (ty+2).
+// z = cz0-1 + s / (ty+2).  The first wavefront loads the rows' CSR ranges
+// and turns their lengths into offsets by a scan in registers, 64 rows at a
+// time (blocks have at least one wavefront).
 __device__ __forceinline__ void tile_window(int tile, const int* __restrict__ start, TileGeom g, TileWin& W) {
     const int t = threadIdx.x;
-    const int tx_i = tile % g.ntx, ty_i = (tile / g.ntx) % g.nty, tz_i = tile / (g.ntx * g.nty);
-    const int cx0 = 1 + tx_i * g.tx, cy0 = 1 + ty_i * g.ty, cz0 = 1 + tz_i * g.tz;
-    const int wy = g.ty + 2;
-    const int nseg = wy * (g.tz + 2);
-    for (int s = t; s < nseg; s += blockDim.x) {
-        const int y = cy0 - 1 + s % wy, z = cz0 - 1 + s / wy;
-        const int xlo = max(cx0 - 1, 0), xhi = min(cx0 + g.tx, g.nx - 1);
-        int b = 0, len = 0;
-        if (y >= 0 && y < g.ny && z >= 0 && z < g.nz) {
-            const int row = (z * g.ny + y) * g.nx;
-            b = start[row + xlo];
-            len = start[row + xhi + 1] - b;
-        }
-        W.seg_beg[s] = b;
-        W.seg_off[s + 1] = len;
-    }
-    if (t == 0) {
-        W.cx0 = cx0;
-        W.cy0 = cy0;
-        W.cz0 = cz0;
-        W.nseg = nseg;
-    }
-    __syncthreads();
     if (t < kWave) {
-        // the first wavefront turns the row lengths into offsets (inclusive
-        // scan, 64 rows at a time; blocks have at least one wavefront)
+        const int tx_i = tile % g.ntx, ty_i = (tile / g.ntx) % g.nty, tz_i = tile / (g.ntx * g.nty);
+        const int cx0 = 1 + tx_i * g.tx, cy0 = 1 + ty_i * g.ty, cz0 = 1 + tz_i * g.tz;
+        const int wy = g.ty + 2;
+        const int nseg = wy * (g.tz + 2);
+        const int xlo = max(cx0 - 1, 0), xhi = min(cx0 + g.tx, g.nx - 1);
         int carry = 0;
         for (int s0 = 0; s0 < nseg; s0 += kWave) {
             const int s = s0 + t;
-            const int inc = wave_inclusive_scan(s < nseg ? W.seg_off[s + 1] : 0);
-            if (s < nseg) W.seg_off[s + 1] = carry + inc;
-            carry += __shfl(inc, kWave - 1, kWave);
+            const int y = cy0 - 1 + s % wy, z = cz0 - 1 + s / wy;
+            int b = 0, len = 0;
+            if (s < nseg && y >= 0 && y < g.ny && z >= 0 && z < g.nz) {
+                const int row = (z * g.ny + y) * g.nx;
+                b = start[row + xlo];
+                len = start[row + xhi + 1] - b;
+            }
+            const int inc = wave_inclusive_scan(len);
+            if (s < nseg) {
+                W.seg_beg[s] = b;
+                W.seg_off[s + 1] = carry + inc;
+            }
+            carry += __builtin_amdgcn_readlane(inc, kWave - 1);
         }
-        if (t == 0) W.seg_off[0] = 0;
+        if (t == 0) {
+            W.cx0 = cx0;
+            W.cy0 = cy0;
+            W.cz0 = cz0;
+            W.nseg = nseg;
+            W.seg_off[0] = 0;
+        }
     }
     __syncthreads();
 }
@@ -166,6 +164,34 @@ __device__ __forceinline__ void stage_row_starts(const TileWin& W, const int* __
     __syncthreads();
 }
 
+// Walk the window's atoms: the block is split into one thread group per
+// window row (rows in turn when there are more rows than groups), and a group
+// walks its row's contiguous CSR range, so no offset-to-row search is needed.
+// Each thread has kStageInFlight atoms' loads under way before the first
+// value is used: load(k, u) issues slot u's loads for mirror index k (clamped
+// to the row, so always valid), put(t, u) stores it at window offset t.  With
+// one atom at a time the staging of a window was three to eight dependent
+// memory round trips.
+constexpr int kStageInFlight = 4;
+template <class Load, class Put>
+__device__ __forceinline__ void stage_rows(const TileWin& W, Load&& load, Put&& put) {
+    const int nseg = W.nseg;
+    const int gsz = max(1, (int)blockDim.x / nseg);
+    const int ngrp = (int)blockDim.x / gsz;
+    const int g = (int)threadIdx.x / gsz, l = (int)threadIdx.x - g * gsz;
+    if (g >= ngrp) return;
+    for (int s = g; s < nseg; s += ngrp) {
+        const int off = W.seg_off[s], beg = W.seg_beg[s], len = W.seg_off[s + 1] - off;
+        for (int q = l; q < len; q += kStageInFlight * gsz) {
+#pragma unroll
+            for (int u = 0; u < kStageInFlight; ++u) load(beg + min(q + u * gsz, len - 1), u);
+#pragma unroll
+            for (int u = 0; u < kStageInFlight; ++u)
+                if (q + u * gsz < len) put(off + q + u * gsz, u);
+        }
+    }
+}
+
 // Stage the window's FP64 positions and, when sj != nullptr, atom indices
 // into LDS if it fits wcap atoms; otherwise consumers read the mirror.
 template <class SP>
@@ -174,24 +200,15 @@ __device__ __forceinline__ bool stage_tile(const TileWin& W, int wcap, const SP&
     const int S = win_size(W);
     const bool staged = S <= wcap;
     if (staged) {
-        // one thread group per window row, as in stage_window
-        const int nseg = W.nseg;
-        const int gsz = max(1, (int)blockDim.x / nseg);
-        const int ngrp = (int)blockDim.x / gsz;
-        const int g = (int)threadIdx.x / gsz, l = (int)threadIdx.x - g * gsz;
-        if (g < ngrp) {
-            for (int s = g; s < nseg; s += ngrp) {
-                const int off = W.seg_off[s], beg = W.seg_beg[s], len = W.seg_off[s + 1] - off;
-                for (int q = l; q < len; q += gsz) {
-                    const int t = off + q, k = beg + q;
-                    const double4 p = spos[k];
-                    sx[t] = p.x;
-                    sy[t] = p.y;
-                    sz[t] = p.z;
-                    if (sj) sj[t] = parts[k];
-                }
-            }
-        }
+        double4 p[kStageInFlight];
+        int j[kStageInFlight];
+        stage_rows(W, [&](int k, int u) { p[u] = spos[k]; if (sj) j[u] = parts[k]; },
+                   [&](int t, int u) {
+                       sx[t] = p[u].x;
+                       sy[t] = p[u].y;
+                       sz[t] = p[u].z;
+                       if (sj) sj[t] = j[u];
+                   });
     }
     __syncthreads();
     return staged;
@@ -231,26 +248,15 @@ __device__ __forceinline__ bool stage_window(const TileWin& W, int wcap, const S
     const int S = win_size(W);
     const bool staged = S + pad <= wcap;
     if (staged) {
-        // the block is split into one thread group per window row (rows in
-        // turn when there are more rows than groups); a group copies its
-        // row's contiguous CSR range, so no offset-to-row search is needed
-        const int nseg = W.nseg;
-        const int gsz = max(1, (int)blockDim.x / nseg);
-        const int ngrp = (int)blockDim.x / gsz;
-        const int g = (int)threadIdx.x / gsz, l = (int)threadIdx.x - g * gsz;
-        if (g < ngrp) {
-            for (int s = g; s < nseg; s += ngrp) {
-                const int off = W.seg_off[s], beg = W.seg_beg[s], len = W.seg_off[s + 1] - off;
-                for (int q = l; q < len; q += gsz) {
-                    const int t = off + q, k = beg + q;
-                    const double4 p = spos[k];
-                    st.xyz[3 * t + 0] = p.x;
-                    st.xyz[3 * t + 1] = p.y;
-                    st.xyz[3 * t + 2] = p.z;
-                    if (parts) st.j[t] = parts[k];
-                }
-            }
-        }
+        double4 p[kStageInFlight];
+        int j[kStageInFlight];
+        stage_rows(W, [&](int k, int u) { p[u] = spos[k]; if (parts) j[u] = parts[k]; },
+                   [&](int t, int u) {
+                       st.xyz[3 * t + 0] = p[u].x;
+                       st.xyz[3 * t + 1] = p[u].y;
+                       st.xyz[3 * t + 2] = p[u].z;
+                       if (parts) st.j[t] = j[u];
+                   });
         if ((int)threadIdx.x < pad) {
             const int t = S + (int)threadIdx.x;
             st.xyz[3 * t + 0] = kFarPos;
