@@ -214,10 +214,8 @@ static void restore_from(Sim& s, const DevBuf& bx, const DevBuf& bv, size_t slot
 
 // ghosts, cells and full list for the current positions (no periodic wrap)
 static void relist(Sim& s, double cutoff) {
-    s.ng = 0;
-    build_ghosts(s);
-    bin_particles(s);
-    build_neighbor_lists(s, 0, cutoff);
+    s.gh_wanted = 0;
+    rebuild_lists(s, false, 0, cutoff);
 }
 
 static int ntiles_of(const Sim& s) { return s.tiles.ntx * s.tiles.nty * s.tiles.ntz; }
@@ -283,10 +281,7 @@ static void forward_traj(Sim& s, const TrajSpec& p, bool store_ckpt, double* uba
     for (int t = 1; t <= p.steps && !has_error(); ++t) {
         initial_integration(s, p.dt);
         if (t % p.ck == 0) {
-            s.ng = 0;
-            build_ghosts(s, true);  // md_enforce_pbc + borders
-            bin_particles(s);
-            build_neighbor_lists(s, 0, cut);
+            rebuild_lists(s, true, 0, cut);  // with md_enforce_pbc
         } else {
             refresh_ghosts(s);
         }

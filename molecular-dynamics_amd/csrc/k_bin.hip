@@ -9,16 +9,11 @@
 
 namespace tmd {
 
-struct BinArgs {
-    double xmin, ymin, zmin, spacing;
-    int nx, ny, ncells, nall;
-};
-
-__global__ void k_bin_count(const double4* __restrict__ pos, BinArgs a, int* __restrict__ cell_of, int* __restrict__ slot,
-                            int* __restrict__ count, int* __restrict__ inv) {
+__global__ void k_bin_count(const double4* __restrict__ pos, BinArgs a, int nall, int* __restrict__ cell_of,
+                            int* __restrict__ slot, int* __restrict__ count, int* __restrict__ inv) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     int c = -1;
-    if (i < a.nall) {
+    if (i < nall) {
         const double4 p = pos[i];
         const double fx = floor((p.x - a.xmin) / a.spacing);
         const double fy = floor((p.y - a.ymin) / a.spacing);
@@ -31,173 +26,251 @@ __global__ void k_bin_count(const double4* __restrict__ pos, BinArgs a, int* __r
         }
     }
     const int sl = wave_cell_slot(c, count);  // all lanes take part
-    if (i >= a.nall) return;
+    if (i >= nall) return;
     cell_of[i] = c;
     slot[i] = sl;
-    inv[i] = -1;  // set by k_bin_sort for binned atoms
+    if (c < 0) inv[i] = -1;  // the sort sets the binned ones
 }
 
-__global__ void k_bin_scatter(const int* __restrict__ cell_of, const int* __restrict__ slot, const int* __restrict__ start,
-                              int nall, int* __restrict__ parts) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nall) return;
-    const int c = cell_of[i];
-    if (c >= 0) parts[start[c] + slot[i]] = i;
+// Counting-sort placement: (atom, source slot) of every binned atom into its
+// cell's segment.  Blocks below nbq take the source slots (MIR: mirror slots
+// of the last binning, holding atom parts[q]; else atom q itself), the rest
+// the ghosts of the emit sweep, their number read on the device.
+template <bool MIR>
+__global__ void __launch_bounds__(256) k_bin_place(const int* __restrict__ cell_of, const int* __restrict__ slot, int nq, int nbq,
+                                                   const int* __restrict__ parts, const int* __restrict__ g_cell,
+                                                   const int* __restrict__ g_slot, int n, int gcap,
+                                                   const int* __restrict__ ctr, const int* __restrict__ start,
+                                                   int2* __restrict__ pairs) {
+    const int b = blockIdx.x;
+    if (b < nbq) {
+        const int q = b * 256 + (int)threadIdx.x;
+        if (q >= nq) return;
+        const int c = cell_of[q];
+        if (c >= 0) pairs[start[c] + slot[q]] = make_int2(MIR ? parts[q] : q, q);
+        return;
+    }
+    const int ng = min(ctr[CT_NGHOST], gcap);
+    for (int g = (b - nbq) * 256 + (int)threadIdx.x; g < ng; g += ((int)gridDim.x - nbq) * 256) {
+        const int c = g_cell[g];
+        if (c >= 0) pairs[start[c] + g_slot[g]] = make_int2(n + g, -1);
+    }
 }
 
-// One thread per cell (sparse grids: a few atoms per cell): insertion sort
-// of the cell segment by atom index, then its locals and the CSR index of
-// every atom; the same result as k_bin_sort.
-__global__ void k_bin_sort_small(const int* __restrict__ start, int ncells, int n, int* __restrict__ parts,
-                                 int* __restrict__ local_count, int* __restrict__ inv) {
+// Work tile of a cell that can hold locals, -1 for the grid's outer cells.
+__device__ __forceinline__ int cell_tile(int c, const TileGeom& g) {
+    const int x = c % g.nx, y = (c / g.nx) % g.ny, z = c / (g.nx * g.ny);
+    if (x < 1 || y < 1 || z < 1 || x > g.nx - 2 || y > g.ny - 2 || z > g.nz - 2) return -1;
+    return ((z - 1) / g.tz * g.nty + (y - 1) / g.ty) * g.ntx + (x - 1) / g.tx;
+}
+
+// One thread per cell (sparse grids: a few atoms per cell): each pair's rank
+// by counting, then the cell's locals and the CSR index of every atom; the
+// same result as k_bin_sort.
+__global__ void k_bin_sort_small(const int* __restrict__ start, int ncells, int n, const int2* __restrict__ pairs,
+                                 int* __restrict__ parts, int* __restrict__ src, int* __restrict__ local_count,
+                                 int* __restrict__ inv, TileGeom g, int* __restrict__ tile_count) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= ncells) return;
-    const int b = start[c], e = start[c + 1];
-    for (int k = b + 1; k < e; ++k) {
-        const int v = parts[k];
-        int q = k - 1;
-        while (q >= b && parts[q] > v) {
-            parts[q + 1] = parts[q];
-            --q;
-        }
-        parts[q + 1] = v;
-    }
+    const int b = start[c], e = start[c + 1], m = e - b;
     int nl = 0;
-    while (b + nl < e && parts[b + nl] < n) ++nl;
+    constexpr int kHeld = 6;  // pairs held in registers
+    if (m <= kHeld) {
+        int2 v[kHeld];
+#pragma unroll
+        for (int k = 0; k < kHeld; ++k) v[k] = k < m ? pairs[b + k] : make_int2(0x7fffffff, 0);
+#pragma unroll
+        for (int k = 0; k < kHeld; ++k) {
+            if (k >= m) break;
+            int rank = 0;
+#pragma unroll
+            for (int q = 0; q < kHeld; ++q) rank += v[q].x < v[k].x ? 1 : 0;
+            parts[b + rank] = v[k].x;
+            src[b + rank] = v[k].y;
+            inv[v[k].x] = b + rank;
+            nl += v[k].x < n ? 1 : 0;
+        }
+    } else {
+        for (int k = b; k < e; ++k) {
+            const int2 v = pairs[k];
+            int rank = 0;
+            for (int q = b; q < e; ++q) rank += pairs[q].x < v.x ? 1 : 0;
+            parts[b + rank] = v.x;
+            src[b + rank] = v.y;
+            inv[v.x] = b + rank;
+            nl += v.x < n ? 1 : 0;
+        }
+    }
     local_count[c] = nl;
-    for (int k = b; k < e; ++k) inv[parts[k]] = k;
+    if (tile_count && nl > 0) {
+        const int t = cell_tile(c, g);
+        if (t >= 0) atomicAdd(&tile_count[t], nl);
+    }
 }
 
-// One wavefront per cell: sort the cell segment by atom index, then the
-// number of locals in it (locals have the lowest indices, so they lead every
-// sorted segment).
-__global__ void __launch_bounds__(256) k_bin_sort(const int* __restrict__ start, int ncells, int n, int* __restrict__ parts,
-                                                  int* __restrict__ local_count, int* __restrict__ inv) {
+// One wavefront per cell: sort the cell segment by atom index; the number of
+// locals in it (locals have the lowest indices, so they lead every sorted
+// segment) goes to the cell and is added to its work tile.
+__global__ void __launch_bounds__(256) k_bin_sort(const int* __restrict__ start, int ncells, int n, const int2* __restrict__ pairs,
+                                                  int* __restrict__ parts, int* __restrict__ src, int* __restrict__ local_count,
+                                                  int* __restrict__ inv, TileGeom g, int* __restrict__ tile_count) {
     const int c = blockIdx.x * (blockDim.x / kWave) + (int)threadIdx.x / kWave;
     if (c >= ncells) return;  // whole wavefronts
-    const int nl = wave_sort_cell(start[c], start[c + 1], n, parts, inv);
-    if ((threadIdx.x & (kWave - 1)) == 0) local_count[c] = nl;
-}
-
-// Tile work order (see tmd_window.hpp): one thread per tile counts the
-// tile's locals and the size of its window (small tiles).
-__global__ void k_tile_stats_small(const int* __restrict__ start, const int* __restrict__ local_count, TileGeom g,
-                                   int ntiles, int* __restrict__ tile_count, int* __restrict__ max_window,
-                                   int* __restrict__ max_locals) {
-    const int tile = blockIdx.x * blockDim.x + threadIdx.x;
-    int cnt = 0, S = 0;
-    if (tile < ntiles) {
-        const int tx_i = tile % g.ntx, ty_i = (tile / g.ntx) % g.nty, tz_i = tile / (g.ntx * g.nty);
-        const int cx0 = 1 + tx_i * g.tx, cy0 = 1 + ty_i * g.ty, cz0 = 1 + tz_i * g.tz;
-        const int cx1 = min(cx0 + g.tx, g.nx - 1), cy1 = min(cy0 + g.ty, g.ny - 1), cz1 = min(cz0 + g.tz, g.nz - 1);
-        for (int z = cz0; z < cz1; ++z)
-            for (int y = cy0; y < cy1; ++y)
-                for (int x = cx0; x < cx1; ++x) cnt += local_count[(z * g.ny + y) * g.nx + x];
-        tile_count[tile] = cnt;
-        const int xlo = cx0 - 1, xhi = min(cx0 + g.tx, g.nx - 1);
-        for (int z = cz0 - 1; z <= cz0 + g.tz; ++z)
-            for (int y = cy0 - 1; y <= cy0 + g.ty; ++y)
-                if (y < g.ny && z < g.nz) {
-                    const int row = (z * g.ny + y) * g.nx;
-                    S += start[row + xhi + 1] - start[row + xlo];
-                }
-        if (cnt == 0) S = 0;  // empty tiles launch no block
-    }
-    // one atomic per wavefront for each maximum
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) {
-        S = max(S, __shfl_down(S, d, kWave));
-        cnt = max(cnt, __shfl_down(cnt, d, kWave));
-    }
-    if ((threadIdx.x & (kWave - 1)) == 0 && cnt > 0) {
-        atomicMax(max_window, S);
-        atomicMax(max_locals, cnt);
-    }
-}
-
-// The same with one wavefront per tile (large tiles: lanes stride over the
-// cells and the window rows; fixed-order wavefront sums).
-__global__ void __launch_bounds__(kWave) k_tile_stats(const int* __restrict__ start, const int* __restrict__ local_count,
-                                                      TileGeom g, int ntiles, int* __restrict__ tile_count,
-                                                      int* __restrict__ max_window, int* __restrict__ max_locals) {
-    const int tile = blockIdx.x;
-    if (tile >= ntiles) return;
-    const int lane = threadIdx.x;
-    const int tx_i = tile % g.ntx, ty_i = (tile / g.ntx) % g.nty, tz_i = tile / (g.ntx * g.nty);
-    const int cx0 = 1 + tx_i * g.tx, cy0 = 1 + ty_i * g.ty, cz0 = 1 + tz_i * g.tz;
-    const int cx1 = min(cx0 + g.tx, g.nx - 1), cy1 = min(cy0 + g.ty, g.ny - 1), cz1 = min(cz0 + g.tz, g.nz - 1);
-    const int ex = cx1 - cx0, ey = cy1 - cy0, ez = cz1 - cz0;
-    int cnt = 0;
-    for (int q = lane; q < ex * ey * ez; q += kWave)
-        cnt += local_count[((cz0 + q / (ex * ey)) * g.ny + (cy0 + (q / ex) % ey)) * g.nx + (cx0 + q % ex)];
-    int S = 0;
-    const int xlo = cx0 - 1, xhi = min(cx0 + g.tx, g.nx - 1);
-    const int wy = g.ty + 2;
-    for (int q = lane; q < wy * (g.tz + 2); q += kWave) {
-        const int y = cy0 - 1 + q % wy, z = cz0 - 1 + q / wy;
-        if (y < g.ny && z < g.nz) {
-            const int row = (z * g.ny + y) * g.nx;
-            S += start[row + xhi + 1] - start[row + xlo];
+    const int nl = wave_sort_pairs(start[c], start[c + 1], n, pairs, parts, src, inv);
+    if ((threadIdx.x & (kWave - 1)) == 0) {
+        local_count[c] = nl;
+        if (tile_count && nl > 0) {
+            const int t = cell_tile(c, g);
+            if (t >= 0) atomicAdd(&tile_count[t], nl);
         }
     }
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) {
-        cnt += __shfl_down(cnt, d, kWave);
-        S += __shfl_down(S, d, kWave);
-    }
-    if (lane == 0) {
-        tile_count[tile] = cnt;
-        // read first: only the few tiles that raise a maximum issue the atomic
-        // (thousands of same-address atomics from separate wavefronts serialise)
-        if (cnt > 0 && S > *(volatile int*)max_window) atomicMax(max_window, S);
-        if (cnt > 0 && cnt > *(volatile int*)max_locals) atomicMax(max_locals, cnt);
-    }
 }
 
-// Work order: one block per tile writes the tile's locals in (z, y, x)
-// cell order (lanes of a wavefront are then atoms of adjacent cells, whose
-// neighbour windows overlap -- measured faster than grouping lanes by list
-// length), with each atom's mirror index and cell.
-__global__ void __launch_bounds__(256) k_tile_fill_block(const int* __restrict__ start, const int* __restrict__ local_count,
-                                                         const int* __restrict__ tile_start, TileGeom g,
-                                                         const int* __restrict__ parts, int* __restrict__ work,
-                                                         int* __restrict__ work_k, int* __restrict__ work_c) {
+// Locals of every tile, a wavefront per tile (large grids: one atomic per
+// cell onto the tiles, as the sorts do for small ones, costs 30 us at 132,000
+// cells and 50 us in the 560,000-cell DEM grid; this launch 5 us).
+__global__ void __launch_bounds__(256) k_tile_count(const int* __restrict__ local_count, TileGeom g, int ntiles,
+                                                    int* __restrict__ tile_count) {
+    const int tile = blockIdx.x * 4 + (int)threadIdx.x / kWave;
+    if (tile >= ntiles) return;  // whole wavefronts
+    const int lane = threadIdx.x & (kWave - 1);
+    const int tx_i = tile % g.ntx, ty_i = (tile / g.ntx) % g.nty, tz_i = tile / (g.ntx * g.nty);
+    const int cx0 = 1 + tx_i * g.tx, cy0 = 1 + ty_i * g.ty, cz0 = 1 + tz_i * g.tz;
+    const int ex = min(cx0 + g.tx, g.nx - 1) - cx0, ey = min(cy0 + g.ty, g.ny - 1) - cy0, ez = min(cz0 + g.tz, g.nz - 1) - cz0;
+    int v = 0;
+    for (int q = lane; q < ex * ey * ez; q += kWave)
+        v += local_count[((cz0 + q / (ex * ey)) * g.ny + (cy0 + (q / ex) % ey)) * g.nx + (cx0 + q % ex)];
+    const int tot = __builtin_amdgcn_readlane(wave_inclusive_scan(v), kWave - 1);
+    if (lane == 0) tile_count[tile] = tot;
+}
+constexpr int kTileAtomicCells = 16384;  // grids up to this many cells count by atomics in the sort
+
+// The last sweep of a rebuild before the lists, three independent parts in
+// one launch (each alone is a few microseconds on a small box):
+//   blocks [0, ntiles): the tile's work order -- its locals in (z, y, x) cell
+//   order (lanes of a wavefront are then atoms of adjacent cells, whose
+//   neighbour windows overlap; measured faster than grouping lanes by list
+//   length) with mirror index, cell and ghost entries -- and the tile and
+//   window statistics;
+//   the next nbm blocks: the cell-ordered mirror, positions (and velocities)
+//   from the last mirror (MIR) or from atom order;
+//   the rest: the mirror indices of every ghost and its owner, and the
+//   ghost index.
+// With few tiles (scanned == 0) a tile's first work slot is the sum of the
+// counts before it, taken by the block itself: a scan launch less.
+constexpr int kTileFlat = 2048;
+struct FinishArgs {
+    TileGeom g;
+    int ntiles, scanned, n, gcap, ncells, nbm, ghost_vel;
+};
+
+template <bool MIR>
+__global__ void __launch_bounds__(256) k_rebuild_finish(FinishArgs a, const int* __restrict__ start,
+                                                        const int* __restrict__ local_count,
+                                                        const int* __restrict__ tile_count, int* __restrict__ tile_start,
+                                                        const int* __restrict__ parts, const int* __restrict__ src,
+                                                        const int* __restrict__ inv, int* __restrict__ work,
+                                                        int* __restrict__ work_k, int* __restrict__ work_c,
+                                                        const int* __restrict__ gh_pack, int* __restrict__ gh_w,
+                                                        const double4* __restrict__ pos, const double4* __restrict__ vel,
+                                                        const CMir spos_old, const CMir svel_old, const Mir spos,
+                                                        const Mir svel, const int* __restrict__ g_owner,
+                                                        const int* __restrict__ g_code, const int* __restrict__ gh_e,
+                                                        int* __restrict__ g_ko, int* __restrict__ g_kg, int* __restrict__ gh_k,
+                                                        int* __restrict__ gh_c, int* __restrict__ ctr) {
+    const int b = blockIdx.x, tid = threadIdx.x;
+    if (b >= a.ntiles + a.nbm) {
+        const int ng = min(ctr[CT_NGHOST], a.gcap);
+        const int stride = ((int)gridDim.x - a.ntiles - a.nbm) * 256;
+        for (int g = (b - a.ntiles - a.nbm) * 256 + tid; g < ng; g += stride) {
+            const int kg = inv[a.n + g];
+            g_ko[g] = inv[g_owner[g]];
+            g_kg[g] = kg;
+            const int e = gh_pack ? gh_e[g] : a.gcap;
+            if (e < a.gcap) {  // entry numbers run past the capacity only where the host will grow it
+                gh_k[e] = kg;
+                gh_c[e] = g_code[g] & 0xff;
+            }
+        }
+        return;
+    }
+    if (b >= a.ntiles) {
+        const int k = (b - a.ntiles) * 256 + tid;
+        if (k >= start[a.ncells]) return;
+        const int j = parts[k];
+        if (MIR && j < a.n) {
+            const int q = src[k];
+            spos[k] = spos_old[q];
+            svel[k] = svel_old[q];
+        } else {
+            spos[k] = pos[j];
+            if (svel.p && (j < a.n || a.ghost_vel)) svel[k] = vel[j];
+        }
+        return;
+    }
+    const TileGeom g = a.g;
+    const int tile = b;
     __shared__ int coff[kMaxTile * kMaxTile * kMaxTile + 1];
-    const int tile = blockIdx.x;
-    const int w0 = tile_start[tile], nloc = tile_start[tile + 1] - w0;
-    if (nloc == 0) return;
+    int w0, nloc;
+    if (a.scanned) {
+        w0 = tile_start[tile];
+        nloc = tile_start[tile + 1] - w0;
+    } else {
+        int v = 0, tot;
+        for (int t = tid; t < tile; t += 256) v += tile_count[t];
+        (void)block_exclusive_scan(v, &tot);
+        w0 = tot;
+        nloc = tile_count[tile];
+        if (tid == 0) {
+            tile_start[tile] = w0;
+            if (tile == a.ntiles - 1) tile_start[a.ntiles] = w0 + nloc;
+        }
+    }
+    if (tid == 0) {
+        if (tile == a.ntiles - 1) ctr[CT_PLACED] = w0 + nloc;
+        if (tile == 0) ctr[CT_BINNED] = start[a.ncells];
+    }
+    if (nloc == 0) return;  // the whole block
     const int tx_i = tile % g.ntx, ty_i = (tile / g.ntx) % g.nty, tz_i = tile / (g.ntx * g.nty);
     const int cx0 = 1 + tx_i * g.tx, cy0 = 1 + ty_i * g.ty, cz0 = 1 + tz_i * g.tz;
     const int cx1 = min(cx0 + g.tx, g.nx - 1), cy1 = min(cy0 + g.ty, g.ny - 1), cz1 = min(cz0 + g.tz, g.nz - 1);
     const int ex = cx1 - cx0, ey = cy1 - cy0, ez = cz1 - cz0;
     const int nc = ex * ey * ez;
-    // cell offsets inside the tile: one thread for small tiles, else a
-    // block-wide exclusive scan of the cells' local counts, 256 at a time
-    if (nc <= 64) {
-        if (threadIdx.x == 0) {
-            int o = 0;
-            for (int q = 0; q < nc; ++q) {
-                coff[q] = o;
-                o += local_count[((cz0 + q / (ex * ey)) * g.ny + (cy0 + (q / ex) % ey)) * g.nx + (cx0 + q % ex)];
+    // cell offsets inside the tile and the window's size (its rows' lengths)
+    int S = 0;
+    {
+        const int xlo = cx0 - 1, xhi = min(cx0 + g.tx, g.nx - 1), wy = g.ty + 2;
+        for (int q = tid; q < wy * (g.tz + 2); q += 256) {
+            const int y = cy0 - 1 + q % wy, z = cz0 - 1 + q / wy;
+            if (y < g.ny && z < g.nz) {
+                const int row = (z * g.ny + y) * g.nx;
+                S += start[row + xhi + 1] - start[row + xlo];
             }
-            coff[nc] = o;
         }
-    } else {
-        int carry = 0;
-        for (int q0 = 0; q0 < nc; q0 += kScanThreads) {
-            const int q = q0 + (int)threadIdx.x;
-            const int v = q < nc ? local_count[((cz0 + q / (ex * ey)) * g.ny + (cy0 + (q / ex) % ey)) * g.nx + (cx0 + q % ex)] : 0;
-            int tot;
-            const int ex_v = block_exclusive_scan(v, &tot);
-            if (q < nc) coff[q] = carry + ex_v;
-            carry += tot;
-        }
-        if (threadIdx.x == 0) coff[nc] = carry;
+        int tot;
+        (void)block_exclusive_scan(S, &tot);
+        S = tot;
+    }
+    int carry = 0;
+    for (int q0 = 0; q0 < nc; q0 += 256) {
+        const int q = q0 + tid;
+        const int v = q < nc ? local_count[((cz0 + q / (ex * ey)) * g.ny + (cy0 + (q / ex) % ey)) * g.nx + (cx0 + q % ex)] : 0;
+        int tot;
+        const int ex_v = block_exclusive_scan(v, &tot);
+        if (q < nc) coff[q] = carry + ex_v;
+        carry += tot;
+    }
+    if (tid == 0) {
+        coff[nc] = carry;
+        // read first: only the few tiles that raise a maximum issue the atomic
+        // (thousands of same-address atomics from separate blocks serialise)
+        if (S > *(volatile int*)&ctr[CT_MAXWIN]) atomicMax(&ctr[CT_MAXWIN], S);
+        if (nloc > *(volatile int*)&ctr[CT_MAXLOC]) atomicMax(&ctr[CT_MAXLOC], nloc);
     }
     __syncthreads();
     // one thread per local (coalesced writes): its cell is the last one whose
     // offset does not exceed its place (empty cells are passed over)
-    for (int e = threadIdx.x; e < nloc; e += blockDim.x) {
+    for (int e = tid; e < nloc; e += 256) {
         int lo = 0, hi = nc - 1;
         while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
@@ -206,9 +279,11 @@ __global__ void __launch_bounds__(256) k_tile_fill_block(const int* __restrict__
         }
         const int c = ((cz0 + lo / (ex * ey)) * g.ny + (cy0 + (lo / ex) % ey)) * g.nx + (cx0 + lo % ex);
         const int k = start[c] + (e - coff[lo]);
-        work[w0 + e] = parts[k];
+        const int i = parts[k];
+        work[w0 + e] = i;
         work_k[w0 + e] = k;  // the atom's mirror index
         work_c[w0 + e] = c;
+        if (gh_pack) gh_w[w0 + e] = gh_pack[i];
     }
 }
 
@@ -267,28 +342,122 @@ void retune_tile_edge(Sim& s) {
     s.tile_auto = std::min(t, s.tile_auto > 0 ? s.tile_auto : t);
 }
 
-// Counting sort of atoms 0..nall-1 by cell: cell_count, cell_start (CSR),
-// cell_parts (index order inside each cell), cell_of, cell_inv.
-static void bin_counting_sort(Sim& s, int nall) {
+BinArgs bin_args(const Sim& s) {
     const Geom& G = s.g;
-    BinArgs a{G.aabb[0], G.aabb[2], G.aabb[4], G.spacing, G.nx, G.ny, G.ncells, nall};
-    const int nt = 256;
-    TMD_HIP(hipMemsetAsync(s.cell_count.p, 0, sizeof(int) * (size_t)G.ncells, s.stream));
-    if (nall > 0)
-        hipLaunchKernelGGL(k_bin_count, dim3(div_up(nall, nt)), dim3(nt), 0, s.stream, (const double4*)s.pos.as<double4>(), a,
-                           s.cell_of.as<int>(), s.cell_slot.as<int>(), s.cell_count.as<int>(), s.cell_inv.as<int>());
+    return BinArgs{G.aabb[0], G.aabb[2], G.aabb[4], G.spacing, G.nx, G.ny, G.ncells};
+}
+
+// Buffers of the counting sort and the tiles for the current grid, and the
+// tile decomposition itself.
+void bin_reserve(Sim& s) {
+    choose_tiles(s);
+    const size_t nc = (size_t)s.g.ncells, nt = (size_t)s.tiles.ntx * s.tiles.nty * s.tiles.ntz, cap = (size_t)std::max(s.cap_all, 1);
+    s.cell_count.reserve(sizeof(int) * nc, false, s.stream);
+    s.cell_start.reserve(sizeof(int) * (nc + 1), false, s.stream);
+    s.tile_start.reserve(sizeof(int) * (nt + 1), false, s.stream);
+    s.work_start.reserve(sizeof(int) * (nt + 1), false, s.stream);  // per-tile counts
+    s.work.reserve(sizeof(int) * ((size_t)s.n + 1), false, s.stream);
+    s.work_k.reserve(sizeof(int) * ((size_t)s.n + 1), false, s.stream);
+    s.work_c.reserve(sizeof(int) * ((size_t)s.n + 1), false, s.stream);
+    s.gh_w.reserve(sizeof(int) * ((size_t)s.n + 1), false, s.stream);
+    s.cell_pair.reserve(sizeof(int2) * cap, false, s.stream);
+    s.cell_src.reserve(sizeof(int) * cap, false, s.stream);
+    s.cell_parts2.reserve(sizeof(int) * cap, false, s.stream);
+    s.cell_inv2.reserve(sizeof(int) * cap, false, s.stream);
+    s.spos.reserve((size_t)kMirBytes * cap, true, s.stream);
+    s.spos2.reserve((size_t)kMirBytes * cap, false, s.stream);
+    s.cell_of.reserve(sizeof(int) * cap, false, s.stream);
+    s.cell_slot.reserve(sizeof(int) * cap, false, s.stream);
+    if (s.vel_mirrored || s.vel_mirror_wanted || s.dem_loop) {
+        s.svel.reserve((size_t)kMirBytes * cap, true, s.stream);
+        s.svel2.reserve((size_t)kMirBytes * cap, false, s.stream);
+    }
+    s.g_ko.reserve(sizeof(int) * cap, false, s.stream);
+    s.g_kg.reserve(sizeof(int) * cap, false, s.stream);
+}
+
+// Scan, placement and sort behind the histogram of nq source slots (and, when
+// with_ghosts, of the ghosts emitted after it): the new CSR (cell_parts,
+// cell_inv, cell_src) replaces the last one.
+static void bin_sort(Sim& s, int nq, bool mir, bool with_ghosts, bool tiles) {
+    const Geom& G = s.g;
+    const int nt = 256, gcap = s.cap_all - s.n;
     exclusive_scan_int(s.cell_count.as<int>(), s.cell_start.as<int>(), G.ncells, s.cell_start.as<int>() + G.ncells, s);
-    if (nall > 0)
-        hipLaunchKernelGGL(k_bin_scatter, dim3(div_up(nall, nt)), dim3(nt), 0, s.stream, (const int*)s.cell_of.as<int>(),
-                           (const int*)s.cell_slot.as<int>(), (const int*)s.cell_start.as<int>(), nall, s.cell_parts.as<int>());
-    if (nall < 4 * G.ncells)  // sparse grid: a thread per cell beats a wavefront per cell
+    const int nbq = div_up(nq, nt);
+    const int nbg = with_ghosts ? std::max(1, std::min(div_up(gcap, nt), 2048)) : 0;
+#define TMD_PLACE(M)                                                                                                    \
+    hipLaunchKernelGGL(k_bin_place<M>, dim3(nbq + nbg), dim3(nt), 0, s.stream, (const int*)s.cell_of.as<int>(),           \
+                       (const int*)s.cell_slot.as<int>(), nq, nbq, (const int*)s.cell_parts.as<int>(),                   \
+                       (const int*)s.g_cell.as<int>(), (const int*)s.g_slot.as<int>(), s.n, gcap,                         \
+                       (const int*)s.counters.as<int>(), (const int*)s.cell_start.as<int>(), s.cell_pair.as<int2>())
+    if (nbq + nbg > 0) { if (mir) TMD_PLACE(true); else TMD_PLACE(false); }
+#undef TMD_PLACE
+    int* tc = tiles && G.ncells <= kTileAtomicCells ? s.work_start.as<int>() : nullptr;
+    if (nq < 4 * G.ncells)  // sparse grid: a thread per cell beats a wavefront per cell
         hipLaunchKernelGGL(k_bin_sort_small, dim3(div_up(G.ncells, nt)), dim3(nt), 0, s.stream,
-                           (const int*)s.cell_start.as<int>(), G.ncells, s.n, s.cell_parts.as<int>(), s.cell_count.as<int>(),
-                           s.cell_inv.as<int>());
+                           (const int*)s.cell_start.as<int>(), G.ncells, s.n, (const int2*)s.cell_pair.as<int2>(),
+                           s.cell_parts2.as<int>(), s.cell_src.as<int>(), s.cell_count.as<int>(), s.cell_inv2.as<int>(), s.tiles, tc);
     else
         hipLaunchKernelGGL(k_bin_sort, dim3(div_up(G.ncells, nt / kWave)), dim3(nt), 0, s.stream,
-                           (const int*)s.cell_start.as<int>(), G.ncells, s.n, s.cell_parts.as<int>(), s.cell_count.as<int>(),
-                           s.cell_inv.as<int>());
+                           (const int*)s.cell_start.as<int>(), G.ncells, s.n, (const int2*)s.cell_pair.as<int2>(),
+                           s.cell_parts2.as<int>(), s.cell_src.as<int>(), s.cell_count.as<int>(), s.cell_inv2.as<int>(), s.tiles, tc);
+    TMD_HIP(hipGetLastError());
+    std::swap(s.cell_parts, s.cell_parts2);
+    std::swap(s.cell_inv, s.cell_inv2);
+}
+
+// The tail of a rebuild after its histogram: cells, tiles, work order,
+// mirrors, ghost indices.  Nothing waits for the host.
+void bin_finish(Sim& s, int nq, bool with_ghosts) {
+    if (has_error()) return;
+    const bool mir = s.pos_stale != 0;
+    const TileGeom tg = s.tiles;
+    const int ntiles = tg.ntx * tg.nty * tg.ntz, gcap = s.cap_all - s.n, nt = 256;
+    bin_sort(s, nq, mir, with_ghosts, true);
+    FinishArgs a;
+    a.g = tg;
+    a.ntiles = ntiles;
+    a.scanned = ntiles > kTileFlat ? 1 : 0;
+    a.n = s.n;
+    a.gcap = gcap;
+    a.ncells = s.g.ncells;
+    a.nbm = div_up(s.cap_all, nt);
+    a.ghost_vel = s.dem_loop;
+    if (s.g.ncells > kTileAtomicCells)
+        hipLaunchKernelGGL(k_tile_count, dim3(div_up(ntiles, 4)), dim3(256), 0, s.stream, (const int*)s.cell_count.as<int>(), tg,
+                           ntiles, s.work_start.as<int>());
+    if (a.scanned)
+        exclusive_scan_int(s.work_start.as<int>(), s.tile_start.as<int>(), ntiles, s.tile_start.as<int>() + ntiles, s);
+    // the velocities follow the new order when they live in the mirror, or
+    // are wanted there (the fused step loops)
+    const bool with_vel = mir || s.vel_mirror_wanted || s.dem_loop;
+    const int nbg = std::max(1, std::min(div_up(gcap, nt), 2048));
+    const int* pack = s.gh_packed ? s.gh_pack.as<int>() : nullptr;
+#define TMD_FINISH(M)                                                                                                   \
+    hipLaunchKernelGGL(k_rebuild_finish<M>, dim3(ntiles + a.nbm + nbg), dim3(nt), 0, s.stream, a,                         \
+                       (const int*)s.cell_start.as<int>(), (const int*)s.cell_count.as<int>(),                           \
+                       (const int*)s.work_start.as<int>(), s.tile_start.as<int>(), (const int*)s.cell_parts.as<int>(),   \
+                       (const int*)s.cell_src.as<int>(), (const int*)s.cell_inv.as<int>(), s.work.as<int>(),             \
+                       s.work_k.as<int>(), s.work_c.as<int>(), pack, s.gh_w.as<int>(), (const double4*)s.pos.as<double4>(), \
+                       (const double4*)s.vel.as<double4>(), CMir{s.spos.as<double>()}, CMir{s.svel.as<double>()},         \
+                       Mir{s.spos2.as<double>()}, Mir{with_vel ? s.svel2.as<double>() : nullptr},                        \
+                       (const int*)s.g_owner.as<int>(), (const int*)s.g_code.as<int>(), (const int*)s.gh_e.as<int>(),    \
+                       s.g_ko.as<int>(), s.g_kg.as<int>(), s.gh_k.as<int>(), s.gh_c.as<int>(), s.counters.as<int>())
+    if (mir) TMD_FINISH(true); else TMD_FINISH(false);
+#undef TMD_FINISH
+    TMD_HIP(hipGetLastError());
+    std::swap(s.spos, s.spos2);
+    s.mirror_fresh = 1;
+    s.ghost_stale = 0;
+    if (with_vel) {
+        std::swap(s.svel, s.svel2);
+        // velocities copied from atom order now live in the mirror
+        if (!mir && s.vel_mirror_wanted) s.vel_mirrored = 1;
+    }
+    s.inv_valid = 1;
+    s.gsrc_valid = 1;
+    s.gh_valid = s.gh_packed;
+    s.windows_valid = 0;
 }
 
 // k-th local of the cell order <- local parts[k]: positions, velocities,
@@ -322,13 +491,16 @@ void sort_locals(Sim& s) {
     sync_pos_from_mirror(s);
     enforce_pbc(s);
     const Geom& G = s.g;
-    s.cell_count.reserve(sizeof(int) * (size_t)G.ncells, false, s.stream);
-    s.cell_start.reserve(sizeof(int) * ((size_t)G.ncells + 1), false, s.stream);
     const size_t n = (size_t)s.n;
     s.sort_buf.reserve((sizeof(double4) * 3 + sizeof(double)) * n, false, s.stream);
     if (has_error()) return;
     s.ng = 0;
-    bin_counting_sort(s, s.n);
+    bin_reserve(s);
+    if (has_error()) return;
+    TMD_HIP(hipMemsetAsync(s.cell_count.p, 0, sizeof(int) * (size_t)G.ncells, s.stream));
+    hipLaunchKernelGGL(k_bin_count, dim3(div_up(s.n, 256)), dim3(256), 0, s.stream, (const double4*)s.pos.as<double4>(),
+                       bin_args(s), s.n, s.cell_of.as<int>(), s.cell_slot.as<int>(), s.cell_count.as<int>(), s.cell_inv2.as<int>());
+    bin_sort(s, s.n, false, false, false);
     int binned = 0;
     TMD_HIP(hipMemcpyAsync(&binned, s.cell_start.as<int>() + G.ncells, sizeof(int), hipMemcpyDeviceToHost, s.stream));
     TMD_HIP(hipStreamSynchronize(s.stream));
@@ -353,48 +525,30 @@ void sort_locals(Sim& s) {
     mirror_invalidate(s);
     s.inv_valid = 0;
     s.gsrc_valid = 0;
+    s.gh_valid = s.gh_packed = 0;
     s.windows_valid = 0;
     s.nb_valid = 0;
 }
 
+// md_distribute_particles: cells, tiles and mirrors of the current atoms
+// (locals and ghosts, in atom order), statistics known on return.
 void bin_particles(Sim& s) {
     if (has_error()) return;
+    sync_pos_from_mirror(s);
     const int nall = s.n + s.ng;
-    const Geom& G = s.g;
-    s.cell_count.reserve(sizeof(int) * (size_t)G.ncells, false, s.stream);
-    s.cell_start.reserve(sizeof(int) * ((size_t)G.ncells + 1), false, s.stream);
-    s.work.reserve(sizeof(int) * ((size_t)s.n + 1), false, s.stream);
-    s.work_k.reserve(sizeof(int) * ((size_t)s.n + 1), false, s.stream);
-    s.work_c.reserve(sizeof(int) * ((size_t)s.n + 1), false, s.stream);
-    if (has_error()) return;
     mirror_invalidate(s);
     s.inv_valid = 0;
-    const int nt = 256;
-    bin_counting_sort(s, nall);
-    s.inv_valid = 1;
-    build_ghost_src(s);
-    // tile work order
-    choose_tiles(s);
-    const TileGeom tg = s.tiles;
-    const int ntiles = tg.ntx * tg.nty * tg.ntz;
-    s.tile_start.reserve(sizeof(int) * ((size_t)ntiles + 1), false, s.stream);
-    s.work_start.reserve(sizeof(int) * ((size_t)ntiles + 1), false, s.stream);  // per-tile counts
+    bin_reserve(s);
     if (has_error()) return;
-    int* counters = s.counters.as<int>();
-    TMD_HIP(hipMemsetAsync(counters + 6, 0, 2 * sizeof(int), s.stream));
-    if (tg.tx * tg.ty * tg.tz <= 64)
-        hipLaunchKernelGGL(k_tile_stats_small, dim3(div_up(ntiles, nt)), dim3(nt), 0, s.stream, (const int*)s.cell_start.as<int>(),
-                           (const int*)s.cell_count.as<int>(), tg, ntiles, s.work_start.as<int>(), counters + 6, counters + 7);
-    else
-        hipLaunchKernelGGL(k_tile_stats, dim3(ntiles), dim3(kWave), 0, s.stream, (const int*)s.cell_start.as<int>(),
-                           (const int*)s.cell_count.as<int>(), tg, ntiles, s.work_start.as<int>(), counters + 6, counters + 7);
-    exclusive_scan_int(s.work_start.as<int>(), s.tile_start.as<int>(), ntiles, s.tile_start.as<int>() + ntiles, s);
-    hipLaunchKernelGGL(k_tile_fill_block, dim3(ntiles), dim3(256), 0, s.stream, (const int*)s.cell_start.as<int>(),
-                       (const int*)s.cell_count.as<int>(), (const int*)s.tile_start.as<int>(), tg,
-                       (const int*)s.cell_parts.as<int>(), s.work.as<int>(), s.work_k.as<int>(), s.work_c.as<int>());
-    TMD_HIP(hipGetLastError());
-    s.windows_valid = 0;
-    build_windows(s);
+    const TileGeom tg = s.tiles;
+    const int ntiles = tg.ntx * tg.nty * tg.ntz, nt = 256;
+    rebuild_zero(s, s.g.ncells, ntiles, s.ng);
+    if (nall > 0)
+        hipLaunchKernelGGL(k_bin_count, dim3(div_up(nall, nt)), dim3(nt), 0, s.stream, (const double4*)s.pos.as<double4>(),
+                           bin_args(s), nall, s.cell_of.as<int>(), s.cell_slot.as<int>(), s.cell_count.as<int>(),
+                           s.cell_inv2.as<int>());
+    bin_finish(s, nall, false);
+    apply_window_stats(s, read_stats(s));
 }
 
 }  // namespace tmd

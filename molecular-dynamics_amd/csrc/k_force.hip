@@ -354,7 +354,7 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_dem_fused(const CMir spos, 
                                                            DEMArgs a, double hdt, double dt, const Mir spos_next,
                                                            const Mir svel_next, double4* __restrict__ force,
                                                            double4* __restrict__ vel, double4* __restrict__ pos,
-                                                           const int* __restrict__ gh_start, const int* __restrict__ gh_k,
+                                                           const int* __restrict__ gh_w, const int* __restrict__ gh_k,
                                                            const int* __restrict__ gh_c, double L0, double L1, double L2) {
     extern __shared__ double dyn[];
     const int tile = xcd_block(blockIdx.x, gridDim.x);
@@ -440,9 +440,11 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_dem_fused(const CMir spos, 
                 svel_next[kw] = v;
                 // the sphere's ghosts: its new position + image shift and its
                 // new velocity (k_ghost_step_mirror_v's arithmetic)
-                if (gh_start) {
-                    const int e1 = gh_start[w + 1];
-                    for (int e = gh_start[w]; e < e1; ++e) {
+                if (gh_w) {
+                    const int pk = gh_w[w];
+                    for (int e = pk >> 5, e1 = e + (pk & 31); e < e1; ++e) {
+                        const int kg = gh_k[e];
+                        if (kg < 0) continue;
                         int ix, iy, iz;
                         img_decode(gh_c[e], ix, iy, iz);
                         double4 q;
@@ -450,7 +452,6 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_dem_fused(const CMir spos, 
                         q.y = x.y + L1 * (double)iy;
                         q.z = x.z + L2 * (double)iz;
                         q.w = x.w;
-                        const int kg = gh_k[e];
                         spos_next[kg] = q;
                         svel_next[kg] = v;
                     }
@@ -480,9 +481,8 @@ void compute_dem_fused(Sim& s, int half, double rc, double gn, double gt, double
     const double hdt = 0.5 * dt;
     // advancing: the pass also writes the ghosts' next mirror entries
     // (from each local's ghost index), so the next step needs no ghost pass
-    if (advance && s.ng > 0 && s.ghost_mode == GHOST_FRESH && !(s.gsrc_valid && s.gh_valid)) build_ghost_index(s);
-    const bool fuse = advance && s.ng > 0 && s.ghost_mode == GHOST_FRESH && s.gsrc_valid && s.gh_valid && !has_error();
-    const int* GS = fuse ? s.gh_start.as<int>() : nullptr;
+    const bool fuse = advance && s.ng > 0 && s.ghost_mode == GHOST_FRESH && s.gsrc_valid && s.gh_valid;
+    const int* GS = fuse ? s.gh_w.as<int>() : nullptr;
     hipEvent_t ev = nullptr;
     s.timer.begin(K_FORCE, s.stream, &ev);
 #define TMD_DEMF(P, H, A)                                                                                               \

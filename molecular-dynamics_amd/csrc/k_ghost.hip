@@ -13,176 +13,357 @@
 
 namespace tmd {
 
-struct BorderArgs {
-    int d;          // dimension 0..2
-    int scan_end;   // scan locals + ghosts of previous dimensions
-    int n;          // number of locals
-    int base;       // first new ghost slot (n + ng)
-    double hi_thr;  // aabb_max - 2 s   (select for image -1)
-    double lo_thr;  // aabb_min + 2 s   (select for image +1)
-    double whi_thr; // world_max - s    (flag -1)
-    double wlo_thr; // world_min + s    (flag +1)
-    double len0, len1, len2;
-};
+// Cell of a position (core/grid.impala:406-426): flat index from the floored
+// coordinates; non-finite or absurd coordinates are outside the grid (-1).
+__device__ __forceinline__ int cell_index(const double4& p, const BinArgs& a) {
+    const double fx = floor((p.x - a.xmin) / a.spacing);
+    const double fy = floor((p.y - a.ymin) / a.spacing);
+    const double fz = floor((p.z - a.zmin) / a.spacing);
+    if (fabs(fx) < 1e9 && fabs(fy) < 1e9 && fabs(fz) < 1e9) {
+        const int ci = (int)fx, cj = (int)fy, ck = (int)fz;
+        const long long flat = ((long long)ck * a.ny + cj) * a.nx + ci;
+        if (flat >= 0 && flat < a.ncells) return (int)flat;
+    }
+    return -1;
+}
 
+// ---------------------------------------------------------------------------
+// Ghost layer in one sweep.
+//
+// The reference selects ghosts dimension by dimension, each time over the
+// locals and the ghosts made so far.  A ghost differs from its local only in
+// the coordinates of the dimensions it was made in, so which ghosts a local
+// gets follows from six bits of the local alone: bit 2d, coordinate d above
+// the upper select threshold; bit 2d + 1, below the lower one.  Each of the
+// 26 sequences (none, upper or lower in x, y and z, not all none) is a class;
+// the reference's order is: classes in the order in which the passes reach
+// them (class_id), and inside a class the locals' index order.  So a ghost's
+// number is the class-major exclusive prefix count, and one scan over the
+// (class, block of locals) counts places every ghost of all three passes:
+// three launches (count, scan, emit) in place of twelve and no host round
+// trip for the totals between them.
+//
+// a, b, c: 0 none, 1 upper, 2 lower in x, y, z.  The x pass scans the locals
+// (classes 0, 1); the y pass scans locals and x ghosts (upper: 2..4, lower:
+// 5..7); the z pass scans locals and the eight classes before it (upper:
+// 8..16, lower: 17..25).
+constexpr int kClasses = 26;
+__device__ __forceinline__ int class_id(int a, int b, int c) {
+    const int xy = b == 0 ? a - 1 : 2 + (b - 1) * 3 + a;  // -1: none in x and y
+    return c == 0 ? xy : 8 + (c - 1) * 9 + xy + 1;
+}
+constexpr int kGhostItems = 1;                              // locals per thread
+constexpr int kGhostBlock = kScanThreads * kGhostItems;     // locals per block
+constexpr int kGhostSubs = kGhostBlock / kWave;             // wavefront-sized groups of locals per block
+// (class, block) counts that the emitting blocks scan by themselves; more are
+// scanned by launches of their own
+constexpr int kClassFlat = 4096;
 
-__device__ __forceinline__ double comp(const double4& p, int d) { return d == 0 ? p.x : (d == 1 ? p.y : p.z); }
-
-// Border selection bits of an atom, bit 2d: coordinate d above the upper
-// select threshold (the ghost of image -1 side), bit 2d + 1: below the lower
-// one.  A ghost made in pass d differs from its source only in coordinate d,
-// so it inherits the source's bits of the later passes.  The bits are
-// computed once, over the locals, together with the ghost totals of the
-// three passes: a local whose family (itself and its ghosts of earlier
-// passes) has m members contributes m to each later pass it is selected in.
 struct FaceArgs {
-    int n, wrap;
+    int nq, n, wrap;   // source slots; locals (atoms below n)
     double hi_thr[3], lo_thr[3];
     PbcArgs pbc;
+    BinArgs bin;
 };
 
-// mpos / mvel (the fused step loop's state, in mirror order): the local's
-// position and velocity are first copied back from there (k_unmirror's copy,
-// through the mirror index inv).
-__global__ void __launch_bounds__(kScanThreads) k_face_flags(double4* __restrict__ pos, FaceArgs a, unsigned char* __restrict__ face,
-                                                             int* __restrict__ totals, const int* __restrict__ inv,
-                                                             const CMir mpos, const CMir mvel,
-                                                             double4* __restrict__ vel) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    int t[6] = {0, 0, 0, 0, 0, 0};
+// Border bits of every local (and, with BIN, its cell and counting-sort
+// slot), after md_enforce_pbc's wrap when asked.  MIR: the locals' positions
+// live in the cell-ordered mirror (the fused step loops), which is then read
+// and wrapped in place in its own order: coalesced, and neighbouring lanes
+// share cells, where a sweep in atom order gathered 24 B records at random
+// and copied positions and velocities back to atom order (80^3: 109 us, plus
+// 38 us for the binning sweep; this one 33 us).
+template <bool MIR, bool BIN>
+__global__ void __launch_bounds__(kScanThreads) k_face_bin(double4* __restrict__ pos, const Mir spos,
+                                                           const int* __restrict__ parts, FaceArgs a,
+                                                           unsigned char* __restrict__ face, int* __restrict__ cell_of,
+                                                           int* __restrict__ slot, int* __restrict__ count,
+                                                           int* __restrict__ inv) {
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = q < a.nq ? (MIR ? parts[q] : q) : a.n;
+    int c = -1;
     if (i < a.n) {
-        double4 p;
-        if (mpos.p || mvel.p) {
-            const int k = inv[i];
-            if (mpos.p) p = mpos[k];
-            if (mvel.p) vel[i] = mvel[k];
+        double4 p = MIR ? (double4)spos[q] : pos[q];
+        if (a.wrap) {
+            const double4 o = p;
+            pbc_wrap(p, a.pbc);
+            if (p.x != o.x || p.y != o.y || p.z != o.z) {
+                if (MIR) spos[q] = p;
+                else pos[q] = p;
+            }
         }
-        if (!mpos.p) p = pos[i];
-        if (a.wrap) pbc_wrap(p, a.pbc);  // md_enforce_pbc, fused
-        if (a.wrap || mpos.p) pos[i] = p;
-        const double c[3] = {p.x, p.y, p.z};
+        const double x[3] = {p.x, p.y, p.z};
         int bits = 0;
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            bits |= (c[d] > a.hi_thr[d] ? 1 : 0) << (2 * d);
-            bits |= (c[d] < a.lo_thr[d] ? 1 : 0) << (2 * d + 1);
+            bits |= (x[d] > a.hi_thr[d] ? 1 : 0) << (2 * d);
+            bits |= (x[d] < a.lo_thr[d] ? 1 : 0) << (2 * d + 1);
         }
         face[i] = (unsigned char)bits;
-        const int fx = 1 + (bits & 1) + ((bits >> 1) & 1);       // the local and its x ghosts
-        const int fy = fx * (1 + ((bits >> 2) & 1) + ((bits >> 3) & 1));  // ... and their y ghosts
-        t[0] = bits & 1;
-        t[1] = (bits >> 1) & 1;
-        t[2] = ((bits >> 2) & 1) * fx;
-        t[3] = ((bits >> 3) & 1) * fx;
-        t[4] = ((bits >> 4) & 1) * fy;
-        t[5] = ((bits >> 5) & 1) * fy;
+        if (BIN) {
+            c = cell_index(p, a.bin);
+            if (c < 0) inv[i] = -1;
+        }
     }
-    // block totals of the six counts: wavefront sums by shuffles, then one
-    // LDS pass (integer sums: the order does not matter)
-    __shared__ int wt[kScanThreads / kWave][6];
+    if (BIN) {
+        const int sl = wave_cell_slot(c, count);  // all lanes take part
+        if (q < a.nq) {
+            cell_of[q] = c;
+            slot[q] = sl;
+        }
+    }
+}
+
+// Members of class (a, b, c) among the wavefront's locals, from the ballots
+// of the six border bits.
+struct FaceBallots {
+    unsigned long long b[6];
+    __device__ __forceinline__ unsigned long long side(int d, int s) const {
+        return s == 0 ? ~0ull : (s == 1 ? b[2 * d] : b[2 * d + 1]);
+    }
+    __device__ __forceinline__ unsigned long long any() const { return b[0] | b[1] | b[2] | b[3] | b[4] | b[5]; }
+};
+
+__device__ __forceinline__ FaceBallots face_ballots(int bits) {
+    FaceBallots f;
+#pragma unroll
+    for (int d = 0; d < 6; ++d) f.b[d] = __ballot((bits >> d) & 1);
+    return f;
+}
+
+// digits of class number `id` (the inverse of class_id), for a lane per class
+__device__ __forceinline__ void class_digits(int id, int& a, int& b, int& c) {
+    c = id < 8 ? 0 : (id < 17 ? 1 : 2);
+    const int e = id < 8 ? id + 1 : (id - 8) % 9;  // 0: none in x and y, else 1 + the xy class
+    a = e == 0 ? 0 : (e < 3 ? e : (e - 3) % 3);
+    b = e < 3 ? 0 : 1 + (e - 3) / 3;
+}
+
+// counts[class * nb + block]: members of each class in each block of locals
+__global__ void __launch_bounds__(kScanThreads) k_class_count(const unsigned char* __restrict__ face, int n, int nb,
+                                                              int* __restrict__ counts) {
+    __shared__ int wc[kScanThreads / kWave][kClasses];
     const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+    int ca = 0, cb = 0, cc = 0;
+    class_digits(min(lane, kClasses - 1), ca, cb, cc);
+    int sum = 0;
 #pragma unroll
-    for (int k = 0; k < 6; ++k) {
-        int v = t[k];
+    for (int it = 0; it < kGhostItems; ++it) {
+        const int i = blockIdx.x * kGhostBlock + it * kScanThreads + (int)threadIdx.x;
+        const FaceBallots f = face_ballots(i < n ? face[i] : 0);
+        if (f.any()) sum += __popcll(f.side(0, ca) & f.side(1, cb) & f.side(2, cc));
+    }
+    if (lane < kClasses) wc[wid][lane] = sum;
+    __syncthreads();
+    if (threadIdx.x < kClasses) {
+        int t = 0;
 #pragma unroll
-        for (int d = kWave / 2; d > 0; d >>= 1) v += __shfl_down(v, d, kWave);
-        if (lane == 0) wt[wid][k] = v;
+        for (int w = 0; w < kScanThreads / kWave; ++w) t += wc[w][threadIdx.x];
+        counts[threadIdx.x * nb + blockIdx.x] = t;
+    }
+}
+
+struct EmitArgs {
+    int n, nb, gcap, scanned;    // locals, blocks, ghost slots, counts already scanned
+    double whi[3], wlo[3];       // image flag thresholds: world max - s, world min + s
+    double len[3];
+};
+
+// Every ghost of every local, straight to its slot: position (local + image
+// * L), velocity, mass, owner, immediate source and image codes; stores only,
+// so a corner atom's 7 classes cost no round trips.  gh_pack / gh_e (may be null): each
+// local's entries in the ghost index (first entry * 32 + number of ghosts)
+// and each ghost's entry.  Ghosts beyond the capacity are counted, not
+// written; the host grows and repeats.
+template <bool MIR>
+__global__ void __launch_bounds__(kScanThreads) k_ghost_emit(double4* __restrict__ pos, double4* __restrict__ vel,
+                                                             double* __restrict__ mass, const CMir spos, const CMir svel,
+                                                             const int* __restrict__ inv_src,
+                                                             const unsigned char* __restrict__ face,
+                                                             const int* __restrict__ counts, EmitArgs a,
+                                                             int* __restrict__ g_owner, int* __restrict__ g_src,
+                                                             int* __restrict__ g_code, int* __restrict__ gh_pack,
+                                                             int* __restrict__ gh_e, int* __restrict__ ctr) {
+    __shared__ int flat[kClassFlat];
+    __shared__ int sub[kGhostSubs][kClasses];
+    __shared__ int entry0;
+    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+    const int blk = blockIdx.x;
+    int bits[kGhostItems];
+    FaceBallots f[kGhostItems];
+    int ca = 0, cb = 0, cc = 0;
+    class_digits(min(lane, kClasses - 1), ca, cb, cc);
+#pragma unroll
+    for (int it = 0; it < kGhostItems; ++it) {
+        const int i = blk * kGhostBlock + it * kScanThreads + (int)threadIdx.x;
+        bits[it] = i < a.n ? face[i] : 0;
+        f[it] = face_ballots(bits[it]);
+        if (lane < kClasses)
+            sub[it * (kScanThreads / kWave) + wid][lane] = __popcll(f[it].side(0, ca) & f[it].side(1, cb) & f[it].side(2, cc));
+    }
+    // thread c: ghost number of the block's first member of class c, and of the
+    // whole class's first one
+    int first = 0, cls0 = 0;
+    if (a.scanned) {
+        if (threadIdx.x < kClasses) {
+            first = counts[threadIdx.x * a.nb + blk];
+            cls0 = counts[threadIdx.x * a.nb];
+        }
+    } else {
+        // few blocks: each scans the class-major counts itself
+        constexpr int kPer = kClassFlat / kScanThreads;
+        const int total = kClasses * a.nb, base = (int)threadIdx.x * kPer;
+        int v[kPer], sum = 0;
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+            v[k] = base + k < total ? counts[base + k] : 0;
+            sum += v[k];
+        }
+        int tot;
+        int run = block_exclusive_scan(sum, &tot);
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+            flat[base + k] = run;
+            run += v[k];
+        }
+        if (blk == 0 && threadIdx.x == 0) ctr[CT_NGHOST] = tot;
+        __syncthreads();
+        if (threadIdx.x < kClasses) {
+            first = flat[threadIdx.x * a.nb + blk];
+            cls0 = flat[threadIdx.x * a.nb];
+        }
+    }
+    if (threadIdx.x < kWave) {
+        // the block's first entry of the ghost index: all ghosts of the blocks
+        // before it, of every class
+        const int before = wave_inclusive_scan(first - cls0);
+        if (threadIdx.x == kWave - 1) entry0 = before;
     }
     __syncthreads();
-    if (threadIdx.x < 6) {
-        int v = 0;
-#pragma unroll
-        for (int w = 0; w < kScanThreads / kWave; ++w) v += wt[w][threadIdx.x];
-        if (v) atomicAdd(&totals[threadIdx.x], v);
-    }
-}
-
-__global__ void __launch_bounds__(kScanThreads) k_border_count(const unsigned char* __restrict__ face, BorderArgs a,
-                                                               int* __restrict__ tiles0, int* __restrict__ tiles1) {
-    const int base = blockIdx.x * kScanTile + threadIdx.x * kScanItems;
-    int c0 = 0, c1 = 0;
-#pragma unroll
-    for (int it = 0; it < kScanItems; ++it) {
-        const int i = base + it;
-        if (i < a.scan_end) {
-            const int b = face[i] >> (2 * a.d);
-            c0 += b & 1;
-            c1 += (b >> 1) & 1;
+    if (threadIdx.x < kClasses) {
+        int run = first;
+        for (int q = 0; q < kGhostSubs; ++q) {
+            const int t = sub[q][threadIdx.x];
+            sub[q][threadIdx.x] = run;
+            run += t;
         }
     }
-    int t0 = block_sum_int(c0);
-    int t1 = block_sum_int(c1);
-    if (threadIdx.x == 0) {
-        tiles0[blockIdx.x] = t0;
-        tiles1[blockIdx.x] = t1;
-    }
-}
-
-__device__ __forceinline__ void write_ghost(int i, int slot, int side, const BorderArgs& a, double4* __restrict__ pos,
-                                            double4* __restrict__ vel, double* __restrict__ mass,
-                                            int* __restrict__ g_owner, int* __restrict__ g_src, int* __restrict__ g_code,
-                                            unsigned char* __restrict__ face) {
-    const double4 p = pos[i];
-    const double pd = comp(p, a.d);
-    int fl = (side == 0) ? (pd > a.whi_thr ? -1 : 0) : (pd < a.wlo_thr ? 1 : 0);
-    int f[3] = {0, 0, 0};
-    f[a.d] = fl;
-    double4 q;
-    q.x = p.x + a.len0 * (double)f[0];
-    q.y = p.y + a.len1 * (double)f[1];
-    q.z = p.z + a.len2 * (double)f[2];
-    q.w = p.w;
-    int owner, ix, iy, iz;
-    if (i < a.n) {
-        owner = i;
-        ix = f[0]; iy = f[1]; iz = f[2];
-    } else {
-        const int gi = i - a.n;
-        owner = g_owner[gi];
-        img_decode(g_code[gi] & 0xff, ix, iy, iz);
-        ix += f[0]; iy += f[1]; iz += f[2];
-    }
-    pos[slot] = q;
-    mass[slot] = mass[i];
-    vel[slot] = vel[owner];
-    const int g = slot - a.n;
-    g_owner[g] = owner;
-    g_src[g] = i;
-    g_code[g] = img_encode(ix, iy, iz) | (img_encode(f[0], f[1], f[2]) << 8);
-    face[slot] = face[i];
-}
-
-__global__ void __launch_bounds__(kScanThreads) k_border_scatter(double4* __restrict__ pos, double4* __restrict__ vel,
-                                                                 double* __restrict__ mass, int* __restrict__ g_owner,
-                                                                 int* __restrict__ g_src, int* __restrict__ g_code,
-                                                                 const int* __restrict__ off0, const int* __restrict__ off1,
-                                                                 const int* __restrict__ totals, BorderArgs a,
-                                                                 unsigned char* __restrict__ face) {
-    const int base = blockIdx.x * kScanTile + threadIdx.x * kScanItems;
-    int f0[kScanItems], f1[kScanItems];
-    int c0 = 0, c1 = 0;
+    __syncthreads();
+    const unsigned long long below = (1ull << lane) - 1ull;
+    int given = entry0;  // ghost index entries given out so far in the block
 #pragma unroll
-    for (int it = 0; it < kScanItems; ++it) {
-        int i = base + it;
-        f0[it] = f1[it] = 0;
-        if (i < a.scan_end) {
-            const int b = face[i] >> (2 * a.d);
-            f0[it] = b & 1;
-            f1[it] = (b >> 1) & 1;
+    for (int it = 0; it < kGhostItems; ++it) {
+        const int i = blk * kGhostBlock + it * kScanThreads + (int)threadIdx.x;
+        const FaceBallots& F = f[it];
+        const int* base = sub[it * (kScanThreads / kWave) + wid];
+        const int bt = bits[it];
+        int entry = 0;
+        if (gh_pack) {
+            const int m = (1 + (bt & 1) + ((bt >> 1) & 1)) * (1 + ((bt >> 2) & 1) + ((bt >> 3) & 1)) *
+                              (1 + ((bt >> 4) & 1) + ((bt >> 5) & 1)) - 1;
+            int tot;
+            entry = given + block_exclusive_scan(m, &tot);
+            given += tot;
+            if (i < a.n) gh_pack[i] = m ? entry * 32 + m : 0;
         }
-        c0 += f0[it];
-        c1 += f1[it];
+        if (F.any() == 0) continue;  // no border atom in the wavefront
+        double4 p = make_double4(0, 0, 0, 0), v = p;
+        double ms = 0.0;
+        if (bt) {
+            if (MIR) {
+                const int k = inv_src[i];
+                p = spos[k];
+                v = svel[k];
+            } else {
+                p = pos[i];
+                v = vel[i];
+            }
+            ms = mass[i];
+        }
+        const int fl[3][2] = {{p.x > a.whi[0] ? -1 : 0, p.x < a.wlo[0] ? 1 : 0},
+                              {p.y > a.whi[1] ? -1 : 0, p.y < a.wlo[1] ? 1 : 0},
+                              {p.z > a.whi[2] ? -1 : 0, p.z < a.wlo[2] ? 1 : 0}};
+        // every class with members in this wavefront (uniform loops: the
+        // class masks are scalar)
+#pragma unroll 1
+        for (int c = 0; c < 3; ++c) {
+            const unsigned long long mc = F.side(2, c);
+#pragma unroll 1
+            for (int b = 0; b < 3; ++b) {
+                const unsigned long long mb = mc & F.side(1, b);
+#pragma unroll 1
+                for (int s = 0; s < 3; ++s) {
+                    const unsigned long long m = mb & F.side(0, s);
+                    if ((s | b | c) == 0 || m == 0) continue;
+                    const bool has = (m >> lane) & 1ull;
+                    const int id = class_id(s, b, c);
+                    const int g = base[id] + __popcll(m & below);
+                    const int ix = s == 0 ? 0 : (s == 1 ? fl[0][0] : fl[0][1]);
+                    const int iy = b == 0 ? 0 : (b == 1 ? fl[1][0] : fl[1][1]);
+                    const int iz = c == 0 ? 0 : (c == 1 ? fl[2][0] : fl[2][1]);
+                    double4 q;
+                    q.x = p.x + a.len[0] * (double)ix;
+                    q.y = p.y + a.len[1] * (double)iy;
+                    q.z = p.z + a.len[2] * (double)iz;
+                    q.w = p.w;
+                    if (has && g < a.gcap) {
+                        // the immediate source: the class without the last pass
+                        int src = i;
+                        if (c ? (s | b) : (b ? s : 0)) {
+                            const int pc = c ? class_id(s, b, 0) : class_id(s, 0, 0);
+                            const unsigned long long pm = F.side(0, s) & (c ? F.side(1, b) : ~0ull);
+                            src = a.n + base[pc] + __popcll(pm & below);
+                        }
+                        pos[a.n + g] = q;
+                        vel[a.n + g] = v;
+                        mass[a.n + g] = ms;
+                        g_owner[g] = i;
+                        g_src[g] = src;
+                        g_code[g] = img_encode(ix, iy, iz) |
+                                    (img_encode(c || b ? 0 : ix, c ? 0 : (b ? iy : 0), c ? iz : 0) << 8);
+                        if (gh_pack) gh_e[g] = entry;
+                    }
+                    if (has) ++entry;
+                }
+            }
+        }
     }
-    int t0, t1;
-    int r0 = off0[blockIdx.x] + block_exclusive_scan(c0, &t0);
-    int r1 = off1[blockIdx.x] + block_exclusive_scan(c1, &t1);
-    const int total0 = totals[0];
-#pragma unroll
-    for (int it = 0; it < kScanItems; ++it) {
-        int i = base + it;
-        if (f0[it]) { write_ghost(i, a.base + r0, 0, a, pos, vel, mass, g_owner, g_src, g_code, face); r0++; }
-        if (f1[it]) { write_ghost(i, a.base + total0 + r1, 1, a, pos, vel, mass, g_owner, g_src, g_code, face); r1++; }
+}
+
+// Cells and counting-sort slots of the ghosts just made (their number is on
+// the device; the launch covers the capacity in strides of whole wavefronts).
+__global__ void __launch_bounds__(256) k_ghost_bin(const double4* __restrict__ pos, int n, int gcap, BinArgs bin,
+                                                   int* __restrict__ g_cell, int* __restrict__ g_slot,
+                                                   int* __restrict__ cell_count, int* __restrict__ inv,
+                                                   const int* __restrict__ ctr) {
+    const int ng = min(ctr[CT_NGHOST], gcap);
+    for (int g0 = blockIdx.x * 256; g0 < ng; g0 += gridDim.x * 256) {
+        const int g = g0 + (int)threadIdx.x;
+        const int c = g < ng ? cell_index(pos[n + g], bin) : -1;
+        const int sl = wave_cell_slot(c, cell_count);  // all lanes take part
+        if (g < ng) {
+            g_cell[g] = c;
+            g_slot[g] = sl;
+            if (c < 0) inv[n + g] = -1;
+        }
     }
+}
+
+// the counters (ng: the ghost count to start from), cell and tile counts
+__global__ void k_rebuild_zero(int* __restrict__ cells, int ncells, int* __restrict__ tiles, int ntiles, int* __restrict__ ctr,
+                               int ng) {
+    const int stride = gridDim.x * blockDim.x, t = blockIdx.x * blockDim.x + threadIdx.x;
+    for (int c = t; c < ncells; c += stride) cells[c] = 0;
+    for (int c = t; c < ntiles; c += stride) tiles[c] = 0;
+    if (t < CT_COUNT) ctr[t] = t == CT_NGHOST ? ng : 0;
+}
+
+// one launch clears what a rebuild accumulates (three memsets before it)
+void rebuild_zero(Sim& s, int ncells, int ntiles, int ng) {
+    const int n = std::max(std::max(ncells, ntiles), 1);
+    hipLaunchKernelGGL(k_rebuild_zero, dim3(std::min(div_up(n, 1024), 512)), dim3(256), 0, s.stream, s.cell_count.as<int>(), ncells,
+                       s.work_start.as<int>(), ntiles, s.counters.as<int>(), ng);
+    TMD_HIP(hipGetLastError());
 }
 
 // FRESH refresh: ghost = owner + image * L (bit-identical to the rebuild's
@@ -266,64 +447,8 @@ __global__ void k_ghost_src(const int* __restrict__ g_owner, const int* __restri
     g_kg[g] = inv[n + g];
 }
 
-// Each local's ghosts by the local's work slot (a CSR over work slots), so
-// that a force pass that advances a local can also write its ghosts' mirror
-// entries.  Within one local the order of its ghosts is that of the atomics
-// (each ghost's entry is written independently of the others).
-__global__ void k_inv_work(const int* __restrict__ work, int n, int* __restrict__ inv_work) {
-    const int w = blockIdx.x * blockDim.x + threadIdx.x;
-    if (w < n) inv_work[work[w]] = w;
-}
-
-__global__ void k_gh_count(const int* __restrict__ g_owner, const int* __restrict__ g_kg, int ng,
-                           const int* __restrict__ inv_work, int* __restrict__ cnt) {
-    const int g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= ng || g_kg[g] < 0) return;
-    atomicAdd(&cnt[inv_work[g_owner[g]]], 1);
-}
-
-__global__ void k_gh_fill(const int* __restrict__ g_owner, const int* __restrict__ g_kg, const int* __restrict__ g_code,
-                          int ng, const int* __restrict__ inv_work, const int* __restrict__ start, int* __restrict__ fill,
-                          int* __restrict__ gh_k, int* __restrict__ gh_c) {
-    const int g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= ng || g_kg[g] < 0) return;
-    const int w = inv_work[g_owner[g]];
-    const int e = start[w] + atomicAdd(&fill[w], 1);
-    gh_k[e] = g_kg[g];
-    gh_c[e] = g_code[g] & 0xff;
-}
-
-void build_ghost_index(Sim& s) {
-    s.gh_valid = 0;
-    if (has_error() || s.n == 0) return;
-    if (!s.gsrc_valid) build_ghost_src(s);
-    const int n = s.n, ng = s.ng;
-    s.gh_start.reserve(sizeof(int) * ((size_t)n + 1), false, s.stream);
-    s.gh_aux.reserve(sizeof(int) * 2 * (size_t)n, false, s.stream);
-    s.gh_k.reserve(sizeof(int) * (size_t)std::max(ng, 1), false, s.stream);
-    s.gh_c.reserve(sizeof(int) * (size_t)std::max(ng, 1), false, s.stream);
-    if (has_error()) return;
-    int* inv_work = s.gh_aux.as<int>();
-    int* cnt = inv_work + n;
-    const int nt = 256;
-    hipLaunchKernelGGL(k_inv_work, dim3(div_up(n, nt)), dim3(nt), 0, s.stream, (const int*)s.work.as<int>(), n, inv_work);
-    TMD_HIP(hipMemsetAsync(cnt, 0, sizeof(int) * (size_t)n, s.stream));
-    if (ng > 0)
-        hipLaunchKernelGGL(k_gh_count, dim3(div_up(ng, nt)), dim3(nt), 0, s.stream, (const int*)s.g_owner.as<int>(),
-                           (const int*)s.g_kg.as<int>(), ng, (const int*)inv_work, cnt);
-    exclusive_scan_int(cnt, s.gh_start.as<int>(), n, s.gh_start.as<int>() + n, s);
-    TMD_HIP(hipMemsetAsync(cnt, 0, sizeof(int) * (size_t)n, s.stream));
-    if (ng > 0)
-        hipLaunchKernelGGL(k_gh_fill, dim3(div_up(ng, nt)), dim3(nt), 0, s.stream, (const int*)s.g_owner.as<int>(),
-                           (const int*)s.g_kg.as<int>(), (const int*)s.g_code.as<int>(), ng, (const int*)inv_work,
-                           (const int*)s.gh_start.as<int>(), cnt, s.gh_k.as<int>(), s.gh_c.as<int>());
-    TMD_HIP(hipGetLastError());
-    if (!has_error()) s.gh_valid = 1;
-}
-
 void build_ghost_src(Sim& s) {
     s.gsrc_valid = 0;
-    s.gh_valid = 0;
     if (has_error() || s.ng == 0) return;
     s.g_ko.reserve(sizeof(int) * (size_t)s.cap_all, false, s.stream);
     s.g_kg.reserve(sizeof(int) * (size_t)s.cap_all, false, s.stream);
@@ -420,84 +545,120 @@ __global__ void k_ghost_unpack_lag(double4* __restrict__ pos, double4* __restric
 
 static void ensure_atom_capacity(Sim& s, int need);
 
-// One pass over the locals (optionally wrapping them into the box first)
-// gives every atom's selection bits and the ghost totals of the three passes,
-// read back with one synchronisation; the passes then run back to back on
-// the stream: per pass a count over the bits, a tile scan and the stable
-// scatter, in the reference's order.
-void build_ghosts(Sim& s, bool wrap) {
-    if (has_error()) return;
-    // after the fused step loop the locals' positions and velocities live in
-    // the mirror: the selection pass copies them back (binning's inv is still
-    // that of the mirror)
-    const CMir mpos{s.pos_stale ? s.spos.as<double>() : nullptr};
-    const CMir mvel{s.vel_mirrored ? s.svel.as<double>() : nullptr};
-    s.pos_stale = 0;
-    s.vel_mirrored = 0;
-    s.ghost_pos_stale = 0;  // the ghosts are made anew
-    s.ng = 0;
-    s.inv_valid = 0;
-    s.gsrc_valid = 0;
-    mirror_invalidate(s);
-    if (s.n == 0) return;
+static FaceArgs face_args(const Sim& s, int nq, bool wrap) {
     const Geom& G = s.g;
-    const double dspacing = G.spacing * 2.0;
-    int* counters = s.counters.as<int>();
-    s.face.reserve((size_t)std::max(s.cap_all, s.n), true, s.stream);
-    if (has_error()) return;
     FaceArgs fa;
+    fa.nq = nq;
     fa.n = s.n;
     fa.wrap = wrap ? 1 : 0;
     for (int d = 0; d < 3; ++d) {
-        fa.hi_thr[d] = G.aabb[2 * d + 1] - dspacing;
-        fa.lo_thr[d] = G.aabb[2 * d] + dspacing;
+        fa.hi_thr[d] = G.aabb[2 * d + 1] - G.spacing * 2.0;
+        fa.lo_thr[d] = G.aabb[2 * d] + G.spacing * 2.0;
     }
     fa.pbc = pbc_args(s);
-    TMD_HIP(hipMemsetAsync(counters + 8, 0, 6 * sizeof(int), s.stream));
-    hipLaunchKernelGGL(k_face_flags, dim3(div_up(s.n, kScanThreads)), dim3(kScanThreads), 0, s.stream, s.pos.as<double4>(), fa,
-                       s.face.as<unsigned char>(), counters + 8, (const int*)s.cell_inv.as<int>(), mpos, mvel,
-                       s.vel.as<double4>());
-    int tot[6] = {0, 0, 0, 0, 0, 0};
-    TMD_HIP(hipMemcpyAsync(tot, counters + 8, sizeof tot, hipMemcpyDeviceToHost, s.stream));
-    TMD_HIP(hipStreamSynchronize(s.stream));
-    if (has_error()) return;
-    const int ng_all = tot[0] + tot[1] + tot[2] + tot[3] + tot[4] + tot[5];
-    ensure_atom_capacity(s, s.n + ng_all);
-    if (has_error()) return;
-    const int max_tiles = div_up(s.n + ng_all, kScanTile);
-    s.scan_blocks.reserve(sizeof(int) * 2 * (size_t)max_tiles, false, s.stream);
-    if (has_error()) return;
-    int ng = 0;
-    for (int d = 0; d < 3; ++d) {
-        BorderArgs a;
-        a.d = d;
-        a.n = s.n;
-        a.scan_end = s.n + ng;
-        a.base = s.n + ng;
-        a.hi_thr = fa.hi_thr[d];
-        a.lo_thr = fa.lo_thr[d];
-        a.whi_thr = G.world[2 * d + 1] - G.spacing;
-        a.wlo_thr = G.world[2 * d] + G.spacing;
-        a.len0 = G.len[0]; a.len1 = G.len[1]; a.len2 = G.len[2];
-        const int add = tot[2 * d] + tot[2 * d + 1];
-        if (add > 0) {
-            const int ntiles = div_up(a.scan_end, kScanTile);
-            int* t0 = s.scan_blocks.as<int>();
-            int* t1 = t0 + ntiles;
-            hipLaunchKernelGGL(k_border_count, dim3(ntiles), dim3(kScanThreads), 0, s.stream,
-                               (const unsigned char*)s.face.as<unsigned char>(), a, t0, t1);
-            scan_tiles(s, t0, ntiles, counters + 0);
-            scan_tiles(s, t1, ntiles, counters + 1);
-            hipLaunchKernelGGL(k_border_scatter, dim3(ntiles), dim3(kScanThreads), 0, s.stream, s.pos.as<double4>(),
-                               s.vel.as<double4>(), s.mass.as<double>(), s.g_owner.as<int>(), s.g_src.as<int>(),
-                               s.g_code.as<int>(), (const int*)t0, (const int*)t1, (const int*)counters, a,
-                               s.face.as<unsigned char>());
-            TMD_HIP(hipGetLastError());
-        }
-        ng += add;
-    }
-    s.ng = ng;
+    fa.bin = bin_args(s);
+    return fa;
 }
+
+// Enqueue the ghost build: border bits, class counts, (scan,) emit.  bin: the
+// counting sort's histogram of locals and ghosts is taken in the same sweeps
+// (the tail of a rebuild, bin_finish, goes on from there).  Nothing waits for
+// the host: the ghost count stays in the counters.
+void enqueue_ghosts(Sim& s, bool wrap, bool bin) {
+    if (has_error()) return;
+    // positions and velocities move together between atom order and mirror
+    if ((s.pos_stale != 0) != (s.vel_mirrored != 0)) sync_pos_from_mirror(s);
+    const bool mir = s.pos_stale != 0;
+    s.ghost_pos_stale = 0;  // the ghosts are made anew
+    s.ng = 0;
+    s.gsrc_valid = 0;
+    s.gh_valid = 0;
+    if (!mir) {
+        s.inv_valid = 0;
+        mirror_invalidate(s);
+    }
+    if (s.n == 0) return;
+    const Geom& G = s.g;
+    const int gcap = s.cap_all - s.n;
+    const int nq = mir ? s.nbinned : s.n;
+    const int nb = div_up(s.n, kGhostBlock);
+    s.face.reserve((size_t)std::max(s.cap_all, s.n), false, s.stream);
+    const int ncls = kClasses * nb;
+    s.cls.reserve(sizeof(int) * 2 * (size_t)ncls, false, s.stream);  // counts, and their scan
+    s.gh_pack.reserve(sizeof(int) * (size_t)s.n, false, s.stream);
+    s.gh_e.reserve(sizeof(int) * (size_t)std::max(gcap, 1), false, s.stream);
+    s.gh_k.reserve(sizeof(int) * (size_t)std::max(gcap, 1), false, s.stream);
+    s.gh_c.reserve(sizeof(int) * (size_t)std::max(gcap, 1), false, s.stream);
+    if (bin) {
+        s.g_cell.reserve(sizeof(int) * (size_t)std::max(gcap, 1), false, s.stream);
+        s.g_slot.reserve(sizeof(int) * (size_t)std::max(gcap, 1), false, s.stream);
+        bin_reserve(s);
+    }
+    if (has_error()) return;
+    int* ctr = s.counters.as<int>();
+    const int ntiles = s.tiles.ntx * s.tiles.nty * s.tiles.ntz;
+    rebuild_zero(s, bin ? G.ncells : 0, bin ? ntiles : 0, 0);
+    const FaceArgs fa = face_args(s, nq, wrap);
+    const dim3 gq(div_up(nq, kScanThreads)), gb(nb), blk(kScanThreads);
+#define TMD_FACE(M, B)                                                                                                   \
+    hipLaunchKernelGGL((k_face_bin<M, B>), gq, blk, 0, s.stream, s.pos.as<double4>(), Mir{s.spos.as<double>()},            \
+                       (const int*)s.cell_parts.as<int>(), fa, s.face.as<unsigned char>(), s.cell_of.as<int>(),           \
+                       s.cell_slot.as<int>(), s.cell_count.as<int>(), s.cell_inv2.as<int>())
+    if (mir) { if (bin) TMD_FACE(true, true); else TMD_FACE(true, false); }
+    else { if (bin) TMD_FACE(false, true); else TMD_FACE(false, false); }
+#undef TMD_FACE
+    hipLaunchKernelGGL(k_class_count, gb, blk, 0, s.stream, (const unsigned char*)s.face.as<unsigned char>(), s.n, nb,
+                       s.cls.as<int>());
+    EmitArgs ea;
+    ea.n = s.n;
+    ea.nb = nb;
+    ea.gcap = gcap;
+    ea.scanned = ncls > kClassFlat ? 1 : 0;
+    for (int d = 0; d < 3; ++d) {
+        ea.whi[d] = G.world[2 * d + 1] - G.spacing;
+        ea.wlo[d] = G.world[2 * d] + G.spacing;
+        ea.len[d] = G.len[d];
+    }
+    const int* counts = s.cls.as<int>();
+    if (ea.scanned) {
+        exclusive_scan_int(counts, s.cls.as<int>() + ncls, ncls, ctr + CT_NGHOST, s);
+        counts += ncls;
+    }
+    // entry * 32 + count in 31 bits: the index ends where ghosts pass 2^26
+    s.gh_packed = s.gh_wanted && gcap < (1 << 26);
+    int* pack = s.gh_packed ? s.gh_pack.as<int>() : nullptr;
+#define TMD_EMIT(M)                                                                                                      \
+    hipLaunchKernelGGL(k_ghost_emit<M>, gb, blk, 0, s.stream, s.pos.as<double4>(), s.vel.as<double4>(),                    \
+                       s.mass.as<double>(), CMir{s.spos.as<double>()}, CMir{s.svel.as<double>()},                         \
+                       (const int*)s.cell_inv.as<int>(), (const unsigned char*)s.face.as<unsigned char>(), counts, ea,    \
+                       s.g_owner.as<int>(), s.g_src.as<int>(), s.g_code.as<int>(), pack, s.gh_e.as<int>(), ctr)
+    if (mir) TMD_EMIT(true); else TMD_EMIT(false);
+#undef TMD_EMIT
+    if (bin)
+        hipLaunchKernelGGL(k_ghost_bin, dim3(std::max(1, std::min(div_up(gcap, 256), 2048))), dim3(256), 0, s.stream,
+                           (const double4*)s.pos.as<double4>(), s.n, gcap, fa.bin, s.g_cell.as<int>(), s.g_slot.as<int>(),
+                           s.cell_count.as<int>(), s.cell_inv2.as<int>(), (const int*)ctr);
+    TMD_HIP(hipGetLastError());
+}
+
+// md_borders: the ghost layer alone, its size known on return.
+void build_ghosts(Sim& s) {
+    for (int attempt = 0; attempt < 3 && !has_error(); ++attempt) {
+        s.gh_wanted = 1;
+        enqueue_ghosts(s, false, false);
+        if (has_error() || s.n == 0) return;
+        const int* st = read_stats(s);
+        if (!st) return;
+        if (st[CT_NGHOST] <= s.cap_all - s.n) {
+            s.ng = st[CT_NGHOST];
+            return;
+        }
+        ensure_atom_capacity(s, s.n + st[CT_NGHOST]);
+    }
+}
+
+// a rebuild found more ghosts than there is room for
+void grow_ghosts(Sim& s, int ng) { ensure_atom_capacity(s, s.n + ng); }
 
 void refresh_ghosts(Sim& s) {
     if (has_error() || s.ng == 0) return;
@@ -627,11 +788,13 @@ static void ensure_atom_capacity(Sim& s, int need) {
     s.g_code.reserve(sizeof(int) * (size_t)cap, true, s.stream);
     s.cell_of.reserve(sizeof(int) * (size_t)cap, false, s.stream);
     s.cell_slot.reserve(sizeof(int) * (size_t)cap, false, s.stream);
-    s.cell_parts.reserve(sizeof(int) * (size_t)cap, false, s.stream);
-    s.cell_inv.reserve(sizeof(int) * (size_t)cap, false, s.stream);
-    s.face.reserve((size_t)cap, true, s.stream);
-    s.inv_valid = 0;
+    // a repeated rebuild may read the locals through the last binning
+    s.cell_parts.reserve(sizeof(int) * (size_t)cap, true, s.stream);
+    s.cell_inv.reserve(sizeof(int) * (size_t)cap, true, s.stream);
+    s.spos.reserve((size_t)kMirBytes * (size_t)cap, true, s.stream);
+    s.svel.reserve((size_t)kMirBytes * (size_t)cap, true, s.stream);
     s.gsrc_valid = 0;
+    s.gh_valid = 0;
     s.cap_all = cap;
 }
 

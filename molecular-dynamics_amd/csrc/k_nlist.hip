@@ -79,25 +79,63 @@ int tile_block_threads(int requested, int max_locals) {
 int window_cap(const Sim& s) { return std::min(s.max_window + 1, kLdsBudget / kStageBytes); }  // + sentinel slot
 int window_cap_pos(const Sim& s) { return std::min(s.max_window + 1, kLdsBudget / kPosStageBytes); }
 
+// the counters, then the number of this read, into pinned host memory
+__global__ void k_publish(const int* __restrict__ ctr, int* __restrict__ host, int seq) {
+    if (threadIdx.x < CT_COUNT) __hip_atomic_store(&host[threadIdx.x], ctr[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(&host[CT_COUNT], seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// The counters of a rebuild on the host, after everything queued so far;
+// nullptr after an error.  The last kernel stores them into pinned memory and
+// the host watches for its number there: a copy and a stream synchronisation
+// took 36 us from the end of the list build to the next force pass, of which
+// the copy kernel is 4 and the wake-up most of the rest.  The stream is
+// asked now and then, so a failed launch ends the wait as an error.
+const int* read_stats(Sim& s) {
+    if (has_error()) return nullptr;
+    if (!s.h_stats) {
+        TMD_HIP(hipHostMalloc(reinterpret_cast<void**>(&s.h_stats), (CT_COUNT + 1) * sizeof(int)));
+        if (has_error()) return nullptr;
+        s.h_stats[CT_COUNT] = s.stats_seq;
+    }
+    const int seq = ++s.stats_seq;
+    hipLaunchKernelGGL(k_publish, dim3(1), dim3(kWave), 0, s.stream, (const int*)s.counters.as<int>(), s.h_stats, seq);
+    TMD_HIP(hipGetLastError());
+    if (has_error()) return nullptr;
+    for (unsigned spin = 1; __atomic_load_n(&s.h_stats[CT_COUNT], __ATOMIC_ACQUIRE) != seq; ++spin) {
+        if (spin % 4096 != 0) {
+            __builtin_ia32_pause();
+            continue;
+        }
+        const hipError_t e = hipStreamQuery(s.stream);
+        if (e == hipErrorNotReady) continue;
+        // done or failed: synchronising reports which
+        TMD_HIP(hipStreamSynchronize(s.stream));
+        if (!has_error() && __atomic_load_n(&s.h_stats[CT_COUNT], __ATOMIC_ACQUIRE) != seq)
+            set_error(__FILE__, __LINE__, "rebuild: the counters did not reach the host");
+        break;
+    }
+    return has_error() ? nullptr : s.h_stats;
+}
+
 // The window statistics (locals placed, binned atoms, largest window, most
 // locals in a tile) decide the LDS size and block size of the tile kernels.
-static void apply_window_stats(Sim& s, const int* host) {
-    if (host[0] != s.n) {
+void apply_window_stats(Sim& s, const int* st) {
+    if (!st) return;
+    if (st[CT_PLACED] != s.n) {
         char msg[200];
         snprintf(msg, sizeof msg,
                  "%d local atoms lie outside the periodic box or the cell grid (non-finite or unwrapped positions; "
                  "md_enforce_pbc wraps them)",
-                 s.n - host[0]);
+                 s.n - st[CT_PLACED]);
         set_error(__FILE__, __LINE__, msg);
         return;
     }
-    s.nbinned = host[1];
-    s.max_window = host[2];
-    s.tile_threads = tile_block_threads(s.tile_threads_req, host[3]);
+    s.nbinned = st[CT_BINNED];
+    s.max_window = st[CT_MAXWIN];
+    s.tile_threads = tile_block_threads(s.tile_threads_req, st[CT_MAXLOC]);
     retune_tile_edge(s);
-    s.spos.reserve((size_t)kMirBytes * (size_t)std::max(s.nbinned, 1), false, s.stream);
-    s.spos2.reserve((size_t)kMirBytes * (size_t)std::max(s.nbinned, 1), false, s.stream);
-    if (has_error()) return;
     if (s.max_window > kWinMax) {
         char msg[200];
         snprintf(msg, sizeof msg, "a tile neighbourhood holds %d atoms, beyond the 16-bit window range (%d)", s.max_window,
@@ -110,51 +148,6 @@ static void apply_window_stats(Sim& s, const int* host) {
         return;
     }
     s.windows_valid = 1;
-}
-
-// A rebuild inside the fused step loop (s.defer_window_sync, with statistics
-// from an earlier binning at hand) only queues the copy of the statistics
-// into pinned host memory: its list build runs with the previous window and
-// block sizes (a larger window is then read from the mirror, a fuller tile
-// takes a second pass of its block) and reads the new statistics after its
-// own synchronisation (finish_windows), saving one host round trip.
-void build_windows(Sim& s) {
-    if (has_error()) return;
-    int* counters = s.counters.as<int>();
-    const Geom& G = s.g;
-    const int ntiles = s.tiles.ntx * s.tiles.nty * s.tiles.ntz;
-    const bool defer = s.defer_window_sync && s.max_window > 0;
-    int local[4] = {0, 0, 0, 0};
-    int* host = local;
-    if (defer) {
-        if (!s.h_winstats) TMD_HIP(hipHostMalloc(reinterpret_cast<void**>(&s.h_winstats), 4 * sizeof(int)));
-        if (has_error()) return;
-        host = s.h_winstats;
-    }
-    // counters[6] = largest tile window, counters[7] = most locals in a tile (from k_tile_stats)
-    TMD_HIP(hipMemcpyAsync(&host[0], s.tile_start.as<int>() + ntiles, sizeof(int), hipMemcpyDeviceToHost, s.stream));
-    TMD_HIP(hipMemcpyAsync(&host[1], s.cell_start.as<int>() + G.ncells, sizeof(int), hipMemcpyDeviceToHost, s.stream));
-    TMD_HIP(hipMemcpyAsync(&host[2], counters + 6, 2 * sizeof(int), hipMemcpyDeviceToHost, s.stream));
-    if (defer) {
-        const int bound = std::max(s.n + s.ng, 1);  // binned atoms, at most
-        s.spos.reserve((size_t)kMirBytes * (size_t)bound, false, s.stream);
-        s.spos2.reserve((size_t)kMirBytes * (size_t)bound, false, s.stream);
-        if (has_error()) return;
-        s.windows_pending = 1;
-        s.windows_valid = 1;
-        return;
-    }
-    TMD_HIP(hipStreamSynchronize(s.stream));
-    if (has_error()) return;
-    apply_window_stats(s, host);
-}
-
-void finish_windows(Sim& s) {
-    if (!s.windows_pending) return;
-    s.windows_pending = 0;
-    TMD_HIP(hipStreamSynchronize(s.stream));  // the copies were queued before
-    if (has_error()) return;
-    apply_window_stats(s, s.h_winstats);
 }
 
 // DEM step loop: positions and velocities of every binned atom, ghosts
@@ -201,10 +194,10 @@ void build_neighbor_lists(Sim& s, int half, double cutoff) {
     TMD_REQUIRE(s.windows_valid, "md_assemble_neighborlists: cells not binned (call md_distribute_particles first)");
     if (has_error()) return;
     int* counters = s.counters.as<int>();
-    refresh_mirror(s);
+    if (!s.mirror_fresh) refresh_mirror(s);
     const int ntiles = s.tiles.ntx * s.tiles.nty * s.tiles.ntz;
-    // counters[2] = overflow (largest count above the capacity)
-    for (;;) {
+    // a rebuild has just cleared the counters
+    for (bool cleared = s.windows_pending != 0;; cleared = false) {
         s.nb_cap = (s.nb_cap + 7) & ~7;
         const int ntile64 = div_up(s.n > 0 ? s.n : 1, 64);
         s.nb_stride = ntile64 * 64;
@@ -216,7 +209,7 @@ void build_neighbor_lists(Sim& s, int half, double cutoff) {
             s.nb_list2.reserve(sizeof(nb_t) * (size_t)ntile64 * 64 * (size_t)s.nb_cap, false, s.stream);
         }
         if (has_error()) return;
-        TMD_HIP(hipMemsetAsync(counters + 2, 0, sizeof(int), s.stream));
+        if (!cleared) rebuild_zero(s, 0, 0, s.ng);
         const int rsb = row_starts_bytes(s.tiles);
         // window slots (positions, 24 B; half lists also the atom index,
         // 28 B) + sentinel slots, then the row starts
@@ -230,15 +223,27 @@ void build_neighbor_lists(Sim& s, int half, double cutoff) {
                        (const int*)s.work_k.as<int>(), (const int*)s.work_c.as<int>(),                                      \
                        (const int*)s.cell_start.as<int>(), (const int*)s.cell_parts.as<int>(), (const int*)s.work.as<int>(), \
                        (const int*)s.tile_start.as<int>(), a, s.nb_count.as<int>(), s.nb_list.as<nb_t>(), \
-                       s.nb_count2.as<int>(), s.nb_list2.as<nb_t>(), counters + 2)
+                       s.nb_count2.as<int>(), s.nb_list2.as<nb_t>(), counters + CT_LIST)
             if (half) TMD_NLIST(true); else TMD_NLIST(false);
 #undef TMD_NLIST
         }
         TMD_HIP(hipGetLastError());
-        int over = 0;
-        TMD_HIP(hipMemcpyAsync(&over, counters + 2, sizeof(int), hipMemcpyDeviceToHost, s.stream));
-        TMD_HIP(hipStreamSynchronize(s.stream));
-        finish_windows(s);  // statistics of a deferred window build
+        const int* st = read_stats(s);
+        if (!st) return;
+        const int over = st[CT_LIST];
+        if (s.windows_pending) {
+            // the statistics of the rebuild that queued this list build
+            s.windows_pending = 0;
+            if (st[CT_NGHOST] > s.cap_all - s.n) {
+                // incomplete ghosts: the rebuild grows and repeats, from the
+                // locals of this binning
+                s.ghosts_missing = st[CT_NGHOST];
+                s.nbinned = st[CT_BINNED];
+                return;
+            }
+            s.ng = st[CT_NGHOST];
+            apply_window_stats(s, st);
+        }
         if (has_error()) return;
         if (over > 0) {
             s.nb_cap = over * 2;
@@ -248,6 +253,53 @@ void build_neighbor_lists(Sim& s, int half, double cutoff) {
     }
     s.nb_half = half;
     s.nb_valid = 1;
+}
+
+// A whole rebuild (wrap when asked, ghosts, cells, tiles, mirrors, lists)
+// with one host synchronisation, at its end: the ghost count stays on the
+// device until then, and the list build runs with the window and block sizes
+// of the rebuild before (a larger window is then read from the mirror, a
+// fuller tile takes a second pass of its block).  The first rebuild has no
+// such sizes and waits for its own before the lists.
+void rebuild_lists(Sim& s, bool wrap, int half, double cutoff) {
+    if (has_error()) return;
+    s.nb_valid = 0;
+    if (s.n == 0) {
+        bin_particles(s);
+        build_neighbor_lists(s, half, cutoff);
+        return;
+    }
+    for (int attempt = 0; attempt < 4 && !has_error(); ++attempt) {
+        hipEvent_t ev = nullptr;
+        s.ghosts_missing = 0;
+        const int nq = s.pos_stale && s.vel_mirrored ? s.nbinned : s.n;
+        s.timer.begin(K_BORDERS, s.stream, &ev);
+        enqueue_ghosts(s, wrap && attempt == 0, true);
+        s.timer.end(K_BORDERS, s.stream, ev);
+        s.timer.begin(K_BIN, s.stream, &ev);
+        bin_finish(s, nq, true);
+        s.timer.end(K_BIN, s.stream, ev);
+        if (has_error()) return;
+        if (s.max_window > 0) {
+            s.windows_pending = 1;
+            s.windows_valid = 1;
+        } else {
+            const int* st = read_stats(s);
+            if (!st) return;
+            if (st[CT_NGHOST] > s.cap_all - s.n) s.ghosts_missing = st[CT_NGHOST];
+            else s.ng = st[CT_NGHOST];
+            apply_window_stats(s, st);  // also the binned count that a repeat reads the mirrors by
+        }
+        if (!s.ghosts_missing) {
+            s.timer.begin(K_NEIGHBOR, s.stream, &ev);
+            build_neighbor_lists(s, half, cutoff);
+            s.timer.end(K_NEIGHBOR, s.stream, ev);
+        }
+        s.windows_pending = 0;
+        if (!s.ghosts_missing) return;
+        s.max_window = 0;
+        grow_ghosts(s, s.ghosts_missing);
+    }
 }
 
 }  // namespace tmd

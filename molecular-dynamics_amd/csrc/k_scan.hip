@@ -79,11 +79,6 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_finish(const int* __restr
     }
 }
 
-void scan_tiles(Sim& s, int* tiles, int ntiles, int* total_dev) {
-    hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(kScanThreads), 0, s.stream, tiles, ntiles, total_dev);
-    TMD_HIP(hipGetLastError());
-}
-
 void scan_exclusive(const int* in, int* out, int n, int* total_dev, int* tiles, hipStream_t st) {
     const int ntiles = div_up(n, kScanTile);
     hipLaunchKernelGGL(k_tile_sums, dim3(ntiles), dim3(kScanThreads), 0, st, in, n, tiles);
@@ -92,9 +87,56 @@ void scan_exclusive(const int* in, int* out, int n, int* total_dev, int* tiles, 
     TMD_HIP(hipGetLastError());
 }
 
+// One block scans up to kScanOneMax ints in registers: one launch instead of
+// three (each about 4 us on an otherwise idle GPU).  Every wavefront takes
+// one contiguous stretch, 64 ints at a time (coalesced, all loads under way
+// before the first is used), scans each 64 in registers and carries on; then
+// the wavefronts' totals are scanned.
+constexpr int kScanOneThreads = 1024, kScanOnePer = 32, kScanOneMax = kScanOneThreads * kScanOnePer;
+__global__ void __launch_bounds__(kScanOneThreads) k_scan_one(const int* __restrict__ in, int* __restrict__ out, int n,
+                                                              int* __restrict__ total) {
+    __shared__ int wsum[kScanOneThreads / kWave];
+    const int lane = threadIdx.x & (kWave - 1), wid = (int)threadIdx.x / kWave;
+    const int per = (n + kScanOneThreads - 1) / kScanOneThreads;  // 64-int groups a wavefront
+    const int base = wid * per * kWave + lane;
+    int v[kScanOnePer], inc[kScanOnePer];
+#pragma unroll
+    for (int it = 0; it < kScanOnePer; ++it) {
+        const int idx = base + it * kWave;
+        v[it] = (it < per && idx < n) ? in[idx] : 0;
+    }
+    int carry = 0;
+#pragma unroll
+    for (int it = 0; it < kScanOnePer; ++it) {
+        if (it < per) {
+            inc[it] = carry + wave_inclusive_scan(v[it]);
+            carry = __builtin_amdgcn_readlane(inc[it], kWave - 1);
+        }
+    }
+    if (lane == 0) wsum[wid] = carry;
+    __syncthreads();
+    int off = 0, tot = 0;
+#pragma unroll
+    for (int w = 0; w < kScanOneThreads / kWave; ++w) {
+        if (w < wid) off += wsum[w];
+        tot += wsum[w];
+    }
+#pragma unroll
+    for (int it = 0; it < kScanOnePer; ++it) {
+        const int idx = base + it * kWave;
+        if (it < per && idx < n) out[idx] = off + inc[it] - v[it];
+    }
+    if (threadIdx.x == 0 && total) *total = tot;
+}
+
 void exclusive_scan_int(const int* in, int* out, int n, int* total_dev, Sim& s) {
     if (n <= 0) {
         if (total_dev) TMD_HIP(hipMemsetAsync(total_dev, 0, sizeof(int), s.stream));
+        return;
+    }
+    if (n <= kScanOneMax) {
+        hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(kScanOneThreads), 0, s.stream, in, out, n, total_dev);
+        TMD_HIP(hipGetLastError());
         return;
     }
     const int ntiles = div_up(n, kScanTile);

@@ -146,8 +146,6 @@ static void alloc_atoms(Sim& s, int cap) {
     s.g_owner.reserve(sizeof(int) * (size_t)cap, true, s.stream);
     s.g_src.reserve(sizeof(int) * (size_t)cap, true, s.stream);
     s.g_code.reserve(sizeof(int) * (size_t)cap, true, s.stream);
-    s.cell_of.reserve(sizeof(int) * (size_t)cap, false, s.stream);
-    s.cell_slot.reserve(sizeof(int) * (size_t)cap, false, s.stream);
     s.cell_parts.reserve(sizeof(int) * (size_t)cap, false, s.stream);
     s.cell_inv.reserve(sizeof(int) * (size_t)cap, false, s.stream);
     s.inv_valid = 0;
@@ -251,24 +249,13 @@ static double host_temperature(const Sim& s) {
 
 static void rebuild(Sim& s, int half, double cutoff) {
     s.ng = 0;  // exchange_particles on one rank (comm/comm.impala:392-396)
-    hipEvent_t ev = nullptr;
     if (s.sort_particles) {
+        hipEvent_t ev = nullptr;
         s.timer.begin(K_BIN, s.stream, &ev);
         sort_locals(s);  // wraps, then renumbers the locals in cell order
         s.timer.end(K_BIN, s.stream, ev);
     }
-    s.timer.begin(K_BORDERS, s.stream, &ev);
-    build_ghosts(s, true);  // md_enforce_pbc + borders
-    s.timer.end(K_BORDERS, s.stream, ev);
-    s.timer.begin(K_BIN, s.stream, &ev);
-    s.defer_window_sync = 1;  // the list build reads the window statistics
-    bin_particles(s);
-    s.timer.end(K_BIN, s.stream, ev);
-    s.timer.begin(K_NEIGHBOR, s.stream, &ev);
-    build_neighbor_lists(s, half, cutoff);
-    s.timer.end(K_NEIGHBOR, s.stream, ev);
-    s.defer_window_sync = 0;
-    finish_windows(s);  // if the list build stopped early
+    rebuild_lists(s, true, half, cutoff);
 }
 
 // ---------------------------------------------------------------------------
@@ -365,6 +352,7 @@ int md_initialize_grid(double const* masses, struct Vector3D const* positions, s
     s.ghost_pos_stale = 0;
     s.dem_mirrored = 0;
     s.gsrc_valid = 0;
+    s.gh_valid = s.gh_packed = 0;
     s.h_mass.assign(masses, masses + nparticles);
     s.h_pos.resize(3 * (size_t)nparticles);
     s.h_vel.resize(3 * (size_t)nparticles);
@@ -663,18 +651,18 @@ void md_deallocate_grid() {
     if (s.stream) (void)hipStreamSynchronize(s.stream);
     s.timer.collect();
     DevBuf* bufs[] = {&s.pos, &s.vel, &s.force, &s.mass, &s.sort_buf, &s.g_owner, &s.g_src, &s.g_code, &s.cell_of, &s.cell_slot,
-                      &s.cell_count, &s.cell_start, &s.cell_parts, &s.cell_inv, &s.work_start, &s.work, &s.work_k, &s.work_c, &s.g_ko, &s.g_kg, &s.gh_start, &s.gh_k, &s.gh_c, &s.gh_aux, &s.tile_start, &s.spos, &s.spos2, &s.face, &s.svel, &s.svel2,
+                      &s.cell_count, &s.cell_start, &s.cell_parts, &s.cell_inv, &s.work_start, &s.work, &s.work_k, &s.work_c, &s.g_ko, &s.g_kg, &s.gh_pack, &s.gh_w, &s.gh_k, &s.gh_c, &s.gh_e, &s.g_cell, &s.g_slot, &s.cell_parts2, &s.cell_inv2, &s.cell_pair,
+                      &s.cell_src, &s.cls, &s.tile_start, &s.spos, &s.spos2, &s.face, &s.svel, &s.svel2,
                       &s.nb_count, &s.nb_list, &s.nb_count2, &s.nb_list2,
                       &s.scan_blocks, &s.scan_aux, &s.red, &s.gbuf, &s.adj_x0, &s.adj_v0, &s.adj_ckx,
                       &s.adj_ckv, &s.adj_segx, &s.adj_segv, &s.adj_xbar, &s.adj_vbar, &s.adj_fbar, &s.adj_part,
                       &s.adj_acc};
     for (DevBuf* b : bufs) b->release();
-    if (s.h_winstats) {
-        (void)hipHostFree(s.h_winstats);
-        s.h_winstats = nullptr;
+    if (s.h_stats) {
+        (void)hipHostFree(s.h_stats);
+        s.h_stats = nullptr;
     }
     s.windows_pending = 0;
-    s.defer_window_sync = 0;
     s.max_window = 0;
     s.tile_auto = 0;
     s.stage_bytes = kPosStageBytes;
@@ -690,6 +678,7 @@ void md_deallocate_grid() {
     s.vel_mirror_wanted = 0;
     s.ghost_pos_stale = 0;
     s.gsrc_valid = 0;
+    s.gh_valid = s.gh_packed = 0;
     s.nbinned = 0;
     s.dev_valid = false;
 }
@@ -771,6 +760,7 @@ void md_exchange_particles() {
     s.ng = 0;
     s.nb_valid = 0;
     s.windows_valid = 0;
+    s.gh_valid = s.gh_packed = 0;
 }
 
 double md_get_send_buffer_value(int) { return 0.0; }
@@ -1009,7 +999,14 @@ int tmd_get_cells(int* start, int* atoms, int* atom_cell) {
     TMD_HIP(hipMemcpy(st.data(), s.cell_start.p, sizeof(int) * (nc + 1), hipMemcpyDeviceToHost));
     if (start) std::copy(st.begin(), st.end(), start);
     if (atoms && st[nc] > 0) TMD_HIP(hipMemcpy(atoms, s.cell_parts.p, sizeof(int) * st[nc], hipMemcpyDeviceToHost));
-    if (atom_cell && s.n + s.ng > 0) TMD_HIP(hipMemcpy(atom_cell, s.cell_of.p, sizeof(int) * (s.n + s.ng), hipMemcpyDeviceToHost));
+    if (atom_cell && s.n + s.ng > 0) {
+        std::vector<int> parts(std::max(st[nc], 1));
+        if (st[nc] > 0) TMD_HIP(hipMemcpy(parts.data(), s.cell_parts.p, sizeof(int) * st[nc], hipMemcpyDeviceToHost));
+        std::fill(atom_cell, atom_cell + s.n + s.ng, -1);
+        if (has_error()) return 0;
+        for (int c = 0; c < nc; ++c)
+            for (int k = st[c]; k < st[c + 1]; ++k) atom_cell[parts[k]] = c;
+    }
     return st[nc];
 }
 
@@ -1079,6 +1076,7 @@ static int run_loop(int steps, int reneigh_every, double dt, bool half, double c
     const int hf = half ? 1 : 0;
     const int saved_sync = s.sync_calls;
     s.sync_calls = 0;
+    s.gh_wanted = dem;  // the DEM step pass also writes the ghosts
     if (!s.nb_valid || s.nb_half != hf) rebuild(s, hf, cutoff + skin);
     int done = 0;
     if (!dem && s.ghost_mode == GHOST_FRESH) {
@@ -1093,7 +1091,7 @@ static int run_loop(int steps, int reneigh_every, double dt, bool half, double c
         s.vel_mirror_wanted = 1;  // the rebuild's mirror pass moves them again
         for (int j = 0; j < steps && !has_error(); ++j) {
             if ((j + 1) % reneigh_every == 0) {
-                rebuild(s, hf, cutoff + skin);  // its ghost selection pass restores pos and vel from the mirror
+                rebuild(s, hf, cutoff + skin);  // mirror to mirror
             } else {
                 hipEvent_t ev = nullptr;
                 s.timer.begin(K_GHOST_SYNC, s.stream, &ev);
@@ -1120,15 +1118,21 @@ static int run_loop(int steps, int reneigh_every, double dt, bool half, double c
         for (int j = 0; j < steps && !has_error(); ++j) {
             hipEvent_t ev = nullptr;
             if ((j + 1) % reneigh_every == 0) {
-                // the rebuild's ghost selection pass copies the locals'
-                // positions and velocities back from the mirrors (as in the
-                // LJ loop); its ghosts are made anew from them
+                // the rebuild goes from the old mirrors to the new ones (as in
+                // the LJ loop), ghosts' velocities included
                 if (s.dem_mirrored) {
                     s.pos_stale = 1;
                     s.vel_mirrored = 1;
                     s.dem_mirrored = 0;
                 }
+                s.dem_loop = 1;
                 rebuild(s, hf, cutoff + skin);
+                s.dem_loop = 0;
+                if (!has_error()) {
+                    s.dem_mirrored = 1;
+                    s.pos_stale = 0;
+                    s.vel_mirrored = 0;
+                }
             } else if (s.dem_mirrored) {
                 // the previous step pass wrote the ghosts too, unless it
                 // could not (no ghost index)

@@ -25,10 +25,11 @@ __device__ __forceinline__ int wave_inclusive_scan(int v) {
     return v;
 }
 
-// Exclusive scan over the block (blockDim.x == kScanThreads); returns the
-// exclusive prefix of v and the block total in *total.
-__device__ __forceinline__ int block_exclusive_scan(int v, int* total) {
-    __shared__ int wsum[kScanThreads / kWave];
+// Exclusive scan over a block of NT threads; returns the exclusive prefix of
+// v and the block total in *total.
+template <int NT>
+__device__ __forceinline__ int block_exclusive_scan_n(int v, int* total) {
+    __shared__ int wsum[NT / kWave];
     const int lane = threadIdx.x & (kWave - 1);
     const int wid = threadIdx.x / kWave;
     int inc = wave_inclusive_scan(v);
@@ -36,7 +37,7 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int* total) {
     __syncthreads();
     int off = 0, tot = 0;
 #pragma unroll
-    for (int w = 0; w < kScanThreads / kWave; ++w) {
+    for (int w = 0; w < NT / kWave; ++w) {
         int s = wsum[w];
         if (w < wid) off += s;
         tot += s;
@@ -45,6 +46,8 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int* total) {
     *total = tot;
     return off + inc - v;
 }
+
+__device__ __forceinline__ int block_exclusive_scan(int v, int* total) { return block_exclusive_scan_n<kScanThreads>(v, total); }
 
 __device__ __forceinline__ int block_sum_int(int v) {
     int tot;
@@ -151,6 +154,42 @@ __device__ __forceinline__ int wave_sort_cell(int b, int e, int lim, int* __rest
         for (int k = b; k < e; ++k) inv[parts[k]] = k;
     }
     return __shfl(nl, 0, kWave);
+}
+
+// Sort the cell segment in[b, e) of (atom index, source slot) pairs by atom
+// index (distinct) with one wavefront: parts and src receive the two halves in
+// order, and inv[atom] its position.  Segments of up to 64 by rank (each
+// lane counts the smaller values, broadcast from a scalar register); longer
+// ones by counting over memory.  Returns, in every lane, how many values are
+// below lim (the locals, which lead the sorted segment).
+__device__ __forceinline__ int wave_sort_pairs(int b, int e, int lim, const int2* __restrict__ in, int* __restrict__ parts,
+                                               int* __restrict__ src, int* __restrict__ inv) {
+    const int lane = threadIdx.x & (kWave - 1);
+    b = __builtin_amdgcn_readfirstlane(b);
+    const int m = __builtin_amdgcn_readfirstlane(e) - b;
+    if (m <= kWave) {
+        const int2 v = lane < m ? in[b + lane] : make_int2(0x7fffffff, 0);
+        int rank = 0;
+        for (int k = 0; k < m; ++k) rank += __builtin_amdgcn_readlane(v.x, k) < v.x ? 1 : 0;
+        if (lane < m) {
+            parts[b + rank] = v.x;
+            if (src) src[b + rank] = v.y;
+            inv[v.x] = b + rank;
+        }
+        return __popcll(__ballot(lane < m && v.x < lim));
+    }
+    int nl = 0;
+    for (int q = lane; q < m; q += kWave) {
+        const int2 v = in[b + q];
+        int rank = 0;
+        for (int k = b; k < e; ++k) rank += in[k].x < v.x ? 1 : 0;
+        parts[b + rank] = v.x;
+        if (src) src[b + rank] = v.y;
+        inv[v.x] = b + rank;
+        nl += v.x < lim ? 1 : 0;
+    }
+    const int inc = wave_inclusive_scan(nl);
+    return __builtin_amdgcn_readlane(inc, kWave - 1);
 }
 
 // Streaming (non-temporal) load, for data a launch reads once (list groups):

@@ -57,6 +57,23 @@ struct Geom {
     int nx, ny, nz, ncells;
 };
 
+// Counters of a rebuild on the device (Sim::counters), read back in one copy.
+enum Counter {
+    CT_NGHOST = 0,   // ghosts of the current layer (all, also those beyond the capacity)
+    CT_LIST = 1,     // largest list count above the capacity (0: none)
+    CT_MAXWIN = 2,   // largest tile window
+    CT_MAXLOC = 3,   // most locals in a tile
+    CT_PLACED = 4,   // locals in the tiles' work order
+    CT_BINNED = 5,   // atoms in the cell CSR
+    CT_COUNT = 6
+};
+
+// Cell grid arguments of the binning kernels.
+struct BinArgs {
+    double xmin, ymin, zmin, spacing;
+    int nx, ny, ncells;
+};
+
 // A device buffer that grows (optionally preserving its contents).
 struct DevBuf {
     void* p = nullptr;
@@ -111,11 +128,15 @@ struct Sim {
     int vel_mirrored = 0;   // local velocities live in svel, in mirror order (fused step loop)
     int vel_mirror_wanted = 0;  // fused step loop: refresh_mirror also moves the velocities to svel
     int gsrc_valid = 0;     // g_ko / g_kg match the ghost table and the binning
-    int gh_valid = 0;       // gh_start / gh_k / gh_c match the ghost table, binning and work order
+    int gh_wanted = 0;      // ghost builds also make the ghost index (gh_pack / gh_e, then gh_w / gh_k / gh_c)
+    int gh_packed = 0;      // gh_pack / gh_e match the ghost table
+    int gh_valid = 0;       // gh_w / gh_k / gh_c match the ghost table, binning and work order
+    int dem_loop = 0;       // DEM step loop: a rebuild's mirrors hold the ghosts' velocities too
     int dem_ghosts_done = 0;  // DEM step loop: the last force pass also wrote the ghosts' mirror entries
-    int defer_window_sync = 0;  // rebuild in progress: build_windows may leave its statistics pending
-    int windows_pending = 0;    // window statistics queued into h_winstats, not yet applied (finish_windows)
-    int* h_winstats = nullptr;  // pinned host copy of the window statistics (4 ints)
+    int windows_pending = 0;    // a rebuild's statistics are still on the device (read after its list build)
+    int ghosts_missing = 0;     // ghosts a rebuild found beyond the capacity (their total number)
+    int* h_stats = nullptr;     // pinned host copy of the counters, then the number of the read (read_stats)
+    int stats_seq = 0;          // reads of the counters so far
     int ghost_pos_stale = 0;  // ghosts in pos lag the mirror (fused step loop; sync_pos_from_mirror)
     int lds_limit = 65536;  // LDS bytes per block (device attribute)
 
@@ -138,8 +159,13 @@ struct Sim {
     DevBuf pos, vel, force, mass;      // double4 x3, double
     DevBuf sort_buf;                   // sort_locals: scratch copies of the four arrays above
     DevBuf g_owner, g_src, g_code;     // ghost table
-    DevBuf cell_of, cell_slot, cell_count, cell_start, cell_parts;
+    DevBuf cell_of, cell_slot;         // binning: cell and counting-sort slot of each source slot
+    DevBuf g_cell, g_slot;             // the same of each ghost
+    DevBuf cell_count, cell_start, cell_parts;
     DevBuf cell_inv;                   // CSR index of each atom (-1: outside the grid)
+    DevBuf cell_parts2, cell_inv2;     // the next binning's, swapped in when it is sorted
+    DevBuf cell_pair, cell_src;        // (atom, source slot) pairs before the sort; source slot by CSR index
+    DevBuf cls;                        // ghost counts by class and block of locals, and their scan
     DevBuf work_start, work;           // per-tile local counts; locals in tile work order (work slots)
     DevBuf tile_start;                 // first work slot of each tile [ntiles + 1]
     DevBuf spos;                       // cell-ordered position mirror (x, y, z packed, 24 B per atom)
@@ -150,10 +176,12 @@ struct Sim {
     DevBuf svel;                       // local velocities in mirror order during the fused step loop
     DevBuf svel2;                      // DEM step loop: the velocity mirror the force pass writes
     int dem_mirrored = 0;              // DEM step loop: positions and velocities (ghosts too) live in the mirrors
-    DevBuf face;                       // per atom: border selection bits of the three ghost passes (u8)
+    DevBuf face;                       // per local: border selection bits of the three ghost passes (u8)
     DevBuf g_ko, g_kg;                 // per ghost: mirror index of its owner and its own (-1: outside the grid)
-    DevBuf gh_start, gh_k, gh_c;       // ghosts by owner work slot: CSR start [n + 1], mirror index, image code
-    DevBuf gh_aux;                     // per work slot: owner's work slot scratch, counts and fill cursors
+    // ghost index: per local (gh_pack) and per work slot (gh_w) the first
+    // entry * 32 + number of ghosts; per entry mirror index and image code;
+    // per ghost its entry (gh_e)
+    DevBuf gh_pack, gh_w, gh_k, gh_c, gh_e;
     DevBuf nb_count, nb_list;
     DevBuf nb_count2, nb_list2;        // half lists: the complementary columns (local j > i)
     DevBuf scan_blocks, scan_aux, counters, red, gbuf;
@@ -188,19 +216,22 @@ inline int div_up(long long a, long long b) { return (int)((a + b - 1) / b); }
 // launchers (kernels live in the .hip translation units)
 // scan / compaction
 void exclusive_scan_int(const int* in, int* out, int n, int* total_dev, Sim& s);
-void scan_tiles(Sim& s, int* tiles, int ntiles, int* total_dev);  // one-block exclusive scan in place
 // exclusive scan of n > 0 ints with caller scratch of div_up(n, kScanTile)
 // ints; no allocation, no host synchronisation (graph-capturable)
 void scan_exclusive(const int* in, int* out, int n, int* total_dev, int* tiles, hipStream_t st);
 
 // borders / ghosts
-void build_ghosts(Sim& s, bool wrap = false);  // wrap: md_enforce_pbc on the locals first (fused)
+void build_ghosts(Sim& s);  // md_borders: the ghost layer alone
+void enqueue_ghosts(Sim& s, bool wrap, bool bin);  // without waiting; wrap: md_enforce_pbc first, bin: histogram too (fused)
+void grow_ghosts(Sim& s, int ng);
+void rebuild_zero(Sim& s, int ncells, int ntiles, int ng);
+// a whole rebuild: (wrap,) ghosts, cells, tiles, mirrors and lists, one host synchronisation
+void rebuild_lists(Sim& s, bool wrap, int half, double cutoff);
 void refresh_ghosts(Sim& s);
 // fresh ghost positions and the cell-ordered mirror of locals and ghosts in
 // one pass (after positions were advanced inside the force pass)
 void step_refresh(Sim& s);
 void build_ghost_src(Sim& s);  // g_ko / g_kg (binning, after the CSR is built)
-void build_ghost_index(Sim& s);  // each local's ghosts by work slot (gh_start / gh_k / gh_c)
 void sync_pos_from_mirror(Sim& s);
 void mirror_velocities(Sim& s, bool into_mirror);
 
@@ -208,19 +239,22 @@ void mirror_velocities(Sim& s, bool into_mirror);
 void make_geom(Geom& G, const double* aabb, const double* rank_aabb, double cell_spacing);
 
 // binning
+BinArgs bin_args(const Sim& s);
+void bin_reserve(Sim& s);
 void bin_particles(Sim& s);
+void bin_finish(Sim& s, int nq, bool with_ghosts);  // everything of a binning behind its histogram of nq source slots
 void sort_locals(Sim& s);  // PBC wrap + renumber the locals in cell order
 int auto_tile_edge(const Geom& G, int n);  // cells per tile edge for ~480 locals per tile
 void retune_tile_edge(Sim& s);  // automatic tiles: a smaller edge at the next binning when windows overflow
 TileGeom make_tile_geom(const Geom& G, int tx, int ty, int tz);
 
 // tile windows (after binning), position mirror, neighbour lists
-void build_windows(Sim& s);
+const int* read_stats(Sim& s);
+void apply_window_stats(Sim& s, const int* st);
 int window_cap(const Sim& s);      // window slots of kernels that stage positions and atom indices
 int window_cap_pos(const Sim& s);  // window slots of kernels that stage positions only
 int tile_block_threads(int requested, int max_locals);  // staged window atoms per block (LDS budget, kStageBytes each)
 void refresh_mirror(Sim& s);
-void finish_windows(Sim& s);  // apply window statistics left pending by build_windows
 void build_neighbor_lists(Sim& s, int half, double cutoff);
 
 // forces

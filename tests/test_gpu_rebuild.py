@@ -1,0 +1,123 @@
+"""GPU parity of a rebuild inside the step loop (ghosts, cells, lists made
+from the cell-ordered mirrors in one pass without a host round trip) against
+the CPU oracle, at the sizes where its launches change shape: a single block
+of locals, whole and ragged blocks, class counts scanned by the emitting
+blocks or by launches of their own, grids whose tiles are counted by the sort
+or by a launch of their own, and more ghosts than there was room for."""
+import numpy as np
+import pytest
+
+import pyoracle as po
+from common import RC, SKIN, announce, make_pair, perturbed_fcc
+
+pytestmark = pytest.mark.gpu
+
+DT = 0.005
+
+
+@pytest.fixture(scope="module")
+def tm():
+    import tinymd_amd
+    _, cus = tinymd_amd.device_info()
+    if cus == 0:
+        pytest.fail("no HIP device visible to libtinymd_amd")
+    return tinymd_amd
+
+
+def same_structure(sim, orc):
+    """Ghost table, cells and lists entry for entry."""
+    assert sim.nghost == orc.ng
+    gt, go = sim.ghost_table(), orc.ghosts()
+    for key in ("owner", "img", "src", "flag"):
+        assert np.array_equal(gt[key], go[key]), key
+    st, parts, pcell = sim.cells()
+    so, po_, pco = orc.cells()
+    assert np.array_equal(st, so) and np.array_equal(parts, po_) and np.array_equal(pcell, pco)
+    cg, lg = sim.neighbor_lists()
+    co, lo = orc.neighbor_lists()
+    assert np.array_equal(cg, co)
+    m = min(lg.shape[1], lo.shape[1])
+    cols = np.arange(m)[None, :] < cg[:, None]
+    assert np.array_equal(np.where(cols, lg[:, :m], -1), np.where(cols, lo[:, :m], -1))
+
+
+# (4, 4, 4): 256 atoms, one block; (5, 4, 7): ragged; (20, 20, 25):
+# 157 blocks, the most whose counts the blocks scan themselves; 22^3: 167
+@pytest.mark.parametrize("shape", [(4, 4, 4), (5, 4, 7), (8, 8, 4), (20, 20, 25), (22, 22, 22)])
+def test_rebuild_in_loop_exact(tm, shape):
+    announce(f"rebuild in the loop {shape}")
+    aabb, m, x, v = perturbed_fcc(*shape, amp=0.05, seed=11)
+    sim, orc = make_pair(aabb, m, x, v)
+    sim.setup(False, RC, SKIN)
+    orc.setup(False, po.HALF_GHOST_FULL, RC + SKIN)
+    same_structure(sim, orc)
+    sim.lennard_jones(False, RC)
+    orc.lj(False, RC)
+    # the second rebuild starts from the first one's mirrors
+    sim.run_lj(45, 20, DT)
+    orc.run_lj(45, 20, DT)
+    same_structure(sim, orc)
+    _, xg, vg, fg = sim.state()
+    xo, vo, fo = orc.state()
+    assert np.array_equal(xg, xo) and np.array_equal(vg, vo) and np.array_equal(fg, fo)
+
+
+def test_rebuild_sparse_grid_dem(tm):
+    """A grid of 35,937 cells for 28,000 spheres: a thread per cell sorts,
+    tiles are counted by their own launch; ghost velocities and the ghost
+    index follow the rebuilds.  Contact forces differ from the oracle's by
+    summation rounding only."""
+    announce("rebuild, sparse DEM grid")
+    nc = 24
+    m, x, v = tm.generate_granular_gas(nc, vmax=3.0)
+    L = nc * 1.6796
+    aabb = np.array([0.0, L] * 3)
+    sim = tm.Simulation(m, x, v, aabb, 1.3, dem_radius=0.5)
+    sim.copy_to_accelerator()
+    orc = po.OracleSim(m, x, v, aabb, 1.3, threads=4)
+    sim.setup(True, 1.0, 0.3)
+    orc.setup(True, po.HALF_GHOST_FULL, 1.3)
+    assert sim.grid_info()["ncells"] > 16384
+    sim.dem(True, 1.0)
+    orc.dem(True, 1.0)
+    sim.run_dem(45, 20, 0.001)
+    orc.run_dem(45, 20, 0.001)
+    gt, go = sim.ghost_table(), orc.ghosts()
+    assert sim.nghost == orc.ng
+    for key in ("owner", "img", "src", "flag"):
+        assert np.array_equal(gt[key], go[key]), key
+    _, xg, vg, _ = sim.state()
+    xo, vo, _ = orc.state()
+    assert np.allclose(xg, xo, rtol=1e-12, atol=1e-12) and np.allclose(vg, vo, rtol=1e-12, atol=1e-12)
+
+
+def test_ghosts_outgrow_their_room(tm):
+    """A sheet of three layers that drifts from 4 to 0.5 cells' lengths of the
+    lower x face between two rebuilds: 1.5 ghosts an atom where the volume of
+    the shell made room for 0.5 (and 4,096), so the rebuild in the loop has to
+    grow its arrays and repeat.  Bit for bit the oracle's."""
+    announce("ghosts outgrow their room")
+    L, ny = 48.0, 43
+    a = L / ny
+    g = np.arange(ny) * a
+    z, y, k = np.meshgrid(g, g, np.arange(3), indexing="ij")
+    x = np.stack([4.0 + 1.1 * k.ravel(), y.ravel(), z.ravel()], axis=1)
+    rng = np.random.default_rng(3)
+    v = rng.normal(0.0, 0.3, x.shape)
+    v[:, 0] -= 35.0
+    aabb = np.array([0.0, L] * 3)
+    m = np.ones(len(x))
+    room = 1.25 * len(x) * ((1 + 5.6 / L) ** 3 - 1) + 4096
+    sim, orc = make_pair(aabb, m, x, v)
+    sim.setup(False, RC, SKIN)
+    orc.setup(False, po.HALF_GHOST_FULL, RC + SKIN)
+    assert sim.nghost == orc.ng < room
+    sim.lennard_jones(False, RC)
+    orc.lj(False, RC)
+    sim.run_lj(22, 20, DT)
+    orc.run_lj(22, 20, DT)
+    assert orc.ng > room
+    same_structure(sim, orc)
+    _, xg, vg, fg = sim.state()
+    xo, vo, fo = orc.state()
+    assert np.array_equal(xg, xo) and np.array_equal(vg, vo) and np.array_equal(fg, fo)
