@@ -24,6 +24,7 @@
 // interval the neighbour list and ghost table are fixed, as in the forward.
 #include "tmd_internal.hpp"
 #include "tmd_lj.hpp"
+#include "tmd_pair.hpp"
 
 namespace tmd {
 
@@ -95,7 +96,7 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_lj_adjoint(const double4* _
             // (~1e-14), at the cost of the FP32 path
             double sr2;
             if (PREC == PREC_FP64) {
-                sr2 = 1.0 / s;
+                sr2 = rcp_round(s);
             } else {
                 sr2 = (double)__builtin_amdgcn_rcpf((float)s);
                 sr2 = fma(sr2, fma(-s, sr2, 1.0), sr2);

@@ -215,7 +215,7 @@ struct DEMArgs {
 // (2R + r), since 2R - r in FP32 would lose a small overlap's leading
 // digits.
 //
-// FP64 divides and takes square roots as written.  FP32 works from the
+// FP64 divides with correct rounding and takes square roots as written.  FP32 works from the
 // hardware reciprocal square root and reciprocal (v_rsq_f32, v_rcp_f32, about
 // 1 ulp each): 1/r once, then products, instead of four IEEE divisions and two
 // square roots; the rounding this adds is a few 1e-8 relative, far inside
@@ -228,7 +228,8 @@ __device__ __forceinline__ void dem_pair(const DEMArgs& a, R dx, R dy, R dz, R r
     if constexpr (sizeof(R) == sizeof(double)) {
         const R r = sqrt(rsq);
         delta = d2 - r;  // the reference's 2R - r
-        nx = dx / r; ny = dy / r; nz = dz / r;
+        const double y = rcp_refined(r);  // the three quotients by r share it
+        nx = div_round(dx, r, y); ny = div_round(dy, r, y); nz = div_round(dz, r, y);
     } else {
         const float ir = __builtin_amdgcn_rsqf(rsq);  // contact: rsq in (0, (2R)^2)
         delta = dd * __builtin_amdgcn_rcpf(d2 + rsq * ir);

@@ -8,22 +8,26 @@
 
 namespace tmd {
 
-template <int SHIFT>
-__device__ __forceinline__ double lj_f64(const LJArgs& a, double rsq) {
-    const double sr2 = 1.0 / rsq;
-    const double sr6 = sr2 * sr2 * sr2 * a.sigma6;
-    double f = 48.0 * sr6 * (sr6 - 0.5) * sr2 * a.eps;
-    if (SHIFT) f = f - a.fc - (rsq - a.rc2) * a.dfc;
-    return f;
+// Refined reciprocal of x and the correctly rounded quotient num / x from it:
+// two Newton steps on the hardware's estimate, then the residual's correction
+// (Markstein's final step), as the compiler's division does them, without the
+// scaling and the special-case fix-up around it, which operands of ordinary
+// size do not need (here squared distances, from about 1e-300 to 1e300; zero
+// and infinity give NaN where the division gave infinity and zero, only in
+// terms that the cutoff masks).  1 / x is 7 instructions instead of 11, and
+// quotients by the same x share the first 5.
+__device__ __forceinline__ double rcp_refined(double x) {
+    double y = __builtin_amdgcn_rcp(x);
+    y = fma(y, fma(-x, y, 1.0), y);
+    return fma(y, fma(-x, y, 1.0), y);
 }
-
-template <int SHIFT>
-__device__ __forceinline__ float lj_f32(const LJArgs& a, float rsq) {
-    const float sr2 = __builtin_amdgcn_rcpf(rsq);
-    const float sr6 = sr2 * sr2 * sr2 * a.sigma6f;
-    float f = 48.0f * sr6 * (sr6 - 0.5f) * sr2 * a.epsf;
-    if (SHIFT) f = f - a.fcf - (rsq - a.rc2f) * a.dfcf;
-    return f;
+__device__ __forceinline__ double rcp_round(double x) {
+    const double y = rcp_refined(x);
+    return fma(fma(-x, y, 1.0), y, y);
+}
+__device__ __forceinline__ double div_round(double num, double x, double y) {  // y = rcp_refined(x)
+    const double q = num * y;
+    return fma(fma(-x, q, num), y, q);
 }
 
 // entry u (0..7) of a packed group of 8 u16 list entries
@@ -38,7 +42,7 @@ __device__ __forceinline__ int nb_entry(const int4& q, int u) {
 // is bit-identical either way.
 template <int SHIFT, int UNIT>
 __device__ __forceinline__ double lj_f64u(const LJArgs& a, double rsq) {
-    const double sr2 = 1.0 / rsq;
+    const double sr2 = rcp_round(rsq);
     const double sr6 = UNIT ? sr2 * sr2 * sr2 : sr2 * sr2 * sr2 * a.sigma6;
     double f = UNIT ? 48.0 * sr6 * (sr6 - 0.5) * sr2 : 48.0 * sr6 * (sr6 - 0.5) * sr2 * a.eps;
     if (SHIFT) f = f - a.fc - (rsq - a.rc2) * a.dfc;
@@ -229,7 +233,7 @@ __device__ __forceinline__ void lj_energy_atom(const double4 pi, int cnt, const 
             const double dx = pi.x - xj, dy = pi.y - yj, dz = pi.z - zj;
             const double rsq = dx * dx + dy * dy + dz * dz;
             if (rsq < a.rc2) {
-                const double sr2 = 1.0 / rsq;
+                const double sr2 = rcp_round(rsq);
                 const double sr6 = sr2 * sr2 * sr2 * a.sigma6;
                 double f = 48.0 * sr6 * (sr6 - 0.5) * sr2 * a.eps;
                 double uu = 4.0 * a.eps * sr6 * (sr6 - 1.0);
