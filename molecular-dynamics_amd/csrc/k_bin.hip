@@ -315,31 +315,100 @@ TileGeom make_tile_geom(const Geom& G, int tx, int ty, int tz) {
     return g;
 }
 
+// Near-cubic tile shapes by size: (t, t, t), (t, t, t - 1), (t, t - 1, t - 1).
+struct TileShape {
+    int x, y, z;
+};
+static TileShape tile_shape(int k) {  // k = 0: one cell, 3 (t - 1): t^3
+    const int t = 1 + (k + 2) / 3, r = (k + 2) % 3;
+    return TileShape{t, r >= 1 ? t : t - (t > 1), r == 2 ? t : t - (t > 1)};
+}
+constexpr int kShapes = 3 * (kMaxTile - 1) + 1;
+
+// Tile of the automatic choice for `rho` atoms a cell where the box is filled,
+// a share `fill` of it, and windows of `slot` LDS bytes an atom within `budget`.
+//   1. the largest shape of at most 320 locals (a block of four or five
+//      wavefronts) whose window fits.  LJ liquid (18.5 a cell), us a step at
+//      3x2x2 against 3x3x3 cells: 40^3 FP32-mixed 54 against 57, 32^3 FP64 41
+//      against 54; from 900 cubes on the cubes are ahead (choose_tiles).  DEM
+//      gas (1.85 a cell where it is filled), 6x5x5 against 6x6x6: 64^3 51.4
+//      against 52.9;
+//   2. one size down where that leaves at least 160 locals and there are fewer
+//      than 1,024 tiles (DEM 48^3, 5x5x4: 26.9 against 28.8 us; the LJ liquid's
+//      next shape would have 148: 28^3 20.5 against 18.6 us);
+//   3. smaller still until 200 tiles hold atoms, not below two cells: a pass
+//      over fewer tiles than CUs leaves CUs idle and lasts as long as its
+//      fullest block (10^3 FP64: 27 tiles of 3x3x3 24.7 us, 196 of 2x1x1 16.6;
+//      DEM 17^3: 64 tiles of 6x6x6 17.7 us a step, 512 of 3x3x3 14.3).
+static TileShape pick_tile(const Geom& G, double rho, double fill, int slot, int budget) {
+    rho = std::max(rho, 1e-3);
+    auto cells = [](const TileShape& t) { return (double)t.x * t.y * t.z; };
+    auto tiles = [&](const TileShape& t) {
+        const TileGeom g = make_tile_geom(G, t.x, t.y, t.z);
+        return (double)g.ntx * g.nty * g.ntz * fill;
+    };
+    int k = kShapes - 1;
+    auto fits = [&](const TileShape& t) {
+        return cells(t) * rho <= 320.0 && (t.x + 2.0) * (t.y + 2.0) * (t.z + 2.0) * rho * slot <= 0.95 * budget;
+    };
+    while (k > 0 && !fits(tile_shape(k))) --k;
+    if (k > 0 && tiles(tile_shape(k)) < 1024.0 && cells(tile_shape(k - 1)) * rho >= 160.0) --k;
+    while (k > 1 && tiles(tile_shape(k)) < 200.0) --k;
+    return tile_shape(k);
+}
+
+// A dense box of this many cubes of about 480 locals keeps them: from there
+// the smaller share of window atoms a local (4.6 against 6.7 in the LJ liquid)
+// counts for more than full CUs.  us a step at 3x3x3 against 3x2x2: 48^3
+// (1,000 cubes) FP32-mixed 76 against 78, half lists 87 against 91; 80^3 246
+// against 250, half lists 307 against 323; 40^3 (729) 57 against 54.
+constexpr int kManyTiles = 900;
+
 static void choose_tiles(Sim& s) {
     int t[3] = {s.tile_req[0], s.tile_req[1], s.tile_req[2]};
     if (t[0] <= 0 || t[1] <= 0 || t[2] <= 0) {
-        if (s.tile_auto <= 0) s.tile_auto = auto_tile_edge(s.g, s.n);
-        t[0] = t[1] = t[2] = s.tile_auto;
+        if (s.tile_auto[0] <= 0) {
+            double cells = 1.0;
+            for (int d = 0; d < 3; ++d) cells *= std::max((s.g.rank[2 * d + 1] - s.g.rank[2 * d]) / s.g.spacing, 1.0);
+            const double rho = (double)s.n / cells;
+            const int T = auto_tile_edge(s.g, s.n);
+            const TileGeom cube = make_tile_geom(s.g, T, T, T);
+            if (rho >= kDenseCell && cube.ntx * cube.nty * cube.ntz < kManyTiles) {
+                const TileShape p = pick_tile(s.g, rho, 1.0, kStageBytes, kLdsBudget);
+                s.tile_auto[0] = p.x; s.tile_auto[1] = p.y; s.tile_auto[2] = p.z;
+            } else {
+                // many tiles, or sparse: there the mean density may be far from
+                // where the atoms are, and the first window statistics decide
+                // (retune_tiles)
+                s.tile_auto[0] = s.tile_auto[1] = s.tile_auto[2] = T;
+            }
+        }
+        for (int d = 0; d < 3; ++d) t[d] = s.tile_auto[d];
     }
     s.tiles = make_tile_geom(s.g, t[0], t[1], t[2]);
 }
 
-// auto_tile_edge sees only the mean density.  Where atoms crowd into part of
-// the box (the DEM gas fills half of it), the largest window can outgrow the
-// LDS share of the force pass in use (stage_bytes per slot within
+// The automatic choice sees only the mean density.  Where atoms crowd into
+// part of the box (the DEM gas fills half of it), the largest window can
+// outgrow the LDS share of the force pass in use (stage_bytes per slot within
 // stage_budget per block); the pass then reads such windows from global
 // memory.  From the peak window density of the current tiles this picks the
-// largest edge whose window fits, for the next binning.  The edge only
-// shrinks, and the tiles do not change the results (list order follows the
-// cells, not the tiles).
-void retune_tile_edge(Sim& s) {
+// tile for the next binning: once when the DEM step loop's sizes come into
+// force, and whenever a window overflows.  Tiles only shrink, and they do not
+// change the results (list order follows the cells, not the tiles).
+void retune_tiles(Sim& s) {
     if (s.tile_req[0] > 0 && s.tile_req[1] > 0 && s.tile_req[2] > 0) return;  // explicit tiles
-    const int T = s.tiles.tx;
-    if (T <= 1 || (double)(s.max_window + 1) * s.stage_bytes <= (double)s.stage_budget) return;
-    const double peak = (s.max_window + 1) / ((T + 2.0) * (T + 2.0) * (T + 2.0));
-    int t = T - 1;
-    while (t > 1 && (t + 2.0) * (t + 2.0) * (t + 2.0) * peak * s.stage_bytes > (double)s.stage_budget) --t;
-    s.tile_auto = std::min(t, s.tile_auto > 0 ? s.tile_auto : t);
+    const TileGeom& T = s.tiles;
+    const bool over = (double)(s.max_window + 1) * s.stage_bytes > (double)s.stage_budget;
+    const bool first = s.stage_bytes == kDemStageBytes && !s.tile_tuned;
+    if ((!over && !first) || s.max_window <= 0) return;
+    s.tile_tuned = 1;
+    const double peak = (s.max_window + 1) / ((T.tx + 2.0) * (T.ty + 2.0) * (T.tz + 2.0));
+    double cells = 1.0;
+    for (int d = 0; d < 3; ++d) cells *= std::max(s.g.len[d] / s.g.spacing, 1.0);
+    TileShape p = pick_tile(s.g, peak, std::min(1.0, s.n / (peak * cells)), s.stage_bytes, s.stage_budget);
+    if ((long long)p.x * p.y * p.z > (long long)T.tx * T.ty * T.tz) p = TileShape{T.tx, T.ty, T.tz};
+    s.tile_auto[0] = p.x; s.tile_auto[1] = p.y; s.tile_auto[2] = p.z;
 }
 
 BinArgs bin_args(const Sim& s) {

@@ -135,7 +135,7 @@ void apply_window_stats(Sim& s, const int* st) {
     s.nbinned = st[CT_BINNED];
     s.max_window = st[CT_MAXWIN];
     s.tile_threads = tile_block_threads(s.tile_threads_req, st[CT_MAXLOC]);
-    retune_tile_edge(s);
+    retune_tiles(s);
     if (s.max_window > kWinMax) {
         char msg[200];
         snprintf(msg, sizeof msg, "a tile neighbourhood holds %d atoms, beyond the 16-bit window range (%d)", s.max_window,

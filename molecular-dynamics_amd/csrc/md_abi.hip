@@ -664,7 +664,8 @@ void md_deallocate_grid() {
     }
     s.windows_pending = 0;
     s.max_window = 0;
-    s.tile_auto = 0;
+    s.tile_auto[0] = s.tile_auto[1] = s.tile_auto[2] = 0;
+    s.tile_tuned = 0;
     s.stage_bytes = kPosStageBytes;
     s.stage_budget = kLdsBudget;
     s.n = s.ng = 0;
@@ -889,7 +890,8 @@ void tmd_set_tile(int tx, int ty, int tz) {
     s.tile_req[0] = tx;
     s.tile_req[1] = ty;
     s.tile_req[2] = tz;
-    s.tile_auto = 0;
+    s.tile_auto[0] = s.tile_auto[1] = s.tile_auto[2] = 0;
+    s.tile_tuned = 0;
     s.windows_valid = 0;
     s.nb_valid = 0;
 }
@@ -1113,7 +1115,7 @@ static int run_loop(int steps, int reneigh_every, double dt, bool half, double c
         // next rebuild on.
         s.stage_bytes = kDemStageBytes;
         s.stage_budget = kDemLdsShare;
-        retune_tile_edge(s);
+        retune_tiles(s);
         if (steps > 0) initial_integration(s, dt);
         for (int j = 0; j < steps && !has_error(); ++j) {
             hipEvent_t ev = nullptr;

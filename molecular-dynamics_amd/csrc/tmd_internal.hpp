@@ -114,7 +114,8 @@ struct Sim {
     int max_window = 0; // largest tile window (atoms)
     TileGeom tiles{};   // tile decomposition of the cell grid
     int tile_req[3] = {0, 0, 0};  // requested cells per tile (0: automatic)
-    int tile_auto = 0;            // automatic cells per tile edge in effect (0: chosen at the next binning)
+    int tile_auto[3] = {0, 0, 0};  // automatic cells per tile in effect (0: chosen at the next binning)
+    int tile_tuned = 0;            // they were chosen for the DEM step loop's window sizes (retune_tiles)
     int stage_bytes = kPosStageBytes;  // LDS bytes per window slot of the force pass in use (LJ: positions)
     int stage_budget = kLdsBudget;  // LDS bytes per block that pass should stay within
     int tile_threads = kTileThreads;  // threads per tile block in use (multiple of 64, <= kMaxTileThreads)
@@ -245,7 +246,7 @@ void bin_particles(Sim& s);
 void bin_finish(Sim& s, int nq, bool with_ghosts);  // everything of a binning behind its histogram of nq source slots
 void sort_locals(Sim& s);  // PBC wrap + renumber the locals in cell order
 int auto_tile_edge(const Geom& G, int n);  // cells per tile edge for ~480 locals per tile
-void retune_tile_edge(Sim& s);  // automatic tiles: a smaller edge at the next binning when windows overflow
+void retune_tiles(Sim& s);  // automatic tiles from the window statistics, for the next binning
 TileGeom make_tile_geom(const Geom& G, int tx, int ty, int tz);
 
 // tile windows (after binning), position mirror, neighbour lists

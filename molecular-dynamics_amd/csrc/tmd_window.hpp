@@ -27,6 +27,7 @@ constexpr int kMaxTileThreads = 1024;  // launch bound of the single-box tile ke
 constexpr int kAutoTileThreads = 768;   // largest automatic block (two blocks per CU at <= 80 VGPRs)
 constexpr int kMaxTile = 8;        // cells per tile dimension, at most
 constexpr int kMaxSeg = (kMaxTile + 2) * (kMaxTile + 2);
+constexpr double kDenseCell = 4.0;  // atoms a cell from which the mean density is taken for the local one
 constexpr int kWinMax = 65535;     // window offsets are 16-bit
 // dynamic LDS per block: two blocks per 160 KiB CU, with 1 KiB left for each
 // block's static LDS (window rows, reductions)
