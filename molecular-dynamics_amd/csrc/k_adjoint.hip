@@ -36,165 +36,334 @@ struct AdjCoef {
     int loss_terms;  // 0 at x_0 (the loss starts at t = 1)
 };
 
+// A local's ghosts in the ghost index: mirror index of each and, when asked,
+// its image shift.
+struct GhostIndex {
+    const int* w;  // per work slot: first entry * 32 + number
+    const int* k;  // per entry: mirror index (-1: outside the grid)
+    const int* c;  // per entry: image code
+    double L0, L1, L2;
+};
+template <class F>
+__device__ __forceinline__ void each_ghost(const GhostIndex& g, int w, F&& f) {
+    const int pk = g.w[w];
+    for (int e = pk >> 5, e1 = e + (pk & 31); e < e1; ++e) {
+        const int kg = g.k[e];
+        if (kg >= 0) f(e, kg);
+    }
+}
+__device__ __forceinline__ double4 ghost_image(const double4& x, const GhostIndex& g, int e) {
+    int ix, iy, iz;
+    img_decode(g.c[e], ix, iy, iz);
+    return make_double4(x.x + g.L0 * (double)ix, x.y + g.L1 * (double)iy, x.z + g.L2 * (double)iz, 0.0);
+}
+
+// One step of a trajectory on the cell-ordered mirrors, one launch: force at
+// x_t, final kick, energy, virial and kinetic sums, and the next step's kick
+// and drift, locals and their ghosts, into the next mirror.  The arithmetic
+// and its order are those of the separate passes (force, integration, ghost
+// refresh); the energy pass, the kinetic pass, their reductions, the ghost
+// pass and the copies of states that came with them (about 60 of 75 us a
+// step at 16,384 atoms) are gone.
+struct TrajStep {
+    Mir vel;               // velocities before the final kick in, after this pass out
+    double hfin, hdt, dt;  // final kick (0: the trajectory's first force), next kick and drift
+    int adv;               // also the next kick and drift
+    Mir xnext;             // mirror of x_{t+1}
+    Mir vt;                // v_t in mirror order (p null: not kept)
+    double4 *ckx, *ckv;    // checkpoint of x_t, v_t in atom order (null: none)
+    GhostIndex gh;
+    double* acc;           // per tile: PE, W, sum v^2, added to
+};
+
+template <int PREC, int SHIFT, int UNIT, bool ENERGY>
+__global__ void __launch_bounds__(kMaxTileThreads) k_traj_step(const CMir spos, const int* __restrict__ start,
+                                                            const int* __restrict__ work, const int* __restrict__ wk,
+                                                            const int* __restrict__ tile_start, const int* __restrict__ nbc,
+                                                            const nb_t* __restrict__ nbl, LJArgs a, TrajStep t) {
+    extern __shared__ double dyn[];
+    const WinStage sp = win_stage(dyn, a.wcap);
+    const int tile = xcd_block(blockIdx.x, gridDim.x);
+    const int w0 = tile_start[tile], nloc = tile_start[tile + 1] - w0;
+    if (nloc == 0) return;
+    __shared__ TileWin W;
+    tile_window(tile, start, a.g, W);
+    const bool staged = stage_window(W, a.wcap, spos, nullptr, sp);
+    PairEnergy en;
+    double v2 = 0.0;
+    for (int at = threadIdx.x; at < nloc; at += blockDim.x) {
+        const int w = w0 + at;
+        const int kw = wk[w];
+        const double4 pi = spos[kw];
+        const int cnt = nbc[w];
+        const int4* lp = reinterpret_cast<const int4*>(nbl + (size_t)(w >> 6) * (size_t)a.cap * 64) + (w & 63);
+        const double4 f = staged ? lj_full_atom<PREC, SHIFT, UNIT, true, false, ENERGY>(pi, cnt, lp, sp, spos, W, a, 0, nullptr, &en)
+                                 : lj_full_atom<PREC, SHIFT, UNIT, false, false, ENERGY>(pi, cnt, lp, sp, spos, W, a, 0, nullptr, &en);
+        double4 v = t.vel[kw];
+        v.x = v.x + f.x * t.hfin;
+        v.y = v.y + f.y * t.hfin;
+        v.z = v.z + f.z * t.hfin;
+        if (ENERGY) v2 += v.x * v.x + v.y * v.y + v.z * v.z;
+        if (t.vt.p) t.vt[kw] = v;
+        if (t.ckx) {
+            const int i = work[w];
+            t.ckx[i] = pi;
+            t.ckv[i] = v;
+        }
+        if (t.adv) {
+            v.x = v.x + f.x * t.hdt;
+            v.y = v.y + f.y * t.hdt;
+            v.z = v.z + f.z * t.hdt;
+            double4 x = pi;
+            x.x = x.x + v.x * t.dt;
+            x.y = x.y + v.y * t.dt;
+            x.z = x.z + v.z * t.dt;
+            t.xnext[kw] = x;
+            each_ghost(t.gh, w, [&](int e, int kg) { t.xnext[kg] = ghost_image(x, t.gh, e); });
+        }
+        t.vel[kw] = v;
+    }
+    if (ENERGY) {
+        const double bpe = block_sum_double_any(en.pe);
+        const double bvir = block_sum_double_any(en.vir);
+        const double bv2 = block_sum_double_any(v2);
+        if (threadIdx.x == 0) {
+            t.acc[3 * tile + 0] += bpe;
+            t.acc[3 * tile + 1] += bvir;
+            t.acc[3 * tile + 2] += bv2;
+        }
+    }
+}
+
+// One reverse step, one launch: (c) at x_t, then (b), (a) and the (e), (d) of
+// step t - 1, which involve the lane's own atom only.  Adjoints live in
+// mirror order inside an interval (ghosts carry their owners' Fbar), so the
+// window's Fbar is staged beside its positions (48 B a slot) and an entry
+// costs six LDS reads; it was an index, an owner and a 32-byte gather from
+// global memory, behind 2-byte list loads.
+//
+// All pair quantities are linear in p = sigma^6 s^-4, q = sigma^12 s^-7,
+// sr6, sr12 and the truncation's 1, s, s^2, so the parameter gradients
+// accumulate those sums (9 operations an entry) and are combined once per
+// lane; an entry is about 60 FP64 operations where it was about 110, without
+// a branch: beyond the cutoff sr2 and the constants' factor `in` are zero.
+//
+// FP64 takes 1/s correctly rounded and s as the forward pass forms it;
+// FP32-mixed skips the last rounding step and forms s with FMAs (a few 1e-16).
+// 16,384 atoms in FP64: 26 us a step by events, where the pair kernel took 86 and
+// five more passes around it 5 us each.
+struct AdjStep {
+    Mir xb, vb;                   // the locals' xbar, vbar (mirror order, own entry read and written)
+    CMir vprev;                   // v_{t-1} (mirror order)
+    Mir fnext;                    // Fbar for step t - 1, locals and ghosts
+    double4 *xbar, *vbar, *fbar;  // atom order, at the interval's first step
+    GhostIndex gh;
+    double cv, h, dt;
+    int post, pre, end;           // (b) and (a); (e) and (d) of t - 1; last of the interval
+    double* acc;                  // per tile: g_eps, g_sig, added to
+};
+
 template <int PREC, int SHIFT>
-__global__ void __launch_bounds__(kMaxTileThreads) k_lj_adjoint(const double4* __restrict__ pos, const CMir spos,
-                                                             const int* __restrict__ start, const int* __restrict__ parts,
-                                                             const int* __restrict__ work, const int* __restrict__ tile_start,
-                                                             const int* __restrict__ nbc, const nb_t* __restrict__ nbl,
-                                                             const int* __restrict__ g_owner, const double4* __restrict__ fbar,
-                                                             LJArgs a, AdjCoef c, double4* __restrict__ xbar,
-                                                             double* __restrict__ partials) {
+__global__ void __launch_bounds__(kMaxTileThreads) k_lj_adjoint(const CMir spos, const CMir fbm, const int* __restrict__ start,
+                                                             const int* __restrict__ work, const int* __restrict__ wk,
+                                                             const int* __restrict__ tile_start, const int* __restrict__ nbc,
+                                                             const nb_t* __restrict__ nbl, LJArgs a, AdjCoef c, AdjStep t) {
     extern __shared__ double dyn[];
     const int tile = xcd_block(blockIdx.x, gridDim.x);
     const int w0 = tile_start[tile], nloc = tile_start[tile + 1] - w0;
-    if (nloc == 0) {
-        if (threadIdx.x == 0) {
-            partials[2 * tile + 0] = 0.0;
-            partials[2 * tile + 1] = 0.0;
-        }
-        return;
-    }
+    if (nloc == 0) return;
     __shared__ TileWin W;
     tile_window(tile, start, a.g, W);
     double* sx = dyn;
-    double* sy = dyn + a.wcap;
-    double* sz = dyn + 2 * a.wcap;
-    int* sj = reinterpret_cast<int*>(dyn + 3 * a.wcap);
-    const bool staged = stage_tile(W, a.wcap, spos, parts, sx, sy, sz, sj);
-    const double inv_eps = 1.0 / a.eps, inv_sig = 1.0 / a.sigma;
+    double* sf = dyn + 3 * a.wcap;
+    const int S = win_size(W);
+    const bool staged = S + 1 <= a.wcap;
+    if (staged) {
+        double4 p[kStageInFlight], q[kStageInFlight];
+        stage_rows(W, [&](int k, int u) { p[u] = spos[k]; q[u] = fbm[k]; },
+                   [&](int j, int u) {
+                       sx[3 * j] = p[u].x; sx[3 * j + 1] = p[u].y; sx[3 * j + 2] = p[u].z;
+                       sf[3 * j] = q[u].x; sf[3 * j + 1] = q[u].y; sf[3 * j + 2] = q[u].z;
+                   });
+        if (threadIdx.x < 3) {
+            sx[3 * S + threadIdx.x] = kFarPos;  // the sentinel slot that pads list groups
+            sf[3 * S + threadIdx.x] = 0.0;
+        }
+    }
+    __syncthreads();
+    const double e48 = 48.0 * a.eps, e24 = 24.0 * a.eps;
+    const double lU = c.loss_terms ? c.cU : 0.0, lW = c.loss_terms ? 2.0 * c.cW : 0.0;
     double g_eps = 0.0, g_sig = 0.0;
     // STAGED as a compile-time constant: LDS reads, not generic-pointer loads
     auto atoms = [&](auto staged_c) {
-    constexpr bool STAGED = decltype(staged_c)::value;
-    for (int at = threadIdx.x; at < nloc; at += blockDim.x) {
-        const int w = w0 + at;
-        const int i = work[w];
-        const double4 pi = pos[i];
-        const double4 fbi = fbar[i];
-        const int cnt = nbc[w];
-        double ax = 0.0, ay = 0.0, az = 0.0;
-        for (int k = 0; k < cnt; ++k) {
-            const int t = nbl[nb16_slot(w, k, a.cap)];
-            int j;
-            double xj, yj, zj;
-            if (STAGED) {
-                j = sj[t];
-                xj = sx[t]; yj = sy[t]; zj = sz[t];
-            } else {
-                const int kk = win_index(t, W);
-                j = parts[kk];
-                const double4 p = spos[kk];
-                xj = p.x; yj = p.y; zj = p.z;
+        constexpr bool STAGED = decltype(staged_c)::value;
+        for (int at = threadIdx.x; at < nloc; at += blockDim.x) {
+            const int w = w0 + at;
+            const int kw = wk[w];
+            const double4 pi = spos[kw];
+            const double4 fbi = fbm[kw];
+            const int cnt = nbc[w];
+            const int4* lp = reinterpret_cast<const int4*>(nbl + (size_t)(w >> 6) * (size_t)a.cap * 64) + (w & 63);
+            double ax = 0.0, ay = 0.0, az = 0.0;
+            double Prf = 0.0, Qrf = 0.0, Rrf = 0.0, Srf = 0.0;  // sums of p rf, q rf, rf, s rf
+            double S6 = 0.0, S12 = 0.0, N0 = 0.0, S1 = 0.0, S2 = 0.0;  // of sr6, sr12, 1, s, s^2
+            const int ng = (cnt + 7) >> 3;
+            int4 nx = ld_stream(lp);  // group 0 of the column always exists (capacity >= 8)
+            for (int gi = 0; gi < ng; ++gi) {
+                const int4 e = nx;
+                nx = ld_stream(lp + (size_t)min(gi + 1, ng - 1) * 64);
+                const int rem = cnt - gi * 8;
+#pragma unroll
+                for (int hb = 0; hb < 8; hb += 2) {
+                    if (hb >= rem) break;
+#pragma unroll
+                    for (int u = hb; u < hb + 2; ++u) {
+                        const bool valid = STAGED || u < rem;
+                        double xj, yj, zj, fxj, fyj, fzj;
+                        if (STAGED) {
+                            const int j = nb_entry(e, u);
+                            xj = sx[3 * j]; yj = sx[3 * j + 1]; zj = sx[3 * j + 2];
+                            fxj = sf[3 * j]; fyj = sf[3 * j + 1]; fzj = sf[3 * j + 2];
+                        } else {
+                            const int kk = win_index(valid ? nb_entry(e, u) : 0, W);
+                            const double4 p = spos[kk], q = fbm[kk];
+                            xj = p.x; yj = p.y; zj = p.z;
+                            fxj = q.x; fyj = q.y; fzj = q.z;
+                        }
+                        const double rx = pi.x - xj, ry = pi.y - yj, rz = pi.z - zj;
+                        const double s = PREC == PREC_FP64 ? rx * rx + ry * ry + rz * rz : fma(rx, rx, fma(ry, ry, rz * rz));
+                        const bool ok = valid && s < a.rc2;
+                        const double r2 = PREC == PREC_FP64 ? rcp_round(s) : rcp_refined(s);
+                        const double sr2 = ok ? r2 : 0.0;
+                        const double in = ok ? 1.0 : 0.0;
+                        const double sv = ok ? s : 0.0;
+                        const double sr6 = sr2 * sr2 * sr2 * a.sigma6;
+                        const double p = sr6 * sr2, q = sr6 * p;
+                        double f = fma(e48, q, -e24 * p);                      // f(s)
+                        const double sdf0 = e24 * fma(-14.0, q, 4.0 * p);      // s f'(s)
+                        double df = sdf0 * sr2, sdf = sdf0;                    // f'(s), s f'(s)
+                        if (SHIFT) {
+                            f = fma(-a.dfc, fma(-a.rc2, in, sv), fma(-a.fc, in, f));
+                            df = fma(-a.dfc, in, df);
+                            sdf = fma(-a.dfc, sv, sdf);
+                        }
+                        // J_F^T Fbar, and the loss: dPE/dx_i = -sum f r ; dW/dx_i = sum 2 (f + s f') r
+                        const double dx = fbi.x - fxj, dy = fbi.y - fyj, dz = fbi.z - fzj;
+                        const double rd = fma(rx, dx, fma(ry, dy, rz * dz));
+                        const double cr = fma(2.0 * df, rd, fma(lW, f + sdf, -lU * f));
+                        ax = fma(f, dx, fma(cr, rx, ax));
+                        ay = fma(f, dy, fma(cr, ry, ay));
+                        az = fma(f, dz, fma(cr, rz, az));
+                        // parameters: Fbar_i . dF_i/dtheta over ordered pairs; the loss halves
+                        const double rf = fma(rx, fbi.x, fma(ry, fbi.y, rz * fbi.z));
+                        Prf = fma(p, rf, Prf);
+                        Qrf = fma(q, rf, Qrf);
+                        S6 += sr6;
+                        S12 = fma(sr6, sr6, S12);
+                        if (SHIFT) {
+                            Rrf = fma(in, rf, Rrf);
+                            Srf = fma(sv, rf, Srf);
+                            N0 += in;
+                            S1 += sv;
+                            S2 = fma(sv, sv, S2);
+                        }
+                    }
+                }
             }
-            const double rx = pi.x - xj, ry = pi.y - yj, rz = pi.z - zj;
-            const double s = rx * rx + ry * ry + rz * rz;
-            if (!(s < a.rc2)) continue;
-            // f(s), f'(s), u(s), d f/d sigma, d u/d sigma in FP64.  FP64 takes
-            // 1/s from the IEEE division (the forward kernel's rounding);
-            // FP32-mixed from the FP32 reciprocal refined by one FP64 Newton
-            // step, whose relative error is about the square of the FP32 one
-            // (~1e-14), at the cost of the FP32 path
-            double sr2;
-            if (PREC == PREC_FP64) {
-                sr2 = rcp_round(s);
-            } else {
-                sr2 = (double)__builtin_amdgcn_rcpf((float)s);
-                sr2 = fma(sr2, fma(-s, sr2, 1.0), sr2);
-            }
-            double f, df, u, dfds, duds;
-            {
-                const double sr6 = sr2 * sr2 * sr2 * a.sigma6;
-                f = 48.0 * a.eps * sr6 * (sr6 - 0.5) * sr2;
-                df = 24.0 * a.eps * sr2 * sr2 * sr6 * (4.0 - 14.0 * sr6);
-                u = 4.0 * a.eps * sr6 * (sr6 - 1.0);
-                dfds = 144.0 * a.eps * inv_sig * sr2 * sr6 * (4.0 * sr6 - 1.0);
-                duds = 24.0 * a.eps * inv_sig * sr6 * (2.0 * sr6 - 1.0);
-            }
+            // sums of f rf, u, s f; and the same of their sigma-derivatives
+            double Frf = e48 * Qrf - e24 * Prf, U = 4.0 * a.eps * (S12 - S6), SF = e48 * S12 - e24 * S6;
+            const double k144 = 144.0 * a.eps / a.sigma, k24 = 24.0 * a.eps / a.sigma;
+            double Drf = k144 * (4.0 * Qrf - Prf), DU = k24 * (2.0 * S12 - S6), DSF = k144 * (4.0 * S12 - S6);
             if (SHIFT) {
-                const double ds = s - a.rc2;
-                f = f - a.fc - ds * a.dfc;
-                df = df - a.dfc;
-                u = u - a.uc + ds * (0.5 * a.fc) + ds * ds * (0.25 * a.dfc);
-                dfds = dfds - c.dfc_ds - ds * c.ddfc_ds;
-                duds = duds - c.duc_ds + ds * (0.5 * c.dfc_ds) + ds * ds * (0.25 * c.ddfc_ds);
+                const double Trf = Srf - a.rc2 * Rrf;                               // sum ds rf
+                const double T1 = S1 - a.rc2 * N0;                                  // sum ds
+                const double T2 = S2 - 2.0 * a.rc2 * S1 + a.rc2 * a.rc2 * N0;       // sum ds^2
+                const double TS = S2 - a.rc2 * S1;                                  // sum s ds
+                Frf = Frf - a.fc * Rrf - a.dfc * Trf;
+                SF = SF - a.fc * S1 - a.dfc * TS;
+                U = U - a.uc * N0 + 0.5 * a.fc * T1 + 0.25 * a.dfc * T2;
+                Drf = Drf - c.dfc_ds * Rrf - c.ddfc_ds * Trf;
+                DSF = DSF - c.dfc_ds * S1 - c.ddfc_ds * TS;
+                DU = DU - c.duc_ds * N0 + 0.5 * c.dfc_ds * T1 + 0.25 * c.ddfc_ds * T2;
             }
-            // J_F^T Fbar
-            const int o = j < a.n ? j : g_owner[j - a.n];
-            const double4 fbj = fbar[o];
-            const double dx = fbi.x - fbj.x, dy = fbi.y - fbj.y, dz = fbi.z - fbj.z;
-            const double rd = rx * dx + ry * dy + rz * dz;
-            double cr = 2.0 * df * rd;  // coefficient of r
-            ax += f * dx;
-            ay += f * dy;
-            az += f * dz;
-            // loss: dPE/dx_i = -sum f r ; dW/dx_i = sum 2 (f + s f') r
-            if (c.loss_terms) cr += -c.cU * f + c.cW * 2.0 * (f + s * df);
-            ax += cr * rx;
-            ay += cr * ry;
-            az += cr * rz;
-            // parameters: Fbar_i . dF_i/dtheta over ordered pairs; loss halves
-            const double rf = rx * fbi.x + ry * fbi.y + rz * fbi.z;
-            double ge = f * inv_eps * rf;
-            double gs = dfds * rf;
-            if (c.loss_terms) {
-                ge += 0.5 * (c.cU * u * inv_eps + c.cW * s * f * inv_eps);
-                gs += 0.5 * (c.cU * duds + c.cW * s * dfds);
+            const double hW = 0.25 * lW, hU = 0.5 * lU;  // half of cW and cU
+            g_eps += (Frf + (hU * U + hW * SF)) / a.eps;
+            g_sig += Drf + (hU * DU + hW * DSF);
+            double4 xb = t.xb[kw], vb = t.vb[kw];
+            xb.x += ax; xb.y += ay; xb.z += az;
+            double4 fb = make_double4(0.0, 0.0, 0.0, 0.0);
+            if (t.post) {
+                // (c) Fbar = 0, (b) vbar += dt xbar, (a) Fbar = h vbar
+                vb.x += t.dt * xb.x; vb.y += t.dt * xb.y; vb.z += t.dt * xb.z;
+                fb = make_double4(t.h * vb.x, t.h * vb.y, t.h * vb.z, 0.0);
             }
-            g_eps += ge;
-            g_sig += gs;
+            if (t.end) {
+                const int i = work[w];
+                t.xbar[i] = xb;
+                t.vbar[i] = vb;
+                t.fbar[i] = fb;
+                continue;
+            }
+            if (t.pre) {
+                // (e) vbar += cv v_{t-1}, (d) Fbar += h vbar
+                const double4 v = t.vprev[kw];
+                vb.x += t.cv * v.x; vb.y += t.cv * v.y; vb.z += t.cv * v.z;
+                fb.x += t.h * vb.x; fb.y += t.h * vb.y; fb.z += t.h * vb.z;
+            }
+            t.xb[kw] = xb;
+            t.vb[kw] = vb;
+            t.fnext[kw] = fb;
+            each_ghost(t.gh, w, [&](int, int kg) { t.fnext[kg] = fb; });
         }
-        double4 xb = xbar[i];
-        xb.x += ax;
-        xb.y += ay;
-        xb.z += az;
-        xbar[i] = xb;
-    }
     };
     if (staged) atoms(std::true_type{});
     else atoms(std::false_type{});
     const double be = block_sum_double_any(g_eps);
     const double bs = block_sum_double_any(g_sig);
     if (threadIdx.x == 0) {
-        partials[2 * tile + 0] = be;
-        partials[2 * tile + 1] = bs;
+        t.acc[2 * tile + 0] += be;
+        t.acc[2 * tile + 1] += bs;
     }
 }
 
-// acc[c] += sum_b partials[width * b + c] (one block, fixed order)
-__global__ void __launch_bounds__(256) k_accumulate(const double* __restrict__ partials, int nblocks, int width,
+// acc[c] += sum_b partials[width * b + c] (one block, fixed order), and the
+// partials start again from zero
+__global__ void __launch_bounds__(256) k_accumulate(double* __restrict__ partials, int nblocks, int width,
                                                     double* __restrict__ acc) {
     for (int c = 0; c < width; ++c) {
         double v = 0.0;
-        for (int b = threadIdx.x; b < nblocks; b += 256) v += partials[(size_t)width * b + c];
+        for (int b = threadIdx.x; b < nblocks; b += 256) {
+            v += partials[(size_t)width * b + c];
+            partials[(size_t)width * b + c] = 0.0;
+        }
         const double t = block_sum_double<256>(v);
         if (threadIdx.x == 0) acc[c] += t;
     }
 }
 
-// (e) + (d): vbar += cv * v_t ; Fbar += h vbar
-__global__ void k_adj_pre(const double4* __restrict__ vel, int n, double cv, double h, double4* __restrict__ vbar,
-                          double4* __restrict__ fbar) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double4 vb = vbar[i];
-    const double4 v = vel[i];
-    vb.x += cv * v.x; vb.y += cv * v.y; vb.z += cv * v.z;
-    vbar[i] = vb;
-    double4 fb = fbar[i];
-    fb.x += h * vb.x; fb.y += h * vb.y; fb.z += h * vb.z;
-    fbar[i] = fb;
+__global__ void k_fill_double(double* __restrict__ p, long long n) {
+    const long long stride = (long long)gridDim.x * blockDim.x;
+    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = 0.0;
 }
 
-// (c) Fbar = 0, (b) vbar += dt xbar, (a) Fbar = h vbar
-__global__ void k_adj_post(const double4* __restrict__ xbar, int n, double dt, double h, double4* __restrict__ vbar,
-                           double4* __restrict__ fbar) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double4 vb = vbar[i];
-    const double4 xb = xbar[i];
-    vb.x += dt * xb.x; vb.y += dt * xb.y; vb.z += dt * xb.z;
-    vbar[i] = vb;
-    fbar[i] = make_double4(h * vb.x, h * vb.y, h * vb.z, 0.0);
+// An interval's adjoints from atom order into its mirrors, with (e) and (d)
+// of its last state: vbar += cv v_t ; Fbar += h vbar
+__global__ void k_adj_begin(const int* __restrict__ work, const int* __restrict__ wk, int n, const double4* __restrict__ xbar,
+                            const double4* __restrict__ vbar, const double4* __restrict__ fbar, const CMir vt, double cv, double h,
+                            int pre, const Mir xb, const Mir vb, const Mir fb, GhostIndex gh) {
+    const int w = blockIdx.x * blockDim.x + threadIdx.x;
+    if (w >= n) return;
+    const int i = work[w], kw = wk[w];
+    double4 b = vbar[i], f = fbar[i];
+    if (pre) {
+        const double4 v = vt[kw];
+        b.x += cv * v.x; b.y += cv * v.y; b.z += cv * v.z;
+        f.x += h * b.x; f.y += h * b.y; f.z += h * b.z;
+    }
+    xb[kw] = xbar[i];
+    vb[kw] = b;
+    fb[kw] = f;
+    each_ghost(gh, w, [&](int, int kg) { fb[kg] = f; });
 }
 
 // ---------------------------------------------------------------------------
@@ -204,61 +373,54 @@ static void copy_state(Sim& s, double4* xd, double4* vd, const double4* xs, cons
     TMD_HIP(hipMemcpyAsync(vd, vs, bytes, hipMemcpyDeviceToDevice, s.stream));
 }
 
-static void snapshot_to(Sim& s, DevBuf& bx, DevBuf& bv, size_t slot) {
-    copy_state(s, bx.as<double4>() + slot * s.n, bv.as<double4>() + slot * s.n, s.pos.as<double4>(), s.vel.as<double4>());
-}
+// the current state (atom order) kept, and put back
+static void keep_state(Sim& s) { copy_state(s, s.adj_x0.as<double4>(), s.adj_v0.as<double4>(), s.pos.as<double4>(), s.vel.as<double4>()); }
 
 static void restore_from(Sim& s, const DevBuf& bx, const DevBuf& bv, size_t slot) {
     mirror_invalidate(s);
+    s.pos_stale = 0;
+    s.vel_mirrored = 0;
     copy_state(s, s.pos.as<double4>(), s.vel.as<double4>(), bx.as<double4>() + slot * s.n, bv.as<double4>() + slot * s.n);
 }
 
-// ghosts, cells and full list for the current positions (no periodic wrap)
-static void relist(Sim& s, double cutoff) {
-    s.gh_wanted = 0;
-    rebuild_lists(s, false, 0, cutoff);
+// Ghosts, cells and full list: from the mirrors with the periodic wrap, or
+// from atom order without.  The velocities come along into their mirror and
+// the ghost index is made.
+static void relist(Sim& s, bool wrap, double cutoff) {
+    s.gh_wanted = 1;
+    s.vel_mirror_wanted = 1;
+    rebuild_lists(s, wrap, 0, cutoff);
+    s.vel_mirror_wanted = 0;
+    if (!has_error() && !s.gh_valid) set_error(__FILE__, __LINE__, "trajectory: too many ghosts for the ghost index");
 }
 
 static int ntiles_of(const Sim& s) { return s.tiles.ntx * s.tiles.nty * s.tiles.ntz; }
 
-static double* partials(Sim& s, size_t count) {
-    s.adj_part.reserve(sizeof(double) * std::max<size_t>(count, 1), false, s.stream);
+static GhostIndex ghost_index(const Sim& s) {
+    return GhostIndex{s.gh_w.as<int>(), s.gh_k.as<int>(), s.gh_c.as<int>(), s.g.len[0], s.g.len[1], s.g.len[2]};
+}
+
+static void zero(Sim& s, void* p, size_t doubles) {
+    hipLaunchKernelGGL(k_fill_double, dim3(std::min<long long>(div_up((long long)doubles, 1024), 1024)), dim3(256), 0, s.stream,
+                       static_cast<double*>(p), (long long)doubles);
+}
+
+// Per-tile accumulators of `width` sums, kept over an interval (its tiles are
+// fixed), then added to the totals and cleared.
+static double* tile_sums(Sim& s, int width) {
+    const size_t need = (size_t)width * (size_t)std::max(ntiles_of(s), 1);
+    if (sizeof(double) * need > s.adj_part.bytes) {
+        s.adj_part.reserve(sizeof(double) * 2 * need, false, s.stream);
+        if (has_error()) return nullptr;
+        zero(s, s.adj_part.p, 2 * need);
+    }
     return s.adj_part.as<double>();
 }
 
-// acc[0..3] += {PE, W, pairs, sum v^2} of the current state
-static void accumulate_thermo(Sim& s, double rc, double eps, double sigma, double* acc) {
-    const int nt = ntiles_of(s), nkb = div_up(s.n, 256);
-    double* part = partials(s, 3 * (size_t)std::max(nt, nkb));
-    launch_lj_energy(s, rc, eps, sigma, part);
-    hipLaunchKernelGGL(k_accumulate, dim3(1), dim3(256), 0, s.stream, (const double*)part, nt, 3, acc);
-    launch_kinetic(s, part);
-    hipLaunchKernelGGL(k_accumulate, dim3(1), dim3(256), 0, s.stream, (const double*)part, nkb, 1, acc + 3);
-    TMD_HIP(hipGetLastError());
-}
-
-static void launch_lj_adjoint(Sim& s, double rc, double eps, double sigma, const AdjCoef& c, double* theta) {
-    LJArgs a = make_lj_args(s, rc, eps, sigma);
-    if (!s.mirror_fresh) refresh_mirror(s);
-    const int ntiles = ntiles_of(s);
-    const size_t lds = (size_t)a.wcap * kStageBytes;
-    double* part = partials(s, 2 * (size_t)ntiles);
-#define TMD_ADJ(P, SH)                                                                                                  \
-    hipLaunchKernelGGL((k_lj_adjoint<P, SH>), dim3(ntiles), dim3(s.tile_threads), lds, s.stream,                          \
-                       (const double4*)s.pos.as<double4>(), CMir{s.spos.as<double>()},                       \
-                       (const int*)s.cell_start.as<int>(), (const int*)s.cell_parts.as<int>(), (const int*)s.work.as<int>(), \
-                       (const int*)s.tile_start.as<int>(), (const int*)s.nb_count.as<int>(),                            \
-                       (const nb_t*)s.nb_list.as<nb_t>(), (const int*)s.g_owner.as<int>(),                             \
-                       (const double4*)s.adj_fbar.as<double4>(), a, c, s.adj_xbar.as<double4>(), part)
-    // the adjoint kernel's precision: the forward's unless set apart
-    const int prec = s.adj_precision >= 0 ? s.adj_precision : s.precision;
-    if (prec == PREC_FP64) {
-        if (s.lj_shift) TMD_ADJ(PREC_FP64, 1); else TMD_ADJ(PREC_FP64, 0);
-    } else {
-        if (s.lj_shift) TMD_ADJ(PREC_FP32_MIXED, 1); else TMD_ADJ(PREC_FP32_MIXED, 0);
-    }
-#undef TMD_ADJ
-    hipLaunchKernelGGL(k_accumulate, dim3(1), dim3(256), 0, s.stream, (const double*)part, ntiles, 2, theta);
+static void flush_sums(Sim& s, int width, double* acc) {
+    // no pass has summed over these tiles yet (a rebuild at the first step)
+    if (sizeof(double) * (size_t)width * (size_t)ntiles_of(s) > s.adj_part.bytes) return;
+    hipLaunchKernelGGL(k_accumulate, dim3(1), dim3(256), 0, s.stream, s.adj_part.as<double>(), ntiles_of(s), width, acc);
     TMD_HIP(hipGetLastError());
 }
 
@@ -267,35 +429,79 @@ struct TrajSpec {
     double dt, rc, skin, eps, sigma;
 };
 
+// The pass of step t at the positions in the mirror x.
+static void traj_step(Sim& s, const TrajSpec& p, const DevBuf& x, TrajStep t, bool energy) {
+    if (has_error()) return;
+    LJArgs a = make_lj_args(s, p.rc, p.eps, p.sigma);
+    a.wcap = window_cap_pos(s);
+    const size_t lds = (size_t)a.wcap * kPosStageBytes;
+    const int unit = (p.eps == 1.0 && a.sigma6 == 1.0) ? 1 : 0;
+    t.vel = Mir{s.svel.as<double>()};
+    t.hdt = 0.5 * p.dt;
+    t.dt = p.dt;
+    t.gh = ghost_index(s);
+    t.acc = energy ? tile_sums(s, 3) : nullptr;
+    if (has_error()) return;
+    s.last_force_rc = p.rc;
+    hipEvent_t ev = nullptr;
+    s.timer.begin(K_FORCE, s.stream, &ev);
+#define TMD_TS(P, SH, U, E)                                                                                             \
+    hipLaunchKernelGGL((k_traj_step<P, SH, U, E>), dim3(ntiles_of(s)), dim3(s.tile_threads), lds, s.stream,               \
+                       CMir{x.as<double>()}, (const int*)s.cell_start.as<int>(), (const int*)s.work.as<int>(),           \
+                       (const int*)s.work_k.as<int>(), (const int*)s.tile_start.as<int>(),                              \
+                       (const int*)s.nb_count.as<int>(), (const nb_t*)s.nb_list.as<nb_t>(), a, t)
+#define TMD_TS_E(P, SH, U) do { if (energy) TMD_TS(P, SH, U, true); else TMD_TS(P, SH, U, false); } while (0)
+#define TMD_TS_U(P, SH) do { if (unit) TMD_TS_E(P, SH, 1); else TMD_TS_E(P, SH, 0); } while (0)
+#define TMD_TS_S(P) do { if (s.lj_shift) TMD_TS_U(P, 1); else TMD_TS_U(P, 0); } while (0)
+    if (s.precision == PREC_FP64) TMD_TS_S(PREC_FP64);
+    else if (s.precision == PREC_FP32_KAHAN) TMD_TS_S(PREC_FP32_KAHAN);
+    else TMD_TS_S(PREC_FP32_MIXED);
+#undef TMD_TS_S
+#undef TMD_TS_U
+#undef TMD_TS_E
+#undef TMD_TS
+    s.timer.end(K_FORCE, s.stream, ev);
+    TMD_HIP(hipGetLastError());
+}
+
 // Forward trajectory from (adj_x0, adj_v0), reneighbouring every ck steps
 // exactly as the step loop does (wrap, ghosts, cells, list after the
 // position update of steps ck, 2ck, ...).  With checkpoints, slot k holds
-// the state at t = k ck (after that step's wrap).
+// the state at t = k ck (after that step's wrap).  The mirrors alternate as in
+// the step loop; a rebuild goes from mirror to mirror.
 static void forward_traj(Sim& s, const TrajSpec& p, bool store_ckpt, double* ubar, double* pbar) {
     const double cut = p.rc + p.skin;
     double* acc = s.adj_acc.as<double>();
+    zero(s, acc, 4);
     restore_from(s, s.adj_x0, s.adj_v0, 0);
-    relist(s, cut);
-    compute_lj(s, 0, p.rc, p.eps, p.sigma);
-    if (store_ckpt) snapshot_to(s, s.adj_ckx, s.adj_ckv, 0);
-    TMD_HIP(hipMemsetAsync(acc, 0, 4 * sizeof(double), s.stream));
-    for (int t = 1; t <= p.steps && !has_error(); ++t) {
-        initial_integration(s, p.dt);
-        if (t % p.ck == 0) {
-            rebuild_lists(s, true, 0, cut);  // with md_enforce_pbc
-        } else {
-            refresh_ghosts(s);
+    relist(s, false, cut);
+    if (has_error()) return;
+    for (int t = 0; t <= p.steps && !has_error(); ++t) {
+        if (t > 0 && t % p.ck == 0) {
+            flush_sums(s, 3, acc);  // the tiles change
+            relist(s, true, cut);
+            if (has_error()) return;
         }
-        compute_lj(s, 0, p.rc, p.eps, p.sigma, p.dt);  // final kick fused
-        accumulate_thermo(s, p.rc, p.eps, p.sigma, acc);
-        if (store_ckpt && t % p.ck == 0) snapshot_to(s, s.adj_ckx, s.adj_ckv, (size_t)(t / p.ck));
+        TrajStep st{};
+        st.hfin = t > 0 ? 0.5 * p.dt : 0.0;
+        st.adv = t < p.steps;
+        st.xnext = Mir{s.spos2.as<double>()};
+        if (store_ckpt && t % p.ck == 0) {
+            st.ckx = s.adj_ckx.as<double4>() + (size_t)(t / p.ck) * s.n;
+            st.ckv = s.adj_ckv.as<double4>() + (size_t)(t / p.ck) * s.n;
+        }
+        traj_step(s, p, s.spos, st, t > 0);
+        if (st.adv) std::swap(s.spos, s.spos2);
+        s.pos_stale = 1;  // the state lives in the mirrors
+        s.vel_mirrored = 1;
     }
-    double h[4] = {0, 0, 0, 0};
+    flush_sums(s, 3, acc);
+    double h[3] = {0, 0, 0};
     TMD_HIP(hipMemcpyAsync(h, acc, sizeof h, hipMemcpyDeviceToHost, s.stream));
     TMD_HIP(hipStreamSynchronize(s.stream));
     const double vol = s.g.len[0] * s.g.len[1] * s.g.len[2];
     *ubar = h[0] / (double)s.n / (double)p.steps;
-    *pbar = (h[3] + h[1]) / (3.0 * vol) / (double)p.steps;
+    *pbar = (h[2] + h[1]) / (3.0 * vol) / (double)p.steps;
 }
 
 static bool begin_traj(Sim& s, const TrajSpec& p, bool adjoint) {
@@ -319,15 +525,19 @@ static bool begin_traj(Sim& s, const TrajSpec& p, bool adjoint) {
         const size_t nck = (size_t)(p.steps / p.ck + 1);
         s.adj_ckx.reserve(atom * nck, false, s.stream);
         s.adj_ckv.reserve(atom * nck, false, s.stream);
-        const size_t nseg = (size_t)std::min(p.ck, p.steps + 1);  // states per interval
-        s.adj_segx.reserve(atom * nseg, false, s.stream);
-        s.adj_segv.reserve(atom * nseg, false, s.stream);
         s.adj_xbar.reserve(atom, false, s.stream);
         s.adj_vbar.reserve(atom, false, s.stream);
         s.adj_fbar.reserve(atom, false, s.stream);
     }
     if (has_error()) return false;
-    snapshot_to(s, s.adj_x0, s.adj_v0, 0);
+    sync_pos_from_mirror(s);
+    keep_state(s);
+    if (s.adj_part.p) zero(s, s.adj_part.p, s.adj_part.bytes / sizeof(double));  // sums of a call that ended in an error
+    if (adjoint) {
+        // the reverse pass stages 48 B a window slot: tiles for that
+        s.stage_bytes = kDemStageBytes;
+        s.stage_budget = kLdsBudget;
+    }
     return !has_error();
 }
 
@@ -335,7 +545,13 @@ static bool begin_traj(Sim& s, const TrajSpec& p, bool adjoint) {
 static void end_traj(Sim& s, const TrajSpec& p) {
     if (has_error()) return;
     restore_from(s, s.adj_x0, s.adj_v0, 0);
-    relist(s, p.rc + p.skin);
+    if (s.stage_bytes != kPosStageBytes) {
+        s.stage_bytes = kPosStageBytes;
+        s.tile_auto[0] = s.tile_auto[1] = s.tile_auto[2] = 0;
+        s.tile_tuned = 0;
+    }
+    s.gh_wanted = 0;
+    rebuild_lists(s, false, 0, p.rc + p.skin);
     compute_lj(s, 0, p.rc, p.eps, p.sigma);
     TMD_HIP(hipStreamSynchronize(s.stream));
 }
@@ -377,45 +593,93 @@ bool traj_adjoint(Sim& s, int steps, int ck, double dt, double rc, double skin, 
     const double h = 0.5 * dt;
     const double cv = 2.0 * c.cW;  // d(sum v^2)/dv = 2 v
     const size_t atom = sizeof(double4) * (size_t)n;
-    TMD_HIP(hipMemsetAsync(s.adj_xbar.p, 0, atom, s.stream));
-    TMD_HIP(hipMemsetAsync(s.adj_vbar.p, 0, atom, s.stream));
-    TMD_HIP(hipMemsetAsync(s.adj_fbar.p, 0, atom, s.stream));
+    zero(s, s.adj_xbar.p, 4 * (size_t)n);
+    zero(s, s.adj_vbar.p, 4 * (size_t)n);
+    zero(s, s.adj_fbar.p, 4 * (size_t)n);
     double* theta = s.adj_acc.as<double>() + 4;
-    TMD_HIP(hipMemsetAsync(theta, 0, 2 * sizeof(double), s.stream));
-    const int nt = 256, nb = div_up(n, nt);
+    zero(s, theta, 2);
+    const int nt = 256;
     const double cut = rc + skin;
     for (int sg = steps / ck; sg >= 0 && !has_error(); --sg) {
         const int t0 = sg * ck, t1 = std::min(t0 + ck - 1, steps);
-        // recompute the interval from its checkpoint (its list is fixed)
+        // recompute the interval from its checkpoint (its list is fixed),
+        // every state kept in mirror order, ghosts included
         restore_from(s, s.adj_ckx, s.adj_ckv, (size_t)sg);
-        relist(s, cut);
-        compute_lj(s, 0, rc, eps, sigma);
-        snapshot_to(s, s.adj_segx, s.adj_segv, 0);
-        for (int t = t0 + 1; t <= t1 && !has_error(); ++t) {
-            initial_integration(s, dt);
-            refresh_ghosts(s);
-            compute_lj(s, 0, rc, eps, sigma, dt);  // final kick fused
-            snapshot_to(s, s.adj_segx, s.adj_segv, (size_t)(t - t0));
+        relist(s, false, cut);
+        if (has_error()) return false;
+        const size_t stride = 3 * (size_t)s.cap_all;  // doubles per mirror
+        const size_t nseg = (size_t)(t1 - t0 + 1);
+        s.adj_segx.reserve(sizeof(double) * stride * nseg, false, s.stream);
+        s.adj_segv.reserve(sizeof(double) * stride * nseg, false, s.stream);
+        s.adj_mir.reserve(sizeof(double) * stride * 4, false, s.stream);
+        if (has_error()) return false;
+        auto segx = [&](int t) { return s.adj_segx.as<double>() + (size_t)(t - t0) * stride; };
+        auto segv = [&](int t) { return s.adj_segv.as<double>() + (size_t)(t - t0) * stride; };
+        TMD_HIP(hipMemcpyAsync(segx(t0), s.spos.p, (size_t)kMirBytes * (size_t)s.nbinned, hipMemcpyDeviceToDevice, s.stream));
+        for (int t = t0; t <= t1 && !has_error(); ++t) {
+            TrajStep st{};
+            st.hfin = t > t0 ? h : 0.0;
+            st.adv = t < t1;
+            st.vt = Mir{segv(t)};
+            if (st.adv) st.xnext = Mir{segx(t + 1)};
+            DevBuf x;
+            x.p = segx(t);
+            // the last state's velocity needs its force too; a lone state has it
+            if (t < t1 || t > t0) traj_step(s, p, x, st, false);
+            else
+                TMD_HIP(hipMemcpyAsync(segv(t), s.svel.p, (size_t)kMirBytes * (size_t)s.nbinned, hipMemcpyDeviceToDevice, s.stream));
         }
         // reverse it
+        double* xb = s.adj_mir.as<double>();
+        double* vb = xb + stride;
+        double* fb[2] = {vb + stride, vb + 2 * stride};
+        hipLaunchKernelGGL(k_adj_begin, dim3(div_up(n, nt)), dim3(nt), 0, s.stream, (const int*)s.work.as<int>(),
+                           (const int*)s.work_k.as<int>(), n, (const double4*)s.adj_xbar.as<double4>(),
+                           (const double4*)s.adj_vbar.as<double4>(), (const double4*)s.adj_fbar.as<double4>(), CMir{segv(t1)}, cv, h,
+                           t1 >= 1 ? 1 : 0, Mir{xb}, Mir{vb}, Mir{fb[0]}, ghost_index(s));
+        TMD_HIP(hipGetLastError());
+        LJArgs a = make_lj_args(s, rc, eps, sigma);
+        a.wcap = std::min(s.max_window + 1, kLdsBudget / kDemStageBytes);
+        const size_t lds = (size_t)a.wcap * kDemStageBytes;
+        // the adjoint kernel's precision: the forward's unless set apart
+        const int prec = s.adj_precision >= 0 ? s.adj_precision : s.precision;
         for (int t = t1; t >= t0 && !has_error(); --t) {
-            if (t < t1) {
-                restore_from(s, s.adj_segx, s.adj_segv, (size_t)(t - t0));
-                refresh_ghosts(s);
-            }
+            AdjStep st{};
+            st.xb = Mir{xb};
+            st.vb = Mir{vb};
+            st.end = t == t0;
+            st.post = t >= 1;
+            st.pre = t - 1 >= 1;
+            if (!st.end) st.vprev = CMir{segv(t - 1)};
+            st.fnext = Mir{fb[1]};
+            st.xbar = s.adj_xbar.as<double4>();
+            st.vbar = s.adj_vbar.as<double4>();
+            st.fbar = s.adj_fbar.as<double4>();
+            st.gh = ghost_index(s);
+            st.cv = cv;
+            st.h = h;
+            st.dt = dt;
+            st.acc = tile_sums(s, 2);
+            c.loss_terms = t >= 1 ? 1 : 0;
+            if (has_error()) return false;
             hipEvent_t ev = nullptr;
             s.timer.begin(K_ADJOINT, s.stream, &ev);
-            if (t >= 1)
-                hipLaunchKernelGGL(k_adj_pre, dim3(nb), dim3(nt), 0, s.stream, (const double4*)s.vel.as<double4>(), n, cv, h,
-                                   s.adj_vbar.as<double4>(), s.adj_fbar.as<double4>());
-            c.loss_terms = t >= 1 ? 1 : 0;
-            launch_lj_adjoint(s, rc, eps, sigma, c, theta);
-            if (t >= 1)
-                hipLaunchKernelGGL(k_adj_post, dim3(nb), dim3(nt), 0, s.stream, (const double4*)s.adj_xbar.as<double4>(), n,
-                                   dt, h, s.adj_vbar.as<double4>(), s.adj_fbar.as<double4>());
+#define TMD_ADJ(P, SH)                                                                                                  \
+    hipLaunchKernelGGL((k_lj_adjoint<P, SH>), dim3(ntiles_of(s)), dim3(s.tile_threads), lds, s.stream, CMir{segx(t)},     \
+                       CMir{fb[0]}, (const int*)s.cell_start.as<int>(), (const int*)s.work.as<int>(),                    \
+                       (const int*)s.work_k.as<int>(), (const int*)s.tile_start.as<int>(),                              \
+                       (const int*)s.nb_count.as<int>(), (const nb_t*)s.nb_list.as<nb_t>(), a, c, st)
+            if (prec == PREC_FP64) {
+                if (s.lj_shift) TMD_ADJ(PREC_FP64, 1); else TMD_ADJ(PREC_FP64, 0);
+            } else {
+                if (s.lj_shift) TMD_ADJ(PREC_FP32_MIXED, 1); else TMD_ADJ(PREC_FP32_MIXED, 0);
+            }
+#undef TMD_ADJ
             s.timer.end(K_ADJOINT, s.stream, ev);
             TMD_HIP(hipGetLastError());
+            std::swap(fb[0], fb[1]);
         }
+        flush_sums(s, 2, theta);
     }
     std::vector<double4> hx(grad_x ? n : 0), hv(grad_v ? n : 0);
     double th[2] = {0, 0};

@@ -400,7 +400,7 @@ void retune_tiles(Sim& s) {
     if (s.tile_req[0] > 0 && s.tile_req[1] > 0 && s.tile_req[2] > 0) return;  // explicit tiles
     const TileGeom& T = s.tiles;
     const bool over = (double)(s.max_window + 1) * s.stage_bytes > (double)s.stage_budget;
-    const bool first = s.stage_bytes == kDemStageBytes && !s.tile_tuned;
+    const bool first = s.stage_budget == kDemLdsShare && !s.tile_tuned;
     if ((!over && !first) || s.max_window <= 0) return;
     s.tile_tuned = 1;
     const double peak = (s.max_window + 1) / ((T.tx + 2.0) * (T.ty + 2.0) * (T.tz + 2.0));

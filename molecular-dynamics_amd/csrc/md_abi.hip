@@ -656,7 +656,7 @@ void md_deallocate_grid() {
                       &s.nb_count, &s.nb_list, &s.nb_count2, &s.nb_list2,
                       &s.scan_blocks, &s.scan_aux, &s.red, &s.gbuf, &s.adj_x0, &s.adj_v0, &s.adj_ckx,
                       &s.adj_ckv, &s.adj_segx, &s.adj_segv, &s.adj_xbar, &s.adj_vbar, &s.adj_fbar, &s.adj_part,
-                      &s.adj_acc};
+                      &s.adj_acc, &s.adj_mir};
     for (DevBuf* b : bufs) b->release();
     if (s.h_stats) {
         (void)hipHostFree(s.h_stats);

@@ -190,6 +190,7 @@ struct Sim {
     // states, adjoints (double4 per local atom), partial sums, accumulators
     DevBuf adj_x0, adj_v0, adj_ckx, adj_ckv, adj_segx, adj_segv;
     DevBuf adj_xbar, adj_vbar, adj_fbar, adj_part, adj_acc;
+    DevBuf adj_mir;                    // adjoints in mirror order: xbar, vbar, Fbar and the next Fbar
 
     hipStream_t stream = nullptr;
     KernelTimer timer;

@@ -39,14 +39,25 @@ __device__ __forceinline__ int nb_entry(const int4& q, int u) {
 
 // FP64 pair scalar of the reference closure; UNIT skips the exact
 // multiplications by eps = 1 and sigma^6 = 1 (x * 1.0 == x), so the result
-// is bit-identical either way.
+// is bit-identical either way.  sr6 also serves the energy.
 template <int SHIFT, int UNIT>
-__device__ __forceinline__ double lj_f64u(const LJArgs& a, double rsq) {
+__device__ __forceinline__ double lj_f64u(const LJArgs& a, double rsq, double& sr6) {
     const double sr2 = rcp_round(rsq);
-    const double sr6 = UNIT ? sr2 * sr2 * sr2 : sr2 * sr2 * sr2 * a.sigma6;
+    sr6 = UNIT ? sr2 * sr2 * sr2 : sr2 * sr2 * sr2 * a.sigma6;
     double f = UNIT ? 48.0 * sr6 * (sr6 - 0.5) * sr2 : 48.0 * sr6 * (sr6 - 0.5) * sr2 * a.eps;
     if (SHIFT) f = f - a.fc - (rsq - a.rc2) * a.dfc;
     return f;
+}
+
+// pair energy from sr6
+template <int SHIFT>
+__device__ __forceinline__ double lj_u64(const LJArgs& a, double rsq, double sr6) {
+    double u = 4.0 * a.eps * sr6 * (sr6 - 1.0);
+    if (SHIFT) {
+        const double ds = rsq - a.rc2;
+        u = u - a.uc + ds * (0.5 * a.fc) + ds * ds * (0.25 * a.dfc);
+    }
+    return u;
 }
 
 template <int SHIFT, int UNIT>
@@ -104,10 +115,17 @@ __device__ __forceinline__ void win_pos(int t, const WinStage& st, const SP& spo
 // followed by column 2's (cnt2 at lp2), one running sum over both; a
 // wavefront then runs as many groups as its busiest lane has in both
 // columns together, not the busiest lane of each column in turn.
-template <int PREC, int SHIFT, int UNIT, bool STAGED, bool PAIR2 = false, class SP = const double4*>
+//
+// ENERGY (full lists): also pe += u / 2 and vir += f r^2 / 2 of every entry
+// within the cutoff, in FP64 whatever the force's precision.
+struct PairEnergy {
+    double pe = 0.0, vir = 0.0;
+};
+template <int PREC, int SHIFT, int UNIT, bool STAGED, bool PAIR2 = false, bool ENERGY = false, class SP = const double4*>
 __device__ __forceinline__ double4 lj_full_atom(const double4 pi, int cnt, const int4* __restrict__ lp, const WinStage& sp,
                                                 const SP& spos, const TileWin& W, const LJArgs& a,
-                                                int cnt2 = 0, const int4* __restrict__ lp2 = nullptr) {
+                                                int cnt2 = 0, const int4* __restrict__ lp2 = nullptr,
+                                                PairEnergy* en = nullptr) {
     double fx = 0.0, fy = 0.0, fz = 0.0;
     float sxa = 0.f, sya = 0.f, sza = 0.f, cxa = 0.f, cya = 0.f, cza = 0.f;
     const int ng1 = (cnt + 7) >> 3;
@@ -144,6 +162,15 @@ __device__ __forceinline__ double4 lj_full_atom(const double4 pi, int cnt, const
                                       : fma(dx[u], dx[u], fma(dy[u], dy[u], dz[u] * dz[u]));
             ok[u] = valid && rs[u] < a.rc2;
         }
+        if (ENERGY && PREC != PREC_FP64) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                double sr6;
+                const double f = lj_f64u<SHIFT, UNIT>(a, rs[u], sr6);
+                en->pe += 0.5 * (ok[u] ? lj_u64<SHIFT>(a, rs[u], sr6) : 0.0);
+                en->vir += 0.5 * (ok[u] ? f * rs[u] : 0.0);
+            }
+        }
         // The pair scalar is evaluated for every entry and masked afterwards:
         // a masked entry may have rsq = 0 (its own position) or lie beyond
         // the cutoff; its (possibly infinite) scalar is replaced by 0 by the
@@ -151,8 +178,13 @@ __device__ __forceinline__ double4 lj_full_atom(const double4 pi, int cnt, const
         if (PREC == PREC_FP64) {
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const double f = lj_f64u<SHIFT, UNIT>(a, rs[u]);
+                double sr6;
+                const double f = lj_f64u<SHIFT, UNIT>(a, rs[u], sr6);
                 const double fm = ok[u] ? f : 0.0;
+                if (ENERGY) {
+                    en->pe += 0.5 * (ok[u] ? lj_u64<SHIFT>(a, rs[u], sr6) : 0.0);
+                    en->vir += 0.5 * (ok[u] ? f * rs[u] : 0.0);
+                }
                 fx = fx + dx[u] * fm;
                 fy = fy + dy[u] * fm;
                 fz = fz + dz[u] * fm;

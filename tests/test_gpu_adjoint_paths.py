@@ -1,0 +1,57 @@
+"""GPU parity of the one-launch trajectory and reverse steps against the
+oracle's scatter-form adjoint, on the branches that ordinary boxes do not
+take: windows read from the mirrors because they outgrow LDS, the plain
+cutoff, eps and sigma other than one, an interval of one state and a run
+shorter than one interval."""
+import numpy as np
+import pytest
+
+import pyoracle as po
+from common import RC, SKIN, announce, perturbed_fcc
+
+pytestmark = pytest.mark.gpu
+
+DT = 0.005
+
+
+@pytest.fixture(scope="module")
+def tm():
+    import tinymd_amd
+    _, cus = tinymd_amd.device_info()
+    if cus == 0:
+        pytest.fail("no HIP device visible to libtinymd_amd")
+    return tinymd_amd
+
+
+@pytest.mark.parametrize("tile,shift,eps,sigma,steps,ck", [
+    (0, True, 1.0, 1.0, 25, 20),     # staged, as ordinary runs
+    (8, True, 1.0, 1.0, 25, 20),     # one tile, window beyond LDS
+    (1, True, 1.05, 0.98, 23, 10),   # one-cell tiles, general eps and sigma
+    (8, False, 1.05, 0.98, 21, 20),  # plain cutoff from the mirrors
+    (0, False, 1.0, 1.0, 12, 5),     # plain cutoff, staged
+    (2, True, 1.0, 1.0, 20, 20),     # the last interval is one state
+    (0, True, 1.0, 1.0, 3, 20),      # shorter than an interval
+    (0, True, 1.0, 1.0, 4, 1),       # a rebuild every step
+])
+def test_adjoint_branches_match_oracle(tm, tile, shift, eps, sigma, steps, ck):
+    announce(f"adjoint tile={tile} shift={shift} eps={eps} sigma={sigma} steps={steps} ck={ck}")
+    aabb, m, x, v = perturbed_fcc(7, 6, 8, amp=0.05, seed=9)
+    sim = tm.Simulation(m, x, v, aabb, RC + SKIN, lj_shift=shift)
+    if tile:
+        sim.set_tile(tile)
+    sim.copy_to_accelerator()
+    r = sim.traj_adjoint(steps, ck, DT, RC, SKIN, eps, sigma, -4.0, 1.0)
+    o = po.OracleSim(m, x, v, aabb, RC + SKIN, threads=4)
+    o.setup(False, po.HALF_GHOST_FULL, RC + SKIN)
+    o.lj(False, RC, eps, sigma, shift=int(shift))
+    q = o.traj_adjoint(steps, ck, DT, RC, SKIN, eps, sigma, shift=int(shift), u_target=-4.0, p_target=1.0)
+    assert r["ubar"] == pytest.approx(q["ubar"], rel=1e-12)
+    assert r["pbar"] == pytest.approx(q["pbar"], rel=1e-10)
+    assert r["grad_eps"] == pytest.approx(q["grad_eps"], rel=1e-9)
+    assert r["grad_sigma"] == pytest.approx(q["grad_sigma"], rel=1e-9)
+    for key in ("grad_x0", "grad_v0"):
+        d = np.linalg.norm(r[key] - q[key]) / np.linalg.norm(q[key])
+        assert d <= 1e-9, key
+    # the call leaves the state at x0
+    _, xa, va, _ = sim.state()
+    assert np.array_equal(xa, x) and np.array_equal(va, v)
