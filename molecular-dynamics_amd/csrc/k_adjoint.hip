@@ -36,28 +36,6 @@ struct AdjCoef {
     int loss_terms;  // 0 at x_0 (the loss starts at t = 1)
 };
 
-// A local's ghosts in the ghost index: mirror index of each and, when asked,
-// its image shift.
-struct GhostIndex {
-    const int* w;  // per work slot: first entry * 32 + number
-    const int* k;  // per entry: mirror index (-1: outside the grid)
-    const int* c;  // per entry: image code
-    double L0, L1, L2;
-};
-template <class F>
-__device__ __forceinline__ void each_ghost(const GhostIndex& g, int w, F&& f) {
-    const int pk = g.w[w];
-    for (int e = pk >> 5, e1 = e + (pk & 31); e < e1; ++e) {
-        const int kg = g.k[e];
-        if (kg >= 0) f(e, kg);
-    }
-}
-__device__ __forceinline__ double4 ghost_image(const double4& x, const GhostIndex& g, int e) {
-    int ix, iy, iz;
-    img_decode(g.c[e], ix, iy, iz);
-    return make_double4(x.x + g.L0 * (double)ix, x.y + g.L1 * (double)iy, x.z + g.L2 * (double)iz, 0.0);
-}
-
 // One step of a trajectory on the cell-ordered mirrors, one launch: force at
 // x_t, final kick, energy, virial and kinetic sums, and the next step's kick
 // and drift, locals and their ghosts, into the next mirror.  The arithmetic
@@ -97,8 +75,8 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_traj_step(const CMir spos, 
         const double4 pi = spos[kw];
         const int cnt = nbc[w];
         const int4* lp = reinterpret_cast<const int4*>(nbl + (size_t)(w >> 6) * (size_t)a.cap * 64) + (w & 63);
-        const double4 f = staged ? lj_full_atom<PREC, SHIFT, UNIT, true, false, ENERGY>(pi, cnt, lp, sp, spos, W, a, 0, nullptr, &en)
-                                 : lj_full_atom<PREC, SHIFT, UNIT, false, false, ENERGY>(pi, cnt, lp, sp, spos, W, a, 0, nullptr, &en);
+        const double4 f = staged ? lj_full_atom<PREC, SHIFT, UNIT, true, false, ENERGY>(pi, cnt, lp, sp, spos, W, a, ld_stream(lp), 0, nullptr, &en)
+                                 : lj_full_atom<PREC, SHIFT, UNIT, false, false, ENERGY>(pi, cnt, lp, sp, spos, W, a, ld_stream(lp), 0, nullptr, &en);
         double4 v = t.vel[kw];
         v.x = v.x + f.x * t.hfin;
         v.y = v.y + f.y * t.hfin;
@@ -119,7 +97,7 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_traj_step(const CMir spos, 
             x.y = x.y + v.y * t.dt;
             x.z = x.z + v.z * t.dt;
             t.xnext[kw] = x;
-            each_ghost(t.gh, w, [&](int e, int kg) { t.xnext[kg] = ghost_image(x, t.gh, e); });
+            each_ghost(t.gh, t.gh.w[w], [&](int e, int kg) { t.xnext[kg] = ghost_image(x, t.gh, e); });
         }
         t.vel[kw] = v;
     }
@@ -313,7 +291,7 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_lj_adjoint(const CMir spos,
             t.xb[kw] = xb;
             t.vb[kw] = vb;
             t.fnext[kw] = fb;
-            each_ghost(t.gh, w, [&](int, int kg) { t.fnext[kg] = fb; });
+            each_ghost(t.gh, t.gh.w[w], [&](int, int kg) { t.fnext[kg] = fb; });
         }
     };
     if (staged) atoms(std::true_type{});
@@ -363,7 +341,7 @@ __global__ void k_adj_begin(const int* __restrict__ work, const int* __restrict_
     xb[kw] = xbar[i];
     vb[kw] = b;
     fb[kw] = f;
-    each_ghost(gh, w, [&](int, int kg) { fb[kg] = f; });
+    each_ghost(gh, gh.w[w], [&](int, int kg) { fb[kg] = f; });
 }
 
 // ---------------------------------------------------------------------------
@@ -387,7 +365,6 @@ static void restore_from(Sim& s, const DevBuf& bx, const DevBuf& bv, size_t slot
 // from atom order without.  The velocities come along into their mirror and
 // the ghost index is made.
 static void relist(Sim& s, bool wrap, double cutoff) {
-    s.gh_wanted = 1;
     s.vel_mirror_wanted = 1;
     rebuild_lists(s, wrap, 0, cutoff);
     s.vel_mirror_wanted = 0;
@@ -395,10 +372,6 @@ static void relist(Sim& s, bool wrap, double cutoff) {
 }
 
 static int ntiles_of(const Sim& s) { return s.tiles.ntx * s.tiles.nty * s.tiles.ntz; }
-
-static GhostIndex ghost_index(const Sim& s) {
-    return GhostIndex{s.gh_w.as<int>(), s.gh_k.as<int>(), s.gh_c.as<int>(), s.g.len[0], s.g.len[1], s.g.len[2]};
-}
 
 static void zero(Sim& s, void* p, size_t doubles) {
     hipLaunchKernelGGL(k_fill_double, dim3(std::min<long long>(div_up((long long)doubles, 1024), 1024)), dim3(256), 0, s.stream,
@@ -550,7 +523,6 @@ static void end_traj(Sim& s, const TrajSpec& p) {
         s.tile_auto[0] = s.tile_auto[1] = s.tile_auto[2] = 0;
         s.tile_tuned = 0;
     }
-    s.gh_wanted = 0;
     rebuild_lists(s, false, 0, p.rc + p.skin);
     compute_lj(s, 0, p.rc, p.eps, p.sigma);
     TMD_HIP(hipStreamSynchronize(s.stream));

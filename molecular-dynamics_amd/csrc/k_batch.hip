@@ -535,8 +535,8 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_b_lj_full(const RepDesc* __
         // atom's column; that run's results are discarded.
         const int cnt = min(nbc[w], a.cap);
         const int4* lp = reinterpret_cast<const int4*>(nbl + (size_t)(w >> 6) * (size_t)a.cap * 64) + (w & 63);
-        const double4 f = staged ? lj_full_atom<PREC, SHIFT, UNIT, true>(pi, cnt, lp, sp, spos, W, a)
-                                 : lj_full_atom<PREC, SHIFT, UNIT, false>(pi, cnt, lp, sp, spos, W, a);
+        const double4 f = staged ? lj_full_atom<PREC, SHIFT, UNIT, true>(pi, cnt, lp, sp, spos, W, a, ld_stream(lp))
+                                 : lj_full_atom<PREC, SHIFT, UNIT, false>(pi, cnt, lp, sp, spos, W, a, ld_stream(lp));
         if (!ADV) force[i] = f;
         // velocity-Verlet final kick (k_final_integration's arithmetic)
         double4 v = vel[i];

@@ -176,8 +176,8 @@ __global__ void __launch_bounds__(256) k_rebuild_finish(FinishArgs a, const int*
                                                         const CMir spos_old, const CMir svel_old, const Mir spos,
                                                         const Mir svel, const int* __restrict__ g_owner,
                                                         const int* __restrict__ g_code, const int* __restrict__ gh_e,
-                                                        int* __restrict__ g_ko, int* __restrict__ g_kg, int* __restrict__ gh_k,
-                                                        int* __restrict__ gh_c, int* __restrict__ ctr) {
+                                                        int* __restrict__ g_ko, int* __restrict__ g_kg, int2* __restrict__ gh_k,
+                                                        int* __restrict__ ctr) {
     const int b = blockIdx.x, tid = threadIdx.x;
     if (b >= a.ntiles + a.nbm) {
         const int ng = min(ctr[CT_NGHOST], a.gcap);
@@ -187,10 +187,8 @@ __global__ void __launch_bounds__(256) k_rebuild_finish(FinishArgs a, const int*
             g_ko[g] = inv[g_owner[g]];
             g_kg[g] = kg;
             const int e = gh_pack ? gh_e[g] : a.gcap;
-            if (e < a.gcap) {  // entry numbers run past the capacity only where the host will grow it
-                gh_k[e] = kg;
-                gh_c[e] = g_code[g] & 0xff;
-            }
+            // entry numbers run past the capacity only where the host will grow it
+            if (e < a.gcap) gh_k[e] = make_int2(kg, g_code[g] & 0xff);
         }
         return;
     }
@@ -511,7 +509,7 @@ void bin_finish(Sim& s, int nq, bool with_ghosts) {
                        (const double4*)s.vel.as<double4>(), CMir{s.spos.as<double>()}, CMir{s.svel.as<double>()},         \
                        Mir{s.spos2.as<double>()}, Mir{with_vel ? s.svel2.as<double>() : nullptr},                        \
                        (const int*)s.g_owner.as<int>(), (const int*)s.g_code.as<int>(), (const int*)s.gh_e.as<int>(),    \
-                       s.g_ko.as<int>(), s.g_kg.as<int>(), s.gh_k.as<int>(), s.gh_c.as<int>(), s.counters.as<int>())
+                       s.g_ko.as<int>(), s.g_kg.as<int>(), s.gh_k.as<int2>(), s.counters.as<int>())
     if (mir) TMD_FINISH(true); else TMD_FINISH(false);
 #undef TMD_FINISH
     TMD_HIP(hipGetLastError());

@@ -51,7 +51,18 @@ namespace tmd {
 // not into pos, and no force: inside the fused step loop the force of a
 // step that is followed by another one is consumed here (the kick) and the
 // loop restores pos from the mirror before it rebuilds or returns.  The
-// arithmetic is that of the separate integration kernels.
+// arithmetic is that of the separate integration kernels.  With the ghost
+// index (gh) it writes the atom's ghosts there too, so a step between
+// rebuilds is this launch alone; without one k_ghost_step_mirror does.
+//
+// Bounds: small boxes by the latency of window, staging and list walk, large
+// ones by the pair arithmetic's vector instructions.  A lane issues its own
+// loads before the window is formed, so they cost no round trip of their own
+// after the staging barrier.  Ghosts written here and own loads first, us a
+// step, rebuilds included: 16^3 cells mixed 23.0 -> 22.0, 32^3 FP64 41.2 ->
+// 39.1, 40^3 mixed 54.2 -> 51.9, 80^3 mixed 241 -> 237, FP64 308 -> 307.
+// Issued after the window instead, 40^3 and 80^3 mixed gain little (54.1,
+// 239): they then queue in front of the staging loads.
 //
 // PAIR2 (half lists): the atom also gathers its complementary column (local
 // neighbours j > i, whose pair terms the half list evaluates from j's side),
@@ -63,33 +74,50 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_lj_full(TMD_KERNEL_LIST_PAR
                                                          double4* __restrict__ vel, const Mir svel, double hdt, double dt,
                                                          const int* __restrict__ wk, const Mir spos_next,
                                                          int vel_by_k, const int* __restrict__ nbc2,
-                                                         const nb_t* __restrict__ nbl2) {
+                                                         const nb_t* __restrict__ nbl2, GhostIndex gh) {
     extern __shared__ double dyn[];
     const WinStage sp = win_stage(dyn, a.wcap);
     const int tile = xcd_block(blockIdx.x, gridDim.x);
     const int w0 = tile_start[tile], nloc = tile_start[tile + 1] - w0;
     if (nloc == 0) return;
+    // position, velocity, list head, ghost entries: two dependent rounds of
+    // loads, in flight while the window is formed and staged
+    struct Own {
+        int kw, cnt, cnt2, pk;
+        double4 x, v;
+        int4 head;
+    } o;
+    auto fetch = [&](int at) {
+        const int w = w0 + at;
+        o.kw = wk[w];
+        o.cnt = nbc[w];
+        o.cnt2 = PAIR2 ? nbc2[w] : 0;  // half lists: the complementary column continues the same sum
+        o.pk = KICK == 2 && gh.w ? gh.w[w] : 0;
+        const size_t col = (size_t)(w >> 6) * (size_t)a.cap * 8 + (w & 63);
+        o.head = list_head<PAIR2>(o.cnt, reinterpret_cast<const int4*>(nbl) + col, reinterpret_cast<const int4*>(nbl2) + col);
+        o.x = spos[o.kw];
+        if (KICK) o.v = vel_by_k ? (double4)svel[o.kw] : vel[work[w]];
+    };
+    if ((int)threadIdx.x < nloc) fetch(threadIdx.x);
     __shared__ TileWin W;
     tile_window(tile, start, a.g, W);
     const bool staged = stage_window(W, a.wcap, spos, nullptr, sp);
     for (int at = threadIdx.x; at < nloc; at += blockDim.x) {
+        if (at >= (int)blockDim.x) fetch(at);
         const int w = w0 + at;
-        const int i = work[w];
-        const int kw = wk[w];
-        const double4 pi = spos[kw];
-        const int cnt = nbc[w];
-        const int4* lp = reinterpret_cast<const int4*>(nbl + (size_t)(w >> 6) * (size_t)a.cap * 64) + (w & 63);
-        // half lists: the complementary column continues the same sum
-        const int cnt2 = PAIR2 ? nbc2[w] : 0;
-        const int4* lp2 = PAIR2 ? reinterpret_cast<const int4*>(nbl2 + (size_t)(w >> 6) * (size_t)a.cap * 64) + (w & 63)
-                                : nullptr;
-        const double4 f = staged ? lj_full_atom<PREC, SHIFT, UNIT, true, PAIR2>(pi, cnt, lp, sp, spos, W, a, cnt2, lp2)
-                                 : lj_full_atom<PREC, SHIFT, UNIT, false, PAIR2>(pi, cnt, lp, sp, spos, W, a, cnt2, lp2);
+        const int kw = o.kw;
+        const double4 pi = o.x;
+        const size_t col = (size_t)(w >> 6) * (size_t)a.cap * 8 + (w & 63);
+        const int4* lp = reinterpret_cast<const int4*>(nbl) + col;
+        const int4* lp2 = PAIR2 ? reinterpret_cast<const int4*>(nbl2) + col : nullptr;
+        const double4 f = staged ? lj_full_atom<PREC, SHIFT, UNIT, true, PAIR2>(pi, o.cnt, lp, sp, spos, W, a, o.head, o.cnt2, lp2)
+                                 : lj_full_atom<PREC, SHIFT, UNIT, false, PAIR2>(pi, o.cnt, lp, sp, spos, W, a, o.head, o.cnt2, lp2);
+        const int i = KICK != 2 || !vel_by_k ? work[w] : 0;
         if (KICK != 2) force[i] = f;
         if (KICK) {
             // velocity-Verlet final kick (k_final_integration's arithmetic)
             // velocities in atom order (vel) or in mirror order (svel)
-            double4 v = vel_by_k ? (double4)svel[kw] : vel[i];
+            double4 v = o.v;
             v.x = v.x + f.x * hdt;
             v.y = v.y + f.y * hdt;
             v.z = v.z + f.z * hdt;
@@ -103,6 +131,8 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_lj_full(TMD_KERNEL_LIST_PAR
                 x.y = x.y + v.y * dt;
                 x.z = x.z + v.z * dt;
                 spos_next[kw] = x;
+                // the atom's ghosts: k_ghost_step_mirror's arithmetic
+                each_ghost(gh, o.pk, [&](int e, int kg) { spos_next[kg] = ghost_image(x, gh, e); });
             }
             if (vel_by_k) svel[kw] = v;
             else vel[i] = v;
@@ -355,8 +385,7 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_dem_fused(const CMir spos, 
                                                            DEMArgs a, double hdt, double dt, const Mir spos_next,
                                                            const Mir svel_next, double4* __restrict__ force,
                                                            double4* __restrict__ vel, double4* __restrict__ pos,
-                                                           const int* __restrict__ gh_w, const int* __restrict__ gh_k,
-                                                           const int* __restrict__ gh_c, double L0, double L1, double L2) {
+                                                           GhostIndex gh) {
     extern __shared__ double dyn[];
     const int tile = xcd_block(blockIdx.x, gridDim.x);
     const int w0 = tile_start[tile], nloc = tile_start[tile + 1] - w0;
@@ -441,22 +470,11 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_dem_fused(const CMir spos, 
                 svel_next[kw] = v;
                 // the sphere's ghosts: its new position + image shift and its
                 // new velocity (k_ghost_step_mirror_v's arithmetic)
-                if (gh_w) {
-                    const int pk = gh_w[w];
-                    for (int e = pk >> 5, e1 = e + (pk & 31); e < e1; ++e) {
-                        const int kg = gh_k[e];
-                        if (kg < 0) continue;
-                        int ix, iy, iz;
-                        img_decode(gh_c[e], ix, iy, iz);
-                        double4 q;
-                        q.x = x.x + L0 * (double)ix;
-                        q.y = x.y + L1 * (double)iy;
-                        q.z = x.z + L2 * (double)iz;
-                        q.w = x.w;
-                        spos_next[kg] = q;
+                if (gh.w)
+                    each_ghost(gh, gh.w[w], [&](int e, int kg) {
+                        spos_next[kg] = ghost_image(x, gh, e);
                         svel_next[kg] = v;
-                    }
-                }
+                    });
             } else {
                 const int i = work[w];
                 force[i] = make_double4(fx, fy, fz, 0.0);
@@ -483,7 +501,8 @@ void compute_dem_fused(Sim& s, int half, double rc, double gn, double gt, double
     // advancing: the pass also writes the ghosts' next mirror entries
     // (from each local's ghost index), so the next step needs no ghost pass
     const bool fuse = advance && s.ng > 0 && s.ghost_mode == GHOST_FRESH && s.gsrc_valid && s.gh_valid;
-    const int* GS = fuse ? s.gh_w.as<int>() : nullptr;
+    GhostIndex GH = ghost_index(s);
+    if (!fuse) GH.w = nullptr;
     hipEvent_t ev = nullptr;
     s.timer.begin(K_FORCE, s.stream, &ev);
 #define TMD_DEMF(P, H, A)                                                                                               \
@@ -493,8 +512,7 @@ void compute_dem_fused(Sim& s, int half, double rc, double gn, double gt, double
                        (const int*)s.tile_start.as<int>(), (const int*)s.nb_count.as<int>(), (const nb_t*)s.nb_list.as<nb_t>(), \
                        (const int*)s.nb_count2.as<int>(), (const nb_t*)s.nb_list2.as<nb_t>(), a, hdt, dt,               \
                        Mir{s.spos2.as<double>()}, Mir{s.svel2.as<double>()}, s.force.as<double4>(), s.vel.as<double4>(),    \
-                       s.pos.as<double4>(), GS, (const int*)s.gh_k.as<int>(), (const int*)s.gh_c.as<int>(), s.g.len[0],  \
-                       s.g.len[1], s.g.len[2])
+                       s.pos.as<double4>(), GH)
 #define TMD_DEMF_A(P, H) do { if (advance) TMD_DEMF(P, H, 1); else TMD_DEMF(P, H, 0); } while (0)
 #define TMD_DEMF_H(P) do { if (half) TMD_DEMF_A(P, true); else TMD_DEMF_A(P, false); } while (0)
     if (s.precision == PREC_FP64) TMD_DEMF_H(PREC_FP64);
@@ -507,7 +525,7 @@ void compute_dem_fused(Sim& s, int half, double rc, double gn, double gt, double
     if (advance) {
         std::swap(s.spos, s.spos2);
         std::swap(s.svel, s.svel2);
-        s.dem_ghosts_done = fuse || s.ng == 0;
+        s.ghosts_done = fuse || s.ng == 0;
     } else {
         // the locals are back in atom order; their ghosts follow from them
         s.dem_mirrored = 0;
@@ -531,6 +549,8 @@ void compute_lj(Sim& s, int half, double rc, double eps, double sigma, double ki
     a.wcap = window_cap_pos(s);  // the force pass stages positions only
     const int nb = s.tiles.ntx * s.tiles.nty * s.tiles.ntz;
     const int shift = s.lj_shift;
+    // advancing with the ghost index at hand: the pass writes the ghosts too
+    const bool fuse = advance && s.ng > 0 && s.ghost_mode == GHOST_FRESH && s.gh_valid && s.vel_mirrored;
     s.last_force_rc = rc;
     hipEvent_t ev = nullptr;
     s.timer.begin(K_MIRROR, s.stream, &ev);
@@ -548,11 +568,13 @@ void compute_lj(Sim& s, int half, double rc, double eps, double sigma, double ki
         const int VK = s.vel_mirrored;
         const int* WK = s.work_k.as<int>();
         const Mir SN{s.spos2.as<double>()};
+        GhostIndex GH = ghost_index(s);
+        if (!fuse) GH.w = nullptr;
         const int* C2 = s.nb_count2.as<int>();
         const nb_t* L2 = s.nb_list2.as<nb_t>();
 #define TMD_LJ_K(P, SH, U, K, H)                                                                                       \
     hipLaunchKernelGGL((k_lj_full<P, SH, U, K, H>), dim3(nb), dim3(s.tile_threads), lds, s.stream, TMD_LIST_ARGS, a, F, V, SV, hdt, \
-                       kick_dt, WK, SN, VK, C2, L2)
+                       kick_dt, WK, SN, VK, C2, L2, GH)
 #define TMD_LJ_H(P, SH, U, K)                                                                                          \
     do { if (half) TMD_LJ_K(P, SH, U, K, true); else TMD_LJ_K(P, SH, U, K, false); } while (0)
 #define TMD_LJ_FULL(P, SH, U)                                                                                          \
@@ -581,8 +603,10 @@ void compute_lj(Sim& s, int half, double rc, double eps, double sigma, double ki
         // the new local positions are in spos2: it becomes the mirror, whose
         // ghost entries step_refresh rewrites
         std::swap(s.spos, s.spos2);
-        s.mirror_fresh = 0;
-        s.ghost_stale = 1;
+        s.mirror_fresh = fuse;
+        s.ghost_stale = !fuse;
+        s.ghosts_done = fuse;
+        if (fuse) s.ghost_pos_stale = 1;
         s.pos_stale = 1;
     }
 }

@@ -587,8 +587,7 @@ void enqueue_ghosts(Sim& s, bool wrap, bool bin) {
     s.cls.reserve(sizeof(int) * 2 * (size_t)ncls, false, s.stream);  // counts, and their scan
     s.gh_pack.reserve(sizeof(int) * (size_t)s.n, false, s.stream);
     s.gh_e.reserve(sizeof(int) * (size_t)std::max(gcap, 1), false, s.stream);
-    s.gh_k.reserve(sizeof(int) * (size_t)std::max(gcap, 1), false, s.stream);
-    s.gh_c.reserve(sizeof(int) * (size_t)std::max(gcap, 1), false, s.stream);
+    s.gh_k.reserve(sizeof(int2) * (size_t)std::max(gcap, 1), false, s.stream);
     if (bin) {
         s.g_cell.reserve(sizeof(int) * (size_t)std::max(gcap, 1), false, s.stream);
         s.g_slot.reserve(sizeof(int) * (size_t)std::max(gcap, 1), false, s.stream);
@@ -625,7 +624,7 @@ void enqueue_ghosts(Sim& s, bool wrap, bool bin) {
         counts += ncls;
     }
     // entry * 32 + count in 31 bits: the index ends where ghosts pass 2^26
-    s.gh_packed = s.gh_wanted && gcap < (1 << 26);
+    s.gh_packed = gcap < (1 << 26);
     int* pack = s.gh_packed ? s.gh_pack.as<int>() : nullptr;
 #define TMD_EMIT(M)                                                                                                      \
     hipLaunchKernelGGL(k_ghost_emit<M>, gb, blk, 0, s.stream, s.pos.as<double4>(), s.vel.as<double4>(),                    \
@@ -644,7 +643,6 @@ void enqueue_ghosts(Sim& s, bool wrap, bool bin) {
 // md_borders: the ghost layer alone, its size known on return.
 void build_ghosts(Sim& s) {
     for (int attempt = 0; attempt < 3 && !has_error(); ++attempt) {
-        s.gh_wanted = 1;
         enqueue_ghosts(s, false, false);
         if (has_error() || s.n == 0) return;
         const int* st = read_stats(s);

@@ -651,7 +651,7 @@ void md_deallocate_grid() {
     if (s.stream) (void)hipStreamSynchronize(s.stream);
     s.timer.collect();
     DevBuf* bufs[] = {&s.pos, &s.vel, &s.force, &s.mass, &s.sort_buf, &s.g_owner, &s.g_src, &s.g_code, &s.cell_of, &s.cell_slot,
-                      &s.cell_count, &s.cell_start, &s.cell_parts, &s.cell_inv, &s.work_start, &s.work, &s.work_k, &s.work_c, &s.g_ko, &s.g_kg, &s.gh_pack, &s.gh_w, &s.gh_k, &s.gh_c, &s.gh_e, &s.g_cell, &s.g_slot, &s.cell_parts2, &s.cell_inv2, &s.cell_pair,
+                      &s.cell_count, &s.cell_start, &s.cell_parts, &s.cell_inv, &s.work_start, &s.work, &s.work_k, &s.work_c, &s.g_ko, &s.g_kg, &s.gh_pack, &s.gh_w, &s.gh_k, &s.gh_e, &s.g_cell, &s.g_slot, &s.cell_parts2, &s.cell_inv2, &s.cell_pair,
                       &s.cell_src, &s.cls, &s.tile_start, &s.spos, &s.spos2, &s.face, &s.svel, &s.svel2,
                       &s.nb_count, &s.nb_list, &s.nb_count2, &s.nb_list2,
                       &s.scan_blocks, &s.scan_aux, &s.red, &s.gbuf, &s.adj_x0, &s.adj_v0, &s.adj_ckx,
@@ -1078,14 +1078,14 @@ static int run_loop(int steps, int reneigh_every, double dt, bool half, double c
     const int hf = half ? 1 : 0;
     const int saved_sync = s.sync_calls;
     s.sync_calls = 0;
-    s.gh_wanted = dem;  // the DEM step pass also writes the ghosts
+    s.ghosts_done = 0;
     if (!s.nb_valid || s.nb_half != hf) rebuild(s, hf, cutoff + skin);
     int done = 0;
     if (!dem && s.ghost_mode == GHOST_FRESH) {
         // LJ: the force pass also performs the final kick of its step and
-        // the first kick + drift of the next one, so a step is a ghost/mirror
-        // refresh (or a rebuild) and one force pass.  Automatic tiles are
-        // sized for that pass's positions-only window slots.
+        // the first kick + drift of the next one, ghosts included, so a step
+        // between rebuilds is one launch.  Automatic tiles are sized for that
+        // pass's positions-only window slots.
         s.stage_bytes = kPosStageBytes;
         s.stage_budget = kLdsBudget;
         if (steps > 0) initial_integration(s, dt);
@@ -1094,7 +1094,7 @@ static int run_loop(int steps, int reneigh_every, double dt, bool half, double c
         for (int j = 0; j < steps && !has_error(); ++j) {
             if ((j + 1) % reneigh_every == 0) {
                 rebuild(s, hf, cutoff + skin);  // mirror to mirror
-            } else {
+            } else if (!s.ghosts_done) {
                 hipEvent_t ev = nullptr;
                 s.timer.begin(K_GHOST_SYNC, s.stream, &ev);
                 step_refresh(s);
@@ -1138,7 +1138,7 @@ static int run_loop(int steps, int reneigh_every, double dt, bool half, double c
             } else if (s.dem_mirrored) {
                 // the previous step pass wrote the ghosts too, unless it
                 // could not (no ghost index)
-                if (!s.dem_ghosts_done) {
+                if (!s.ghosts_done) {
                     s.timer.begin(K_GHOST_SYNC, s.stream, &ev);
                     dem_ghost_step(s);
                     s.timer.end(K_GHOST_SYNC, s.stream, ev);

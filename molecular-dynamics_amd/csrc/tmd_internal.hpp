@@ -129,11 +129,10 @@ struct Sim {
     int vel_mirrored = 0;   // local velocities live in svel, in mirror order (fused step loop)
     int vel_mirror_wanted = 0;  // fused step loop: refresh_mirror also moves the velocities to svel
     int gsrc_valid = 0;     // g_ko / g_kg match the ghost table and the binning
-    int gh_wanted = 0;      // ghost builds also make the ghost index (gh_pack / gh_e, then gh_w / gh_k / gh_c)
-    int gh_packed = 0;      // gh_pack / gh_e match the ghost table
-    int gh_valid = 0;       // gh_w / gh_k / gh_c match the ghost table, binning and work order
+    int gh_packed = 0;      // the ghost index's gh_pack / gh_e match the ghost table
+    int gh_valid = 0;       // gh_w / gh_k match the ghost table, binning and work order
     int dem_loop = 0;       // DEM step loop: a rebuild's mirrors hold the ghosts' velocities too
-    int dem_ghosts_done = 0;  // DEM step loop: the last force pass also wrote the ghosts' mirror entries
+    int ghosts_done = 0;    // step loops: the last force pass also wrote the ghosts' mirror entries
     int windows_pending = 0;    // a rebuild's statistics are still on the device (read after its list build)
     int ghosts_missing = 0;     // ghosts a rebuild found beyond the capacity (their total number)
     int* h_stats = nullptr;     // pinned host copy of the counters, then the number of the read (read_stats)
@@ -180,9 +179,9 @@ struct Sim {
     DevBuf face;                       // per local: border selection bits of the three ghost passes (u8)
     DevBuf g_ko, g_kg;                 // per ghost: mirror index of its owner and its own (-1: outside the grid)
     // ghost index: per local (gh_pack) and per work slot (gh_w) the first
-    // entry * 32 + number of ghosts; per entry mirror index and image code;
+    // entry * 32 + number of ghosts; per entry (mirror index, image code);
     // per ghost its entry (gh_e)
-    DevBuf gh_pack, gh_w, gh_k, gh_c, gh_e;
+    DevBuf gh_pack, gh_w, gh_k, gh_e;
     DevBuf nb_count, nb_list;
     DevBuf nb_count2, nb_list2;        // half lists: the complementary columns (local j > i)
     DevBuf scan_blocks, scan_aux, counters, red, gbuf;
@@ -302,6 +301,30 @@ __device__ __forceinline__ void img_decode(int c, int& ix, int& iy, int& iz) {
     ix = c % 3 - 1;
     iy = (c / 3) % 3 - 1;
     iz = c / 9 - 1;
+}
+
+// A local's ghosts in the ghost index: mirror index of each and, when asked,
+// its image shift.
+struct GhostIndex {
+    const int* w;  // per work slot: first entry * 32 + number
+    const int2* k;  // per entry: mirror index (-1: outside the grid), image code
+    double L0, L1, L2;
+};
+template <class F>
+__device__ __forceinline__ void each_ghost(const GhostIndex& g, int pk, F&& f) {  // pk = g.w[work slot]
+    for (int e = pk >> 5, e1 = e + (pk & 31); e < e1; ++e) {
+        const int2 k = g.k[e];
+        if (k.x >= 0) f(k.y, k.x);
+    }
+}
+__device__ __forceinline__ double4 ghost_image(const double4& x, const GhostIndex& g, int code) {
+    int ix, iy, iz;
+    img_decode(code, ix, iy, iz);
+    return make_double4(x.x + g.L0 * (double)ix, x.y + g.L1 * (double)iy, x.z + g.L2 * (double)iz, 0.0);
+}
+
+inline GhostIndex ghost_index(const Sim& s) {
+    return GhostIndex{s.gh_w.as<int>(), s.gh_k.as<int2>(), s.g.len[0], s.g.len[1], s.g.len[2]};
 }
 
 __host__ __device__ inline void pbc_wrap(double4& p, const PbcArgs& a) {

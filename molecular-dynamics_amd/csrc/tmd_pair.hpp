@@ -121,10 +121,14 @@ __device__ __forceinline__ void win_pos(int t, const WinStage& st, const SP& spo
 struct PairEnergy {
     double pe = 0.0, vir = 0.0;
 };
+template <bool PAIR2>
+__device__ __forceinline__ int4 list_head(int cnt, const int4* __restrict__ lp, const int4* __restrict__ lp2) {
+    return ld_stream(!PAIR2 || cnt > 0 ? lp : lp2);
+}
 template <int PREC, int SHIFT, int UNIT, bool STAGED, bool PAIR2 = false, bool ENERGY = false, class SP = const double4*>
 __device__ __forceinline__ double4 lj_full_atom(const double4 pi, int cnt, const int4* __restrict__ lp, const WinStage& sp,
                                                 const SP& spos, const TileWin& W, const LJArgs& a,
-                                                int cnt2 = 0, const int4* __restrict__ lp2 = nullptr,
+                                                const int4 first, int cnt2 = 0, const int4* __restrict__ lp2 = nullptr,
                                                 PairEnergy* en = nullptr) {
     double fx = 0.0, fy = 0.0, fz = 0.0;
     float sxa = 0.f, sya = 0.f, sza = 0.f, cxa = 0.f, cya = 0.f, cza = 0.f;
@@ -136,8 +140,9 @@ __device__ __forceinline__ double4 lj_full_atom(const double4 pi, int cnt, const
         return (!PAIR2 || g < ng1) ? lp + (size_t)g * 64 : lp2 + (size_t)(g - ng1) * 64;
     };
     // the next group of 8 entries is loaded while the current one is used
-    // (streaming loads: each group is read once per pass)
-    int4 q = ld_stream(grp(0));
+    // (streaming loads: each group is read once per pass); the caller has
+    // loaded the first (list_head)
+    int4 q = first;
     for (int gi = 0; gi < ng; ++gi) {
         const int4 e = q;
         q = ld_stream(grp(min(gi + 1, ng - 1)));  // next group (clamped: always a valid load)

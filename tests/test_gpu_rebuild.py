@@ -121,3 +121,28 @@ def test_ghosts_outgrow_their_room(tm):
     _, xg, vg, fg = sim.state()
     xo, vo, fo = orc.state()
     assert np.array_equal(xg, xo) and np.array_equal(vg, vo) and np.array_equal(fg, fo)
+
+
+# threads 64: lanes that own several atoms; (4, 4, 4): the smallest box, up to seven
+# images of an atom; 45 steps: two rebuilds, whose ghost index the
+# steps after them use
+@pytest.mark.parametrize("precision", ["fp64", "fp32mixed"])
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("shape,threads", [((4, 4, 4), 0), ((9, 4, 5), 64), ((13, 11, 12), 0)])
+def test_step_pass_writes_ghosts(tm, shape, threads, half, precision):
+    """A step whose force pass also drifts the atoms and their ghosts against
+    the separate calls: the same operations, so bit for bit."""
+    announce(f"step pass with ghosts {shape} {threads} {half} {precision}")
+    aabb, m, x, v = perturbed_fcc(*shape, amp=0.05, seed=5)
+    out = []
+    for run in ("run_lj", "run_abi_lj"):
+        sim = tm.Simulation(m, x, v, aabb, RC + SKIN, precision=precision)
+        if threads:
+            sim.set_tile(3, 2, 2, threads)
+        sim.copy_to_accelerator()
+        sim.setup(half, RC, SKIN)
+        sim.lennard_jones(half, RC)
+        getattr(sim, run)(45, 20, DT, half)
+        out.append(sim.state()[1:] + tuple(sim.ghost_state()[:2]))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
