@@ -564,7 +564,6 @@ bool traj_adjoint(Sim& s, int steps, int ck, double dt, double rc, double skin, 
     c.loss_terms = 0;
     const double h = 0.5 * dt;
     const double cv = 2.0 * c.cW;  // d(sum v^2)/dv = 2 v
-    const size_t atom = sizeof(double4) * (size_t)n;
     zero(s, s.adj_xbar.p, 4 * (size_t)n);
     zero(s, s.adj_vbar.p, 4 * (size_t)n);
     zero(s, s.adj_fbar.p, 4 * (size_t)n);
@@ -653,21 +652,20 @@ bool traj_adjoint(Sim& s, int steps, int ck, double dt, double rc, double skin, 
         }
         flush_sums(s, 2, theta);
     }
-    std::vector<double4> hx(grad_x ? n : 0), hv(grad_v ? n : 0);
+    const size_t row = 3 * (size_t)n;
+    s.h_out.reserve(2 * row);
+    if (has_error()) return false;
     double th[2] = {0, 0};
     TMD_HIP(hipMemcpyAsync(th, theta, sizeof th, hipMemcpyDeviceToHost, s.stream));
-    if (grad_x) TMD_HIP(hipMemcpyAsync(hx.data(), s.adj_xbar.p, atom, hipMemcpyDeviceToHost, s.stream));
-    if (grad_v) TMD_HIP(hipMemcpyAsync(hv.data(), s.adj_vbar.p, atom, hipMemcpyDeviceToHost, s.stream));
+    const HostArray out[2] = {{s.adj_xbar.as<double>(), s.h_out.p, grad_x ? row : 0, row, 3},
+                              {s.adj_vbar.as<double>(), s.h_out.p + row, grad_v ? row : 0, row, 3}};
+    to_host(out, 2, s.h_out.pinned, s.stream);
     TMD_HIP(hipStreamSynchronize(s.stream));
     if (has_error()) return false;
     grad_theta[0] = th[0];
     grad_theta[1] = th[1];
-    for (int i = 0; i < (grad_x ? n : 0); ++i) {
-        grad_x[3 * i] = hx[i].x; grad_x[3 * i + 1] = hx[i].y; grad_x[3 * i + 2] = hx[i].z;
-    }
-    for (int i = 0; i < (grad_v ? n : 0); ++i) {
-        grad_v[3 * i] = hv[i].x; grad_v[3 * i + 1] = hv[i].y; grad_v[3 * i + 2] = hv[i].z;
-    }
+    host_copy({{grad_x, s.h_out.p, grad_x ? sizeof(double) * row : 0},
+               {grad_v, s.h_out.p + row, grad_v ? sizeof(double) * row : 0}});
     end_traj(s, p);
     return !has_error();
 }

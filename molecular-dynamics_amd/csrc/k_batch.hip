@@ -658,6 +658,7 @@ struct Batch {
     DevBuf sb_cnt0, sb_cnt1, scan_tmp, nb_count, nb_list;
     DevBuf dyn, flags, epart, kpart, tout;
     DevBuf snap_pos, snap_vel, snap_force;
+    HostBuf h_out;  // a replica's state on its way out
     hipStream_t stream = nullptr;
     struct CapturedRun {
         hipGraph_t graph;
@@ -676,6 +677,7 @@ struct Batch {
                           &kpart, &tout, &snap_pos, &snap_vel, &snap_force};
         if (stream) (void)hipStreamSynchronize(stream);
         for (DevBuf* b : bufs) b->release();
+        h_out.release();
         if (stream) (void)hipStreamDestroy(stream);
     }
     void drop_graphs() {
@@ -1483,16 +1485,19 @@ int tmd_batch_get_state(int h, int rep, struct Vector3D* pos, struct Vector3D* v
     }
     const int n = B->n[rep];
     const size_t a0 = (size_t)B->R[rep].a0;
-    std::vector<double4> tmp((size_t)n);
     struct Vector3D* outs[3] = {pos, vel, force};
     DevBuf* srcs[3] = {&B->pos, &B->vel, &B->force};
-    for (int k = 0; k < 3; ++k) {
-        if (!outs[k]) continue;
-        TMD_HIP(hipMemcpyAsync(tmp.data(), srcs[k]->as<double4>() + a0, sizeof(double4) * n, hipMemcpyDeviceToHost, B->stream));
-        TMD_HIP(hipStreamSynchronize(B->stream));
-        if (has_error()) return 0;
-        for (int i = 0; i < n; ++i) outs[k][i] = Vector3D{tmp[i].x, tmp[i].y, tmp[i].z};
-    }
+    const size_t row = 3 * (size_t)n;
+    B->h_out.reserve(3 * row);
+    if (has_error()) return 0;
+    HostArray a[3];
+    for (int k = 0; k < 3; ++k)
+        a[k] = HostArray{reinterpret_cast<double*>(srcs[k]->as<double4>() + a0), B->h_out.p + k * row, outs[k] ? row : 0, row, 3};
+    to_host(a, 3, B->h_out.pinned, B->stream);
+    TMD_HIP(hipStreamSynchronize(B->stream));
+    if (has_error()) return 0;
+    for (int k = 0; k < 3; ++k)
+        if (outs[k]) host_copy({{outs[k], B->h_out.p + k * row, sizeof(double) * row}});
     return n;
 }
 

@@ -154,54 +154,54 @@ static void alloc_atoms(Sim& s, int cap) {
 }
 
 static void upload(Sim& s) {
-    // the host mirror holds the locals and, after a download, the ghosts
-    const int nall = std::min<int>(s.n + s.ng, (int)std::min(s.h_pos.size(), s.h_vel.size()) / 3);
-    if (nall < s.n || (int)s.h_mass.size() < nall || (int)s.h_force.size() < 3 * s.n) {
+    // the host copy holds the locals and, after a download, the ghosts
+    HostAtoms& h = s.host;
+    const int nall = std::min(s.n + s.ng, h.count);
+    if (nall < s.n) {
         set_error(__FILE__, __LINE__, "host mirror smaller than the number of local atoms");
         return;
     }
     if (nall == 0) return;
     alloc_atoms(s, std::max(s.cap_all, nall));
-    std::vector<double4> p(nall), v(nall);
-    for (int i = 0; i < nall; ++i) {
-        p[i] = make_double4(s.h_pos[3 * i], s.h_pos[3 * i + 1], s.h_pos[3 * i + 2], 0.0);
-        v[i] = make_double4(s.h_vel[3 * i], s.h_vel[3 * i + 1], s.h_vel[3 * i + 2], 0.0);
-    }
+    if (has_error()) return;
     mirror_invalidate(s);
     s.pos_stale = 0;  // pos and vel are uploaded whole
     s.vel_mirrored = 0;
     s.vel_mirror_wanted = 0;
-    TMD_HIP(hipMemcpyAsync(s.pos.p, p.data(), sizeof(double4) * nall, hipMemcpyHostToDevice, s.stream));
-    TMD_HIP(hipMemcpyAsync(s.vel.p, v.data(), sizeof(double4) * nall, hipMemcpyHostToDevice, s.stream));
-    TMD_HIP(hipMemcpyAsync(s.mass.p, s.h_mass.data(), sizeof(double) * nall, hipMemcpyHostToDevice, s.stream));
-    std::vector<double4> f(s.n);
-    for (int i = 0; i < s.n; ++i) f[i] = make_double4(s.h_force[3 * i], s.h_force[3 * i + 1], s.h_force[3 * i + 2], 0.0);
-    TMD_HIP(hipMemcpyAsync(s.force.p, f.data(), sizeof(double4) * s.n, hipMemcpyHostToDevice, s.stream));
+    const size_t a = (size_t)nall, n = (size_t)s.n;
+    const HostArray arrays[4] = {{s.pos.as<double>(), h.pos(), 3 * a, 3 * a, 3},
+                                 {s.vel.as<double>(), h.vel(), 3 * a, 3 * a, 3},
+                                 {s.force.as<double>(), h.force(), 3 * n, h.no_force ? 0 : 3 * n, 3},
+                                 {s.mass.as<double>(), h.mass(), a, a, 1}};
+    to_device(arrays, 4, h.buf.pinned, s.stream);
     TMD_HIP(hipStreamSynchronize(s.stream));
     s.dev_valid = true;
 }
 
 static void download(Sim& s) {
+    HostAtoms& h = s.host;
     const int nall = s.n + s.ng;
-    s.h_pos.resize(3 * (size_t)nall);
-    s.h_vel.resize(3 * (size_t)nall);
-    s.h_mass.resize(nall);
-    s.h_force.assign(3 * (size_t)nall, 0.0);
-    if (nall == 0 || !s.dev_valid) return;
-    std::vector<double4> p(nall), v(nall), f(std::max(s.n, 1));
-    TMD_HIP(hipMemcpyAsync(p.data(), s.pos.p, sizeof(double4) * nall, hipMemcpyDeviceToHost, s.stream));
-    TMD_HIP(hipMemcpyAsync(v.data(), s.vel.p, sizeof(double4) * nall, hipMemcpyDeviceToHost, s.stream));
-    TMD_HIP(hipMemcpyAsync(s.h_mass.data(), s.mass.p, sizeof(double) * nall, hipMemcpyDeviceToHost, s.stream));
-    if (s.n) TMD_HIP(hipMemcpyAsync(f.data(), s.force.p, sizeof(double4) * s.n, hipMemcpyDeviceToHost, s.stream));
-    TMD_HIP(hipStreamSynchronize(s.stream));
+    h.reserve(nall);
     if (has_error()) return;
-    for (int i = 0; i < nall; ++i) {
-        s.h_pos[3 * i] = p[i].x; s.h_pos[3 * i + 1] = p[i].y; s.h_pos[3 * i + 2] = p[i].z;
-        s.h_vel[3 * i] = v[i].x; s.h_vel[3 * i + 1] = v[i].y; s.h_vel[3 * i + 2] = v[i].z;
+    const int had = h.count;
+    h.count = nall;
+    if (nall == 0 || !s.dev_valid) {
+        h.no_force = true;
+        if (had < nall) {
+            const size_t add = sizeof(double) * (size_t)(nall - had);
+            host_copy({{h.pos() + 3 * (size_t)had, nullptr, 3 * add}, {h.vel() + 3 * (size_t)had, nullptr, 3 * add},
+                       {h.mass() + had, nullptr, add}});
+        }
+        return;
     }
-    for (int i = 0; i < s.n; ++i) {
-        s.h_force[3 * i] = f[i].x; s.h_force[3 * i + 1] = f[i].y; s.h_force[3 * i + 2] = f[i].z;
-    }
+    const size_t a = (size_t)nall, n = (size_t)s.n;
+    const HostArray arrays[4] = {{s.pos.as<double>(), h.pos(), 3 * a, 3 * a, 3},
+                                 {s.vel.as<double>(), h.vel(), 3 * a, 3 * a, 3},
+                                 {s.force.as<double>(), h.force(), 3 * a, 3 * n, 3},
+                                 {s.mass.as<double>(), h.mass(), a, a, 1}};
+    h.no_force = false;
+    to_host(arrays, 4, h.buf.pinned, s.stream);
+    TMD_HIP(hipStreamSynchronize(s.stream));
 }
 
 // device operations need the atoms on the device; the reference requires an
@@ -236,12 +236,74 @@ void make_geom(Geom& G, const double* aabb, const double* rank_aabb, double cell
     G.ncells = G.nx * G.ny * G.nz;
 }
 
+template <class F>
+static void each_buffer(Sim& s, F&& f) {
+    DevBuf* bufs[] = {&s.pos, &s.vel, &s.force, &s.mass, &s.sort_buf, &s.g_owner, &s.g_src, &s.g_code, &s.cell_of, &s.cell_slot,
+                      &s.cell_count, &s.cell_start, &s.cell_parts, &s.cell_inv, &s.work_start, &s.work, &s.work_k, &s.work_c, &s.g_ko, &s.g_kg, &s.gh_pack, &s.gh_w, &s.gh_k, &s.gh_e, &s.g_cell, &s.g_slot, &s.cell_parts2, &s.cell_inv2, &s.cell_pair,
+                      &s.cell_src, &s.cls, &s.tile_start, &s.spos, &s.spos2, &s.face, &s.svel, &s.svel2,
+                      &s.nb_count, &s.nb_list, &s.nb_count2, &s.nb_list2,
+                      &s.scan_blocks, &s.scan_aux, &s.red, &s.gbuf, &s.adj_x0, &s.adj_v0, &s.adj_ckx,
+                      &s.adj_ckv, &s.adj_segx, &s.adj_segv, &s.adj_xbar, &s.adj_vbar, &s.adj_fbar, &s.adj_part,
+                      &s.adj_acc, &s.adj_mir};
+    for (DevBuf* b : bufs) f(*b);
+}
+
+static void release_memory(Sim& s) {
+    each_buffer(s, [](DevBuf& b) { b.release(); });
+    s.host.release();
+    s.h_out.release();
+    if (s.h_stats) {
+        (void)hipHostFree(s.h_stats);
+        s.h_stats = nullptr;
+    }
+    s.cap_all = 0;
+}
+
+// nothing derived from the atoms holds any longer
+static void reset_state(Sim& s) {
+    s.ng = 0;
+    s.windows_pending = 0;
+    s.max_window = 0;
+    s.tile_auto[0] = s.tile_auto[1] = s.tile_auto[2] = 0;
+    s.tile_tuned = 0;
+    s.stage_bytes = kPosStageBytes;
+    s.stage_budget = kLdsBudget;
+    s.nb_valid = 0;
+    s.windows_valid = 0;
+    s.inv_valid = 0;
+    mirror_invalidate(s);
+    s.pos_stale = 0;
+    s.vel_mirrored = 0;
+    s.vel_mirror_wanted = 0;
+    s.ghost_pos_stale = 0;
+    s.dem_mirrored = 0;
+    s.gsrc_valid = 0;
+    s.gh_valid = s.gh_packed = 0;
+    s.nbinned = 0;
+    s.dev_valid = false;
+}
+
+// A simulation made over another one takes its memory, on the device and
+// the pinned host arrays, if it needs from half of it to all of it (by atoms
+// and expected ghosts) and that is no more than 8 GiB in all; else, and from
+// md_deallocate_grid, all of it goes back first.  At 80^3 cells (2,048,000
+// atoms) giving back and allocating anew cost 16 ms of the next simulation's
+// creation (17.5 against 1.4), 1.2 of its first list build (2.3, 1.1) and 9 of
+// its first reads of freshly pinned pages (11.5, 2.4).
+constexpr size_t kTakeOverBytes = size_t(8) << 30;
+static void replace_memory(Sim& s, long long room) {
+    TMD_HIP(hipStreamSynchronize(s.stream));
+    size_t held = sizeof(double) * (s.host.buf.doubles + s.h_out.doubles);
+    each_buffer(s, [&](const DevBuf& b) { held += b.bytes; });
+    if (room > s.cap_all || room < s.cap_all / 2 || held > kTakeOverBytes) release_memory(s);
+}
+
 static double host_temperature(const Sim& s) {
     // core/thermo.impala:1-16 on the host mirror
     const double t_scale = 1.0 / (double)(s.n * 3 - 3);
     double t = 0.0;
     for (int i = 0; i < s.n; ++i) {
-        const double* v = &s.h_vel[3 * i];
+        const double* v = s.host.vel() + 3 * (size_t)i;
         t += (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]) * 1.0;
     }
     return t * t_scale;
@@ -339,34 +401,23 @@ int md_initialize_grid(double const* masses, struct Vector3D const* positions, s
         set_error(__FILE__, __LINE__, "md_initialize_grid: cell grid too large");
         return 0;
     }
-    s.n = nparticles;
-    s.ng = 0;
-    s.nb_cap = neighborlist_capacity > 0 ? neighborlist_capacity : 1;
-    s.nb_valid = 0;
-    s.windows_valid = 0;
-    s.inv_valid = 0;
-    mirror_invalidate(s);
-    s.pos_stale = 0;
-    s.vel_mirrored = 0;
-    s.vel_mirror_wanted = 0;
-    s.ghost_pos_stale = 0;
-    s.dem_mirrored = 0;
-    s.gsrc_valid = 0;
-    s.gh_valid = s.gh_packed = 0;
-    s.h_mass.assign(masses, masses + nparticles);
-    s.h_pos.resize(3 * (size_t)nparticles);
-    s.h_vel.resize(3 * (size_t)nparticles);
-    s.h_force.assign(3 * (size_t)nparticles, 0.0);
-    for (int i = 0; i < nparticles; ++i) {
-        s.h_pos[3 * i] = positions[i].x; s.h_pos[3 * i + 1] = positions[i].y; s.h_pos[3 * i + 2] = positions[i].z;
-        s.h_vel[3 * i] = velocities[i].x; s.h_vel[3 * i + 1] = velocities[i].y; s.h_vel[3 * i + 2] = velocities[i].z;
-    }
-    s.dev_valid = false;
     // ghosts of a cube of side L with a shell of width s: ~ N ((1 + 2s/L)^3 - 1)
     double shell = 1.0;
     for (int d = 0; d < 3; ++d) shell *= 1.0 + 2.0 * cell_spacing / s.g.len[d];
     const long long est = (long long)nparticles + (long long)(nparticles * (shell - 1.0) * 1.25) + 4096;
+    replace_memory(s, est);
+    reset_state(s);
+    s.n = nparticles;
+    s.nb_cap = neighborlist_capacity > 0 ? neighborlist_capacity : 1;
     alloc_atoms(s, (int)std::min<long long>(est, 0x7fffffffLL));
+    HostAtoms& h = s.host;
+    h.count = 0;
+    h.reserve(s.cap_all);  // room for the ghosts of a download
+    if (has_error()) return 0;
+    h.count = nparticles;
+    h.no_force = true;
+    const size_t row = sizeof(double) * (size_t)nparticles;
+    host_copy({{h.mass(), masses, row}, {h.pos(), positions, 3 * row}, {h.vel(), velocities, 3 * row}});
     return has_error() ? 0 : nparticles;
 }
 
@@ -419,29 +470,27 @@ void md_enforce_pbc() {
     finish(s);
 }
 
+static void write_atoms(const HostAtoms& h, int first, int last, double* masses, struct Vector3D* positions,
+                        struct Vector3D* velocities, struct Vector3D* forces) {
+    static_assert(sizeof(Vector3D) == 3 * sizeof(double), "packed triples");
+    if (last <= first) return;
+    const size_t f = (size_t)first, row = sizeof(double) * (size_t)(last - first);
+    host_copy({{masses, h.mass() + f, row},
+               {positions, h.pos() + 3 * f, 3 * row},
+               {velocities, h.vel() + 3 * f, 3 * row},
+               {forces, h.no_force ? nullptr : h.force() + 3 * f, 3 * row}});
+}
+
 int md_write_grid_data_to_arrays(double* masses, struct Vector3D* positions, struct Vector3D* velocities, struct Vector3D* forces) {
     Sim& s = sim();
-    const int n = std::min<int>(s.n, (int)s.h_mass.size());
-    for (int i = 0; i < n; ++i) {
-        masses[i] = s.h_mass[i];
-        positions[i] = {s.h_pos[3 * i], s.h_pos[3 * i + 1], s.h_pos[3 * i + 2]};
-        velocities[i] = {s.h_vel[3 * i], s.h_vel[3 * i + 1], s.h_vel[3 * i + 2]};
-        forces[i] = {s.h_force[3 * i], s.h_force[3 * i + 1], s.h_force[3 * i + 2]};
-    }
+    write_atoms(s.host, 0, std::min(s.n, s.host.count), masses, positions, velocities, forces);
     return s.n;
 }
 
 int md_write_grid_ghost_data_to_arrays(double* masses, struct Vector3D* positions, struct Vector3D* velocities,
                                        struct Vector3D* forces) {
     Sim& s = sim();
-    const int nall = std::min<int>(s.n + s.ng, (int)s.h_mass.size());
-    for (int i = s.n; i < nall; ++i) {
-        const int g = i - s.n;
-        masses[g] = s.h_mass[i];
-        positions[g] = {s.h_pos[3 * i], s.h_pos[3 * i + 1], s.h_pos[3 * i + 2]};
-        velocities[g] = {s.h_vel[3 * i], s.h_vel[3 * i + 1], s.h_vel[3 * i + 2]};
-        forces[g] = {s.h_force[3 * i], s.h_force[3 * i + 1], s.h_force[3 * i + 2]};
-    }
+    write_atoms(s.host, s.n, std::min(s.n + s.ng, s.host.count), masses, positions, velocities, forces);
     return s.n;  // the reference returns nparticles here (core/grid.impala:517)
 }
 
@@ -564,7 +613,7 @@ int tmd_save_state(const char* path) {
     const size_t n = (size_t)s.n;
     bool ok = fwrite(&h, sizeof h, 1, fp) == 1;
     sum = fnv1a(&h, sizeof h, sum);
-    const void* parts[4] = {s.h_mass.data(), s.h_pos.data(), s.h_vel.data(), s.h_force.data()};
+    const void* parts[4] = {s.host.mass(), s.host.pos(), s.host.vel(), s.host.force()};
     const size_t lens[4] = {n, 3 * n, 3 * n, 3 * n};
     for (int k = 0; k < 4 && ok; ++k) {
         ok = fwrite(parts[k], sizeof(double), lens[k], fp) == lens[k];
@@ -614,7 +663,8 @@ int tmd_load_state(const char* path) {
     md_initialize_grid(m.data(), reinterpret_cast<const Vector3D*>(x.data()), reinterpret_cast<const Vector3D*>(v.data()), h.n,
                        h.world, h.rank, h.spacing, 0, h.nb_cap);
     if (has_error()) return 0;
-    s.h_force = f;
+    host_copy({{s.host.force(), f.data(), sizeof(double) * f.size()}});
+    s.host.no_force = false;
     s.precision = h.precision;
     s.half_mode = h.half_mode;
     s.ghost_mode = h.ghost_mode;
@@ -650,54 +700,25 @@ void md_deallocate_grid() {
     Sim& s = *g_sim;
     if (s.stream) (void)hipStreamSynchronize(s.stream);
     s.timer.collect();
-    DevBuf* bufs[] = {&s.pos, &s.vel, &s.force, &s.mass, &s.sort_buf, &s.g_owner, &s.g_src, &s.g_code, &s.cell_of, &s.cell_slot,
-                      &s.cell_count, &s.cell_start, &s.cell_parts, &s.cell_inv, &s.work_start, &s.work, &s.work_k, &s.work_c, &s.g_ko, &s.g_kg, &s.gh_pack, &s.gh_w, &s.gh_k, &s.gh_e, &s.g_cell, &s.g_slot, &s.cell_parts2, &s.cell_inv2, &s.cell_pair,
-                      &s.cell_src, &s.cls, &s.tile_start, &s.spos, &s.spos2, &s.face, &s.svel, &s.svel2,
-                      &s.nb_count, &s.nb_list, &s.nb_count2, &s.nb_list2,
-                      &s.scan_blocks, &s.scan_aux, &s.red, &s.gbuf, &s.adj_x0, &s.adj_v0, &s.adj_ckx,
-                      &s.adj_ckv, &s.adj_segx, &s.adj_segv, &s.adj_xbar, &s.adj_vbar, &s.adj_fbar, &s.adj_part,
-                      &s.adj_acc, &s.adj_mir};
-    for (DevBuf* b : bufs) b->release();
-    if (s.h_stats) {
-        (void)hipHostFree(s.h_stats);
-        s.h_stats = nullptr;
-    }
-    s.windows_pending = 0;
-    s.max_window = 0;
-    s.tile_auto[0] = s.tile_auto[1] = s.tile_auto[2] = 0;
-    s.tile_tuned = 0;
-    s.stage_bytes = kPosStageBytes;
-    s.stage_budget = kLdsBudget;
-    s.n = s.ng = 0;
-    s.cap_all = 0;
-    s.nb_valid = 0;
-    s.windows_valid = 0;
-    s.inv_valid = 0;
-    mirror_invalidate(s);
-    s.pos_stale = 0;
-    s.vel_mirrored = 0;
-    s.vel_mirror_wanted = 0;
-    s.ghost_pos_stale = 0;
-    s.gsrc_valid = 0;
-    s.gh_valid = s.gh_packed = 0;
-    s.nbinned = 0;
-    s.dev_valid = false;
+    release_memory(s);
+    reset_state(s);
+    s.n = 0;
 }
 
 void md_print_grid() {
     Sim& s = sim();
-    for (int i = 0; i < s.n && 3 * i + 2 < (int)s.h_pos.size(); ++i)
-        printf("0> pos_local: %g, %g, %g\n", s.h_pos[3 * i], s.h_pos[3 * i + 1], s.h_pos[3 * i + 2]);
-    for (int i = 0; i < s.n && 3 * i + 2 < (int)s.h_vel.size(); ++i)
-        printf("0> vel_local: %g, %g, %g\n", s.h_vel[3 * i], s.h_vel[3 * i + 1], s.h_vel[3 * i + 2]);
+    for (int i = 0; i < s.n && i < s.host.count; ++i)
+        printf("0> pos_local: %g, %g, %g\n", s.host.pos()[3 * i], s.host.pos()[3 * i + 1], s.host.pos()[3 * i + 2]);
+    for (int i = 0; i < s.n && i < s.host.count; ++i)
+        printf("0> vel_local: %g, %g, %g\n", s.host.vel()[3 * i], s.host.vel()[3 * i + 1], s.host.vel()[3 * i + 2]);
 }
 
 void md_print_ghost() {
     Sim& s = sim();
-    for (int i = s.n; i < s.n + s.ng && 3 * i + 2 < (int)s.h_pos.size(); ++i)
-        printf("0> pos_ghost: %g, %g, %g\n", s.h_pos[3 * i], s.h_pos[3 * i + 1], s.h_pos[3 * i + 2]);
-    for (int i = s.n; i < s.n + s.ng && 3 * i + 2 < (int)s.h_vel.size(); ++i)
-        printf("0> vel_ghost: %g, %g, %g\n", s.h_vel[3 * i], s.h_vel[3 * i + 1], s.h_vel[3 * i + 2]);
+    for (int i = s.n; i < s.n + s.ng && i < s.host.count; ++i)
+        printf("0> pos_ghost: %g, %g, %g\n", s.host.pos()[3 * i], s.host.pos()[3 * i + 1], s.host.pos()[3 * i + 2]);
+    for (int i = s.n; i < s.n + s.ng && i < s.host.count; ++i)
+        printf("0> vel_ghost: %g, %g, %g\n", s.host.vel()[3 * i], s.host.vel()[3 * i + 1], s.host.vel()[3 * i + 2]);
 }
 
 void md_create_velocity(double t_request) {
@@ -706,14 +727,14 @@ void md_create_velocity(double t_request) {
     if (has_error() || s.n <= 1) return;
     double vt[3] = {0.0, 0.0, 0.0};
     for (int i = 0; i < s.n; ++i)
-        for (int e = 0; e < 3; ++e) vt[e] = vt[e] + s.h_vel[3 * i + e];
+        for (int e = 0; e < 3; ++e) vt[e] = vt[e] + s.host.vel()[3 * i + e];
     for (int e = 0; e < 3; ++e) vt[e] = vt[e] / (double)s.n;
     for (int i = 0; i < s.n; ++i)
-        for (int e = 0; e < 3; ++e) s.h_vel[3 * i + e] = s.h_vel[3 * i + e] - vt[e];
+        for (int e = 0; e < 3; ++e) s.host.vel()[3 * i + e] = s.host.vel()[3 * i + e] - vt[e];
     const double t = host_temperature(s);
     const double factor = std::sqrt(t_request / t);
     for (int i = 0; i < s.n; ++i)
-        for (int e = 0; e < 3; ++e) s.h_vel[3 * i + e] = s.h_vel[3 * i + e] * factor;
+        for (int e = 0; e < 3; ++e) s.host.vel()[3 * i + e] = s.host.vel()[3 * i + e] * factor;
     s.dev_valid = false;
 }
 
@@ -784,9 +805,9 @@ void md_compute_boundary_weights(double xmin, double xmax, double ymin, double y
     // bounds, core/grid.impala:413-417), counted on the host mirror
     Sim& s = sim();
     unsigned long int c = 0, g = 0;
-    const int nall = std::min<int>(s.n + s.ng, (int)(s.h_pos.size() / 3));
+    const int nall = std::min(s.n + s.ng, s.host.count);
     for (int i = 0; i < nall; ++i) {
-        const double* p = &s.h_pos[3 * i];
+        const double* p = &s.host.pos()[3 * i];
         const bool in = p[0] >= xmin && p[0] <= xmax && p[1] >= ymin && p[1] <= ymax && p[2] >= zmin && p[2] <= zmax;
         if (in) (i < s.n ? c : g)++;
     }
@@ -826,7 +847,7 @@ void md_report_iterations() {
 void md_report_particles() {
     Sim& s = sim();
     printf("# Local # Ghost Temp\n");
-    printf("%d %d %g \n", s.n, s.ng, (int)s.h_vel.size() >= 3 * s.n && s.n > 1 ? host_temperature(s) : 0.0);
+    printf("%d %d %g \n", s.n, s.ng, s.host.count >= s.n && s.n > 1 ? host_temperature(s) : 0.0);
     fflush(stdout);
 }
 

@@ -83,6 +83,46 @@ struct DevBuf {
     template <class T> T* as() const { return reinterpret_cast<T*>(p); }
 };
 
+// Host memory that kernels read and write directly (pinned; ordinary memory
+// where no more can be pinned).
+struct HostBuf {
+    double* p = nullptr;
+    size_t doubles = 0;
+    bool pinned = false;
+    void reserve(size_t need, size_t keep = 0);  // keep: doubles carried over
+    void release();
+};
+// The host's copy of the atoms, locals then ghosts: three packed triples and
+// a mass each.
+struct HostAtoms {
+    HostBuf buf;
+    int cap = 0, count = 0;
+    bool no_force = true;  // every force is zero and none has been written
+    double* pos() const { return buf.p; }
+    double* vel() const { return buf.p + 3 * (size_t)cap; }
+    double* force() const { return buf.p + 6 * (size_t)cap; }
+    double* mass() const { return buf.p + 9 * (size_t)cap; }
+    void reserve(int atoms);  // keeps what is there
+    void release();
+};
+// width 3: triples against 32-B device rows; 1: plain doubles.  Beyond the
+// first `have` doubles of `count` the source is taken as zero.
+struct HostArray {
+    double* dev;
+    double* host;
+    size_t count, have;
+    int width;
+};
+constexpr int kHostArrays = 4;
+void to_host(const HostArray* a, int na, bool pinned, hipStream_t st);    // not waited for where pinned
+void to_device(const HostArray* a, int na, bool pinned, hipStream_t st);
+struct HostSpan {
+    void* to;
+    const void* from;  // nullptr: zeros
+    size_t bytes;
+};
+void host_copy(std::initializer_list<HostSpan> spans);
+
 // Per-kernel timing with HIP events on the library stream.
 enum KernelId {
     K_FORCE = 0, K_INTEGRATE_1, K_INTEGRATE_2, K_GHOST_SYNC, K_NEIGHBOR, K_BIN, K_BORDERS,
@@ -150,9 +190,8 @@ struct Sim {
     int lj_shift = 0;
 
     // host mirrors (filled by md_copy_data_from_accelerator)
-    std::vector<double> h_mass;
-    std::vector<double> h_pos, h_vel, h_force;  // AoS 3 doubles per atom (locals + ghosts)
-    bool host_valid = true;                     // host mirror is the newest copy
+    HostAtoms host;
+    HostBuf h_out;  // results on their way out (gradients)
     bool dev_valid = false;
 
     // device state

@@ -120,7 +120,7 @@ class Batch:
 
     def state(self, rep):
         n = int(self.counts[rep])
-        x = np.zeros((n, 3)); v = np.zeros((n, 3)); f = np.zeros((n, 3))
+        x = np.empty((n, 3)); v = np.empty((n, 3)); f = np.empty((n, 3))
         self.L.tmd_batch_get_state(self.h, rep, _vptr(x), _vptr(v), _vptr(f))
         check()
         return x, v, f

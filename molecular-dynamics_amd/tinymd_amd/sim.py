@@ -67,22 +67,27 @@ class Simulation:
                  dem_radius=None, sync=True, sort=False):
         self.L = L = load()
         L.tmd_clear_error()
-        L.md_deallocate_grid()
-        self.set_modes(precision, half_mode, ghost_mode, lj_shift, dem_radius, sync)
-        L.tmd_set_sort_particles(int(bool(sort)))
-        # tile shape and block size are library-wide settings: a new
-        # simulation starts from the automatic ones (set_tile after this)
-        L.tmd_set_tile(0, 0, 0)
-        L.tmd_set_tile_threads(0)
-        m = np.ascontiguousarray(masses, dtype=np.float64)
-        x = np.ascontiguousarray(positions, dtype=np.float64).reshape(-1, 3)
-        v = np.ascontiguousarray(velocities, dtype=np.float64).reshape(-1, 3)
-        self.aabb = np.ascontiguousarray(aabb, dtype=np.float64)
-        ra = self.aabb if rank_aabb is None else np.ascontiguousarray(rank_aabb, dtype=np.float64)
-        self.cell_spacing = cell_spacing
-        n = L.md_initialize_grid(_dptr(m), _vptr(x), _vptr(v), len(m), _dptr(self.aabb), _dptr(ra),
-                                 cell_spacing, cell_cap, nb_cap)
-        check()
+        # a simulation takes over the memory of the one it replaces
+        # (md_initialize_grid); close() gives it back
+        try:
+            self.set_modes(precision, half_mode, ghost_mode, lj_shift, dem_radius, sync)
+            L.tmd_set_sort_particles(int(bool(sort)))
+            # tile shape and block size are library-wide settings: a new
+            # simulation starts from the automatic ones (set_tile after this)
+            L.tmd_set_tile(0, 0, 0)
+            L.tmd_set_tile_threads(0)
+            m = np.ascontiguousarray(masses, dtype=np.float64)
+            x = np.ascontiguousarray(positions, dtype=np.float64).reshape(-1, 3)
+            v = np.ascontiguousarray(velocities, dtype=np.float64).reshape(-1, 3)
+            self.aabb = np.ascontiguousarray(aabb, dtype=np.float64)
+            ra = self.aabb if rank_aabb is None else np.ascontiguousarray(rank_aabb, dtype=np.float64)
+            self.cell_spacing = cell_spacing
+            n = L.md_initialize_grid(_dptr(m), _vptr(x), _vptr(v), len(m), _dptr(self.aabb), _dptr(ra),
+                                     cell_spacing, cell_cap, nb_cap)
+            check()
+        except Exception:
+            L.md_deallocate_grid()
+            raise
         self.n = n
 
     # ---- modes
@@ -274,7 +279,7 @@ class Simulation:
         """(m, x, v, f) of the locals after a device -> host copy."""
         self.copy_from_accelerator()
         n = self.nlocal
-        m = np.zeros(n); x = np.zeros((n, 3)); v = np.zeros((n, 3)); f = np.zeros((n, 3))
+        m = np.empty(n); x = np.empty((n, 3)); v = np.empty((n, 3)); f = np.empty((n, 3))
         self.L.md_write_grid_data_to_arrays(_dptr(m), _vptr(x), _vptr(v), _vptr(f))
         check()
         return m, x, v, f
