@@ -475,7 +475,6 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_b_nlist(const RepDesc* __re
                                                           int* __restrict__ nb_count, nb_t* __restrict__ nb_list,
                                                           int* __restrict__ flags) {
     extern __shared__ double dyn[];
-    int* cst = reinterpret_cast<int*>(reinterpret_cast<char*>(dyn) + (size_t)kStageBytes * a.wcap);
     const int tile = blockIdx.x;
     const int w0 = tile_start[tile], nloc = tile_start[tile + 1] - w0;
     if (nloc == 0) return;
@@ -485,19 +484,19 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_b_nlist(const RepDesc* __re
     aa.g = D.g;
     const int* st = start + D.c0;
     __shared__ TileWin W;
+    __shared__ unsigned maxr;
+    if (threadIdx.x == 0) maxr = 0u;
+    ListWin L = list_win(dyn, a.wcap, D.g, spos[work_k[w0 + nloc / 2]]);
     tile_window(tile - D.t0, st, D.g, W);
-    stage_row_starts(W, st, D.g, cst);
-    const WinStage sp = win_stage(dyn, a.wcap);
-    const bool staged = stage_window(W, a.wcap, spos, nullptr, sp, kListPad);
+    stage_row_starts(W, st, D.g, L.cst);
+    const bool staged = stage_list_window<false>(W, a.wcap, spos, nullptr, a.cut2, L, &maxr);
     for (int at = threadIdx.x; at < nloc; at += blockDim.x) {
         const int w = w0 + at;
-        const int i = work[w];
+        const int c = cell_of[work[w]];
         const int k = work_k[w];  // its mirror index (the mirror is current)
         int unused = 0;
-        const int cnt = staged ? nlist_atom<false, true>(i, w, cell_of[i], k, spos[k], cst, aa, W, sp, spos, parts, nb_list,
-                                                         nullptr, unused)
-                               : nlist_atom<false, false>(i, w, cell_of[i], k, spos[k], cst, aa, W, sp, spos, parts, nb_list,
-                                                          nullptr, unused);
+        const int cnt = staged ? nlist_atom<false, true>(0, w, c, k, spos[k], aa, W, L, spos, parts, nb_list, nullptr, unused)
+                               : nlist_atom<false, false>(0, w, c, k, spos[k], aa, W, L, spos, parts, nb_list, nullptr, unused);
         nb_count[w] = cnt;
         if (cnt > a.cap) atomicMax(&flags[FL_LIST], cnt);
     }
@@ -651,6 +650,7 @@ struct Batch {
     std::vector<RepDesc> R;
     int n_sb = 0, n_eb = 0, n_cb = 0, n_gb = 0, n_tiles = 0, n_cells = 0, n_slots = 0, n_work = 0;
     int list_cap = 8, wcap = 0;
+    int max_window = 0;              // largest window of the set-ups so far
     int threads = kTileThreads;      // tile block size in use (cfg.threads, or automatic at set-up)
     DevBuf dR, sb_rep, eb_rep, cb_rep, gb_rep, tile_rep, cell_rep;
     DevBuf pos, vel, force, g_owner, g_code, cell_of, cell_slot, cell_inv, parts, spos, spos2;
@@ -905,21 +905,20 @@ static void enq_unmirror(Batch& B, const DevBuf& m) {
                        B.pos.as<double4>());
 }
 
-// LDS layout of the list-build launch: the row starts of the largest tile
-// shape among the replicas (rsb bytes) after the staged window, whose atom
-// capacity is what the budget leaves.  These values are baked into a
+// LDS layout of the list-build launch: the staged window with a sixteenth of
+// room over the largest one of the set-up, the row starts of the largest tile
+// shape among the replicas (rsb bytes), the wavefronts' rings.  These values are baked into a
 // captured run, so graph_signature includes them.
 struct NlistLds {
-    int rsb, wcap;
-    size_t bytes;
+    int rsb;
+    ListLds l;
 };
 
 static NlistLds nlist_lds(const Batch& B) {
     NlistLds l;
     l.rsb = 0;
     for (const RepDesc& D : B.R) l.rsb = std::max(l.rsb, row_starts_bytes(D.g));
-    l.wcap = std::min(B.wcap, (kLdsBudget - l.rsb) / kStageBytes);
-    l.bytes = (size_t)l.wcap * kStageBytes + l.rsb;
+    l.l = list_lds(B.max_window + B.max_window / 16 + 16, l.rsb, B.threads / kWave);
     return l;
 }
 
@@ -929,11 +928,10 @@ static void enq_nlist(Batch& B, const DevBuf& m) {
     a.half = 0;
     a.half_mode = HALF_GHOST_FULL;
     const NlistLds l = nlist_lds(B);
-    a.wcap = l.wcap;
+    a.wcap = l.l.wcap;
     const double cut = B.rc + B.skin;
     a.cut2 = cut * cut;
-    const size_t lds = l.bytes;
-    hipLaunchKernelGGL(k_b_nlist, dim3(B.n_tiles), dim3(B.threads), lds, B.stream, (const RepDesc*)B.dR.as<RepDesc>(),
+    hipLaunchKernelGGL(k_b_nlist, dim3(B.n_tiles), dim3(l.l.waves * kWave), l.l.bytes, B.stream, (const RepDesc*)B.dR.as<RepDesc>(),
                        (const int*)B.tile_rep.as<int>(), CMir{m.as<double>()}, (const int*)B.work_k.as<int>(),
                        (const int*)B.cell_of.as<int>(), (const int*)B.cell_start.as<int>(),
                        (const int*)B.parts.as<int>(),
@@ -1096,6 +1094,7 @@ static bool setup_lists(Batch& B) {
         const int maxwin = fl[FL_MAXWIN];
         B.threads = tile_block_threads(B.cfg.threads, fl[FL_MAXLOC]);
         // capacities only grow, so a restart keeps a captured run valid
+        B.max_window = std::max(B.max_window, maxwin);
         B.wcap = std::max(B.wcap, std::min(maxwin + maxwin / 4 + 64, kLdsBudget / kStageBytes));
         enq_mirror(B, B.spos);
         for (int k = 0; k < 4 && !has_error(); ++k) {
@@ -1125,7 +1124,7 @@ static bool setup_from_initial(Batch& B, bool fresh = true) {
     if (has_error()) return false;
     if (fresh) {
         B.list_cap = 8;
-        B.wcap = 0;
+        B.wcap = B.max_window = 0;
     }
     upload_initial(B);
     if (has_error()) return false;
@@ -1150,7 +1149,7 @@ static std::vector<unsigned long long> graph_signature(const Batch& B) {
     }
     const NlistLds l = nlist_lds(B);
     const int iv[] = {B.reneigh, B.precision, B.shift, B.list_cap, B.wcap, B.threads, B.n_sb, B.n_eb, B.n_cb, B.n_gb,
-                      B.n_tiles, B.n_cells, B.n_slots, B.nrep, l.rsb, l.wcap, (int)l.bytes};
+                      B.n_tiles, B.n_cells, B.n_slots, B.nrep, l.rsb, l.l.wcap, l.l.bytes};
     for (int v : iv) s.push_back((unsigned long long)(unsigned)v);
     // the host-side tile shapes behind the launch sizes above: two layouts
     // with equal totals but different tile edges must not share a graph

@@ -3,12 +3,12 @@
 // (tmd_window.hpp).
 //
 // List build: one block per tile, one lane per local atom of the tile.  The
-// block stages its window (atom index + FP64 position) into LDS; each lane
-// walks its 27-cell stencil as 9 rows of 3 cells inside the window, in the
-// reference's order -- stencil (z, y, x), then cell order
+// block stages its window (FP32 position relative to the tile, atom index)
+// into LDS; each lane walks its 27-cell stencil as 9 rows of 3 cells inside
+// the window, in the reference's order -- stencil (z, y, x), then cell order
 // (core/neighborlist.impala:1-78) -- and keeps a candidate when
-// `rsq <= r_nb^2` in FP64 without contraction, so the sets are bit-exact with
-// the reference.  Half lists keep j < i among locals (the reference's
+// `rsq <= r_nb^2` in FP64 without contraction, decided in FP32 where that is
+// certain (nlist_atom), so the sets are bit-exact with the reference.  Half lists keep j < i among locals (the reference's
 // filter) plus, by default, every ghost.
 #include "tmd_internal.hpp"
 #include "tmd_pair.hpp"
@@ -38,26 +38,23 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_nlist(const CMir spos, cons
                                                         int* __restrict__ nb_count2, nb_t* __restrict__ nb_list2,
                                                         int* __restrict__ overflow) {
     extern __shared__ double dyn[];
-    // half lists stage the atom index too (the i < j test), full lists positions only
-    constexpr int SB = HALF ? kStageBytes : kPosStageBytes;
-    int* cst = reinterpret_cast<int*>(reinterpret_cast<char*>(dyn) + (size_t)SB * a.wcap);
     const int tile = blockIdx.x;
     const int w0 = tile_start[tile], nloc = tile_start[tile + 1] - w0;
     if (nloc == 0) return;
     __shared__ TileWin W;
+    __shared__ unsigned maxr;
+    if (threadIdx.x == 0) maxr = 0u;
+    ListWin L = list_win(dyn, a.wcap, a.g, spos[work_k[w0 + nloc / 2]]);
     tile_window(tile, start, a.g, W);
-    stage_row_starts(W, start, a.g, cst);
-    const WinStage sp = win_stage(dyn, a.wcap);
-    const bool staged = stage_window(W, a.wcap, spos, HALF ? parts : nullptr, sp, kListPad);
+    stage_row_starts(W, start, a.g, L.cst);
+    const bool staged = stage_list_window<HALF>(W, a.wcap, spos, parts, a.cut2, L, &maxr);
     for (int at = threadIdx.x; at < nloc; at += blockDim.x) {
         const int w = w0 + at;
-        const int i = work[w];
+        const int i = HALF ? work[w] : 0;
         const int k = work_k[w];
         int cnt2 = 0;
-        const int cnt = staged ? nlist_atom<HALF, true>(i, w, work_c[w], k, spos[k], cst, a, W, sp, spos, parts, nb_list,
-                                                        nb_list2, cnt2)
-                               : nlist_atom<HALF, false>(i, w, work_c[w], k, spos[k], cst, a, W, sp, spos, parts, nb_list,
-                                                         nb_list2, cnt2);
+        const int cnt = staged ? nlist_atom<HALF, true>(i, w, work_c[w], k, spos[k], a, W, L, spos, parts, nb_list, nb_list2, cnt2)
+                               : nlist_atom<HALF, false>(i, w, work_c[w], k, spos[k], a, W, L, spos, parts, nb_list, nb_list2, cnt2);
         nb_count[w] = cnt;
         if (HALF) nb_count2[w] = cnt2;
         const int most = max(cnt, cnt2);
@@ -192,7 +189,7 @@ void refresh_mirror(Sim& s) {
 // A window that outgrows its room by one atom is read from the mirror, which
 // takes its block several times as long (6^3 cells, FP64: 174 us a build, with
 // an eighth of room 48; 23.2 and 20.1 us a step, at 16^3 mixed 21.6 and 18.2).
-constexpr int kWindowGrowth = 8;
+constexpr int kWindowGrowth = 16;
 
 void build_neighbor_lists(Sim& s, int half, double cutoff) {
     if (has_error()) return;
@@ -215,18 +212,13 @@ void build_neighbor_lists(Sim& s, int half, double cutoff) {
         }
         if (has_error()) return;
         if (!cleared) rebuild_zero(s, 0, 0, s.ng);
-        const int rsb = row_starts_bytes(s.tiles);
-        // window slots (positions, 24 B; half lists also the atom index,
-        // 28 B) + sentinel slots, then the row starts
-        const int sb = half ? kStageBytes : kPosStageBytes;
-        // the rebuild before's largest window: with room for it to grow
-        const int grow = s.windows_pending ? s.max_window / kWindowGrowth : 0;
-        const int wcap = std::min(s.max_window + grow + kListPad, (kLdsBudget - rsb) / sb);
-        NbArgs a{s.n, s.nb_cap, half, s.half_mode, wcap, cutoff * cutoff, s.tiles};
-        const size_t lds = (size_t)wcap * sb + rsb;
+        // the rebuild before's largest window, with room for it to grow
+        const int grow = s.windows_pending ? s.max_window / kWindowGrowth + 16 : 0;
+        const ListLds l = list_lds(s.max_window + grow + kListPad, row_starts_bytes(s.tiles), s.tile_threads / kWave);
+        NbArgs a{s.n, s.nb_cap, half, s.half_mode, l.wcap, cutoff * cutoff, s.tiles};
         if (s.n > 0) {
 #define TMD_NLIST(H)                                                                                                   \
-    hipLaunchKernelGGL(k_nlist<H>, dim3(ntiles), dim3(s.tile_threads), lds, s.stream, CMir{s.spos.as<double>()},           \
+    hipLaunchKernelGGL(k_nlist<H>, dim3(ntiles), dim3(l.waves * kWave), l.bytes, s.stream, CMir{s.spos.as<double>()},           \
                        (const int*)s.work_k.as<int>(), (const int*)s.work_c.as<int>(),                                      \
                        (const int*)s.cell_start.as<int>(), (const int*)s.cell_parts.as<int>(), (const int*)s.work.as<int>(), \
                        (const int*)s.tile_start.as<int>(), a, s.nb_count.as<int>(), s.nb_list.as<nb_t>(), \

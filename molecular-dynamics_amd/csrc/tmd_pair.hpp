@@ -296,100 +296,186 @@ struct NbArgs {
     TileGeom g;
 };
 
-// One list column being written: groups of 8 entries assembled in registers
-// (q0..q3 hold the last 8 entries, the newest in the high half of q3, and p
-// the two before them) and stored whole, one 16-byte store per group; groups
-// beyond the capacity are counted, not stored.
-struct ListCol {
+// A list column being written by its lane: entries wait in the lane's ring of
+// 16-bit slots in LDS (slot-major, so a wavefront's accesses spread over the
+// banks) and leave in whole groups of 8, one 16-byte store each, when the
+// ring of some lane would overflow, once in several chunks.  Kept in
+// registers instead, nearly every pair of entries met some lane that
+// completed a group, and the store's instructions ran at every step.
+template <int SLOTS>
+struct RingCol {
     int4* col;
-    int ngroups;
-    unsigned p, q0, q1, q2, q3;
-    int cnt;
-    __device__ __forceinline__ ListCol(int4* c, int ng)
-        : col(c), ngroups(ng), p(0u), q0(0u), q1(0u), q2(0u), q3(0u), cnt(0) {}
-    __device__ __forceinline__ void shift_in(unsigned t) {
-        q0 = __builtin_amdgcn_alignbit(q1, q0, 16);
-        q1 = __builtin_amdgcn_alignbit(q2, q1, 16);
-        q2 = __builtin_amdgcn_alignbit(q3, q2, 16);
-        q3 = __builtin_amdgcn_alignbit(t, q3, 16);
+    unsigned ngroups;
+    nb_t* ring;         // the lane's slot 0; slots are kWave apart
+    unsigned at, done;  // entries so far and entries stored, times kWave
+    __device__ __forceinline__ RingCol(int4* c, int ng, nb_t* r) : col(c), ngroups((unsigned)ng), ring(r), at(0u), done(0u) {}
+    __device__ __forceinline__ int count() const { return (int)(at / kWave); }
+    __device__ __forceinline__ nb_t& slot(unsigned e) const { return ring[e & (unsigned)((SLOTS - 1) * kWave)]; }
+    __device__ __forceinline__ void store_group() {
+        const nb_t* q = &slot(done);
+        unsigned d[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) d[k] = (unsigned)q[2 * k * kWave] | (unsigned)q[(2 * k + 1) * kWave] << 16;
+        // groups beyond the capacity are counted, not stored
+        const unsigned grp = done / (8 * kWave);
+        if (grp < ngroups) col[(size_t)grp * 64] = make_int4((int)d[0], (int)d[1], (int)d[2], (int)d[3]);
+        done += 8 * kWave;
     }
-    __device__ __forceinline__ void store(unsigned d0, unsigned d1, unsigned d2, unsigned d3) {
-        const int grp = (cnt >> 3) - 1;
-        if (grp < ngroups) col[(size_t)grp * 64] = make_int4((int)d0, (int)d1, (int)d2, (int)d3);
+    __device__ __forceinline__ void flush() {
+        while (at - done >= 8 * kWave) store_group();
     }
-    // one entry (p is not kept up to date here: push2 refills it before any
-    // store reads it)
-    __device__ __forceinline__ void push(unsigned t) {
-        shift_in(t);
-        ++cnt;
-        if ((cnt & 7) == 0) store(q0, q1, q2, q3);
-    }
-    // two entries, t1 first: whole dwords move, no funnel shifts.  A group
-    // completes either at t2 (the last 8 entries, q0..q3) or at t1 (the 8
-    // before t2, one entry lower: the high half of p through the low half
-    // of q3).
-    __device__ __forceinline__ void push2(unsigned t1, unsigned t2) {
-        p = q0;
-        q0 = q1;
-        q1 = q2;
-        q2 = q3;
-        q3 = t1 | (t2 << 16);
-        cnt += 2;
-        if ((cnt & 6) == 0) {
-            if (cnt & 1)
-                store(__builtin_amdgcn_alignbit(q0, p, 16), __builtin_amdgcn_alignbit(q1, q0, 16),
-                      __builtin_amdgcn_alignbit(q2, q1, 16), __builtin_amdgcn_alignbit(q3, q2, 16));
-            else
-                store(q0, q1, q2, q3);
-        }
-    }
-    // the set bits of m (bit b: entry base + b) in ascending order: an odd
-    // one alone, then two per step
-    __device__ __forceinline__ void push_mask(unsigned m, unsigned base) {
-        if (__builtin_popcount(m) & 1) {
-            push(base + (unsigned)__builtin_ctz(m));
-            m &= m - 1u;
-        }
+    __device__ __forceinline__ void append(unsigned m, unsigned base) {
         while (m != 0u) {
-            const unsigned b1 = (unsigned)__builtin_ctz(m);
+            slot(at) = (nb_t)(base + (unsigned)__builtin_ctz(m));
             m &= m - 1u;
-            const unsigned b2 = (unsigned)__builtin_ctz(m);
-            m &= m - 1u;
-            push2(base + b1, base + b2);
+            at += kWave;
         }
+    }
+    __device__ __forceinline__ bool full(unsigned m) const { return at - done + kWave * __builtin_popcount(m) > SLOTS * kWave; }
+    // the set bits of m (bit b: entry base + b) in ascending order
+    __device__ __forceinline__ void push_mask(unsigned m, unsigned base) {
+        if (__ballot(full(m))) {
+            flush();
+            if (__ballot(full(m))) {  // at most 7 wait: a byte at a time always fits
+                for (int k = 0; k < 32; k += 8) {
+                    append(m & (0xffu << k), base);
+                    flush();
+                }
+                return;
+            }
+        }
+        append(m, base);
     }
     // the last group's free slots hold the window's sentinel offset
     __device__ __forceinline__ void finish(unsigned pad) {
-        if ((cnt & 7) != 0 && (cnt >> 3) < ngroups) {
-            for (int p = cnt & 7; p < 8; ++p) shift_in(pad);
-            col[(size_t)(cnt >> 3) * 64] = make_int4((int)q0, (int)q1, (int)q2, (int)q3);
+        flush();
+        const unsigned cnt = at;
+        if (at > done) {
+            while (at - done < 8 * kWave) {
+                slot(at) = (nb_t)pad;
+                at += kWave;
+            }
+            store_group();
         }
+        at = cnt;
     }
 };
+constexpr int kRingSlots = 32;                           // of a lane; half lists: 16 for each column
+constexpr int kRingBytes = kRingSlots * kWave * 2;       // of a wavefront
+
+// The list build's window in LDS: FP32 positions relative to a point of the
+// tile, and the atom index.
+struct NbCand {
+    float x, y, z;
+    int j;
+};
+constexpr int kCandBytes = 16;
+struct ListWin {
+    NbCand* c;
+    int* cst;     // row starts (stage_row_starts)
+    nb_t* ring;   // the wavefronts' rings
+    double4 ref;  // the point
+    float sure;   // a squared distance off the cutoff's by more than this has the FP64 test's outcome
+};
+// LDS of a block's list build: `wcap` window slots, tables of `tab` bytes and
+// the rings of as many wavefronts as there is room for, of the `want` that
+// take the fullest tile at once; with fewer (at least kListWaves, at the cost
+// of window slots), as few as do not need another round.
+constexpr int kListWaves = 4;
+struct ListLds {
+    int wcap, waves, bytes;
+};
+inline ListLds list_lds(int window, int tab, int want) {
+    ListLds l;
+    const int room = (kLdsBudget - tab - window * kCandBytes) / kRingBytes;
+    l.waves = std::min(want, std::max(room, kListWaves));
+    const int rounds = (want + l.waves - 1) / l.waves;
+    l.waves = (want + rounds - 1) / rounds;
+    l.wcap = std::min(window, (kLdsBudget - tab - l.waves * kRingBytes) / kCandBytes);
+    l.bytes = l.wcap * kCandBytes + tab + l.waves * kRingBytes;
+    return l;
+}
+__device__ __forceinline__ ListWin list_win(double* dyn, int wcap, const TileGeom& g, const double4& ref) {
+    ListWin L;
+    L.c = reinterpret_cast<NbCand*>(dyn);
+    L.cst = reinterpret_cast<int*>(L.c + wcap);
+    L.ring = reinterpret_cast<nb_t*>(L.cst + row_starts_bytes(g) / 4);
+    L.ref = ref;
+    L.sure = 0.0f;
+    return L;
+}
+
+// What the FP32 test may be off by.  With u = 2^-24 and R the largest
+// coordinate of the window, a difference d is off by 2 u R + u |d|, its
+// square's sum over a distance r by u (7 R r + 2 r^2), and the three sums
+// from -cut2 by u (4 cut2 + 3 r^2): where the sign is wrong, r is within that
+// of the cutoff, and the sum is below u (7.4 R rc + 10 cut2).  Outside FP32's
+// comfortable range, or with a window 1e5 cutoffs wide, nothing is sure.
+__device__ __forceinline__ float list_sure(float R, double cut2) {
+    if (!(cut2 > 1e-12 && cut2 < 1e12 && (double)R * (double)R < 1e10 * cut2)) return __builtin_inff();
+    const float c2 = (float)cut2;
+    return 16.0f / 16777216.0f * (R * sqrtf(c2) + c2);
+}
+
+// Stage the list build's window if it fits wcap atoms.  Whole block; maxr
+// (shared, largest coordinate's bits) is zero and visible before.
+template <bool HALF, class SP>
+__device__ __forceinline__ bool stage_list_window(const TileWin& W, int wcap, const SP& spos, const int* __restrict__ parts,
+                                                  double cut2, ListWin& L, unsigned* maxr) {
+    const int S = win_size(W);
+    const bool staged = S + kListPad <= wcap;
+    if (staged) {
+        double4 p[kStageInFlight];
+        int j[kStageInFlight];
+        float R = 0.0f;
+        stage_rows(W, [&](int k, int u) { p[u] = spos[k]; if (HALF) j[u] = parts[k]; },
+                   [&](int t, int u) {
+                       const float x = (float)(p[u].x - L.ref.x), y = (float)(p[u].y - L.ref.y), z = (float)(p[u].z - L.ref.z);
+                       L.c[t] = NbCand{x, y, z, HALF ? j[u] : 0};
+                       R = fmaxf(fmaxf(R, fabsf(x)), fmaxf(fabsf(y), fabsf(z)));
+                   });
+        if ((int)threadIdx.x < kListPad) L.c[S + (int)threadIdx.x] = NbCand{0.0f, 0.0f, 0.0f, 0};  // masked
+#pragma unroll
+        for (int o = kWave / 2; o > 0; o >>= 1) R = fmaxf(R, __shfl_xor(R, o));
+        if ((threadIdx.x & (kWave - 1)) == 0) atomicMax(maxr, __float_as_uint(R));
+    }
+    __syncthreads();
+    if (staged) L.sure = list_sure(__uint_as_float(*maxr), cut2);
+    return staged;
+}
 
 // Verlet list of local atom i (work slot w, cell c of the tile's grid,
-// cell-ordered index k_i) from the staged window: 9 stencil rows of 3 cells
-// in the reference's order, `rsq <= cut2` in FP64 without contraction.  Row
-// bounds come from the staged row starts (cst).  Each row is tested in
-// chunks of 32 candidates that produce a bit mask (bit b: candidate tc + b
-// accepted); i itself is removed from the mask by its window offset, so full
-// lists read no atom index (half lists read the staged index for the j < i /
-// ghost filter).  The set bits are then appended in ascending order, which is
-// the reference's order (ListCol, two entries per step).  Only accepted
-// candidates pay for the packing.  Returns the count.
+// cell-ordered index k_i) from its tile's window: 9 stencil rows of 3 cells
+// in the reference's order, `rsq <= cut2` in FP64 without contraction.  Each
+// row is taken in chunks of 32 candidates that produce a bit mask (bit b:
+// candidate tc + b accepted); i itself is removed from the mask by its window
+// offset, and the set bits are appended in ascending order, which is the
+// reference's order.
 //
-// HALF also writes the complementary column (nb_list2, count in cnt2): the
-// local neighbours j > i that the half list leaves to j's own list.  The
-// pair force then needs no reaction scatter: atom i gathers its half-list
-// entries and its complementary entries, which are exactly the pairs whose
-// reactions the half list would have sent to i.  STAGED is a template
-// parameter so that the staged loop addresses LDS directly (ds_read) rather
-// than through generic pointers.
+// Bounds: vector instructions.  A staged candidate is tested in FP32 (6
+// instructions and one for its bit, 12 bytes of LDS; the FP64 test took 10
+// and 24 bytes), which is exact but for candidates within `sure` of the
+// cutoff; a chunk that holds one (about one atom in 1,000 meets one) is
+// repeated by the FP64 test.  Accepted candidates cost 9 instructions per
+// round of a wavefront (RingCol), a third of what packing in registers took.
+// A build at 80^3 cells took 722 us and takes 477 (268 M vector instructions
+// a wavefront's lanes share, 99 % busy), half lists of 53 x 47 x 39 cells 288
+// and 170.  The products -2 x_i . x_j on the matrix cores (32 x 32 tests for
+// two products of depth 2 and one for the constants) left the signs to be
+// gathered and three quarters of the candidates' slots padded, and took 870.
+//
+// HALF keeps j < i among locals (the reference's filter) plus, by default,
+// every ghost, and also writes the complementary column (nb_list2, count in
+// cnt2): the local neighbours j > i that the half list leaves to j's own
+// list.  The pair force then needs no reaction scatter: atom i gathers its
+// half-list entries and its complementary entries, which are exactly the
+// pairs whose reactions the half list would have sent to i.  STAGED is a
+// template parameter so that the staged loop addresses LDS directly (ds_read)
+// rather than through generic pointers.
 template <bool HALF, bool STAGED, class SP>
-__device__ __forceinline__ int nlist_atom(int i, int w, int c, int k_i, const double4 pi, const int* cst, const NbArgs& a,
-                                          const TileWin& W, const WinStage& sp, const SP& spos,
-                                          const int* __restrict__ parts, nb_t* __restrict__ nb_list,
-                                          nb_t* __restrict__ nb_list2, int& cnt2) {
+__device__ __forceinline__ int nlist_atom(int i, int w, int c, int k_i, const double4 pi, const NbArgs& a, const TileWin& W,
+                                          const ListWin& L, const SP& spos, const int* __restrict__ parts,
+                                          nb_t* __restrict__ nb_list, nb_t* __restrict__ nb_list2, int& cnt2) {
     const int cx = c % a.g.nx, cy = (c / a.g.nx) % a.g.ny, cz = c / (a.g.nx * a.g.ny);
     const int wy = a.g.ty + 2;
     const int xo = cx - W.cx0;  // (cx - 1) - (cx0 - 1)
@@ -397,75 +483,87 @@ __device__ __forceinline__ int nlist_atom(int i, int w, int c, int k_i, const do
     const int s_own = (cz - (W.cz0 - 1)) * wy + (cy - (W.cy0 - 1));
     const int t_i = W.seg_off[s_own] + (k_i - W.seg_beg[s_own]);
     const size_t col_off = (size_t)(w >> 6) * (size_t)a.cap * 8 + (w & 63);
-    ListCol A(reinterpret_cast<int4*>(nb_list) + col_off, a.cap >> 3);
-    ListCol B(HALF ? reinterpret_cast<int4*>(nb_list2) + col_off : nullptr, a.cap >> 3);
+    constexpr int SLOTS = HALF ? kRingSlots / 2 : kRingSlots;
+    nb_t* ring = L.ring + (threadIdx.x / kWave) * (kRingSlots * kWave) + threadIdx.x % kWave;
+    RingCol<SLOTS> A(reinterpret_cast<int4*>(nb_list) + col_off, a.cap >> 3, ring);
+    RingCol<SLOTS> B(HALF ? reinterpret_cast<int4*>(nb_list2) + col_off : nullptr, a.cap >> 3, ring + SLOTS * kWave);
+    const float xi = (float)(pi.x - L.ref.x), yi = (float)(pi.y - L.ref.y), zi = (float)(pi.z - L.ref.z);
+    const float ncut2 = -(float)a.cut2;
     for (int r = 0; r < 9; ++r) {
         const int s = s_own + (r / 3 - 1) * wy + (r % 3 - 1);
-        const int t0 = cst[s * per + xo], t1 = cst[s * per + xo + 3];
+        const int t0 = L.cst[s * per + xo], t1 = L.cst[s * per + xo + 3];
+        const int k0 = W.seg_beg[s] - W.seg_off[s];  // mirror index less window offset, in this row
         for (int tc = t0; tc < t1; tc += 32) {
             const int te = min(tc + 32, t1);
-            // the candidates' bits are shifted in at the low end (first
-            // candidate highest): half lists a batch of 4 at a time, full
-            // lists one sign bit per candidate (one funnel shift)
-            unsigned m = 0u, m2 = 0u;
-            const int nbat = (te - tc + 3) >> 2;  // batches (the loop test is then one compare)
-            for (int q = 0; q < nbat; ++q) {
-                const int tb = tc + 4 * q;
-                unsigned bq = 0u, bq2 = 0u;
+            unsigned m = 0u, m2 = 0u;  // accepted; half lists: of those, locals j > i
+            bool sure = false;
+            if (STAGED) {
+                // the candidates' sign bits are shifted in at the low end
+                // (first candidate highest), a batch of 4 at a time: up to
+                // three past te are read (window atoms or the slots behind
+                // it) and masked below
+                const int nbat = (te - tc + 3) >> 2;
+                float near = __builtin_inff();
+                const NbCand* q = L.c + tc;
+                const NbCand* const end = q + 4 * nbat;
+                do {
+                    float d[4];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    // staged: up to three candidates past te are read (window
-                    // atoms or sentinel slots) and masked below; from the
-                    // mirror, t is clamped to stay inside the window
-                    const int t = STAGED ? tb + u : min(tb + u, te - 1);
-                    double xj, yj, zj;
-                    int j = 0;
-                    if (STAGED) {
-                        xj = sp.xyz[3 * t + 0]; yj = sp.xyz[3 * t + 1]; zj = sp.xyz[3 * t + 2];
-                        if (HALF) j = sp.j[t];
-                    } else {
-                        const int kk = win_index(t, W);
-                        const double4 p = spos[kk];
-                        xj = p.x; yj = p.y; zj = p.z;
-                        if (HALF) j = parts[kk];
+                    for (int u = 0; u < 4; ++u) {
+                        const float dx = xi - q[u].x, dy = yi - q[u].y, dz = zi - q[u].z;
+                        d[u] = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, __builtin_fmaf(dx, dx, ncut2)));
+                        m = __builtin_amdgcn_alignbit(m, __float_as_uint(d[u]), 31);
+                        if (HALF) {
+                            // i < j < n: neither j - (i + 1) nor (n - 1) - j is negative
+                            const int j = q[u].j;
+                            m2 = __builtin_amdgcn_alignbit(m2, (unsigned)((j - (i + 1)) | ((a.n - 1) - j)), 31);
+                        }
                     }
-                    const double dx = pi.x - xj, dy = pi.y - yj, dz = pi.z - zj;
+                    near = fminf(fminf(near, fabsf(d[0])), fabsf(d[1]));
+                    near = fminf(fminf(near, fabsf(d[2])), fabsf(d[3]));
+                    q += 4;
+                } while (q != end);
+                sure = near > L.sure;
+                // reversed, bit b is candidate tc + b
+                m = __builtin_bitreverse32(m) >> (32 - 4 * nbat);
+                if (HALF) m2 = ~(__builtin_bitreverse32(m2) >> (32 - 4 * nbat));
+            }
+            if (!sure) {
+                m = 0u;
+                if (!STAGED) m2 = 0u;
+                for (int t = tc; t < te; ++t) {
+                    const double4 p = spos[k0 + t];
+                    const double dx = pi.x - p.x, dy = pi.y - p.y, dz = pi.z - p.z;
                     const double rsq = dx * dx + dy * dy + dz * dz;
-                    if (HALF) {
-                        bool ok = rsq <= a.cut2;
-                        bq2 |= (ok && j < a.n && j > i) ? 8u >> u : 0u;
-                        ok = ok && ((a.half_mode == HALF_REF_LITERAL) ? (i > j) : (j >= a.n || i > j));
-                        bq |= ok ? 8u >> u : 0u;
-                    } else {
-                        // the sign of cut2 - rsq is set exactly when rsq > cut2
-                        // (the difference of two equal finite doubles is +0);
-                        // it is shifted in at the low end
-                        const double d = a.cut2 - rsq;
-                        m = __builtin_amdgcn_alignbit(m, (unsigned)__double2hiint(d), 31);
+                    const unsigned bit = 1u << (t - tc);
+                    m |= rsq <= a.cut2 ? bit : 0u;
+                    if (HALF && !STAGED) {
+                        const int j = parts[k0 + t];
+                        m2 |= j > i && j < a.n ? bit : 0u;
                     }
-                }
-                if (HALF) {
-                    m = (m << 4) | bq;
-                    m2 = (m2 << 4) | bq2;
                 }
             }
-            if (!HALF) m = ~m;  // the bits were set for the rejected candidates
-            // reversed, bit b is candidate tc + b (nbat >= 1: the chunk is not empty)
-            m = __builtin_bitreverse32(m) >> (32 - 4 * nbat);
-            if (HALF) m2 = __builtin_bitreverse32(m2) >> (32 - 4 * nbat);
-            const unsigned chunk = te - tc == 32 ? 0xffffffffu : (1u << (te - tc)) - 1u;  // candidates of this chunk only
-            m &= chunk;
-            const unsigned d = (unsigned)(t_i - tc);
-            m &= ~(d < 32u ? 1u << d : 0u);  // i is not its own neighbour
+            m &= 0xffffffffu >> (32 - (te - tc));  // candidates of this chunk only
+            if (r == 4) m &= ~(unsigned)(1ull << min((unsigned)(t_i - tc), 32u));  // i is not its own neighbour
+            if (HALF) {
+                m2 &= m;
+                B.push_mask(m2, (unsigned)tc);
+                m &= ~m2;
+                if (a.half_mode == HALF_REF_LITERAL && m != 0u) {  // no ghosts either
+                    for (unsigned q = m; q != 0u; q &= q - 1u) {
+                        const int t = tc + __builtin_ctz(q);
+                        if ((STAGED ? L.c[t].j : parts[k0 + t]) >= a.n) m &= ~(q & (0u - q));
+                    }
+                }
+            }
             A.push_mask(m, (unsigned)tc);
-            if (HALF) B.push_mask(m2 & chunk, (unsigned)tc);  // j > i excludes i itself
         }
     }
     const unsigned pad = (unsigned)win_size(W);
     A.finish(pad);
     if (HALF) B.finish(pad);
-    cnt2 = B.cnt;
-    return A.cnt;
+    cnt2 = B.count();
+    return A.count();
 }
 
 }  // namespace tmd

@@ -146,3 +146,30 @@ def test_step_pass_writes_ghosts(tm, shape, threads, half, precision):
         out.append(sim.state()[1:] + tuple(sim.ghost_state()[:2]))
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+# lattice 0.7: a quarter of the list cutoff, so whole shells of pairs lie at
+# the cutoff to the last bit and FP32 decides none of them; gas of 40 atoms a
+# cell: most of a chunk's candidates accepted at once; thin gas: empty chunks;
+# window of 6 x 6 x 6 cells of 40: larger than the LDS
+@pytest.mark.parametrize("half,literal", [(False, False), (True, False), (True, True)])
+@pytest.mark.parametrize("atoms,tile", [("lattice", (2, 1, 1)), ("gas", (1, 2, 1)), ("gas", (4, 4, 4)), ("thin", (3, 3, 3))])
+def test_lists_exact_at_the_cutoff(tm, atoms, tile, half, literal):
+    announce(f"lists at the cutoff, {atoms} {tile} {half} {literal}")
+    rng = np.random.default_rng(7)
+    if atoms == "lattice":
+        L = 0.7 * 18
+        g = (np.arange(18) + 0.5) * 0.7
+        x = np.stack(np.meshgrid(g, g, g, indexing="ij"), axis=-1).reshape(-1, 3)
+    else:
+        L = 2.8 * 4.4
+        x = rng.random((3400 if atoms == "gas" else 60, 3)) * L
+    aabb = np.array([0.0, L] * 3)
+    mode = "ref_literal" if literal else "ghost_full"
+    sim = tm.Simulation(np.ones(len(x)), x, np.zeros_like(x), aabb, RC + SKIN, nb_cap=400, half_mode=mode)
+    sim.set_tile(*tile)
+    sim.copy_to_accelerator()
+    sim.setup(half, RC, SKIN)
+    orc = po.OracleSim(np.ones(len(x)), x, np.zeros_like(x), aabb, RC + SKIN, nb_cap=400, threads=4)
+    orc.setup(half, po.HALF_REF_LITERAL if literal else po.HALF_GHOST_FULL, RC + SKIN)
+    same_structure(sim, orc)
