@@ -140,6 +140,74 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_lj_full(TMD_KERNEL_LIST_PAR
     }
 }
 
+// k_lj_full's KICK 2 for small boxes: a group of lanes an atom, lane c < 3 of
+// it for component c of the sum, the kicks and the drift.
+//
+// Bounds: the latency of one wavefront's list walk, which four lanes an atom
+// cut to a third, and the launch.  us a step, one lane an atom against four:
+// 6^3 cells FP64 19.7 and 15.0, 9^3 FP32-mixed half lists 18.8 and 17.0, 9^3
+// Kahan 19.6 and 14.4.  Eight lanes gain another 0.5 to 1.3 in FP64 up to 12^3
+// and lose 1 to 5 in FP32-mixed (the terms' way through LDS).
+template <int PREC, int SHIFT, int UNIT, bool PAIR2>
+__global__ void __launch_bounds__(kMaxTileThreads) k_lj_group(const CMir spos, const int* __restrict__ start,
+                                                          const int* __restrict__ tile_start, const int* __restrict__ nbc,
+                                                          const nb_t* __restrict__ nbl, LJArgs a, const Mir svel, double hdt,
+                                                          double dt, const int* __restrict__ wk, const Mir spos_next,
+                                                          const int* __restrict__ nbc2, const nb_t* __restrict__ nbl2,
+                                                          GhostIndex gh) {
+    constexpr int G = kGroupLanes;
+    extern __shared__ double dyn[];
+    const WinStage sp = win_stage(dyn, a.wcap);
+    double* buf = dyn + 3 * a.wcap + threadIdx.x / kWave * (kGroupBufBytes / sizeof(double));
+    const int tile = xcd_block(blockIdx.x, gridDim.x);
+    const int w0 = tile_start[tile], nloc = tile_start[tile + 1] - w0;
+    if (nloc == 0) return;
+    const int c = min((int)threadIdx.x & (G - 1), 2);
+    const bool mine = ((int)threadIdx.x & (G - 1)) < 3;
+    // as in k_lj_full: own loads first
+    int kw = 0, cnt = 0, cnt2 = 0, pk = 0;
+    double4 pi;
+    double v = 0.0;
+    int4 next;
+    const int4 *lp, *lp2;
+    auto fetch = [&](int at) {
+        const int w = w0 + at;
+        kw = wk[w];
+        cnt = nbc[w];
+        cnt2 = PAIR2 ? nbc2[w] : 0;
+        pk = gh.w ? gh.w[w] : 0;
+        const size_t col = (size_t)(w >> 6) * (size_t)a.cap * 8 + (w & 63);
+        lp = reinterpret_cast<const int4*>(nbl) + col;
+        lp2 = PAIR2 ? reinterpret_cast<const int4*>(nbl2) + col : nullptr;
+        pi = spos[kw];
+        v = svel.p[3 * (size_t)kw + c];
+        next = group_entries<PAIR2>(threadIdx.x & (G - 1), cnt, lp, cnt2, lp2);
+    };
+    if ((int)threadIdx.x / G < nloc) fetch(threadIdx.x / G);
+    __shared__ TileWin W;
+    tile_window(tile, start, a.g, W);
+    const bool staged = stage_window(W, a.wcap, spos, nullptr, sp);
+    for (int at = threadIdx.x / G; at < nloc; at += blockDim.x / G) {
+        if (at >= (int)blockDim.x / G) fetch(at);
+        const double f = staged ? lj_group_atom<PREC, SHIFT, UNIT, true, PAIR2>(pi, cnt, lp, sp, spos, W, a, next, cnt2, lp2, buf)
+                                : lj_group_atom<PREC, SHIFT, UNIT, false, PAIR2>(pi, cnt, lp, sp, spos, W, a, next, cnt2, lp2, buf);
+        v = v + f * hdt;
+        v = v + f * hdt;
+        double x = c == 0 ? pi.x : (c == 1 ? pi.y : pi.z);
+        x = x + v * dt;
+        if (mine) {
+            spos_next.p[3 * (size_t)kw + c] = x;
+            svel.p[3 * (size_t)kw + c] = v;
+            each_ghost(gh, pk, [&](int e, int kg) {
+                int i[3];
+                img_decode(e, i[0], i[1], i[2]);
+                const double L = c == 0 ? gh.L0 : (c == 1 ? gh.L1 : gh.L2);
+                spos_next.p[3 * (size_t)kg + c] = x + L * (double)(c == 0 ? i[0] : (c == 1 ? i[1] : i[2]));
+            });
+        }
+    }
+}
+
 // End of a DEM step: the final kick v += f dt/2 and, with ADV, the next
 // step's kick and drift, with the mirror kept current when inv is given
 // (k_final_integration and k_initial_integration arithmetic, in that order).
@@ -538,6 +606,12 @@ void compute_dem_fused(Sim& s, int half, double rc, double gn, double gt, double
         (const int*)s.cell_parts.as<int>(), (const int*)s.work.as<int>(), (const int*)s.tile_start.as<int>(),     \
         (const int*)s.nb_count.as<int>(), (const nb_t*)s.nb_list.as<nb_t>()
 
+// Boxes up to this many atoms take four lanes an atom: 28,000 and 44,000 of
+// the chip's 65,536 lanes.  us a step, one lane against four: 12^3 cells (6,912
+// atoms) FP32-mixed half lists 19.2 and 17.5, FP64 20.2 and 15.4; 14^3 (10,976)
+// FP32-mixed 18.2 and 19.3, FP64 20.7 and 18.2; 16^3 FP64 20.2 and 21.1.
+static int group_atoms(int precision) { return precision == PREC_FP32_MIXED ? 7000 : 11000; }
+
 static size_t lds_bytes(const Sim& s, bool) { return (size_t)window_cap(s) * kStageBytes; }
 
 void compute_lj(Sim& s, int half, double rc, double eps, double sigma, double kick_dt, bool advance) {
@@ -572,14 +646,24 @@ void compute_lj(Sim& s, int half, double rc, double eps, double sigma, double ki
         if (!fuse) GH.w = nullptr;
         const int* C2 = s.nb_count2.as<int>();
         const nb_t* L2 = s.nb_list2.as<nb_t>();
+        const int gthreads = std::min(kMaxTileThreads, (s.max_locals * kGroupLanes + kWave - 1) / kWave * kWave);
+        const size_t glds = lds + (size_t)gthreads / kWave * kGroupBufBytes;
+        const bool group = kick_dt > 0.0 && advance && VK && s.n <= group_atoms(s.precision) && s.tile_threads_req == 0 &&
+                           glds <= (size_t)kLdsBudget;
 #define TMD_LJ_K(P, SH, U, K, H)                                                                                       \
     hipLaunchKernelGGL((k_lj_full<P, SH, U, K, H>), dim3(nb), dim3(s.tile_threads), lds, s.stream, TMD_LIST_ARGS, a, F, V, SV, hdt, \
                        kick_dt, WK, SN, VK, C2, L2, GH)
 #define TMD_LJ_H(P, SH, U, K)                                                                                          \
     do { if (half) TMD_LJ_K(P, SH, U, K, true); else TMD_LJ_K(P, SH, U, K, false); } while (0)
+#define TMD_LJ_G(P, SH, U, H)                                                                                       \
+    hipLaunchKernelGGL((k_lj_group<P, SH, U, H>), dim3(nb), dim3(gthreads), glds, s.stream, CMir{s.spos.as<double>()},  \
+                       (const int*)s.cell_start.as<int>(), (const int*)s.tile_start.as<int>(),                            \
+                       (const int*)s.nb_count.as<int>(), (const nb_t*)s.nb_list.as<nb_t>(), a, SV, hdt, kick_dt, WK, SN, C2, L2, GH)
 #define TMD_LJ_FULL(P, SH, U)                                                                                          \
     do {                                                                                                               \
-        if (kick_dt > 0.0 && advance) TMD_LJ_H(P, SH, U, 2);                                                           \
+        if (group && half) TMD_LJ_G(P, SH, U, true);                                                                   \
+        else if (group) TMD_LJ_G(P, SH, U, false);                                                                     \
+        else if (kick_dt > 0.0 && advance) TMD_LJ_H(P, SH, U, 2);                                                           \
         else if (kick_dt > 0.0) TMD_LJ_H(P, SH, U, 1);                                                                 \
         else TMD_LJ_H(P, SH, U, 0);                                                                                    \
     } while (0)
@@ -596,6 +680,7 @@ void compute_lj(Sim& s, int half, double rc, double eps, double sigma, double ki
 #undef TMD_LJ_FULL
 #undef TMD_LJ_H
 #undef TMD_LJ_K
+#undef TMD_LJ_G
     }
     s.timer.end(K_FORCE, s.stream, ev);
     TMD_HIP(hipGetLastError());

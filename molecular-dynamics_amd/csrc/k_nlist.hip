@@ -131,6 +131,7 @@ void apply_window_stats(Sim& s, const int* st) {
     }
     s.nbinned = st[CT_BINNED];
     s.max_window = st[CT_MAXWIN];
+    s.max_locals = st[CT_MAXLOC];
     s.tile_threads = tile_block_threads(s.tile_threads_req, st[CT_MAXLOC]);
     retune_tiles(s);
     if (s.max_window > kWinMax) {

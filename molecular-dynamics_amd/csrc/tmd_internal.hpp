@@ -152,6 +152,7 @@ struct Sim {
     int nb_valid = 0;   // list present
     int nbinned = 0;    // atoms in the cell CSR (locals + ghosts inside the grid)
     int max_window = 0; // largest tile window (atoms)
+    int max_locals = 0; // most locals of a tile
     TileGeom tiles{};   // tile decomposition of the cell grid
     int tile_req[3] = {0, 0, 0};  // requested cells per tile (0: automatic)
     int tile_auto[3] = {0, 0, 0};  // automatic cells per tile in effect (0: chosen at the next binning)

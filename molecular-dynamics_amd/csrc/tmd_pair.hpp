@@ -232,6 +232,101 @@ __device__ __forceinline__ double4 lj_full_atom(const double4 pi, int cnt, const
 }
 
 
+// The force on one atom by a group of G lanes, for boxes whose atoms do not
+// fill the chip's lanes: lane s evaluates entries s, s + G, s + 2 G and
+// s + 3 G of every 4 G, as lj_full_atom does, and leaves their terms in the wavefront's buffer in
+// LDS; lane c of the group then adds component c of the 4 G terms in list
+// order (the terms of absent entries are dx * 0), so the sum is
+// lj_full_atom's bit for bit.  All lanes of a group call together, lane s with
+// list group s in `next`: it fetches group s of every G for all of them,
+// through LDS.  Lane c < 3 returns component c.
+constexpr int kGroupLanes = 4;
+constexpr int kGroupBufBytes = 8192 + 1024;  // of a wavefront: 256 entries of up to four doubles, 64 groups of list entries
+template <bool PAIR2>  // list group g (clamped), column 2's groups behind column 1's
+__device__ __forceinline__ int4 group_entries(int g, int cnt, const int4* __restrict__ lp, int cnt2, const int4* __restrict__ lp2) {
+    const int ng1 = (cnt + 7) >> 3, ng = ng1 + (PAIR2 ? (cnt2 + 7) >> 3 : 0);
+    g = max(min(g, ng - 1), 0);
+    return ld_stream((!PAIR2 || g < ng1) ? lp + (size_t)g * 64 : lp2 + (size_t)(g - ng1) * 64);
+}
+template <int PREC, int SHIFT, int UNIT, bool STAGED, bool PAIR2, class SP>
+__device__ __forceinline__ double lj_group_atom(const double4 pi, int cnt, const int4* __restrict__ lp, const WinStage& sp,
+                                                const SP& spos, const TileWin& W, const LJArgs& a, int4 next, int cnt2,
+                                                const int4* __restrict__ lp2, double* buf) {
+    constexpr int G = kGroupLanes, A = kWave / G, U = 4, E = U * G;  // atoms of a wavefront, entries of a round
+    const int s = threadIdx.x & (G - 1), c = min(s, 2);
+    const int far = win_size(W);             // sentinel slot
+    double* const mine = buf + (threadIdx.x & (kWave - 1)) / G;
+    float* const minef = reinterpret_cast<float*>(buf) + (threadIdx.x & (kWave - 1)) / G;
+    const int ng1 = (cnt + 7) >> 3;
+    const int ng = ng1 + (PAIR2 ? (cnt2 + 7) >> 3 : 0);
+    int4* const lists = reinterpret_cast<int4*>(buf + 1024) + (threadIdx.x & (kWave - 1));
+    const nb_t* const list = reinterpret_cast<const nb_t*>(lists - s);
+    double F = 0.0;
+    float fs = 0.f, fc = 0.f;
+    for (int base = 0; base < 8 * ng; base += E) {
+        if (base % (8 * G) == 0) {
+            *lists = next;
+            next = group_entries<PAIR2>(base / 8 + G + s, cnt, lp, cnt2, lp2);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+        double d[U][3], rs[U];
+        bool ok[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int e = base + s + u * G, g = e >> 3;
+            const bool valid = (!PAIR2 || g < ng1) ? e < cnt : e - 8 * ng1 < cnt2;
+            const int t = list[e % (8 * G)];
+            double xj, yj, zj;
+            win_pos<STAGED>(valid ? t : (STAGED ? far : 0), sp, spos, W, xj, yj, zj);
+            d[u][0] = pi.x - xj;
+            d[u][1] = pi.y - yj;
+            d[u][2] = pi.z - zj;
+            rs[u] = PREC == PREC_FP64 ? d[u][0] * d[u][0] + d[u][1] * d[u][1] + d[u][2] * d[u][2]
+                                      : fma(d[u][0], d[u][0], fma(d[u][1], d[u][1], d[u][2] * d[u][2]));
+            ok[u] = valid && rs[u] < a.rc2;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = u * G + s;
+            if (PREC == PREC_FP64) {
+                double sr6;
+                const double f = lj_f64u<SHIFT, UNIT>(a, rs[u], sr6);
+                const double fm = ok[u] ? f : 0.0;
+#pragma unroll
+                for (int x = 0; x < 3; ++x) mine[(3 * k + x) * A] = d[u][x] * fm;
+            } else {
+                float f;
+                if (SHIFT || PREC == PREC_FP32_KAHAN) {
+                    f = lj_f32u<SHIFT, UNIT>(a, (float)rs[u]);
+                    f = ok[u] ? f : 0.0f;
+                } else {
+                    f = lj_f32u<SHIFT, UNIT>(a, ok[u] ? (float)rs[u] : __builtin_inff());
+                }
+                if (PREC == PREC_FP32_MIXED) {
+#pragma unroll
+                    for (int x = 0; x < 3; ++x) mine[(4 * k + x) * A] = d[u][x];
+                    mine[(4 * k + 3) * A] = (double)f;
+                } else {
+#pragma unroll
+                    for (int x = 0; x < 3; ++x) minef[(3 * k + x) * A] = (float)d[u][x] * f;
+                }
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int k = 0; k < E; ++k) {
+            if (PREC == PREC_FP64) F = F + mine[(3 * k + c) * A];
+            else if (PREC == PREC_FP32_MIXED) F = fma(mine[(4 * k + c) * A], mine[(4 * k + 3) * A], F);
+            else kahan_add(fs, fc, minef[(3 * k + c) * A]);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    return PREC != PREC_FP32_KAHAN ? F : kahan_value(fs, fc);
+}
+
 // Energy and virial terms of one atom's list entries (FP64): U = 4 eps
 // (sr12 - sr6) [+ shift terms], W = f r^2.  Full lists weight every entry
 // 1/2; half lists weight local-local entries 1 and local-ghost entries 1/2

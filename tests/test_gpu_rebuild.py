@@ -173,3 +173,36 @@ def test_lists_exact_at_the_cutoff(tm, atoms, tile, half, literal):
     orc = po.OracleSim(np.ones(len(x)), x, np.zeros_like(x), aabb, RC + SKIN, nb_cap=400, threads=4)
     orc.setup(half, po.HALF_REF_LITERAL if literal else po.HALF_GHOST_FULL, RC + SKIN)
     same_structure(sim, orc)
+
+
+# 6,912 and 7,200 atoms: either side of FP32-mixed's line for four lanes an
+# atom, 10,976 and 11,760 of the others'; (4, 4, 5): fewer atoms a tile than
+# one wavefront's 16; cutoffs 1.2 and 3: lists within one round of 16 entries and
+# over several fetches of 32
+@pytest.mark.parametrize("shape,rc,half,precision,par", [
+    ((4, 4, 5), 2.5, False, "fp64", (1.0, 1.0, True)),
+    ((4, 4, 5), 1.2, True, "fp32mixed", (1.0, 1.0, False)),
+    ((7, 6, 8), 3.0, True, "fp64", (1.3, 0.9, False)),
+    ((7, 6, 8), 3.0, False, "fp32mixed", (1.3, 0.9, True)),
+    ((7, 6, 8), 3.0, True, "fp32kahan", (0.8, 1.1, True)),
+    ((7, 6, 8), 2.5, False, "fp32kahan", (1.0, 1.0, False)),
+    ((12, 12, 12), 2.5, False, "fp32mixed", (1.0, 1.0, False)),
+    ((12, 15, 10), 2.5, False, "fp32mixed", (1.0, 1.0, False)),
+    ((14, 14, 14), 2.5, True, "fp64", (1.0, 1.0, False)),
+    ((14, 15, 14), 2.5, True, "fp64", (1.0, 1.0, False)),
+])
+def test_lanes_of_an_atom(tm, shape, rc, half, precision, par):
+    """The step pass of small boxes against the separate calls: bit for bit."""
+    announce(f"lanes of an atom {shape} {rc} {half} {precision} {par}")
+    eps, sigma, shift = par
+    aabb, m, x, v = perturbed_fcc(*shape, amp=0.03, seed=5)
+    out = []
+    for run in ("run_lj", "run_abi_lj"):
+        sim = tm.Simulation(m, x, v, aabb, rc + SKIN, precision=precision, lj_shift=shift)
+        sim.copy_to_accelerator()
+        sim.setup(half, rc, SKIN)
+        sim.lennard_jones(half, rc, eps, sigma)
+        getattr(sim, run)(25, 10, 0.002, half, rc, SKIN, eps, sigma)
+        out.append(sim.state()[1:] + tuple(sim.ghost_state()[:2]))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
