@@ -437,12 +437,52 @@ static void traj_step(Sim& s, const TrajSpec& p, const DevBuf& x, TrajStep t, bo
     TMD_HIP(hipGetLastError());
 }
 
+// The states of the steps t0 .. of a trajectory, mirrors of positions and
+// velocities one behind the other (adj_segx, adj_segv).
+struct Kept {
+    bool on = false;
+    size_t stride = 0;  // doubles a mirror
+    int t0 = 0;
+    double *x = nullptr, *v = nullptr;
+    double* X(int t) const { return x + (size_t)(t - t0) * stride; }
+    double* V(int t) const { return v + (size_t)(t - t0) * stride; }
+};
+static Kept reserve_kept(Sim& s, int t0, int t1) {
+    Kept k;
+    k.stride = 3 * (size_t)s.cap_all;
+    k.t0 = t0;
+    const size_t bytes = sizeof(double) * k.stride * (size_t)(t1 - t0 + 1);
+    s.adj_segx.reserve(bytes, false, s.stream);
+    s.adj_segv.reserve(bytes, false, s.stream);
+    k.x = s.adj_segx.as<double>();
+    k.v = s.adj_segv.as<double>();
+    k.on = !has_error();
+    return k;
+}
+// A gradient keeps every state of its forward pass, where that takes at most
+// 4 GiB and a quarter of the free memory; else each interval is recomputed
+// from its checkpoint.  16,384 atoms over 200 steps: 0.4 GB, and the second
+// forward pass (16 us a step) is gone, 14.8 -> 11.7 ms a gradient.
+constexpr size_t kKeptBytes = size_t(4) << 30;
+static bool keep_all(const Sim& s, int steps) {
+    const size_t bytes = 2 * sizeof(double) * 3 * (size_t)s.cap_all * (size_t)(steps + 1);
+    if (bytes > kKeptBytes) return false;
+    if (bytes <= s.adj_segx.bytes + s.adj_segv.bytes) return true;
+    size_t avail = 0, total = 0;
+    return hipMemGetInfo(&avail, &total) == hipSuccess && bytes <= avail / 4;
+}
+
+static void copy_mirror(Sim& s, double* to, const DevBuf& from) {
+    TMD_HIP(hipMemcpyAsync(to, from.p, (size_t)kMirBytes * (size_t)s.nbinned, hipMemcpyDeviceToDevice, s.stream));
+}
+
 // Forward trajectory from (adj_x0, adj_v0), reneighbouring every ck steps
 // exactly as the step loop does (wrap, ghosts, cells, list after the
 // position update of steps ck, 2ck, ...).  With checkpoints, slot k holds
-// the state at t = k ck (after that step's wrap).  The mirrors alternate as in
-// the step loop; a rebuild goes from mirror to mirror.
-static void forward_traj(Sim& s, const TrajSpec& p, bool store_ckpt, double* ubar, double* pbar) {
+// the state at t = k ck (after that step's wrap), and the states go into
+// `kept` while it is on.  The mirrors alternate as in the step loop; a rebuild
+// goes from mirror to mirror.
+static void forward_traj(Sim& s, const TrajSpec& p, bool store_ckpt, double* ubar, double* pbar, Kept* kept = nullptr) {
     const double cut = p.rc + p.skin;
     double* acc = s.adj_acc.as<double>();
     zero(s, acc, 4);
@@ -458,13 +498,23 @@ static void forward_traj(Sim& s, const TrajSpec& p, bool store_ckpt, double* uba
         TrajStep st{};
         st.hfin = t > 0 ? 0.5 * p.dt : 0.0;
         st.adv = t < p.steps;
-        st.xnext = Mir{s.spos2.as<double>()};
+        if (kept && 3 * (size_t)s.cap_all > kept->stride) kept->on = false;  // a rebuild made room for more ghosts
+        const bool keep = kept && kept->on;
+        DevBuf x = s.spos;
+        if (keep) {
+            if (t % p.ck == 0) copy_mirror(s, kept->X(t), s.spos);
+            x.p = kept->X(t);
+            st.vt = Mir{kept->V(t)};
+        }
+        // a rebuild starts from the mirror
+        const bool into_kept = keep && (t + 1) % p.ck != 0;
+        st.xnext = Mir{into_kept && st.adv ? kept->X(t + 1) : s.spos2.as<double>()};
         if (store_ckpt && t % p.ck == 0) {
             st.ckx = s.adj_ckx.as<double4>() + (size_t)(t / p.ck) * s.n;
             st.ckv = s.adj_ckv.as<double4>() + (size_t)(t / p.ck) * s.n;
         }
-        traj_step(s, p, s.spos, st, t > 0);
-        if (st.adv) std::swap(s.spos, s.spos2);
+        traj_step(s, p, x, st, t > 0);
+        if (st.adv && !into_kept) std::swap(s.spos, s.spos2);
         s.pos_stale = 1;  // the state lives in the mirrors
         s.vel_mirrored = 1;
     }
@@ -542,7 +592,10 @@ bool traj_adjoint(Sim& s, int steps, int ck, double dt, double rc, double skin, 
     const TrajSpec p{steps, ck, dt, rc, skin, eps, sigma};
     if (!begin_traj(s, p, true)) return false;
     double ubar = 0.0, pbar = 0.0;
-    forward_traj(s, p, true, &ubar, &pbar);
+    Kept kept;
+    if (keep_all(s, steps)) kept = reserve_kept(s, 0, steps);
+    if (has_error()) return false;
+    forward_traj(s, p, true, &ubar, &pbar, kept.on ? &kept : nullptr);
     if (has_error()) return false;
     const int n = s.n;
     const double vol = s.g.len[0] * s.g.len[1] * s.g.len[2];
@@ -571,34 +624,34 @@ bool traj_adjoint(Sim& s, int steps, int ck, double dt, double rc, double skin, 
     zero(s, theta, 2);
     const int nt = 256;
     const double cut = rc + skin;
+    Kept seg = kept;
     for (int sg = steps / ck; sg >= 0 && !has_error(); --sg) {
         const int t0 = sg * ck, t1 = std::min(t0 + ck - 1, steps);
-        // recompute the interval from its checkpoint (its list is fixed),
-        // every state kept in mirror order, ghosts included
+        // the interval's lists, from its checkpoint
         restore_from(s, s.adj_ckx, s.adj_ckv, (size_t)sg);
         relist(s, false, cut);
         if (has_error()) return false;
-        const size_t stride = 3 * (size_t)s.cap_all;  // doubles per mirror
-        const size_t nseg = (size_t)(t1 - t0 + 1);
-        s.adj_segx.reserve(sizeof(double) * stride * nseg, false, s.stream);
-        s.adj_segv.reserve(sizeof(double) * stride * nseg, false, s.stream);
+        const size_t stride = kept.on ? kept.stride : 3 * (size_t)s.cap_all;  // doubles per mirror
         s.adj_mir.reserve(sizeof(double) * stride * 4, false, s.stream);
         if (has_error()) return false;
-        auto segx = [&](int t) { return s.adj_segx.as<double>() + (size_t)(t - t0) * stride; };
-        auto segv = [&](int t) { return s.adj_segv.as<double>() + (size_t)(t - t0) * stride; };
-        TMD_HIP(hipMemcpyAsync(segx(t0), s.spos.p, (size_t)kMirBytes * (size_t)s.nbinned, hipMemcpyDeviceToDevice, s.stream));
-        for (int t = t0; t <= t1 && !has_error(); ++t) {
-            TrajStep st{};
-            st.hfin = t > t0 ? h : 0.0;
-            st.adv = t < t1;
-            st.vt = Mir{segv(t)};
-            if (st.adv) st.xnext = Mir{segx(t + 1)};
-            DevBuf x;
-            x.p = segx(t);
-            // the last state's velocity needs its force too; a lone state has it
-            if (t < t1 || t > t0) traj_step(s, p, x, st, false);
-            else
-                TMD_HIP(hipMemcpyAsync(segv(t), s.svel.p, (size_t)kMirBytes * (size_t)s.nbinned, hipMemcpyDeviceToDevice, s.stream));
+        if (!kept.on) {
+            // recompute the interval (its list is fixed), every state kept in
+            // mirror order, ghosts included
+            seg = reserve_kept(s, t0, t1);
+            if (has_error()) return false;
+            copy_mirror(s, seg.X(t0), s.spos);
+            for (int t = t0; t <= t1 && !has_error(); ++t) {
+                TrajStep st{};
+                st.hfin = t > t0 ? h : 0.0;
+                st.adv = t < t1;
+                st.vt = Mir{seg.V(t)};
+                if (st.adv) st.xnext = Mir{seg.X(t + 1)};
+                DevBuf x;
+                x.p = seg.X(t);
+                // the last state's velocity needs its force too; a lone state has it
+                if (t < t1 || t > t0) traj_step(s, p, x, st, false);
+                else copy_mirror(s, seg.V(t), s.svel);
+            }
         }
         // reverse it
         double* xb = s.adj_mir.as<double>();
@@ -606,7 +659,7 @@ bool traj_adjoint(Sim& s, int steps, int ck, double dt, double rc, double skin, 
         double* fb[2] = {vb + stride, vb + 2 * stride};
         hipLaunchKernelGGL(k_adj_begin, dim3(div_up(n, nt)), dim3(nt), 0, s.stream, (const int*)s.work.as<int>(),
                            (const int*)s.work_k.as<int>(), n, (const double4*)s.adj_xbar.as<double4>(),
-                           (const double4*)s.adj_vbar.as<double4>(), (const double4*)s.adj_fbar.as<double4>(), CMir{segv(t1)}, cv, h,
+                           (const double4*)s.adj_vbar.as<double4>(), (const double4*)s.adj_fbar.as<double4>(), CMir{seg.V(t1)}, cv, h,
                            t1 >= 1 ? 1 : 0, Mir{xb}, Mir{vb}, Mir{fb[0]}, ghost_index(s));
         TMD_HIP(hipGetLastError());
         LJArgs a = make_lj_args(s, rc, eps, sigma);
@@ -621,7 +674,7 @@ bool traj_adjoint(Sim& s, int steps, int ck, double dt, double rc, double skin, 
             st.end = t == t0;
             st.post = t >= 1;
             st.pre = t - 1 >= 1;
-            if (!st.end) st.vprev = CMir{segv(t - 1)};
+            if (!st.end) st.vprev = CMir{seg.V(t - 1)};
             st.fnext = Mir{fb[1]};
             st.xbar = s.adj_xbar.as<double4>();
             st.vbar = s.adj_vbar.as<double4>();
@@ -636,7 +689,7 @@ bool traj_adjoint(Sim& s, int steps, int ck, double dt, double rc, double skin, 
             hipEvent_t ev = nullptr;
             s.timer.begin(K_ADJOINT, s.stream, &ev);
 #define TMD_ADJ(P, SH)                                                                                                  \
-    hipLaunchKernelGGL((k_lj_adjoint<P, SH>), dim3(ntiles_of(s)), dim3(s.tile_threads), lds, s.stream, CMir{segx(t)},     \
+    hipLaunchKernelGGL((k_lj_adjoint<P, SH>), dim3(ntiles_of(s)), dim3(s.tile_threads), lds, s.stream, CMir{seg.X(t)},     \
                        CMir{fb[0]}, (const int*)s.cell_start.as<int>(), (const int*)s.work.as<int>(),                    \
                        (const int*)s.work_k.as<int>(), (const int*)s.tile_start.as<int>(),                              \
                        (const int*)s.nb_count.as<int>(), (const nb_t*)s.nb_list.as<nb_t>(), a, c, st)

@@ -55,3 +55,33 @@ def test_adjoint_branches_match_oracle(tm, tile, shift, eps, sigma, steps, ck):
     # the call leaves the state at x0
     _, xa, va, _ = sim.state()
     assert np.array_equal(xa, x) and np.array_equal(va, v)
+
+
+def test_states_no_longer_kept(tm):
+    """A sheet that drifts to the face between two rebuilds, so the rebuild
+    makes room for more ghosts and the rest of the forward pass is not kept:
+    every interval is recomputed.  And the same run again, kept whole now
+    that the room is there: bit for bit the same gradients."""
+    announce("adjoint, ghosts outgrow their room")
+    L, ny = 48.0, 43
+    a = L / ny
+    g = np.arange(ny) * a
+    z, y, k = np.meshgrid(g, g, np.arange(3), indexing="ij")
+    x = np.stack([4.0 + 1.1 * k.ravel(), y.ravel(), z.ravel()], axis=1)
+    v = np.random.default_rng(3).normal(0.0, 0.3, x.shape)
+    v[:, 0] -= 35.0
+    aabb = np.array([0.0, L] * 3)
+    m = np.ones(len(x))
+    tm.load().md_deallocate_grid()
+    sim = tm.Simulation(m, x, v, aabb, RC + SKIN, lj_shift=True)
+    sim.copy_to_accelerator()
+    r = sim.traj_adjoint(25, 20, DT, RC, SKIN, 1.0, 1.0, -4.0, 1.0)
+    again = sim.traj_adjoint(25, 20, DT, RC, SKIN, 1.0, 1.0, -4.0, 1.0)
+    o = po.OracleSim(m, x, v, aabb, RC + SKIN, threads=4)
+    o.setup(False, po.HALF_GHOST_FULL, RC + SKIN)
+    o.lj(False, RC, 1.0, 1.0, shift=1)
+    q = o.traj_adjoint(25, 20, DT, RC, SKIN, 1.0, 1.0, shift=1, u_target=-4.0, p_target=1.0)
+    assert r["grad_eps"] == pytest.approx(q["grad_eps"], rel=1e-9)
+    for key in ("grad_x0", "grad_v0"):
+        assert np.linalg.norm(r[key] - q[key]) / np.linalg.norm(q[key]) <= 1e-9, key
+        assert np.array_equal(r[key], again[key]), key
