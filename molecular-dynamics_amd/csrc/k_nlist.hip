@@ -29,7 +29,7 @@ __global__ void k_mirror(const double4* __restrict__ pos, const int* __restrict_
 
 // Per-atom inputs come in work order (mirror index work_k, cell work_c), so
 // a wavefront's reads of them are contiguous.
-template <bool HALF>
+template <bool HALF, int SLOTS>
 __global__ void __launch_bounds__(kMaxTileThreads) k_nlist(const CMir spos, const int* __restrict__ work_k,
                                                         const int* __restrict__ work_c,
                                                         const int* __restrict__ start, const int* __restrict__ parts,
@@ -53,8 +53,8 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_nlist(const CMir spos, cons
         const int i = HALF ? work[w] : 0;
         const int k = work_k[w];
         int cnt2 = 0;
-        const int cnt = staged ? nlist_atom<HALF, true>(i, w, work_c[w], k, spos[k], a, W, L, spos, parts, nb_list, nb_list2, cnt2)
-                               : nlist_atom<HALF, false>(i, w, work_c[w], k, spos[k], a, W, L, spos, parts, nb_list, nb_list2, cnt2);
+        const int cnt = staged ? nlist_atom<HALF, true, SLOTS>(i, w, work_c[w], k, spos[k], a, W, L, spos, parts, nb_list, nb_list2, cnt2)
+                               : nlist_atom<HALF, false, SLOTS>(i, w, work_c[w], k, spos[k], a, W, L, spos, parts, nb_list, nb_list2, cnt2);
         nb_count[w] = cnt;
         if (HALF) nb_count2[w] = cnt2;
         const int most = max(cnt, cnt2);
@@ -215,16 +215,17 @@ void build_neighbor_lists(Sim& s, int half, double cutoff) {
         if (!cleared) rebuild_zero(s, 0, 0, s.ng);
         // the rebuild before's largest window, with room for it to grow
         const int grow = s.windows_pending ? s.max_window / kWindowGrowth + 16 : 0;
-        const ListLds l = list_lds(s.max_window + grow + kListPad, row_starts_bytes(s.tiles), s.tile_threads / kWave);
+        const ListLds l = list_lds(s.max_window + grow + kListPad, row_starts_bytes(s.tiles), s.tile_threads / kWave,
+                                     half);
         NbArgs a{s.n, s.nb_cap, half, s.half_mode, l.wcap, cutoff * cutoff, s.tiles};
         if (s.n > 0) {
-#define TMD_NLIST(H)                                                                                                   \
-    hipLaunchKernelGGL(k_nlist<H>, dim3(ntiles), dim3(l.waves * kWave), l.bytes, s.stream, CMir{s.spos.as<double>()},           \
+#define TMD_NLIST(H, R)                                                                                                   \
+    hipLaunchKernelGGL((k_nlist<H, R>), dim3(ntiles), dim3(l.waves * kWave), l.bytes, s.stream, CMir{s.spos.as<double>()},           \
                        (const int*)s.work_k.as<int>(), (const int*)s.work_c.as<int>(),                                      \
                        (const int*)s.cell_start.as<int>(), (const int*)s.cell_parts.as<int>(), (const int*)s.work.as<int>(), \
                        (const int*)s.tile_start.as<int>(), a, s.nb_count.as<int>(), s.nb_list.as<nb_t>(), \
                        s.nb_count2.as<int>(), s.nb_list2.as<nb_t>(), counters + CT_LIST)
-            if (half) TMD_NLIST(true); else TMD_NLIST(false);
+            if (half) TMD_NLIST(true, 16); else if (l.slots == 32) TMD_NLIST(false, 32); else TMD_NLIST(false, 16);
 #undef TMD_NLIST
         }
         TMD_HIP(hipGetLastError());

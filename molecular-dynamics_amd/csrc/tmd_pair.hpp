@@ -455,8 +455,7 @@ struct RingCol {
         at = cnt;
     }
 };
-constexpr int kRingSlots = 32;                           // of a lane; half lists: 16 for each column
-constexpr int kRingBytes = kRingSlots * kWave * 2;       // of a wavefront
+constexpr int ring_bytes(int slots) { return slots * kWave * 2; }  // of a wavefront
 
 // The list build's window in LDS: FP32 positions relative to a point of the
 // tile, and the atom index.
@@ -475,19 +474,25 @@ struct ListWin {
 // LDS of a block's list build: `wcap` window slots, tables of `tab` bytes and
 // the rings of as many wavefronts as there is room for, of the `want` that
 // take the fullest tile at once; with fewer (at least kListWaves, at the cost
-// of window slots), as few as do not need another round.
+// of window slots), as few as do not need another round.  A lane has 32 ring
+// slots (half lists: 16 for each column), or 16 where 32 leave too few
+// wavefronts: 64 replicas with tiles of up to 668 atoms, 11 wavefronts instead
+// of two rounds of 6, 37.5 against 38.2 ms for 200 steps; with room for all,
+// 16 slots cost 4 % of a build in more frequent stores.
 constexpr int kListWaves = 4;
 struct ListLds {
-    int wcap, waves, bytes;
+    int wcap, waves, slots, bytes;
 };
-inline ListLds list_lds(int window, int tab, int want) {
+inline ListLds list_lds(int window, int tab, int want, bool half) {
     ListLds l;
-    const int room = (kLdsBudget - tab - window * kCandBytes) / kRingBytes;
-    l.waves = std::min(want, std::max(room, kListWaves));
+    const int left = kLdsBudget - tab - window * kCandBytes;
+    l.slots = half || left / ring_bytes(32) >= want ? 32 : 16;
+    const int ring = ring_bytes(l.slots);
+    l.waves = std::min(want, std::max(left / ring, kListWaves));
     const int rounds = (want + l.waves - 1) / l.waves;
     l.waves = (want + rounds - 1) / rounds;
-    l.wcap = std::min(window, (kLdsBudget - tab - l.waves * kRingBytes) / kCandBytes);
-    l.bytes = l.wcap * kCandBytes + tab + l.waves * kRingBytes;
+    l.wcap = std::min(window, (kLdsBudget - tab - l.waves * ring) / kCandBytes);
+    l.bytes = l.wcap * kCandBytes + tab + l.waves * ring;
     return l;
 }
 __device__ __forceinline__ ListWin list_win(double* dyn, int wcap, const TileGeom& g, const double4& ref) {
@@ -567,7 +572,7 @@ __device__ __forceinline__ bool stage_list_window(const TileWin& W, int wcap, co
 // pairs whose reactions the half list would have sent to i.  STAGED is a
 // template parameter so that the staged loop addresses LDS directly (ds_read)
 // rather than through generic pointers.
-template <bool HALF, bool STAGED, class SP>
+template <bool HALF, bool STAGED, int SLOTS, class SP>
 __device__ __forceinline__ int nlist_atom(int i, int w, int c, int k_i, const double4 pi, const NbArgs& a, const TileWin& W,
                                           const ListWin& L, const SP& spos, const int* __restrict__ parts,
                                           nb_t* __restrict__ nb_list, nb_t* __restrict__ nb_list2, int& cnt2) {
@@ -578,8 +583,7 @@ __device__ __forceinline__ int nlist_atom(int i, int w, int c, int k_i, const do
     const int s_own = (cz - (W.cz0 - 1)) * wy + (cy - (W.cy0 - 1));
     const int t_i = W.seg_off[s_own] + (k_i - W.seg_beg[s_own]);
     const size_t col_off = (size_t)(w >> 6) * (size_t)a.cap * 8 + (w & 63);
-    constexpr int SLOTS = HALF ? kRingSlots / 2 : kRingSlots;
-    nb_t* ring = L.ring + (threadIdx.x / kWave) * (kRingSlots * kWave) + threadIdx.x % kWave;
+    nb_t* ring = L.ring + (threadIdx.x / kWave) * ((HALF ? 2 : 1) * SLOTS * kWave) + threadIdx.x % kWave;
     RingCol<SLOTS> A(reinterpret_cast<int4*>(nb_list) + col_off, a.cap >> 3, ring);
     RingCol<SLOTS> B(HALF ? reinterpret_cast<int4*>(nb_list2) + col_off : nullptr, a.cap >> 3, ring + SLOTS * kWave);
     const float xi = (float)(pi.x - L.ref.x), yi = (float)(pi.y - L.ref.y), zi = (float)(pi.z - L.ref.z);

@@ -192,3 +192,28 @@ def test_batch_ghost_overflow_inside_run(tm):
         xb, vb, fb = b.state(r)
         assert np.array_equal(xb, xs) and np.array_equal(vb, vs) and np.array_equal(fb, fs), r
     b.close()
+
+
+@pytest.mark.parametrize("shapes", [
+    [(4, 4, 4), (5, 7, 4), (9, 6, 8)],  # up to 7 images of an atom
+    [(3, 3, 3), (4, 3, 5), (6, 6, 6)],  # boxes under two cells long: up to 26
+])
+@pytest.mark.parametrize("precision", ["fp64", "fp32mixed"])
+def test_batch_force_pass_writes_ghosts(tm, shapes, precision):
+    """One run of 15 steps, whose force passes write the ghosts, against 15
+    runs of one step, which start with the ghost pass: bit for bit."""
+    from common import perturbed_fcc
+    announce(f"batch ghosts {shapes} {precision}")
+    boxes = []
+    for r, shape in enumerate(shapes):
+        aabb, _, x, v = perturbed_fcc(*shape, amp=0.05, seed=r)
+        boxes.append((aabb, x, v))
+    out = []
+    for runs in ([15], [1] * 15):
+        b = tm.Batch(boxes, cutoff=RC, skin=SKIN, dt=0.005, precision=precision)
+        for n in runs:
+            b.run(n)
+        out.append([a for r in range(len(boxes)) for a in b.state(r)])
+        b.close()
+    for a, c in zip(*out):
+        assert np.array_equal(a, c)
