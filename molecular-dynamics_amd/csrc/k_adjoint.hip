@@ -558,7 +558,7 @@ static bool begin_traj(Sim& s, const TrajSpec& p, bool adjoint) {
     if (s.adj_part.p) zero(s, s.adj_part.p, s.adj_part.bytes / sizeof(double));  // sums of a call that ended in an error
     if (adjoint) {
         // the reverse pass stages 48 B a window slot: tiles for that
-        s.stage_bytes = kDemStageBytes;
+        s.stage_bytes = kAdjStageBytes;
         s.stage_budget = kLdsBudget;
     }
     return !has_error();
@@ -663,8 +663,8 @@ bool traj_adjoint(Sim& s, int steps, int ck, double dt, double rc, double skin, 
                            t1 >= 1 ? 1 : 0, Mir{xb}, Mir{vb}, Mir{fb[0]}, ghost_index(s));
         TMD_HIP(hipGetLastError());
         LJArgs a = make_lj_args(s, rc, eps, sigma);
-        a.wcap = std::min(s.max_window + 1, kLdsBudget / kDemStageBytes);
-        const size_t lds = (size_t)a.wcap * kDemStageBytes;
+        a.wcap = std::min(s.max_window + 1, kLdsBudget / kAdjStageBytes);
+        const size_t lds = (size_t)a.wcap * kAdjStageBytes;
         // the adjoint kernel's precision: the forward's unless set apart
         const int prec = s.adj_precision >= 0 ? s.adj_precision : s.precision;
         for (int t = t1; t >= t0 && !has_error(); --t) {

@@ -313,6 +313,14 @@ TileGeom make_tile_geom(const Geom& G, int tx, int ty, int tz) {
     return g;
 }
 
+constexpr double kTileLocals = 320.0, kDemTileLocals = 288.0;
+
+static double mean_density(const Sim& s) {  // locals a cell of the box
+    double cells = 1.0;
+    for (int d = 0; d < 3; ++d) cells *= std::max((s.g.rank[2 * d + 1] - s.g.rank[2 * d]) / s.g.spacing, 1.0);
+    return (double)s.n / cells;
+}
+
 // Near-cubic tile shapes by size: (t, t, t), (t, t, t - 1), (t, t - 1, t - 1).
 struct TileShape {
     int x, y, z;
@@ -325,20 +333,22 @@ constexpr int kShapes = 3 * (kMaxTile - 1) + 1;
 
 // Tile of the automatic choice for `rho` atoms a cell where the box is filled,
 // a share `fill` of it, and windows of `slot` LDS bytes an atom within `budget`.
-//   1. the largest shape of at most 320 locals (a block of four or five
-//      wavefronts) whose window fits.  LJ liquid (18.5 a cell), us a step at
-//      3x2x2 against 3x3x3 cells: 40^3 FP32-mixed 54 against 57, 32^3 FP64 41
-//      against 54; from 900 cubes on the cubes are ahead (choose_tiles).  DEM
-//      gas (1.85 a cell where it is filled), 6x5x5 against 6x6x6: 64^3 51.4
-//      against 52.9;
+//   1. the largest shape of at most `most` locals whose window fits.  LJ 320 (a
+//      block of four or five wavefronts): the liquid (18.5 a cell), us a step
+//      at 3x2x2 against 3x3x3 cells: 40^3 FP32-mixed 54 against 57, 32^3 FP64
+//      41 against 54; from 900 cubes on the cubes are ahead (choose_tiles).
+//      DEM 288, by a peak density a tenth over the mean (four wavefronts, six
+//      blocks a CU): the gas (1.85 a cell where it is filled) at 64^3, 5x5x5
+//      38.3, 6x5x5 40.9, 6x6x6 39.7, 5x4x4 40.7;
 //   2. one size down where that leaves at least 160 locals and there are fewer
-//      than 1,024 tiles (DEM 48^3, 5x5x4: 26.9 against 28.8 us; the LJ liquid's
-//      next shape would have 148: 28^3 20.5 against 18.6 us);
+//      than 1,536 tiles (DEM 48^3, 5x5x4: 21.0 against 22.7 us; 64^3, 2,456
+//      tiles, 39.1 against 38.3; the LJ liquid's next shape would have 148: 28^3
+//      20.5 against 18.6 us);
 //   3. smaller still until 200 tiles hold atoms, not below two cells: a pass
 //      over fewer tiles than CUs leaves CUs idle and lasts as long as its
 //      fullest block (10^3 FP64: 27 tiles of 3x3x3 24.7 us, 196 of 2x1x1 16.6;
 //      DEM 17^3: 64 tiles of 6x6x6 17.7 us a step, 512 of 3x3x3 14.3).
-static TileShape pick_tile(const Geom& G, double rho, double fill, int slot, int budget) {
+static TileShape pick_tile(const Geom& G, double rho, double fill, int slot, int budget, double most) {
     rho = std::max(rho, 1e-3);
     auto cells = [](const TileShape& t) { return (double)t.x * t.y * t.z; };
     auto tiles = [&](const TileShape& t) {
@@ -347,10 +357,10 @@ static TileShape pick_tile(const Geom& G, double rho, double fill, int slot, int
     };
     int k = kShapes - 1;
     auto fits = [&](const TileShape& t) {
-        return cells(t) * rho <= 320.0 && (t.x + 2.0) * (t.y + 2.0) * (t.z + 2.0) * rho * slot <= 0.95 * budget;
+        return cells(t) * rho <= most && (t.x + 2.0) * (t.y + 2.0) * (t.z + 2.0) * rho * slot <= 0.95 * budget;
     };
     while (k > 0 && !fits(tile_shape(k))) --k;
-    if (k > 0 && tiles(tile_shape(k)) < 1024.0 && cells(tile_shape(k - 1)) * rho >= 160.0) --k;
+    if (k > 0 && tiles(tile_shape(k)) < 1536.0 && cells(tile_shape(k - 1)) * rho >= 160.0) --k;
     while (k > 1 && tiles(tile_shape(k)) < 200.0) --k;
     return tile_shape(k);
 }
@@ -366,13 +376,11 @@ static void choose_tiles(Sim& s) {
     int t[3] = {s.tile_req[0], s.tile_req[1], s.tile_req[2]};
     if (t[0] <= 0 || t[1] <= 0 || t[2] <= 0) {
         if (s.tile_auto[0] <= 0) {
-            double cells = 1.0;
-            for (int d = 0; d < 3; ++d) cells *= std::max((s.g.rank[2 * d + 1] - s.g.rank[2 * d]) / s.g.spacing, 1.0);
-            const double rho = (double)s.n / cells;
+            const double rho = mean_density(s);
             const int T = auto_tile_edge(s.g, s.n);
             const TileGeom cube = make_tile_geom(s.g, T, T, T);
             if (rho >= kDenseCell && cube.ntx * cube.nty * cube.ntz < kManyTiles) {
-                const TileShape p = pick_tile(s.g, rho, 1.0, kStageBytes, kLdsBudget);
+                const TileShape p = pick_tile(s.g, rho, 1.0, kStageBytes, kLdsBudget, kTileLocals);
                 s.tile_auto[0] = p.x; s.tile_auto[1] = p.y; s.tile_auto[2] = p.z;
             } else {
                 // many tiles, or sparse: there the mean density may be far from
@@ -391,22 +399,28 @@ static void choose_tiles(Sim& s) {
 // outgrow the LDS share of the force pass in use (stage_bytes per slot within
 // stage_budget per block); the pass then reads such windows from global
 // memory.  From the peak window density of the current tiles this picks the
-// tile for the next binning: once when the DEM step loop's sizes come into
-// force, and whenever a window overflows.  Tiles only shrink, and they do not
-// change the results (list order follows the cells, not the tiles).
-void retune_tiles(Sim& s) {
-    if (s.tile_req[0] > 0 && s.tile_req[1] > 0 && s.tile_req[2] > 0) return;  // explicit tiles
+// tile for the next binning: from the first statistics of a sparse box of
+// spheres with a radius (the first rebuild then bins again; 64^3: 38 us a step
+// instead of about 100 until the step loop's first rebuild), when the DEM step
+// loop's sizes come into force otherwise, and whenever a window overflows.
+// Tiles only shrink, and they do not change the results (list order follows
+// the cells, not the tiles).  True: the first rebuild should bin again.
+bool retune_tiles(Sim& s) {
+    if (s.tile_req[0] > 0 && s.tile_req[1] > 0 && s.tile_req[2] > 0) return false;  // explicit tiles
     const TileGeom& T = s.tiles;
     const bool over = (double)(s.max_window + 1) * s.stage_bytes > (double)s.stage_budget;
-    const bool first = s.stage_budget == kDemLdsShare && !s.tile_tuned;
-    if ((!over && !first) || s.max_window <= 0) return;
+    const bool sparse = !s.tile_tuned && s.dem_radius > 0.0 && mean_density(s) < kDenseCell;
+    const bool dem = s.stage_budget == kDemLdsShare || sparse, first = dem && !s.tile_tuned;
+    if ((!over && !first) || s.max_window <= 0) return false;
     s.tile_tuned = 1;
     const double peak = (s.max_window + 1) / ((T.tx + 2.0) * (T.ty + 2.0) * (T.tz + 2.0));
     double cells = 1.0;
     for (int d = 0; d < 3; ++d) cells *= std::max(s.g.len[d] / s.g.spacing, 1.0);
-    TileShape p = pick_tile(s.g, peak, std::min(1.0, s.n / (peak * cells)), s.stage_bytes, s.stage_budget);
+    TileShape p = pick_tile(s.g, peak, std::min(1.0, s.n / (peak * cells)), sparse ? kStageBytes : s.stage_bytes,
+                            sparse ? kDemLdsShare : s.stage_budget, dem ? kDemTileLocals : kTileLocals);
     if ((long long)p.x * p.y * p.z > (long long)T.tx * T.ty * T.tz) p = TileShape{T.tx, T.ty, T.tz};
     s.tile_auto[0] = p.x; s.tile_auto[1] = p.y; s.tile_auto[2] = p.z;
+    return sparse && (p.x != T.tx || p.y != T.ty || p.z != T.tz);
 }
 
 BinArgs bin_args(const Sim& s) {

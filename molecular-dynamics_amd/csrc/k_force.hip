@@ -432,20 +432,32 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_dem(TMD_KERNEL_LIST_PARAMS,
 
 // ---------------------------------------------------------------------------
 // DEM step loop with the state in the cell-ordered mirrors (spos, svel,
-// ghosts included).  The block stages its window's positions and
-// velocities into LDS (48 bytes per atom), so a contact's velocity is an LDS
-// read rather than a global gather; the lane reads its own atom at its mirror
-// index.  With ADV the pass ends the step (final kick v += f dt/2) and runs
-// the next step's kick and drift, writing the new position and velocity
-// into the other mirrors (spos_next, svel_next; other blocks still read the
-// current ones); without it (the last step) it stores the force, the
-// velocity and the position in atom order.  The pair arithmetic, the
-// contact decisions and the summation order are k_dem's, and the kicks are
+// ghosts included).  The block stages its window's positions and mirror
+// indices into LDS; the lane reads its own atom at its mirror index.  Of the
+// spheres on its list few are in contact, but in a wavefront some lane's
+// nearly always is, so the lane first tests 16 entries (both columns' first
+// groups, as a rule all there are) and then evaluates the terms of those in
+// contact, in list order, with their velocities from the mirror.
+//
+// Bounds: latency, so registers (blocks a CU) count for more than early loads;
+// only counts and first list groups are read ahead of the window.  us a step,
+// rebuilds included, against a pass that staged velocities too and evaluated
+// every entry that was in contact in some lane: 64^3 half lists FP32-mixed
+// 49.1 -> 38.3, 64^3 FP64 52.3 -> 39.7, 48^3 FP32-mixed 28.8 -> 21.0, 40^3 half
+// lists FP64 24.0 -> 18.1.  FP32-mixed is held to 80 registers, six wavefronts
+// a SIMD (39.1 without, at 87); FP64 would spill (43.9 against 39.7).
+//
+// With ADV the pass ends the step (final kick v += f dt/2) and runs the next
+// step's kick and drift, writing the new position and velocity into the other
+// mirrors (spos_next, svel_next; other blocks still read the current ones),
+// those of the sphere's ghosts too; without it (the last step) it stores the
+// force, the velocity and the position in atom order.  The pair arithmetic,
+// the contact decisions and the summation order are k_dem's, and the kicks are
 // k_dem_finish's, so the trajectory is that of the separate passes.
-static int dem_window_cap(const Sim& s) { return std::min(s.max_window + 1, kLdsBudget / kDemStageBytes); }
+static int dem_window_cap(const Sim& s) { return std::min(s.max_window + 1, kLdsBudget / kStageBytes); }
 
 template <int PREC, bool PAIR2, int ADV>
-__global__ void __launch_bounds__(kMaxTileThreads) k_dem_fused(const CMir spos, const CMir svel,
+__global__ void __launch_bounds__(kMaxTileThreads, PREC == PREC_FP64 ? 4 : 6) k_dem_fused(const CMir spos, const CMir svel,
                                                            const int* __restrict__ start, const int* __restrict__ work,
                                                            const int* __restrict__ wk, const int* __restrict__ tile_start,
                                                            const int* __restrict__ nbc, const nb_t* __restrict__ nbl,
@@ -458,69 +470,122 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_dem_fused(const CMir spos, 
     const int tile = xcd_block(blockIdx.x, gridDim.x);
     const int w0 = tile_start[tile], nloc = tile_start[tile + 1] - w0;
     if (nloc == 0) return;
+    struct Own {
+        int kw, cnt, cnt2, pk;
+        int4 e0, e1 = {};
+    } o;
+    auto fetch = [&](int at) {
+        const int w = w0 + at;
+        o.kw = wk[w];
+        o.cnt = nbc[w];
+        o.cnt2 = PAIR2 ? nbc2[w] : 0;
+        o.pk = ADV && gh.w ? gh.w[w] : 0;
+        const size_t col = (size_t)(w >> 6) * (size_t)a.cap * 8 + (w & 63);
+        o.e0 = ld_stream(reinterpret_cast<const int4*>(nbl) + col);
+        if (PAIR2) o.e1 = ld_stream(reinterpret_cast<const int4*>(nbl2) + col);
+    };
+    if ((int)threadIdx.x < nloc) fetch(threadIdx.x);
     __shared__ TileWin W;
     tile_window(tile, start, a.g, W);
-    double* sx = dyn;
-    double* sy = dyn + a.wcap;
-    double* sz = dyn + 2 * a.wcap;
-    double* su = dyn + 3 * a.wcap;
-    double* sv = dyn + 4 * a.wcap;
-    double* sw = dyn + 5 * a.wcap;
+    const WinStage sp = win_stage(dyn, a.wcap);
     const bool staged = win_size(W) <= a.wcap;
     if (staged) {
-        double4 p[kStageInFlight], q[kStageInFlight];
-        stage_rows(W, [&](int k, int u) { p[u] = spos[k]; q[u] = svel[k]; },
+        double4 p[kStageInFlight];
+        int kk[kStageInFlight];
+        stage_rows(W, [&](int k, int u) { p[u] = spos[k]; kk[u] = k; },
                    [&](int t, int u) {
-                       sx[t] = p[u].x; sy[t] = p[u].y; sz[t] = p[u].z;
-                       su[t] = q[u].x; sv[t] = q[u].y; sw[t] = q[u].z;
+                       sp.xyz[3 * t + 0] = p[u].x;
+                       sp.xyz[3 * t + 1] = p[u].y;
+                       sp.xyz[3 * t + 2] = p[u].z;
+                       sp.j[t] = kk[u];
                    });
     }
     __syncthreads();
     auto atoms = [&](auto staged_c) {
         constexpr bool STAGED = decltype(staged_c)::value;
         for (int at = threadIdx.x; at < nloc; at += blockDim.x) {
-            const int w = w0 + at;
-            const int kw = wk[w];
-            const double4 pi = spos[kw];
-            const double4 vi = svel[kw];
+            if (at >= (int)blockDim.x) fetch(at);
+            const int w = w0 + at, kw = o.kw;
+            const double4 pi = spos[kw], vi = svel[kw];
             double fx = 0.0, fy = 0.0, fz = 0.0;
-            auto entries = [&](const nb_t* __restrict__ L, int cnt) {
-                const int4* lp = reinterpret_cast<const int4*>(L + (size_t)(w >> 6) * (size_t)a.cap * 64) + (w & 63);
-                int4 e = make_int4(0, 0, 0, 0);
-                for (int k = 0; k < cnt; ++k) {
-                    if ((k & 7) == 0) e = ld_stream(lp + (size_t)(k >> 3) * 64);
-                    const int t = (k & 1) ? (int)((unsigned)e.x >> 16) : (e.x & 0xffff);
-                    if (k & 1) e = make_int4(e.y, e.z, e.w, 0);
-                    double xj, yj, zj, uj, vj, wj;
-                    if (STAGED) {
-                        xj = sx[t]; yj = sy[t]; zj = sz[t];
-                        uj = su[t]; vj = sv[t]; wj = sw[t];
-                    } else {
-                        const int kk = win_index(t, W);
-                        const double4 p = spos[kk];
-                        const double4 u = svel[kk];
-                        xj = p.x; yj = p.y; zj = p.z;
-                        uj = u.x; vj = u.y; wj = u.z;
-                    }
-                    const double dx = pi.x - xj, dy = pi.y - yj, dz = pi.z - zj;
-                    const double rsq = dx * dx + dy * dy + dz * dz;
-                    const double dd = a.d2 * a.d2 - rsq;
-                    if (rsq < a.rc2 && dd > 0.0) {
-                        double Fx, Fy, Fz;
-                        if (PREC == PREC_FP64) {
-                            dem_pair<double>(a, dx, dy, dz, rsq, dd, vi.x - uj, vi.y - vj, vi.z - wj, Fx, Fy, Fz);
-                        } else {
-                            float gx, gy, gz;
-                            dem_pair<float>(a, (float)dx, (float)dy, (float)dz, (float)rsq, (float)dd, (float)(vi.x - uj),
-                                            (float)(vi.y - vj), (float)(vi.z - wj), gx, gy, gz);
-                            Fx = gx; Fy = gy; Fz = gz;
-                        }
-                        fx = fx + Fx; fy = fy + Fy; fz = fz + Fz;
-                    }
-                }
+            const size_t col = (size_t)(w >> 6) * (size_t)a.cap * 8 + (w & 63);
+            const int ng1 = (o.cnt + 7) >> 3, ng = ng1 + (PAIR2 ? (o.cnt2 + 7) >> 3 : 0);
+            // list group g, column 2's groups behind column 1's, and its entries
+            auto group = [&](int g) {
+                return ld_stream((!PAIR2 || g < ng1) ? reinterpret_cast<const int4*>(nbl) + col + (size_t)g * 64
+                                                     : reinterpret_cast<const int4*>(nbl2) + col + (size_t)(g - ng1) * 64);
             };
-            entries(nbl, nbc[w]);
-            if (PAIR2) entries(nbl2, nbc2[w]);
+            auto in_group = [&](int g) {
+                const int left = (!PAIR2 || g < ng1) ? o.cnt - 8 * g : o.cnt2 - 8 * (g - ng1);
+                return g < ng ? min(left, 8) : 0;
+            };
+            auto at_slot = [&](int t, double& dx, double& dy, double& dz) {
+                double xj, yj, zj;
+                win_pos<STAGED>(t, sp, spos, W, xj, yj, zj);
+                dx = pi.x - xj;
+                dy = pi.y - yj;
+                dz = pi.z - zj;
+                return dx * dx + dy * dy + dz * dz;
+            };
+            int4 e0 = o.e0, e1 = o.e1;
+            if (PAIR2 ? ng1 != 1 : ng1 > 1) {  // not one group of column 1, then column 2's first
+                if (ng1 == 0) e0 = e1;
+                if (ng > 1) e1 = group(1);
+            }
+            for (int g = 0; g < ng; g += 2) {
+                if (g > 0) {
+                    e0 = group(g);
+                    if (g + 1 < ng) e1 = group(g + 1);
+                }
+                // which of the 16 entries are in contact
+                const int n0 = in_group(g), n1 = in_group(g + 1);
+                auto touching = [&](const int4 e, int n) {
+                    unsigned q = 0u;
+                    auto test = [&](int u) {
+                        double dx, dy, dz;
+                        const double rsq = at_slot(u < n ? nb_entry(e, u) : 0, dx, dy, dz);
+                        q |= rsq < a.rc2 && a.d2 * a.d2 - rsq > 0.0 ? 1u << u : 0u;
+                    };
+                    if (STAGED) {
+#pragma unroll
+                        for (int h = 0; h < 8; h += 4) {
+                            if (h >= n) break;
+#pragma unroll
+                            for (int u = h; u < h + 4; ++u) test(u);
+                        }
+                    } else {
+#pragma unroll 1
+                        for (int u = 0; u < n; ++u) test(u);
+                    }
+                    return q & ((1u << n) - 1u);
+                };
+                unsigned m = touching(e0, n0) | touching(e1, n1) << 8;
+                // their terms, in list order, the next one's velocity under way
+                auto slot = [&](unsigned q) {
+                    const int b = __builtin_ctz(q);
+                    const bool lo = b < 8;
+                    return nb_entry(make_int4(lo ? e0.x : e1.x, lo ? e0.y : e1.y, lo ? e0.z : e1.z, lo ? e0.w : e1.w), b & 7);
+                };
+                auto velocity = [&](int t) -> double4 { return svel[STAGED ? sp.j[t] : win_index(t, W)]; };
+                while (m) {
+                    const int tc = slot(m);
+                    const double4 uj = velocity(tc);
+                    m &= m - 1u;
+                    double dx, dy, dz;
+                    const double rsq = at_slot(tc, dx, dy, dz);
+                    const double dd = a.d2 * a.d2 - rsq;
+                    double Fx, Fy, Fz;
+                    if (PREC == PREC_FP64) {
+                        dem_pair<double>(a, dx, dy, dz, rsq, dd, vi.x - uj.x, vi.y - uj.y, vi.z - uj.z, Fx, Fy, Fz);
+                    } else {
+                        float gx, gy, gz;
+                        dem_pair<float>(a, (float)dx, (float)dy, (float)dz, (float)rsq, (float)dd, (float)(vi.x - uj.x),
+                                        (float)(vi.y - uj.y), (float)(vi.z - uj.z), gx, gy, gz);
+                        Fx = gx; Fy = gy; Fz = gz;
+                    }
+                    fx = fx + Fx; fy = fy + Fy; fz = fz + Fz;
+                }
+            }
             // k_dem_finish's arithmetic
             double4 v = vi;
             v.x = v.x + fx * hdt;
@@ -538,11 +603,10 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_dem_fused(const CMir spos, 
                 svel_next[kw] = v;
                 // the sphere's ghosts: its new position + image shift and its
                 // new velocity (k_ghost_step_mirror_v's arithmetic)
-                if (gh.w)
-                    each_ghost(gh, gh.w[w], [&](int e, int kg) {
-                        spos_next[kg] = ghost_image(x, gh, e);
-                        svel_next[kg] = v;
-                    });
+                each_ghost(gh, o.pk, [&](int e, int kg) {
+                    spos_next[kg] = ghost_image(x, gh, e);
+                    svel_next[kg] = v;
+                });
             } else {
                 const int i = work[w];
                 force[i] = make_double4(fx, fy, fz, 0.0);
@@ -564,7 +628,7 @@ void compute_dem_fused(Sim& s, int half, double rc, double gn, double gt, double
     s.last_force_rc = rc;
     DEMArgs a{rc * rc, 2.0 * radius, gn, gt, k, mu, s.nb_cap, s.n, s.n, dem_window_cap(s), s.tiles};
     const int nb = s.tiles.ntx * s.tiles.nty * s.tiles.ntz;
-    const size_t lds = (size_t)a.wcap * kDemStageBytes;
+    const size_t lds = (size_t)a.wcap * kStageBytes;
     const double hdt = 0.5 * dt;
     // advancing: the pass also writes the ghosts' next mirror entries
     // (from each local's ghost index), so the next step needs no ghost pass

@@ -118,8 +118,8 @@ const int* read_stats(Sim& s) {
 
 // The window statistics (locals placed, binned atoms, largest window, most
 // locals in a tile) decide the LDS size and block size of the tile kernels.
-void apply_window_stats(Sim& s, const int* st) {
-    if (!st) return;
+bool apply_window_stats(Sim& s, const int* st) {
+    if (!st) return false;
     if (st[CT_PLACED] != s.n) {
         char msg[200];
         snprintf(msg, sizeof msg,
@@ -127,25 +127,26 @@ void apply_window_stats(Sim& s, const int* st) {
                  "md_enforce_pbc wraps them)",
                  s.n - st[CT_PLACED]);
         set_error(__FILE__, __LINE__, msg);
-        return;
+        return false;
     }
     s.nbinned = st[CT_BINNED];
     s.max_window = st[CT_MAXWIN];
     s.max_locals = st[CT_MAXLOC];
     s.tile_threads = tile_block_threads(s.tile_threads_req, st[CT_MAXLOC]);
-    retune_tiles(s);
+    const bool again = retune_tiles(s);
     if (s.max_window > kWinMax) {
         char msg[200];
         snprintf(msg, sizeof msg, "a tile neighbourhood holds %d atoms, beyond the 16-bit window range (%d)", s.max_window,
                  kWinMax);
         set_error(__FILE__, __LINE__, msg);
-        return;
+        return false;
     }
     if (kLdsBudget > s.lds_limit) {
         set_error(__FILE__, __LINE__, "device LDS per block is below the window budget");
-        return;
+        return false;
     }
     s.windows_valid = 1;
+    return again;
 }
 
 // DEM step loop: positions and velocities of every binned atom, ghosts
@@ -289,7 +290,12 @@ void rebuild_lists(Sim& s, bool wrap, int half, double cutoff) {
             if (!st) return;
             if (st[CT_NGHOST] > s.cap_all - s.n) s.ghosts_missing = st[CT_NGHOST];
             else s.ng = st[CT_NGHOST];
-            apply_window_stats(s, st);  // also the binned count that a repeat reads the mirrors by
+            // also the binned count that a repeat reads the mirrors by
+            const bool tiles = apply_window_stats(s, st);
+            if (tiles && nq == s.n && !s.ghosts_missing && attempt < 2) {
+                s.max_window = 0;  // with the new tiles' sizes
+                continue;
+            }
         }
         if (!s.ghosts_missing) {
             s.timer.begin(K_NEIGHBOR, s.stream, &ev);

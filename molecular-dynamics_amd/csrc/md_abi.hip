@@ -1130,11 +1130,10 @@ static int run_loop(int steps, int reneigh_every, double dt, bool half, double c
         // DEM: positions and velocities (ghosts included) live in the cell-
         // ordered mirrors; the force pass ends each step and runs the next
         // step's kick and drift (compute_dem_fused), and a step between
-        // rebuilds is the mirror-only ghost pass and one force pass.  That
-        // pass stages positions and velocities (48 B per window slot), so
-        // automatic tiles are sized for three of its blocks per CU from the
-        // next rebuild on.
-        s.stage_bytes = kDemStageBytes;
+        // rebuilds is that one launch, ghosts included.  The pass stages
+        // positions and mirror indices (28 B per window slot); automatic tiles
+        // are sized for six of its blocks per CU from the next rebuild on.
+        s.stage_bytes = kStageBytes;
         s.stage_budget = kDemLdsShare;
         retune_tiles(s);
         if (steps > 0) initial_integration(s, dt);

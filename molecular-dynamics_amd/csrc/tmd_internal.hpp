@@ -286,12 +286,12 @@ void bin_particles(Sim& s);
 void bin_finish(Sim& s, int nq, bool with_ghosts);  // everything of a binning behind its histogram of nq source slots
 void sort_locals(Sim& s);  // PBC wrap + renumber the locals in cell order
 int auto_tile_edge(const Geom& G, int n);  // cells per tile edge for ~480 locals per tile
-void retune_tiles(Sim& s);  // automatic tiles from the window statistics, for the next binning
+bool retune_tiles(Sim& s);  // automatic tiles from the window statistics, for the next binning
 TileGeom make_tile_geom(const Geom& G, int tx, int ty, int tz);
 
 // tile windows (after binning), position mirror, neighbour lists
 const int* read_stats(Sim& s);
-void apply_window_stats(Sim& s, const int* st);
+bool apply_window_stats(Sim& s, const int* st);  // true: the first rebuild should bin again
 int window_cap(const Sim& s);      // window slots of kernels that stage positions and atom indices
 int window_cap_pos(const Sim& s);  // window slots of kernels that stage positions only
 int tile_block_threads(int requested, int max_locals);  // staged window atoms per block (LDS budget, kStageBytes each)

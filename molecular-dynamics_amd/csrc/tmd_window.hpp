@@ -34,10 +34,10 @@ constexpr int kWinMax = 65535;     // window offsets are 16-bit
 constexpr int kLdsBudget = 80 * 1024 - 1024;
 constexpr int kStageBytes = 28;       // LDS bytes per staged window atom: x, y, z 24, index 4
 constexpr int kPosStageBytes = 24;    // the same without the index (kernels that stage positions only)
-constexpr int kDemStageBytes = 48;    // DEM step pass: position and velocity, 24 + 24
-// LDS share per block of the DEM step pass: three blocks per CU (160 KiB of
-// LDS) less the static tile table
-constexpr int kDemLdsShare = 160 * 1024 / 3 - 1024;
+constexpr int kAdjStageBytes = 48;    // reverse pass of the gradients: position and force adjoint, 24 + 24
+// LDS share per block of the DEM step pass (kStageBytes a slot): six blocks
+// per CU (160 KiB of LDS) less the static tile table
+constexpr int kDemLdsShare = 160 * 1024 / 6 - 1024;
 
 // The cell-ordered mirrors of the single-box path (positions, velocities)
 // hold x, y, z doubles packed at 24 B per atom, a quarter less than double4

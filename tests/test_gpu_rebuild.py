@@ -206,3 +206,34 @@ def test_lanes_of_an_atom(tm, shape, rc, half, precision, par):
         out.append(sim.state()[1:] + tuple(sim.ghost_state()[:2]))
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+# spheres a cell of 1.3: lists of about 2 (one group or none), 8 (either side
+# of a group), 20 and 45 entries (several rounds of two groups, most of them in
+# contact); one tile shape whose blocks hold more locals than threads
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("n,tile", [(700, None), (2600, None), (6500, (2, 2, 2)), (14500, (3, 2, 2))])
+def test_dem_step_pass_dense_lists(tm, n, tile, half):
+    """Overlapping spheres at random against the oracle, which sums in another
+    order: rounding of up to 50 terms below 100 a force, 2e-12, times a time
+    step of 1e-4."""
+    announce(f"DEM step pass {n} {tile} {half}")
+    rng = np.random.default_rng(n)
+    L = 1.3 * 11.3
+    x, v = rng.random((n, 3)) * L, rng.normal(0.0, 0.3, (n, 3))
+    m, aabb = np.ones(n), np.array([0.0, L] * 3)
+    sim = tm.Simulation(m, x, v, aabb, 1.3, dem_radius=0.5, nb_cap=160)
+    if tile:
+        sim.set_tile(*tile, 64)
+    sim.copy_to_accelerator()
+    orc = po.OracleSim(m, x, v, aabb, 1.3, nb_cap=160, threads=4)
+    sim.setup(half, 1.0, 0.3)
+    orc.setup(half, po.HALF_GHOST_FULL, 1.3)
+    sim.dem(half, 1.0)
+    orc.dem(half, 1.0)
+    sim.run_dem(7, 3, 1e-4, half)
+    orc.run_dem(7, 3, 1e-4, half)
+    _, xg, vg, fg = sim.state()
+    xo, vo, fo = orc.state()
+    assert np.allclose(xg, xo, rtol=1e-13, atol=1e-13) and np.allclose(vg, vo, rtol=1e-13, atol=1e-13)
+    assert np.allclose(fg, fo, rtol=1e-12, atol=2e-12 * max(1.0, np.abs(fo).max() / 100.0))
