@@ -36,13 +36,36 @@ struct AdjCoef {
     int loss_terms;  // 0 at x_0 (the loss starts at t = 1)
 };
 
+// Both passes give an atom to a group of G lanes (atom_lanes), which share its
+// list by groups of entries and add their sums.
+// 131 registers fit three wavefronts a SIMD; held to four, G > 1 spills.
+constexpr int kGroupThreads = 768;  // threads a block with G > 1
+
+// the first list group of the lane in its atom's group of G (clamped: always a
+// valid load), and the sum of a vector over the group
+template <int G>
+__device__ __forceinline__ int4 lane_group(int cnt, const int4* __restrict__ lp) {
+    const int s = G > 1 ? min((int)threadIdx.x & (G - 1), max((cnt - 1) >> 3, 0)) : 0;
+    return ld_stream(lp + (size_t)s * 64);
+}
+template <int G>
+__device__ __forceinline__ double4 group_sum(double4 f) {
+#pragma unroll
+    for (int o = 1; o < G; o <<= 1) {
+        f.x += __shfl_xor(f.x, o);
+        f.y += __shfl_xor(f.y, o);
+        f.z += __shfl_xor(f.z, o);
+    }
+    return f;
+}
+
 // One step of a trajectory on the cell-ordered mirrors, one launch: force at
 // x_t, final kick, energy, virial and kinetic sums, and the next step's kick
 // and drift, locals and their ghosts, into the next mirror.  The arithmetic
 // and its order are those of the separate passes (force, integration, ghost
-// refresh); the energy pass, the kinetic pass, their reductions, the ghost
-// pass and the copies of states that came with them (about 60 of 75 us a
-// step at 16,384 atoms) are gone.
+// refresh), but for the order of a force's sum where G > 1; the energy pass,
+// the kinetic pass, their reductions, the ghost pass and the copies of states
+// that came with them (about 60 of 75 us a step at 16,384 atoms) are gone.
 struct TrajStep {
     Mir vel;               // velocities before the final kick in, after this pass out
     double hfin, hdt, dt;  // final kick (0: the trajectory's first force), next kick and drift
@@ -54,8 +77,8 @@ struct TrajStep {
     double* acc;           // per tile: PE, W, sum v^2, added to
 };
 
-template <int PREC, int SHIFT, int UNIT, bool ENERGY>
-__global__ void __launch_bounds__(kMaxTileThreads) k_traj_step(const CMir spos, const int* __restrict__ start,
+template <int PREC, int SHIFT, int UNIT, bool ENERGY, int G>
+__global__ void __launch_bounds__(G > 1 ? kGroupThreads : kMaxTileThreads) k_traj_step(const CMir spos, const int* __restrict__ start,
                                                             const int* __restrict__ work, const int* __restrict__ wk,
                                                             const int* __restrict__ tile_start, const int* __restrict__ nbc,
                                                             const nb_t* __restrict__ nbl, LJArgs a, TrajStep t) {
@@ -69,14 +92,19 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_traj_step(const CMir spos, 
     const bool staged = stage_window(W, a.wcap, spos, nullptr, sp);
     PairEnergy en;
     double v2 = 0.0;
-    for (int at = threadIdx.x; at < nloc; at += blockDim.x) {
+    for (int at = threadIdx.x / G; at < nloc; at += blockDim.x / G) {
         const int w = w0 + at;
         const int kw = wk[w];
         const double4 pi = spos[kw];
         const int cnt = nbc[w];
         const int4* lp = reinterpret_cast<const int4*>(nbl + (size_t)(w >> 6) * (size_t)a.cap * 64) + (w & 63);
-        const double4 f = staged ? lj_full_atom<PREC, SHIFT, UNIT, true, false, ENERGY>(pi, cnt, lp, sp, spos, W, a, ld_stream(lp), 0, nullptr, &en)
-                                 : lj_full_atom<PREC, SHIFT, UNIT, false, false, ENERGY>(pi, cnt, lp, sp, spos, W, a, ld_stream(lp), 0, nullptr, &en);
+        const int4 head = lane_group<G>(cnt, lp);
+        double4 f = staged ? lj_full_atom<PREC, SHIFT, UNIT, true, false, ENERGY, G>(pi, cnt, lp, sp, spos, W, a, head, 0, nullptr, &en)
+                           : lj_full_atom<PREC, SHIFT, UNIT, false, false, ENERGY, G>(pi, cnt, lp, sp, spos, W, a, head, 0, nullptr, &en);
+        if (G > 1) {
+            f = group_sum<G>(f);
+            if (threadIdx.x & (G - 1)) continue;
+        }
         double4 v = t.vel[kw];
         v.x = v.x + f.x * t.hfin;
         v.y = v.y + f.y * t.hfin;
@@ -128,8 +156,8 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_traj_step(const CMir spos, 
 //
 // FP64 takes 1/s correctly rounded and s as the forward pass forms it;
 // FP32-mixed skips the last rounding step and forms s with FMAs (a few 1e-16).
-// 16,384 atoms in FP64: 26 us a step by events, where the pair kernel took 86 and
-// five more passes around it 5 us each.
+// 16,384 atoms in FP64: 26 us a step by events with one lane an atom, where the
+// pair kernel took 86 and five more passes around it 5 us each.
 struct AdjStep {
     Mir xb, vb;                   // the locals' xbar, vbar (mirror order, own entry read and written)
     CMir vprev;                   // v_{t-1} (mirror order)
@@ -141,8 +169,8 @@ struct AdjStep {
     double* acc;                  // per tile: g_eps, g_sig, added to
 };
 
-template <int PREC, int SHIFT>
-__global__ void __launch_bounds__(kMaxTileThreads) k_lj_adjoint(const CMir spos, const CMir fbm, const int* __restrict__ start,
+template <int PREC, int SHIFT, int G>
+__global__ void __launch_bounds__(G > 1 ? kGroupThreads : kMaxTileThreads) k_lj_adjoint(const CMir spos, const CMir fbm, const int* __restrict__ start,
                                                              const int* __restrict__ work, const int* __restrict__ wk,
                                                              const int* __restrict__ tile_start, const int* __restrict__ nbc,
                                                              const nb_t* __restrict__ nbl, LJArgs a, AdjCoef c, AdjStep t) {
@@ -175,7 +203,7 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_lj_adjoint(const CMir spos,
     // STAGED as a compile-time constant: LDS reads, not generic-pointer loads
     auto atoms = [&](auto staged_c) {
         constexpr bool STAGED = decltype(staged_c)::value;
-        for (int at = threadIdx.x; at < nloc; at += blockDim.x) {
+        for (int at = threadIdx.x / G; at < nloc; at += blockDim.x / G) {
             const int w = w0 + at;
             const int kw = wk[w];
             const double4 pi = spos[kw];
@@ -186,10 +214,10 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_lj_adjoint(const CMir spos,
             double Prf = 0.0, Qrf = 0.0, Rrf = 0.0, Srf = 0.0;  // sums of p rf, q rf, rf, s rf
             double S6 = 0.0, S12 = 0.0, N0 = 0.0, S1 = 0.0, S2 = 0.0;  // of sr6, sr12, 1, s, s^2
             const int ng = (cnt + 7) >> 3;
-            int4 nx = ld_stream(lp);  // group 0 of the column always exists (capacity >= 8)
-            for (int gi = 0; gi < ng; ++gi) {
+            int4 nx = lane_group<G>(cnt, lp);
+            for (int gi = G > 1 ? (int)threadIdx.x & (G - 1) : 0; gi < ng; gi += G) {
                 const int4 e = nx;
-                nx = ld_stream(lp + (size_t)min(gi + 1, ng - 1) * 64);
+                nx = ld_stream(lp + (size_t)min(gi + G, ng - 1) * 64);
                 const int rem = cnt - gi * 8;
 #pragma unroll
                 for (int hb = 0; hb < 8; hb += 2) {
@@ -267,6 +295,11 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_lj_adjoint(const CMir spos,
             const double hW = 0.25 * lW, hU = 0.5 * lU;  // half of cW and cU
             g_eps += (Frf + (hU * U + hW * SF)) / a.eps;
             g_sig += Drf + (hU * DU + hW * DSF);
+            if (G > 1) {
+                const double4 sum = group_sum<G>(make_double4(ax, ay, az, 0.0));
+                ax = sum.x; ay = sum.y; az = sum.z;
+                if (threadIdx.x & (G - 1)) continue;
+            }
             double4 xb = t.xb[kw], vb = t.vb[kw];
             xb.x += ax; xb.y += ay; xb.z += az;
             double4 fb = make_double4(0.0, 0.0, 0.0, 0.0);
@@ -397,6 +430,21 @@ static void flush_sums(Sim& s, int width, double* acc) {
     TMD_HIP(hipGetLastError());
 }
 
+// Lanes an atom of both passes: four or two while all of them fit on the chip
+// at once (65,536 lanes, one wavefront a SIMD); there a pass lasts as long as
+// one wavefront's lists.  us a step of a gradient, rebuilds included, at 1, 2
+// and 4 lanes: 6^3 cells FP64 67, 52, 44; 12^3 61, 46, 39; 16^3 (16,384 atoms)
+// 61, 54, 52; 20^3 (32,000) 71, 63, 66; 24^3 mixed 95, 98, 101.
+constexpr int kChipLanes = 65536;
+static int atom_lanes(const Sim& s) {
+    if (s.tile_threads_req > 0) return 1;
+    return s.n <= kChipLanes / 4 ? 4 : (s.n <= kChipLanes / 2 ? 2 : 1);
+}
+static int group_threads(const Sim& s, int lanes) {
+    if (lanes == 1) return s.tile_threads;
+    return std::min(kGroupThreads, (std::max(s.max_locals, 1) * lanes + kWave - 1) / kWave * kWave);
+}
+
 struct TrajSpec {
     int steps, ck;
     double dt, rc, skin, eps, sigma;
@@ -418,12 +466,15 @@ static void traj_step(Sim& s, const TrajSpec& p, const DevBuf& x, TrajStep t, bo
     s.last_force_rc = p.rc;
     hipEvent_t ev = nullptr;
     s.timer.begin(K_FORCE, s.stream, &ev);
-#define TMD_TS(P, SH, U, E)                                                                                             \
-    hipLaunchKernelGGL((k_traj_step<P, SH, U, E>), dim3(ntiles_of(s)), dim3(s.tile_threads), lds, s.stream,               \
+    const int lanes = atom_lanes(s);
+    const int threads = group_threads(s, lanes);
+#define TMD_TS(P, SH, U, E, G)                                                                                             \
+    hipLaunchKernelGGL((k_traj_step<P, SH, U, E, G>), dim3(ntiles_of(s)), dim3(threads), lds, s.stream,               \
                        CMir{x.as<double>()}, (const int*)s.cell_start.as<int>(), (const int*)s.work.as<int>(),           \
                        (const int*)s.work_k.as<int>(), (const int*)s.tile_start.as<int>(),                              \
                        (const int*)s.nb_count.as<int>(), (const nb_t*)s.nb_list.as<nb_t>(), a, t)
-#define TMD_TS_E(P, SH, U) do { if (energy) TMD_TS(P, SH, U, true); else TMD_TS(P, SH, U, false); } while (0)
+#define TMD_TS_G(P, SH, U, E) do { if (lanes == 4) TMD_TS(P, SH, U, E, 4); else if (lanes == 2) TMD_TS(P, SH, U, E, 2); else TMD_TS(P, SH, U, E, 1); } while (0)
+#define TMD_TS_E(P, SH, U) do { if (energy) TMD_TS_G(P, SH, U, true); else TMD_TS_G(P, SH, U, false); } while (0)
 #define TMD_TS_U(P, SH) do { if (unit) TMD_TS_E(P, SH, 1); else TMD_TS_E(P, SH, 0); } while (0)
 #define TMD_TS_S(P) do { if (s.lj_shift) TMD_TS_U(P, 1); else TMD_TS_U(P, 0); } while (0)
     if (s.precision == PREC_FP64) TMD_TS_S(PREC_FP64);
@@ -432,6 +483,7 @@ static void traj_step(Sim& s, const TrajSpec& p, const DevBuf& x, TrajStep t, bo
 #undef TMD_TS_S
 #undef TMD_TS_U
 #undef TMD_TS_E
+#undef TMD_TS_G
 #undef TMD_TS
     s.timer.end(K_FORCE, s.stream, ev);
     TMD_HIP(hipGetLastError());
@@ -462,7 +514,8 @@ static Kept reserve_kept(Sim& s, int t0, int t1) {
 // A gradient keeps every state of its forward pass, where that takes at most
 // 4 GiB and a quarter of the free memory; else each interval is recomputed
 // from its checkpoint.  16,384 atoms over 200 steps: 0.4 GB, and the second
-// forward pass (16 us a step) is gone, 14.8 -> 11.7 ms a gradient.
+// forward pass (16 us a step) is gone, 14.8 -> 11.7 ms a gradient
+// (10.0 with the lanes of atom_lanes).
 constexpr size_t kKeptBytes = size_t(4) << 30;
 static bool keep_all(const Sim& s, int steps) {
     const size_t bytes = 2 * sizeof(double) * 3 * (size_t)s.cap_all * (size_t)(steps + 1);
@@ -688,16 +741,20 @@ bool traj_adjoint(Sim& s, int steps, int ck, double dt, double rc, double skin, 
             if (has_error()) return false;
             hipEvent_t ev = nullptr;
             s.timer.begin(K_ADJOINT, s.stream, &ev);
-#define TMD_ADJ(P, SH)                                                                                                  \
-    hipLaunchKernelGGL((k_lj_adjoint<P, SH>), dim3(ntiles_of(s)), dim3(s.tile_threads), lds, s.stream, CMir{seg.X(t)},     \
+            const int lanes = atom_lanes(s);
+            const int threads = group_threads(s, lanes);
+#define TMD_ADJ(P, SH, G)                                                                                                  \
+    hipLaunchKernelGGL((k_lj_adjoint<P, SH, G>), dim3(ntiles_of(s)), dim3(threads), lds, s.stream, CMir{seg.X(t)},     \
                        CMir{fb[0]}, (const int*)s.cell_start.as<int>(), (const int*)s.work.as<int>(),                    \
                        (const int*)s.work_k.as<int>(), (const int*)s.tile_start.as<int>(),                              \
                        (const int*)s.nb_count.as<int>(), (const nb_t*)s.nb_list.as<nb_t>(), a, c, st)
+#define TMD_ADJ_G(P, SH) do { if (lanes == 4) TMD_ADJ(P, SH, 4); else if (lanes == 2) TMD_ADJ(P, SH, 2); else TMD_ADJ(P, SH, 1); } while (0)
             if (prec == PREC_FP64) {
-                if (s.lj_shift) TMD_ADJ(PREC_FP64, 1); else TMD_ADJ(PREC_FP64, 0);
+                if (s.lj_shift) TMD_ADJ_G(PREC_FP64, 1); else TMD_ADJ_G(PREC_FP64, 0);
             } else {
-                if (s.lj_shift) TMD_ADJ(PREC_FP32_MIXED, 1); else TMD_ADJ(PREC_FP32_MIXED, 0);
+                if (s.lj_shift) TMD_ADJ_G(PREC_FP32_MIXED, 1); else TMD_ADJ_G(PREC_FP32_MIXED, 0);
             }
+#undef TMD_ADJ_G
 #undef TMD_ADJ
             s.timer.end(K_ADJOINT, s.stream, ev);
             TMD_HIP(hipGetLastError());

@@ -710,7 +710,7 @@ void compute_lj(Sim& s, int half, double rc, double eps, double sigma, double ki
         if (!fuse) GH.w = nullptr;
         const int* C2 = s.nb_count2.as<int>();
         const nb_t* L2 = s.nb_list2.as<nb_t>();
-        const int gthreads = std::min(kMaxTileThreads, (s.max_locals * kGroupLanes + kWave - 1) / kWave * kWave);
+        const int gthreads = std::min(kMaxTileThreads, (std::max(s.max_locals, 1) * kGroupLanes + kWave - 1) / kWave * kWave);
         const size_t glds = lds + (size_t)gthreads / kWave * kGroupBufBytes;
         const bool group = kick_dt > 0.0 && advance && VK && s.n <= group_atoms(s.precision) && s.tile_threads_req == 0 &&
                            glds <= (size_t)kLdsBudget;

@@ -116,6 +116,9 @@ __device__ __forceinline__ void win_pos(int t, const WinStage& st, const SP& spo
 // wavefront then runs as many groups as its busiest lane has in both
 // columns together, not the busiest lane of each column in turn.
 //
+// G > 1: lane s of a group of G takes list groups s, s + G, ..; the caller
+// adds the lanes' sums.
+//
 // ENERGY (full lists): also pe += u / 2 and vir += f r^2 / 2 of every entry
 // within the cutoff, in FP64 whatever the force's precision.
 struct PairEnergy {
@@ -125,7 +128,7 @@ template <bool PAIR2>
 __device__ __forceinline__ int4 list_head(int cnt, const int4* __restrict__ lp, const int4* __restrict__ lp2) {
     return ld_stream(!PAIR2 || cnt > 0 ? lp : lp2);
 }
-template <int PREC, int SHIFT, int UNIT, bool STAGED, bool PAIR2 = false, bool ENERGY = false, class SP = const double4*>
+template <int PREC, int SHIFT, int UNIT, bool STAGED, bool PAIR2 = false, bool ENERGY = false, int G = 1, class SP = const double4*>
 __device__ __forceinline__ double4 lj_full_atom(const double4 pi, int cnt, const int4* __restrict__ lp, const WinStage& sp,
                                                 const SP& spos, const TileWin& W, const LJArgs& a,
                                                 const int4 first, int cnt2 = 0, const int4* __restrict__ lp2 = nullptr,
@@ -143,9 +146,9 @@ __device__ __forceinline__ double4 lj_full_atom(const double4 pi, int cnt, const
     // (streaming loads: each group is read once per pass); the caller has
     // loaded the first (list_head)
     int4 q = first;
-    for (int gi = 0; gi < ng; ++gi) {
+    for (int gi = G > 1 ? (int)threadIdx.x & (G - 1) : 0; gi < ng; gi += G) {
         const int4 e = q;
-        q = ld_stream(grp(min(gi + 1, ng - 1)));  // next group (clamped: always a valid load)
+        q = ld_stream(grp(min(gi + G, ng - 1)));  // next group (clamped: always a valid load)
         const int rem = (!PAIR2 || gi < ng1) ? cnt - gi * 8 : cnt2 - (gi - ng1) * 8;  // entries in this group
         // two passes of 4 entries (fewer live registers than 8 at once),
         // unrolled: the compiler then overlaps one pass's LDS reads with the

@@ -85,3 +85,26 @@ def test_states_no_longer_kept(tm):
     for key in ("grad_x0", "grad_v0"):
         assert np.linalg.norm(r[key] - q[key]) / np.linalg.norm(q[key]) <= 1e-9, key
         assert np.array_equal(r[key], again[key]), key
+
+
+@pytest.mark.parametrize("shape,shift", [
+    ((16, 16, 16), True),   # 16,384 atoms: the last box with four lanes an atom
+    ((16, 16, 17), True),   # the first with two
+    ((16, 16, 32), False),  # 32,768 atoms: the last with two, plain cutoff
+    ((16, 16, 33), True),   # one lane an atom
+])
+def test_lanes_of_an_atom(tm, shape, shift):
+    announce(f"adjoint lanes {shape} shift={shift}")
+    aabb, m, x, v = perturbed_fcc(*shape, amp=0.05, seed=5)
+    sim = tm.Simulation(m, x, v, aabb, RC + SKIN, lj_shift=shift)
+    sim.copy_to_accelerator()
+    r = sim.traj_adjoint(5, 3, DT, RC, SKIN, 1.0, 1.0, -4.0, 1.0)
+    o = po.OracleSim(m, x, v, aabb, RC + SKIN, threads=4)
+    o.setup(False, po.HALF_GHOST_FULL, RC + SKIN)
+    o.lj(False, RC, 1.0, 1.0, shift=int(shift))
+    q = o.traj_adjoint(5, 3, DT, RC, SKIN, 1.0, 1.0, shift=int(shift), u_target=-4.0, p_target=1.0)
+    assert r["ubar"] == pytest.approx(q["ubar"], rel=1e-12)
+    assert r["grad_eps"] == pytest.approx(q["grad_eps"], rel=1e-9)
+    assert r["grad_sigma"] == pytest.approx(q["grad_sigma"], rel=1e-9)
+    for key in ("grad_x0", "grad_v0"):
+        assert np.linalg.norm(r[key] - q[key]) / np.linalg.norm(q[key]) <= 1e-9, key
