@@ -84,7 +84,7 @@ __global__ void __launch_bounds__(G > 1 ? kGroupThreads : kMaxTileThreads) k_tra
                                                             const nb_t* __restrict__ nbl, LJArgs a, TrajStep t) {
     extern __shared__ double dyn[];
     const WinStage sp = win_stage(dyn, a.wcap);
-    const int tile = xcd_block(blockIdx.x, gridDim.x);
+    const int tile = block_tile(blockIdx.x, a.g);
     const int w0 = tile_start[tile], nloc = tile_start[tile + 1] - w0;
     if (nloc == 0) return;
     __shared__ TileWin W;
@@ -175,7 +175,7 @@ __global__ void __launch_bounds__(G > 1 ? kGroupThreads : kMaxTileThreads) k_lj_
                                                              const int* __restrict__ tile_start, const int* __restrict__ nbc,
                                                              const nb_t* __restrict__ nbl, LJArgs a, AdjCoef c, AdjStep t) {
     extern __shared__ double dyn[];
-    const int tile = xcd_block(blockIdx.x, gridDim.x);
+    const int tile = block_tile(blockIdx.x, a.g);
     const int w0 = tile_start[tile], nloc = tile_start[tile + 1] - w0;
     if (nloc == 0) return;
     __shared__ TileWin W;

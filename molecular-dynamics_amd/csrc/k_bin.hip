@@ -301,6 +301,33 @@ int auto_tile_edge(const Geom& G, int n) {
     return T;
 }
 
+// A dense box of this many cubes of about 480 locals keeps them: from there
+// the smaller share of window atoms a local (4.6 against 6.7 in the LJ liquid)
+// counts for more than full CUs.  us a step at 3x3x3 against 3x2x2: 48^3
+// (1,000 cubes) FP32-mixed 62 against 65; 52^3 half lists FP64 107 against 111;
+// 80^3 214 against 226.
+constexpr int kManyTiles = 900;
+
+// Order of the blocks over the XCDs (block_tile).  Up to one tile a CU no
+// order helps, and its divisions cost 0.3 us a pass.  Dealt in runs from
+// kManyTiles on where the box fills its last layer of tiles so little that
+// equal ranges were more than 3 % uneven; else the ranges keep more of the
+// windows in one L2 (36^3 cells, 1.8 %: 42.2 against 43.4 us; 53x47x39 76.8
+// against 78.2).
+static void order_tiles(const Geom& G, TileGeom& g) {
+    double cells[3];  // of the box
+    for (int d = 0; d < 3; ++d) cells[d] = (G.rank[2 * d + 1] - G.rank[2 * d]) / G.spacing;
+    auto reached = [](double len, int edge, int nt) {
+        return (int)std::min((double)nt, std::max(1.0, std::ceil(std::ceil(len - 1e-9) / edge)));
+    };
+    g.ox = reached(cells[0], g.tx, g.ntx);
+    g.oy = reached(cells[1], g.ty, g.nty);
+    g.oz = reached(cells[2], g.tz, g.ntz);
+    const int tiles = g.ox * g.oy * g.oz;
+    if (tiles >= kManyTiles && g.oz - cells[2] / g.tz > 0.03 * g.oz) g.order = ORDER_DEAL;
+    else g.order = tiles > kNumCu && tiles < g.ntx * g.nty * g.ntz ? ORDER_BOX : ORDER_ALL;
+}
+
 TileGeom make_tile_geom(const Geom& G, int tx, int ty, int tz) {
     TileGeom g;
     g.nx = G.nx; g.ny = G.ny; g.nz = G.nz;
@@ -310,6 +337,7 @@ TileGeom make_tile_geom(const Geom& G, int tx, int ty, int tz) {
     g.ntx = std::max(1, div_up(G.nx - 2, g.tx));
     g.nty = std::max(1, div_up(G.ny - 2, g.ty));
     g.ntz = std::max(1, div_up(G.nz - 2, g.tz));
+    order_tiles(G, g);
     return g;
 }
 
@@ -365,12 +393,17 @@ static TileShape pick_tile(const Geom& G, double rho, double fill, int slot, int
     return tile_shape(k);
 }
 
-// A dense box of this many cubes of about 480 locals keeps them: from there
-// the smaller share of window atoms a local (4.6 against 6.7 in the LJ liquid)
-// counts for more than full CUs.  us a step at 3x3x3 against 3x2x2: 48^3
-// (1,000 cubes) FP32-mixed 76 against 78, half lists 87 against 91; 80^3 246
-// against 250, half lists 307 against 323; 40^3 (729) 57 against 54.
-constexpr int kManyTiles = 900;
+// Between one cube a CU and kManyTiles the pass runs in rounds of one tile a
+// CU, each as long as a tile: cubes where theirs take less.  Time of a tile as
+// of its locals and 25 more (of 500, 333 and 222 locals: 19.0, 13.3 and 9.0
+// us).  us a step at 3x3x3 against 3x2x2: 40^3 FP32-mixed (512 and 1,152
+// tiles) 37 against 45, 44^3 50 against 54, 38^3 FP64 45 against 50; 36^3 (512,
+// 968) 45 against 42, 42^3 (729, 1,521) 53 against 49, 32^3 (343, 700) 44
+// against 34.
+static double rounds(const TileGeom& g, double rho) {
+    const double tiles = (double)g.ox * g.oy * g.oz;
+    return std::ceil(tiles / kNumCu) * (rho * g.tx * g.ty * g.tz + 25.0);
+}
 
 static void choose_tiles(Sim& s) {
     int t[3] = {s.tile_req[0], s.tile_req[1], s.tile_req[2]};
@@ -379,8 +412,11 @@ static void choose_tiles(Sim& s) {
             const double rho = mean_density(s);
             const int T = auto_tile_edge(s.g, s.n);
             const TileGeom cube = make_tile_geom(s.g, T, T, T);
-            if (rho >= kDenseCell && cube.ntx * cube.nty * cube.ntz < kManyTiles) {
-                const TileShape p = pick_tile(s.g, rho, 1.0, kStageBytes, kLdsBudget, kTileLocals);
+            const int cubes = cube.ox * cube.oy * cube.oz;
+            if (rho >= kDenseCell && cubes < kManyTiles) {
+                TileShape p = pick_tile(s.g, rho, 1.0, kStageBytes, kLdsBudget, kTileLocals);
+                const TileGeom q = make_tile_geom(s.g, p.x, p.y, p.z);
+                if (cubes > kNumCu && rounds(cube, rho) < rounds(q, rho)) p = TileShape{T, T, T};
                 s.tile_auto[0] = p.x; s.tile_auto[1] = p.y; s.tile_auto[2] = p.z;
             } else {
                 // many tiles, or sparse: there the mean density may be far from

@@ -77,7 +77,7 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_lj_full(TMD_KERNEL_LIST_PAR
                                                          const nb_t* __restrict__ nbl2, GhostIndex gh) {
     extern __shared__ double dyn[];
     const WinStage sp = win_stage(dyn, a.wcap);
-    const int tile = xcd_block(blockIdx.x, gridDim.x);
+    const int tile = block_tile(blockIdx.x, a.g);
     const int w0 = tile_start[tile], nloc = tile_start[tile + 1] - w0;
     if (nloc == 0) return;
     // position, velocity, list head, ghost entries: two dependent rounds of
@@ -159,7 +159,7 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_lj_group(const CMir spos, c
     extern __shared__ double dyn[];
     const WinStage sp = win_stage(dyn, a.wcap);
     double* buf = dyn + 3 * a.wcap + threadIdx.x / kWave * (kGroupBufBytes / sizeof(double));
-    const int tile = xcd_block(blockIdx.x, gridDim.x);
+    const int tile = block_tile(blockIdx.x, a.g);
     const int w0 = tile_start[tile], nloc = tile_start[tile + 1] - w0;
     if (nloc == 0) return;
     const int c = min((int)threadIdx.x & (G - 1), 2);
@@ -247,7 +247,7 @@ template <int SHIFT>
 __global__ void __launch_bounds__(kMaxTileThreads) k_lj_energy(TMD_KERNEL_LIST_PARAMS, LJArgs a, int half,
                                                            double* __restrict__ partials) {
     extern __shared__ double dyn[];
-    const int tile = xcd_block(blockIdx.x, gridDim.x);
+    const int tile = block_tile(blockIdx.x, a.g);
     const int w0 = tile_start[tile], nloc = tile_start[tile + 1] - w0;
     if (nloc == 0) {
         if (threadIdx.x == 0) {

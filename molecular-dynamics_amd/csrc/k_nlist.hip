@@ -38,7 +38,7 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_nlist(const CMir spos, cons
                                                         int* __restrict__ nb_count2, nb_t* __restrict__ nb_list2,
                                                         int* __restrict__ overflow) {
     extern __shared__ double dyn[];
-    const int tile = blockIdx.x;
+    const int tile = block_tile(blockIdx.x, a.g);
     const int w0 = tile_start[tile], nloc = tile_start[tile + 1] - w0;
     if (nloc == 0) return;
     __shared__ TileWin W;

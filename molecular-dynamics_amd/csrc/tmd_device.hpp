@@ -205,11 +205,21 @@ __device__ __forceinline__ int4 ld_stream(const int4* p) {
 // with a private L2.  Remap so that XCD x processes one contiguous range of
 // logical blocks: atoms that are neighbours in cell order (and so share
 // neighbour positions) then share an L2.  A bijection on [0, nblocks).
-constexpr int kNumXcd = 8;
+constexpr int kNumXcd = 8, kNumCu = 256;
 __device__ __forceinline__ int xcd_block(int b, int nblocks) {
     const int q = nblocks / kNumXcd, r = nblocks % kNumXcd;
     const int x = b % kNumXcd, k = b / kNumXcd;
     return x * q + min(x, r) + k;
+}
+
+// The same for tiles of uneven work: from kDealFrom blocks on they are dealt
+// to the XCDs in runs of kDealRun, so that thin tiles at a box's far faces do
+// not all come to one XCD.
+constexpr int kDealRun = 16;
+__device__ __forceinline__ int xcd_deal(int b, int nblocks) {
+    const int full = nblocks / (kNumXcd * kDealRun) * (kNumXcd * kDealRun);
+    if (b < full) return (b / kNumXcd / kDealRun * kNumXcd + b % kNumXcd) * kDealRun + b / kNumXcd % kDealRun;
+    return full + xcd_block(b - full, nblocks - full);
 }
 
 }  // namespace tmd

@@ -78,7 +78,42 @@ struct TileGeom {
     int nx, ny, nz;     // cells
     int tx, ty, tz;     // cells per tile
     int ntx, nty, ntz;  // tiles
+    int order;          // of the blocks, TileOrder
+    int ox, oy, oz;     // tiles that the box reaches (ORDER_BOX, ORDER_DEAL)
 };
+
+// The grid may be one cell longer than the box on each side, and then its last
+// layers of tiles hold no atom; a contiguous range of all tiles for each XCD
+// leaves the last XCD idle in part.  With ORDER_BOX the ranges are of the tiles
+// that the box reaches, with ORDER_DEAL these are dealt in runs; the others
+// come last.
+enum TileOrder { ORDER_ALL = 0, ORDER_BOX = 1, ORDER_DEAL = 2 };
+
+// Tile of a block, a bijection (rule: order_tiles).  us a step, ORDER_ALL and
+// now: 80^3 FP32-mixed 217, 213; FP64 286, 280; 40^3 at 3x3x3 cells 51.0, 37.2; 30^3
+// half lists 28.9, 25.6; dealt: 46^3 half lists FP64 86, 81; 48^3 64.6, 62.0.
+__device__ __forceinline__ int block_tile(int b, const TileGeom& g) {
+    if (g.order == ORDER_ALL) return xcd_block(b, gridDim.x);
+    const int nin = g.ox * g.oy * g.oz;
+    if (b < nin) {
+        const int t = g.order == ORDER_DEAL ? xcd_deal(b, nin) : xcd_block(b, nin);
+        const int r = t / g.ox;
+        return t % g.ox + g.ntx * (r % g.oy + g.nty * (r / g.oy));
+    }
+    b -= nin;
+    const int hx = g.ntx - g.ox, hy = g.nty - g.oy;  // outer tiles of a row, outer rows of a layer
+    const int nx = hx * g.oy * g.oz, ny = g.ntx * hy * g.oz;
+    if (b < nx) {
+        const int r = b / hx;
+        return g.ox + b % hx + g.ntx * (r % g.oy + g.nty * (r / g.oy));
+    }
+    b -= nx;
+    if (b < ny) {
+        const int r = b / g.ntx;
+        return b % g.ntx + g.ntx * (g.oy + r % hy + g.nty * (r / hy));
+    }
+    return g.ntx * g.nty * g.oz + (b - ny);
+}
 
 struct TileWin {
     int cx0, cy0, cz0;          // first cell of the tile

@@ -208,6 +208,28 @@ def test_lanes_of_an_atom(tm, shape, rc, half, precision, par):
         assert np.array_equal(a, b)
 
 
+# one-cell tiles, ordered over the reached part of the grid (layers beyond it
+# on all sides, on x and y, on z) or dealt in runs (with such layers on x and
+# y, with none), against few tiles in their plain order
+@pytest.mark.parametrize("shape", [(15, 10, 20), (16, 15, 14), (14, 14, 20), (15, 15, 22), (14, 12, 22)])
+@pytest.mark.parametrize("half", [False, True])
+def test_order_of_the_tiles(tm, shape, half):
+    """The order of the blocks changes no bit."""
+    announce(f"order of the tiles {shape} {half}")
+    aabb, m, x, v = perturbed_fcc(*shape, amp=0.05, seed=7)
+    out = []
+    for tile in (1, 5):
+        sim = tm.Simulation(m, x, v, aabb, RC + SKIN)
+        sim.set_tile(tile)
+        sim.copy_to_accelerator()
+        sim.setup(half, RC, SKIN)
+        sim.lennard_jones(half, RC, 1.0, 1.0)
+        sim.run_lj(25, 10, 0.005, half, RC, SKIN, 1.0, 1.0)
+        out.append(sim.state()[1:])
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
 # spheres a cell of 1.3: lists of about 2 (one group or none), 8 (either side
 # of a group), 20 and 45 entries (several rounds of two groups, most of them in
 # contact); one tile shape whose blocks hold more locals than threads
