@@ -226,7 +226,7 @@ int tmd_batch_run_timed(int handle, int steps, double* gpu_ms);
 int tmd_batch_get_state(int handle, int rep, struct Vector3D* pos, struct Vector3D* vel, struct Vector3D* force);
 /* Per replica 6 values as tmd_thermo: T, KE, PE, virial, P, pairs. */
 int tmd_batch_thermo(int handle, double* out);
-/* Per replica 8 ints: n, ghosts, cells per x, cells, tiles, tile edge, ghost
+/* Per replica 8 ints: n, ghosts, cells per x, cells, tiles, tile edge in x, ghost
  * room, list capacity. */
 int tmd_batch_info(int handle, int* out);
 void tmd_batch_destroy(int handle);

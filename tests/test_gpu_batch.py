@@ -217,3 +217,23 @@ def test_batch_force_pass_writes_ghosts(tm, shapes, precision):
         b.close()
     for a, c in zip(*out):
         assert np.array_equal(a, c)
+
+
+def test_batch_tile_shapes(tm):
+    """Automatic tiles, another shape for each box, against cubes of two
+    cells: bit for bit."""
+    from common import perturbed_fcc
+    announce("batch tile shapes")
+    boxes = []
+    for r, shape in enumerate([(4, 4, 4), (6, 6, 6), (9, 7, 12), (16, 5, 8), (11, 11, 11)]):
+        aabb, _, x, v = perturbed_fcc(*shape, amp=0.05, seed=r)
+        boxes.append((aabb, x, v))
+    out = []
+    for tile in (0, 2):
+        b = tm.Batch(boxes, cutoff=RC, skin=SKIN, dt=0.005)
+        b.configure(tile=tile)
+        b.run(25)
+        out.append([a for r in range(len(boxes)) for a in b.state(r)])
+        b.close()
+    for a, c in zip(*out):
+        assert np.array_equal(a, c)
