@@ -500,7 +500,8 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_b_nlist(const RepDesc* __re
 // included, with no force store (as k_lj_full<..., 2>); ADV 0 stores the force.
 // As there, a lane's own loads come first (but the velocity: with it 2 % slower
 // here).  64 replicas of 864 to 55,296 atoms (1.18 M), a step between
-// rebuilds: 138 us and 14 for the ghost pass that went before, now 141.
+// rebuilds: 138 us and 14 for the ghost pass that went before, now 141, with
+// a tile shape for each replica (batch_tiles) 128.
 template <int PREC, int SHIFT, int UNIT, int ADV>
 __global__ void __launch_bounds__(kMaxTileThreads) k_b_lj_full(const RepDesc* __restrict__ R, const int* __restrict__ tile_rep,
                                                                const CMir spos, const int* __restrict__ start,

@@ -363,8 +363,9 @@ constexpr int kShapes = 3 * (kMaxTile - 1) + 1;
 // a share `fill` of it, and windows of `slot` LDS bytes an atom within `budget`.
 //   1. the largest shape of at most `most` locals whose window fits.  LJ 320 (a
 //      block of four or five wavefronts): the liquid (18.5 a cell), us a step
-//      at 3x2x2 against 3x3x3 cells: 40^3 FP32-mixed 54 against 57, 32^3 FP64
-//      41 against 54; from 900 cubes on the cubes are ahead (choose_tiles).
+//      at 3x2x2 against 3x3x3 cells: 32^3 FP64 34 against 44, 36^3 42 against
+//      45; where the cubes are ahead choose_tiles takes them (rounds,
+//      kManyTiles).
 //      DEM 288, by a peak density a tenth over the mean (four wavefronts, six
 //      blocks a CU): the gas (1.85 a cell where it is filled) at 64^3, 5x5x5
 //      38.3, 6x5x5 40.9, 6x6x6 39.7, 5x4x4 40.7;

@@ -62,7 +62,8 @@ namespace tmd {
 // step, rebuilds included: 16^3 cells mixed 23.0 -> 22.0, 32^3 FP64 41.2 ->
 // 39.1, 40^3 mixed 54.2 -> 51.9, 80^3 mixed 241 -> 237, FP64 308 -> 307.
 // Issued after the window instead, 40^3 and 80^3 mixed gain little (54.1,
-// 239): they then queue in front of the staging loads.
+// 239): they then queue in front of the staging loads.  With the list build
+// and the order of the tiles since: 19.9, 34.2, 37.1, 213 and 280.
 //
 // PAIR2 (half lists): the atom also gathers its complementary column (local
 // neighbours j > i, whose pair terms the half list evaluates from j's side),

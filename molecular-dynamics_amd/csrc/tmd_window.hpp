@@ -70,9 +70,6 @@ typedef unsigned short nb_t;
 
 // u16 list layout: tiles of 64 work slots, entry k of column l at
 // (k / 8) * 512 + l * 8 + (k % 8); one int4 load reads 8 entries of a lane.
-__device__ __forceinline__ size_t nb16_slot(int w, int k, int cap) {
-    return (size_t)(w >> 6) * (size_t)cap * 64 + (size_t)(k >> 3) * 512 + (size_t)(w & 63) * 8 + (size_t)(k & 7);
-}
 
 struct TileGeom {
     int nx, ny, nz;     // cells
