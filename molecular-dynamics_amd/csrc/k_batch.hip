@@ -113,7 +113,11 @@ __global__ void k_b_pbc(const RepDesc* __restrict__ R, const int* __restrict__ e
 }
 
 // ---------------------------------------------------------------------------
-// ghosts (k_ghost.hip order and arithmetic), one dimension per pass
+// ghosts (k_ghost.hip order and arithmetic), one dimension per pass.  The count
+// keeps each thread's items' sides (low bits: beyond the upper threshold), so
+// the scatter reads no positions but its ghosts': bound by the one reading of
+// the positions (64 replicas, 1.18 M atoms, a dimension: 20 and 30 us before,
+// now 18 and 16).
 __global__ void k_b_zero_ng(int* __restrict__ dyn, int nrep) {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r < nrep) dyn[r * DY_STRIDE + DY_NG] = 0;
@@ -121,21 +125,24 @@ __global__ void k_b_zero_ng(int* __restrict__ dyn, int nrep) {
 
 __global__ void __launch_bounds__(kScanThreads) k_b_border_count(const RepDesc* __restrict__ R, const int* __restrict__ sb_rep,
                                                                  const double4* __restrict__ pos, const int* __restrict__ dyn,
-                                                                 int d, int* __restrict__ cnt0, int* __restrict__ cnt1) {
+                                                                 int d, int* __restrict__ cnt0, int* __restrict__ cnt1,
+                                                                 unsigned char* __restrict__ sides) {
     const int r = sb_rep[blockIdx.x];
     const RepDesc& D = R[r];
     const int scan_end = D.n + dyn[r * DY_STRIDE + DY_NG];
     const int base = (blockIdx.x - D.sb0) * kScanTile + threadIdx.x * kScanItems;
-    int c0 = 0, c1 = 0;
+    int m = 0;
 #pragma unroll
     for (int it = 0; it < kScanItems; ++it) {
         const int i = base + it;
         if (i < scan_end) {
             const double p = b_comp(pos[D.a0 + i], d);
-            c0 += (p > D.hi_thr[d]) ? 1 : 0;
-            c1 += (p < D.lo_thr[d]) ? 1 : 0;
+            m |= ((p > D.hi_thr[d]) ? 1 : 0) << it;
+            m |= ((p < D.lo_thr[d]) ? 16 : 0) << it;
         }
     }
+    sides[(size_t)blockIdx.x * kScanThreads + threadIdx.x] = (unsigned char)m;
+    const int c0 = __popc(m & 15), c1 = __popc(m >> 4);
     const int t0 = block_sum_int(c0);
     const int t1 = block_sum_int(c1);
     if (threadIdx.x == 0) {
@@ -210,34 +217,22 @@ __global__ void __launch_bounds__(kScanThreads) k_b_border_scatter(const RepDesc
                                                                    double4* __restrict__ pos, int* __restrict__ g_owner,
                                                                    int* __restrict__ g_code, const int* __restrict__ off0,
                                                                    const int* __restrict__ off1, const int* __restrict__ dyn,
-                                                                   int d) {
+                                                                   int d, const unsigned char* __restrict__ sides) {
     const int r = sb_rep[blockIdx.x];
     const RepDesc& D = R[r];
     const int scan_end = dyn[r * DY_STRIDE + DY_BASE + d];  // n + ghosts before this dimension
     const int total0 = dyn[r * DY_STRIDE + DY_TOT0 + d];
     const int base = (blockIdx.x - D.sb0) * kScanTile + threadIdx.x * kScanItems;
-    int f0[kScanItems], f1[kScanItems];
-    int c0 = 0, c1 = 0;
-#pragma unroll
-    for (int it = 0; it < kScanItems; ++it) {
-        const int i = base + it;
-        f0[it] = f1[it] = 0;
-        if (i < scan_end) {
-            const double p = b_comp(pos[D.a0 + i], d);
-            f0[it] = (p > D.hi_thr[d]) ? 1 : 0;
-            f1[it] = (p < D.lo_thr[d]) ? 1 : 0;
-        }
-        c0 += f0[it];
-        c1 += f1[it];
-    }
+    const int m = sides[(size_t)blockIdx.x * kScanThreads + threadIdx.x];
+    if (!__syncthreads_or(m)) return;
     int t0, t1;
-    int r0 = off0[blockIdx.x] + block_exclusive_scan(c0, &t0);
-    int r1 = off1[blockIdx.x] + block_exclusive_scan(c1, &t1);
+    int r0 = off0[blockIdx.x] + block_exclusive_scan(__popc(m & 15), &t0);
+    int r1 = off1[blockIdx.x] + block_exclusive_scan(__popc(m >> 4), &t1);
 #pragma unroll
     for (int it = 0; it < kScanItems; ++it) {
         const int i = base + it;
-        if (f0[it]) { b_write_ghost(D, i, scan_end + r0, 0, d, pos, g_owner, g_code); r0++; }
-        if (f1[it]) { b_write_ghost(D, i, scan_end + total0 + r1, 1, d, pos, g_owner, g_code); r1++; }
+        if (m >> it & 1) { b_write_ghost(D, i, scan_end + r0, 0, d, pos, g_owner, g_code); r0++; }
+        if (m >> it & 16) { b_write_ghost(D, i, scan_end + total0 + r1, 1, d, pos, g_owner, g_code); r1++; }
     }
 }
 
@@ -468,7 +463,7 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_b_nlist(const RepDesc* __re
                                                           int* __restrict__ nb_count, nb_t* __restrict__ nb_list,
                                                           int* __restrict__ flags) {
     extern __shared__ double dyn[];
-    const int tile = blockIdx.x;
+    const int tile = xcd_deal(blockIdx.x, gridDim.x);
     const int w0 = tile_start[tile], nloc = tile_start[tile + 1] - w0;
     if (nloc == 0) return;
     const RepDesc& D = R[tile_rep[tile]];
@@ -684,7 +679,7 @@ struct Batch {
     DevBuf dR, sb_rep, eb_rep, cb_rep, gb_rep, tile_rep, cell_rep;
     DevBuf pos, vel, force, g_owner, g_code, cell_of, cell_slot, cell_inv, parts, spos, spos2, svel;
     DevBuf cell_count, cell_start, tile_count, tile_start, work, work_k, gh_n, gh;
-    DevBuf sb_cnt0, sb_cnt1, scan_tmp, nb_count, nb_list;
+    DevBuf sb_cnt0, sb_cnt1, sb_sides, scan_tmp, nb_count, nb_list;
     DevBuf dyn, flags, epart, kpart, tout;
     DevBuf snap_pos, snap_vel, snap_force;
     HostBuf h_out;  // a replica's state on its way out
@@ -702,7 +697,7 @@ struct Batch {
         drop_graphs();
         DevBuf* bufs[] = {&dR, &sb_rep, &eb_rep, &cb_rep, &gb_rep, &tile_rep, &cell_rep, &pos, &vel, &force, &g_owner,
                           &g_code, &cell_of, &cell_slot, &cell_inv, &parts, &spos, &spos2, &svel, &cell_count, &cell_start,
-                          &tile_count, &tile_start, &work, &work_k, &gh_n, &gh, &sb_cnt0, &sb_cnt1, &scan_tmp, &nb_count, &nb_list, &dyn, &flags, &epart,
+                          &tile_count, &tile_start, &work, &work_k, &gh_n, &gh, &sb_cnt0, &sb_cnt1, &sb_sides, &scan_tmp, &nb_count, &nb_list, &dyn, &flags, &epart,
                           &kpart, &tout, &snap_pos, &snap_vel, &snap_force};
         if (stream) (void)hipStreamSynchronize(stream);
         for (DevBuf* b : bufs) b->release();
@@ -738,9 +733,10 @@ static int scan_scratch(int n) { return div_up(std::max(n, 1), kScanTile) + 1; }
 // the one whose tiles, full and cut off at the far faces, cost least: a tile
 // 1.3 us, 0.9 ns a window atom and 1 us a wavefront of locals, fitted at cubes
 // of 2 and 3 cells.  Ragged cubes of 3 cells in 64 replicas of 864 to 55,296
-// atoms: 200 steps 37.2 ms, now 34.8 (with the runs of xcd_deal, 1 % of it);
-// windows to 2,400 atoms 36.4, to 2,000 39.8, to 2,900 42.8.
-constexpr double kBatchLocals = 640.0, kBatchWindow = 2700.0;
+// atoms: 200 steps 37.2 ms; windows to 2,000 atoms 39.8, to 2,400 36.4, to
+// 2,700 34.8, to 3,000 34.1 (with the runs of xcd_deal, 1 % of it).  The LDS
+// share holds 3,413.
+constexpr double kBatchLocals = 740.0, kBatchWindow = 3000.0;
 static TileGeom batch_tiles(const Geom& G, int n, int edge) {
     if (edge > 0) return make_tile_geom(G, edge, edge, edge);
     double len[3], cells = 1.0;  // of the box, in cells
@@ -888,6 +884,7 @@ static void layout(Batch& B) {
     B.work.reserve(sizeof(int) * ((size_t)B.n_work + 1), false, st);
     B.work_k.reserve(sizeof(int) * ((size_t)B.n_work + 1), false, st);
     B.sb_cnt0.reserve(sizeof(int) * (size_t)B.n_sb, false, st);
+    B.sb_sides.reserve((size_t)B.n_sb * kScanThreads, false, st);
     B.sb_cnt1.reserve(sizeof(int) * (size_t)B.n_sb, false, st);
     B.scan_tmp.reserve(sizeof(int) * (size_t)scan_scratch(std::max(B.n_cells, B.n_tiles)), false, st);
     B.nb_count.reserve(sizeof(int) * ((size_t)div_up(B.n_work, 64) * 64), false, st);
@@ -941,12 +938,13 @@ static void enq_rebuild(Batch& B) {
     for (int d = 0; d < 3; ++d) {
         hipLaunchKernelGGL(k_b_border_count, dim3(B.n_sb), dim3(kScanThreads), 0, st, R, (const int*)B.sb_rep.as<int>(),
                            (const double4*)B.pos.as<double4>(), (const int*)B.dyn.as<int>(), d, B.sb_cnt0.as<int>(),
-                           B.sb_cnt1.as<int>());
+                           B.sb_cnt1.as<int>(), B.sb_sides.as<unsigned char>());
         hipLaunchKernelGGL(k_b_border_scan, dim3(B.nrep), dim3(kScanThreads), 0, st, R, d, B.sb_cnt0.as<int>(),
                            B.sb_cnt1.as<int>(), B.dyn.as<int>(), B.flags.as<int>());
         hipLaunchKernelGGL(k_b_border_scatter, dim3(B.n_sb), dim3(kScanThreads), 0, st, R, (const int*)B.sb_rep.as<int>(),
                            B.pos.as<double4>(), B.g_owner.as<int>(), B.g_code.as<int>(), (const int*)B.sb_cnt0.as<int>(),
-                           (const int*)B.sb_cnt1.as<int>(), (const int*)B.dyn.as<int>(), d);
+                           (const int*)B.sb_cnt1.as<int>(), (const int*)B.dyn.as<int>(), d,
+                           (const unsigned char*)B.sb_sides.as<unsigned char>());
     }
     fill(B, B.cell_count, B.n_cells, 0);
     hipLaunchKernelGGL(k_b_bin_count, dim3(B.n_cb), dim3(kBlk), 0, st, R, (const int*)B.cb_rep.as<int>(),
@@ -1037,7 +1035,7 @@ static void enq_ghost_step(Batch& B, DevBuf& m) {
 // advance: also the next step's kick and drift, into the mirror `next`
 static void enq_force(Batch& B, bool kick, bool advance, const DevBuf& cur, DevBuf& next) {
     const LJArgs a = batch_lj_args(B);
-    const size_t lds = (size_t)B.wcap * kStageBytes;
+    const size_t lds = (size_t)B.wcap * kPosStageBytes;
     const bool unit = B.eps == 1.0 && B.sigma == 1.0;
     const double hdt = kick ? 0.5 * B.dt : 0.0;
 #define TMD_B_LJ_ADV(P, SH, U, ADV)                                                                                 \
@@ -1177,7 +1175,7 @@ static bool setup_lists(Batch& B) {
         B.threads = tile_block_threads(B.cfg.threads, fl[FL_MAXLOC]);
         // capacities only grow, so a restart keeps a captured run valid
         B.max_window = std::max(B.max_window, maxwin);
-        B.wcap = std::max(B.wcap, std::min(maxwin + maxwin / 4 + 64, kLdsBudget / kStageBytes));
+        B.wcap = std::max(B.wcap, std::min(maxwin + maxwin / 4 + 64, kLdsBudget / kPosStageBytes));
         enq_mirror(B, B.spos);
         for (int k = 0; k < 4 && !has_error(); ++k) {
             reserve_lists(B);
@@ -1220,7 +1218,7 @@ static std::vector<unsigned long long> graph_signature(const Batch& B) {
                             &B.force, &B.g_owner, &B.g_code, &B.cell_of, &B.cell_slot, &B.cell_inv, &B.parts, &B.spos,
                             &B.spos2, &B.svel, &B.cell_count, &B.cell_start, &B.tile_count, &B.tile_start, &B.work, &B.work_k,
                             &B.gh_n, &B.gh,
-                            &B.sb_cnt0, &B.sb_cnt1,
+                            &B.sb_cnt0, &B.sb_cnt1, &B.sb_sides,
                             &B.scan_tmp, &B.nb_count, &B.nb_list, &B.dyn, &B.flags};
     for (const DevBuf* b : bufs) s.push_back((unsigned long long)(uintptr_t)b->p);
     const double dv[] = {B.rc, B.skin, B.eps, B.sigma, B.dt};
@@ -1339,8 +1337,9 @@ static bool run_steps(Batch& B, int steps, double* gpu_ms) {
 }
 
 static void batch_thermo(Batch& B, double* out) {
-    const LJArgs a = batch_lj_args(B);
-    const size_t lds = (size_t)B.wcap * kStageBytes;
+    LJArgs a = batch_lj_args(B);
+    a.wcap = std::min(a.wcap, kLdsBudget / kStageBytes);
+    const size_t lds = (size_t)a.wcap * kStageBytes;
     enq_mirror(B, B.spos);
 #define TMD_B_EN(SH)                                                                                                 \
     hipLaunchKernelGGL(k_b_energy<SH>, dim3(B.n_tiles), dim3(B.threads), lds, B.stream,                          \
