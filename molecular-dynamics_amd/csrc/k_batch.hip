@@ -734,10 +734,14 @@ static int scan_scratch(int n) { return div_up(std::max(n, 1), kScanTile) + 1; }
 // 1.3 us, 0.9 ns a window atom and 1 us a wavefront of locals, fitted at cubes
 // of 2 and 3 cells.  Ragged cubes of 3 cells in 64 replicas of 864 to 55,296
 // atoms: 200 steps 37.2 ms; windows to 2,000 atoms 39.8, to 2,400 36.4, to
-// 2,700 34.8, to 3,000 34.1 (with the runs of xcd_deal, 1 % of it).  The LDS
-// share holds 3,413.
-constexpr double kBatchLocals = 740.0, kBatchWindow = 3000.0;
-static TileGeom batch_tiles(const Geom& G, int n, int edge) {
+// 2,700 34.8, to 3,000 34.1 (with the runs of xcd_deal, 1 % of it); the LDS
+// share holds 3,413.  In a batch of `all` atoms a full tile has at most a 200th
+// of them, down to two cells: fewer tiles leave CUs idle, and the pass lasts
+// as long as its fullest block.  us a step, without and with that bound: 2,728
+// atoms FP64 25.5, 20.2; 11,200 FP32-mixed 24.6, 17.7; 63,396 FP64 45.0, 36.6;
+// 65,628 FP32-mixed 28.9, 27.8 (a 400th: 41.8 and 32.6 for these two).
+constexpr double kBatchLocals = 740.0, kBatchWindow = 3000.0, kBatchTiles = 200.0;
+static TileGeom batch_tiles(const Geom& G, int n, double all, int edge) {
     if (edge > 0) return make_tile_geom(G, edge, edge, edge);
     double len[3], cells = 1.0;  // of the box, in cells
     for (int d = 0; d < 3; ++d) {
@@ -748,6 +752,7 @@ static TileGeom batch_tiles(const Geom& G, int n, int edge) {
     const int T = auto_tile_edge(G, n);
     TileGeom best = make_tile_geom(G, T, T, T);
     if (!(rho >= kDenseCell)) return best;
+    const double locals = std::min(kBatchLocals, std::max(2.05 * rho, all / kBatchTiles));
     double least = 1e300;
     for (int z = 1; z <= kMaxTile; ++z)
         for (int y = 1; y <= kMaxTile; ++y)
@@ -767,7 +772,7 @@ static TileGeom batch_tiles(const Geom& G, int n, int edge) {
                     most *= nt[d] > 1 ? own[d][0] : own[d][1];
                     widest *= nt[d] > 1 ? win[d][0] : win[d][1];
                 }
-                if (most > kBatchLocals || widest > kBatchWindow) continue;
+                if (most > locals || widest > kBatchWindow) continue;
                 double cost = 0.0;
                 for (int k = 0; k < 8; ++k) {
                     const int a = k & 1, b = k >> 1 & 1, c = k >> 2;
@@ -786,6 +791,8 @@ static void layout(Batch& B) {
     const double spacing = cut * B.cfg.spacing;
     std::vector<int> sb, eb, cb, gb, tr, cr;
     int a0 = 0, w0 = 0, c0 = 0, t0 = 0;
+    double all = 0.0;
+    for (int r = 0; r < B.nrep; ++r) all += B.n[r];
     // an atom is within one spacing of at most one face of a dimension if the
     // box is two spacings long: 7 images; else up to 26
     B.images = 8;
@@ -794,7 +801,7 @@ static void layout(Batch& B) {
         const double* box = &B.aabb[6 * (size_t)r];
         Geom G;
         make_geom(G, box, box, spacing);
-        D.g = batch_tiles(G, B.n[r], B.cfg.tile);
+        D.g = batch_tiles(G, B.n[r], all, B.cfg.tile);
         D.n = B.n[r];
         double vol = 1.0, volx = 1.0;
         for (int d = 0; d < 3; ++d) {

@@ -219,13 +219,19 @@ def test_batch_force_pass_writes_ghosts(tm, shapes, precision):
         assert np.array_equal(a, c)
 
 
-def test_batch_tile_shapes(tm):
+# tiles of two cells, of about 100 atoms, of full size
+@pytest.mark.parametrize("shapes", [
+    [(4, 4, 4), (5, 6, 4)],
+    [(4, 4, 4), (6, 6, 6), (9, 7, 12), (16, 5, 8), (11, 11, 11)],
+    [(6, 6, 6), (34, 34, 34)],
+])
+def test_batch_tile_shapes(tm, shapes):
     """Automatic tiles, another shape for each box, against cubes of two
     cells: bit for bit."""
     from common import perturbed_fcc
-    announce("batch tile shapes")
+    announce(f"batch tile shapes {shapes}")
     boxes = []
-    for r, shape in enumerate([(4, 4, 4), (6, 6, 6), (9, 7, 12), (16, 5, 8), (11, 11, 11)]):
+    for r, shape in enumerate(shapes):
         aabb, _, x, v = perturbed_fcc(*shape, amp=0.05, seed=r)
         boxes.append((aabb, x, v))
     out = []
