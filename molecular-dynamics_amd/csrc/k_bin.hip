@@ -525,9 +525,10 @@ static void bin_sort(Sim& s, int nq, bool mir, bool with_ghosts, bool tiles) {
 }
 
 // The tail of a rebuild after its histogram: cells, tiles, work order,
-// mirrors, ghost indices.  Nothing waits for the host.
-void bin_finish(Sim& s, int nq, bool with_ghosts) {
-    if (has_error()) return;
+// mirrors, ghost indices.  Nothing waits for the host.  False: an error came
+// before it, and nothing was done.
+bool bin_finish(Sim& s, int nq, bool with_ghosts) {
+    if (has_error()) return false;
     const bool mir = s.pos_stale != 0;
     const TileGeom tg = s.tiles;
     const int ntiles = tg.ntx * tg.nty * tg.ntz, gcap = s.cap_all - s.n, nt = 256;
@@ -576,6 +577,7 @@ void bin_finish(Sim& s, int nq, bool with_ghosts) {
     s.gsrc_valid = 1;
     s.gh_valid = s.gh_packed;
     s.windows_valid = 0;
+    return true;
 }
 
 // k-th local of the cell order <- local parts[k]: positions, velocities,

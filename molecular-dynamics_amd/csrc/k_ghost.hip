@@ -716,6 +716,30 @@ void sync_pos_from_mirror(Sim& s) {
     s.vel_mirrored = 0;
 }
 
+// A rebuild that ended in an error (atoms outside the grid, no memory) leaves
+// the locals in atom order, wrapped, with no cells and no lists; the ghosts are
+// those it made.  mir: they lived in the mirrors, of nq slots.  binned: the new
+// binning took the place of the one whose slots these are, which is then in the
+// second buffers, whole; the new one may lack the atoms that the error is about.
+// The error is set already, so this launches by itself.
+void rebuild_failed(Sim& s, bool mir, bool binned, int nq) {
+    if (mir && nq > 0)
+        hipLaunchKernelGGL(k_unmirror, dim3(div_up(nq, 256)), dim3(256), 0, s.stream,
+                           CMir{(binned ? s.spos2 : s.spos).as<double>()},
+                           (const int*)(binned ? s.cell_parts2 : s.cell_parts).as<int>(), nq, s.n, s.pos.as<double4>(),
+                           CMir{(binned ? s.svel2 : s.svel).as<double>()}, s.vel.as<double4>());
+    TMD_HIP(hipGetLastError());
+    mirror_invalidate(s);
+    s.pos_stale = 0;
+    s.vel_mirrored = 0;
+    s.inv_valid = 0;
+    s.gsrc_valid = 0;
+    s.gh_valid = 0;
+    s.nbinned = 0;
+    s.windows_valid = 0;
+    s.nb_valid = 0;
+}
+
 // velocities of the locals between atom order (vel) and mirror order (svel)
 __global__ void k_vel_mirror(const int* __restrict__ work, const int* __restrict__ wk, int n, double4* __restrict__ vel,
                              const Mir svel, int into_mirror) {

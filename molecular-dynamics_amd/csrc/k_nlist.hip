@@ -116,19 +116,21 @@ const int* read_stats(Sim& s) {
     return has_error() ? nullptr : s.h_stats;
 }
 
+static bool all_placed(const Sim& s, const int* st) {
+    if (st[CT_PLACED] == s.n) return true;
+    char msg[200];
+    snprintf(msg, sizeof msg,
+             "%d local atoms lie outside the periodic box or the cell grid (non-finite or unwrapped positions; "
+             "md_enforce_pbc wraps them)",
+             s.n - st[CT_PLACED]);
+    set_error(__FILE__, __LINE__, msg);
+    return false;
+}
+
 // The window statistics (locals placed, binned atoms, largest window, most
 // locals in a tile) decide the LDS size and block size of the tile kernels.
 bool apply_window_stats(Sim& s, const int* st) {
-    if (!st) return false;
-    if (st[CT_PLACED] != s.n) {
-        char msg[200];
-        snprintf(msg, sizeof msg,
-                 "%d local atoms lie outside the periodic box or the cell grid (non-finite or unwrapped positions; "
-                 "md_enforce_pbc wraps them)",
-                 s.n - st[CT_PLACED]);
-        set_error(__FILE__, __LINE__, msg);
-        return false;
-    }
+    if (!st || !all_placed(s, st)) return false;
     s.nbinned = st[CT_BINNED];
     s.max_window = st[CT_MAXWIN];
     s.max_locals = st[CT_MAXLOC];
@@ -239,6 +241,7 @@ void build_neighbor_lists(Sim& s, int half, double cutoff) {
             if (st[CT_NGHOST] > s.cap_all - s.n) {
                 // incomplete ghosts: the rebuild grows and repeats, from the
                 // locals of this binning
+                if (!all_placed(s, st)) return;
                 s.ghosts_missing = st[CT_NGHOST];
                 s.nbinned = st[CT_BINNED];
                 return;
@@ -271,41 +274,44 @@ void rebuild_lists(Sim& s, bool wrap, int half, double cutoff) {
         build_neighbor_lists(s, half, cutoff);
         return;
     }
-    for (int attempt = 0; attempt < 4 && !has_error(); ++attempt) {
+    for (int attempt = 0; attempt < 4; ++attempt) {
         hipEvent_t ev = nullptr;
         s.ghosts_missing = 0;
-        const int nq = s.pos_stale && s.vel_mirrored ? s.nbinned : s.n;
         s.timer.begin(K_BORDERS, s.stream, &ev);
         enqueue_ghosts(s, wrap && attempt == 0, true);
         s.timer.end(K_BORDERS, s.stream, ev);
+        // the locals' places: mirrors, or atom order
+        const bool mir = s.pos_stale != 0;
+        const int nq = mir ? s.nbinned : s.n;
         s.timer.begin(K_BIN, s.stream, &ev);
-        bin_finish(s, nq, true);
+        const bool binned = bin_finish(s, nq, true);
         s.timer.end(K_BIN, s.stream, ev);
-        if (has_error()) return;
-        if (s.max_window > 0) {
+        bool again = false;
+        if (!has_error() && s.max_window > 0) {
             s.windows_pending = 1;
             s.windows_valid = 1;
-        } else {
-            const int* st = read_stats(s);
-            if (!st) return;
+        } else if (const int* st = read_stats(s)) {
             if (st[CT_NGHOST] > s.cap_all - s.n) s.ghosts_missing = st[CT_NGHOST];
             else s.ng = st[CT_NGHOST];
             // also the binned count that a repeat reads the mirrors by
             const bool tiles = apply_window_stats(s, st);
-            if (tiles && nq == s.n && !s.ghosts_missing && attempt < 2) {
-                s.max_window = 0;  // with the new tiles' sizes
-                continue;
-            }
+            again = tiles && !mir && !s.ghosts_missing && attempt < 2;
         }
-        if (!s.ghosts_missing) {
+        if (!has_error() && !again && !s.ghosts_missing) {
             s.timer.begin(K_NEIGHBOR, s.stream, &ev);
             build_neighbor_lists(s, half, cutoff);
             s.timer.end(K_NEIGHBOR, s.stream, ev);
         }
         s.windows_pending = 0;
-        if (!s.ghosts_missing) return;
-        s.max_window = 0;
-        grow_ghosts(s, s.ghosts_missing);
+        if (!has_error() && s.ghosts_missing && attempt == 3)
+            set_error(__FILE__, __LINE__, "rebuild: the ghosts keep outgrowing their room");
+        if (has_error()) {
+            rebuild_failed(s, mir, binned, nq);
+            return;
+        }
+        if (!again && !s.ghosts_missing) return;
+        s.max_window = 0;  // again: with the new tiles' sizes
+        if (s.ghosts_missing) grow_ghosts(s, s.ghosts_missing);
     }
 }
 

@@ -274,6 +274,7 @@ void refresh_ghosts(Sim& s);
 void step_refresh(Sim& s);
 void build_ghost_src(Sim& s);  // g_ko / g_kg (binning, after the CSR is built)
 void sync_pos_from_mirror(Sim& s);
+void rebuild_failed(Sim& s, bool mir, bool binned, int nq);
 void mirror_velocities(Sim& s, bool into_mirror);
 
 // geometry (core/grid.impala:94-98): world AABB, rank AABB, cell spacing
@@ -283,7 +284,7 @@ void make_geom(Geom& G, const double* aabb, const double* rank_aabb, double cell
 BinArgs bin_args(const Sim& s);
 void bin_reserve(Sim& s);
 void bin_particles(Sim& s);
-void bin_finish(Sim& s, int nq, bool with_ghosts);  // everything of a binning behind its histogram of nq source slots
+bool bin_finish(Sim& s, int nq, bool with_ghosts);  // everything of a binning behind its histogram of nq source slots
 void sort_locals(Sim& s);  // PBC wrap + renumber the locals in cell order
 int auto_tile_edge(const Geom& G, int n);  // cells per tile edge for ~480 locals per tile
 bool retune_tiles(Sim& s);  // automatic tiles from the window statistics, for the next binning

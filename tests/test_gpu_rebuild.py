@@ -259,3 +259,49 @@ def test_dem_step_pass_dense_lists(tm, n, tile, half):
     xo, vo, fo = orc.state()
     assert np.allclose(xg, xo, rtol=1e-13, atol=1e-13) and np.allclose(vg, vo, rtol=1e-13, atol=1e-13)
     assert np.allclose(fg, fo, rtol=1e-12, atol=2e-12 * max(1.0, np.abs(fo).max() / 100.0))
+
+
+# a rebuild inside the loop, from the mirrors and, at the first step, from atom
+# order
+@pytest.mark.parametrize("dem", [False, True])
+@pytest.mark.parametrize("reneigh", [5, 1])
+def test_atom_lost_in_the_loop(tm, dem, reneigh):
+    """An atom that leaves the box by many lengths before a rebuild: an error,
+    after which the locals, the lost one too, are as they were at that rebuild,
+    wrapped, bit for bit as the separate calls leave them."""
+    announce(f"atom lost in the loop dem={dem} {reneigh}")
+    if dem:
+        m, x, v = tm.generate_granular_gas(9, vmax=2.0)
+        aabb, rc, dt = np.array([0.0, 9 * 1.6796] * 3), 1.0, 0.001
+    else:
+        aabb, m, x, v = perturbed_fcc(6, amp=0.05, seed=5)
+        rc, dt = RC, DT
+    v = v.copy()
+    v[len(x) // 2] = 1e6
+
+    def force(sim):
+        sim.dem(True, rc) if dem else sim.lennard_jones(False, rc)
+
+    def make():
+        sim = tm.Simulation(m, x, v, aabb, rc + SKIN, dem_radius=0.5 if dem else None)
+        sim.copy_to_accelerator()
+        sim.setup(dem, rc, SKIN)
+        force(sim)
+        return sim
+
+    ref = make()
+    for j in range(reneigh):
+        ref.initial_integration(dt)
+        if j + 1 < reneigh:
+            ref.synchronize_ghost_layer()
+            force(ref)
+            ref.final_integration(dt)
+    ref.enforce_pbc()
+    _, xr, vr, _ = ref.state()
+    sim = make()
+    with pytest.raises(tm.TinyMDError, match="outside the periodic box"):
+        sim.run_dem(9, reneigh, dt) if dem else sim.run_lj(9, reneigh, dt)
+    tm.load().tmd_clear_error()
+    _, xs, vs, _ = sim.state()
+    assert np.array_equal(xs, xr) and np.array_equal(vs, vr)
+    sim.close()
