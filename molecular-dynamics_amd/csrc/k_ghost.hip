@@ -817,7 +817,7 @@ static void ensure_atom_capacity(Sim& s, int need) {
     s.svel.reserve((size_t)kMirBytes * (size_t)cap, true, s.stream);
     s.gsrc_valid = 0;
     s.gh_valid = 0;
-    s.cap_all = cap;
+    if (!has_error()) s.cap_all = cap;  // as in alloc_atoms
 }
 
 // End of the DEM mirror phase: the locals' positions and velocities back to

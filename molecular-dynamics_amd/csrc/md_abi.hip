@@ -150,7 +150,8 @@ static void alloc_atoms(Sim& s, int cap) {
     s.cell_inv.reserve(sizeof(int) * (size_t)cap, false, s.stream);
     s.inv_valid = 0;
     s.force.reserve(sizeof(double4) * (size_t)std::max(s.n, 1), false, s.stream);
-    if (cap > s.cap_all) s.cap_all = cap;
+    // the room that every array has: not raised if one of them could not grow
+    if (cap > s.cap_all && !has_error()) s.cap_all = cap;
 }
 
 static void upload(Sim& s) {
