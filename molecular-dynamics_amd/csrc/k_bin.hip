@@ -522,6 +522,7 @@ static void bin_sort(Sim& s, int nq, bool mir, bool with_ghosts, bool tiles) {
     TMD_HIP(hipGetLastError());
     std::swap(s.cell_parts, s.cell_parts2);
     std::swap(s.cell_inv, s.cell_inv2);
+    s.binned_cells = has_error() ? 0 : G.ncells;
 }
 
 // The tail of a rebuild after its histogram: cells, tiles, work order,

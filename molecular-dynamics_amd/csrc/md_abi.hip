@@ -281,6 +281,7 @@ static void reset_state(Sim& s) {
     s.gsrc_valid = 0;
     s.gh_valid = s.gh_packed = 0;
     s.nbinned = 0;
+    s.binned_cells = 0;
     s.dev_valid = false;
 }
 
@@ -1019,17 +1020,26 @@ int tmd_get_cells(int* start, int* atoms, int* atom_cell) {
     Sim& s = sim();
     if (!s.stream || has_error()) return 0;
     const int nc = s.g.ncells;
-    std::vector<int> st(nc + 1);
-    TMD_HIP(hipMemcpy(st.data(), s.cell_start.p, sizeof(int) * (nc + 1), hipMemcpyDeviceToHost));
-    if (start) std::copy(st.begin(), st.end(), start);
-    if (atoms && st[nc] > 0) TMD_HIP(hipMemcpy(atoms, s.cell_parts.p, sizeof(int) * st[nc], hipMemcpyDeviceToHost));
-    if (atom_cell && s.n + s.ng > 0) {
-        std::vector<int> parts(std::max(st[nc], 1));
-        if (st[nc] > 0) TMD_HIP(hipMemcpy(parts.data(), s.cell_parts.p, sizeof(int) * st[nc], hipMemcpyDeviceToHost));
-        std::fill(atom_cell, atom_cell + s.n + s.ng, -1);
-        if (has_error()) return 0;
-        for (int c = 0; c < nc; ++c)
-            for (int k = st[c]; k < st[c + 1]; ++k) atom_cell[parts[k]] = c;
+    // the grid as it was binned: a box rescaled since may have fewer cells
+    if (s.binned_cells == 0 || nc > s.binned_cells) {
+        set_error(__FILE__, __LINE__, "tmd_get_cells: cells not binned (call md_distribute_particles first)");
+        return 0;
+    }
+    std::vector<int> st(s.binned_cells + 1);
+    TMD_HIP(hipMemcpy(st.data(), s.cell_start.p, sizeof(int) * st.size(), hipMemcpyDeviceToHost));
+    if (has_error()) return 0;
+    std::vector<int> parts(st.back());
+    if (!parts.empty()) TMD_HIP(hipMemcpy(parts.data(), s.cell_parts.p, sizeof(int) * parts.size(), hipMemcpyDeviceToHost));
+    if (has_error()) return 0;
+    if (start) std::copy(st.begin(), st.begin() + nc + 1, start);
+    if (atoms) std::copy(parts.begin(), parts.begin() + st[nc], atoms);
+    if (atom_cell) {
+        // the ghosts may be others by now, or none
+        const int nall = s.n + s.ng;
+        std::fill(atom_cell, atom_cell + nall, -1);
+        for (int c = 0; c < s.binned_cells; ++c)
+            for (int k = st[c]; k < st[c + 1]; ++k)
+                if (parts[k] < nall) atom_cell[parts[k]] = c;
     }
     return st[nc];
 }

@@ -151,6 +151,7 @@ struct Sim {
     int nb_half = 0;    // list built as a half list
     int nb_valid = 0;   // list present
     int nbinned = 0;    // atoms in the cell CSR (locals + ghosts inside the grid)
+    int binned_cells = 0;  // cells of the grid that the CSR is of (0: none)
     int max_window = 0; // largest tile window (atoms)
     int max_locals = 0; // most locals of a tile
     TileGeom tiles{};   // tile decomposition of the cell grid

@@ -1,6 +1,8 @@
 """Host arrays to the device and back, and a simulation made over another
 one: the values that went in come back bit for bit, and nothing of the
 replaced simulation is left in the new one's results."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -91,3 +93,48 @@ def test_refused_simulation_leaves_none(tm):
         tm.Simulation(m, x, v, np.array([0.0, 5.0] * 3), RC + SKIN)
     assert tm.load().md_get_number_of_particles() == 0
     tm.load().tmd_clear_error()
+
+
+def test_cells_of_the_last_binning(tm):
+    """The cells stay those of the last binning when the ghosts go or become
+    fewer, no entry is written behind the caller's arrays, and a simulation
+    made over another one has none before its own."""
+    announce("cells after the ghosts changed")
+    L = tm.load()
+    aabb, m, x, v = perturbed_fcc(7, amp=0.05, seed=9)
+    x = 0.3 + x * ((7 * 1.6796 - 0.6) / (7 * 1.6796))  # no atom within 0.3 of a face
+    v = np.where(x > 5.9, -1.0, 1.0)                   # all move inwards
+    sim = tm.Simulation(m, x, v, aabb, RC + SKIN)
+    sim.copy_to_accelerator()
+    sim.setup(False, RC, SKIN)
+    start, parts, cell = sim.cells()
+    n, ng = sim.nlocal, sim.nghost
+
+    def cells():
+        nall = sim.nlocal + sim.nghost
+        at = np.full(n + ng + 64, -7, dtype=np.int32)
+        st, pa = np.zeros_like(start), np.zeros_like(parts)
+        ptr = lambda a: a.ctypes.data_as(ctypes.POINTER(ctypes.c_int))
+        assert L.tmd_get_cells(ptr(st), ptr(pa), ptr(at)) == len(parts)
+        assert np.array_equal(st, start) and np.array_equal(pa, parts)
+        assert np.array_equal(at[:nall], cell[:nall]) and np.all(at[nall:] == -7)
+
+    cells()
+    sim.exchange()
+    assert sim.nghost == 0
+    cells()
+    sim.initial_integration(0.5)
+    sim.borders()
+    assert 0 < sim.nghost < ng
+    cells()
+    aabb2, m2, x2, v2 = perturbed_fcc(6, amp=0.05, seed=9)
+    sim = tm.Simulation(m2, x2, v2, aabb2, RC + SKIN)
+    sim.copy_to_accelerator()
+    with pytest.raises(tm.TinyMDError, match="not binned"):
+        sim.cells()
+    L.tmd_clear_error()
+    sim.setup(False, RC, SKIN)
+    st, pa, at = sim.cells()
+    for c in range(len(st) - 1):
+        assert np.all(at[pa[st[c]:st[c + 1]]] == c)
+    sim.close()
