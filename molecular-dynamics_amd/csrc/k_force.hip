@@ -157,9 +157,9 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_lj_group(const CMir spos, c
                                                           const int* __restrict__ nbc2, const nb_t* __restrict__ nbl2,
                                                           GhostIndex gh) {
     constexpr int G = kGroupLanes;
-    extern __shared__ double dyn[];
-    const WinStage sp = win_stage(dyn, a.wcap);
-    double* buf = dyn + 3 * a.wcap + threadIdx.x / kWave * (kGroupBufBytes / sizeof(double));
+    extern __shared__ __align__(16) double group_lds[];
+    const WinStage sp = win_stage(group_lds, a.wcap);
+    double* buf = group_lds + group_buf_at(a.wcap) + threadIdx.x / kWave * (kGroupBufBytes / sizeof(double));
     const int tile = block_tile(blockIdx.x, a.g);
     const int w0 = tile_start[tile], nloc = tile_start[tile + 1] - w0;
     if (nloc == 0) return;
@@ -712,7 +712,7 @@ void compute_lj(Sim& s, int half, double rc, double eps, double sigma, double ki
         const int* C2 = s.nb_count2.as<int>();
         const nb_t* L2 = s.nb_list2.as<nb_t>();
         const int gthreads = std::min(kMaxTileThreads, (std::max(s.max_locals, 1) * kGroupLanes + kWave - 1) / kWave * kWave);
-        const size_t glds = lds + (size_t)gthreads / kWave * kGroupBufBytes;
+        const size_t glds = group_buf_at(a.wcap) * sizeof(double) + (size_t)gthreads / kWave * kGroupBufBytes;
         const bool group = kick_dt > 0.0 && advance && VK && s.n <= group_atoms(s.precision) && s.tile_threads_req == 0 &&
                            glds <= (size_t)kLdsBudget;
 #define TMD_LJ_K(P, SH, U, K, H)                                                                                       \
