@@ -222,7 +222,8 @@ int tmd_batch_set_graph(int handle, int on);
  * The timed variant also returns the GPU time of the launch. */
 int tmd_batch_run(int handle, int steps);
 int tmd_batch_run_timed(int handle, int steps, double* gpu_ms);
-/* Locals of replica `rep` (any pointer may be NULL); returns their number. */
+/* Locals of replica `rep` (any pointer may be NULL); returns their number.
+ * Several host threads may read replicas of a handle at a time. */
 int tmd_batch_get_state(int handle, int rep, struct Vector3D* pos, struct Vector3D* vel, struct Vector3D* force);
 /* Per replica 6 values as tmd_thermo: T, KE, PE, virial, P, pairs. */
 int tmd_batch_thermo(int handle, double* out);

@@ -29,6 +29,7 @@
 #include <cmath>
 #include <map>
 #include <memory>
+#include <mutex>
 
 #include "tmd_internal.hpp"
 #include "tmd_pair.hpp"
@@ -682,7 +683,8 @@ struct Batch {
     DevBuf sb_cnt0, sb_cnt1, sb_sides, scan_tmp, nb_count, nb_list;
     DevBuf dyn, flags, epart, kpart, tout;
     DevBuf snap_pos, snap_vel, snap_force;
-    HostBuf h_out;  // a replica's state on its way out
+    HostBuf h_out;  // a replica's state on its way out, one reader at a time
+    std::mutex h_out_lock;
     hipStream_t stream = nullptr;
     struct CapturedRun {
         hipGraph_t graph;
@@ -1575,6 +1577,7 @@ int tmd_batch_get_state(int h, int rep, struct Vector3D* pos, struct Vector3D* v
     struct Vector3D* outs[3] = {pos, vel, force};
     DevBuf* srcs[3] = {&B->pos, &B->vel, &B->force};
     const size_t row = 3 * (size_t)n;
+    std::lock_guard<std::mutex> lock(B->h_out_lock);
     // Fresh pinned pages cost 0.37 ms a MB, and a larger buffer is all new
     // pages, so it grows in steps: to the largest replica's or 4 MiB, then at
     // least twofold.  First sweep of a handle over 64 replicas of 864 to 55,296

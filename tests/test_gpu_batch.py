@@ -3,6 +3,7 @@ through the md_* path: each replica's positions, velocities and forces are
 bit-identical (FP64 and FP32-mixed), for any tile and block size, across
 capacity retries, and with a non-default cell spacing when the single run
 uses the same spacing."""
+import threading
 import time
 
 import numpy as np
@@ -269,3 +270,28 @@ def test_first_reads_by_ascending_size(tm):
             b.close()
         best.append(min(times))
     assert best[0] < 2.0 * best[1], best
+
+
+def test_replicas_read_by_several_threads(tm):
+    """Host threads that read different replicas of one handle at a time."""
+    announce("replicas read by several threads")
+    boxes = []
+    for nc in (5, 12, 6, 14, 7, 13):
+        _, x, v = tm.generate_fcc(nc, nc, nc)
+        boxes.append((np.array([0.0, nc * 1.6796] * 3), x, v))
+    b = tm.Batch(boxes)
+    wrong = []
+
+    def read(r):
+        for _ in range(100):
+            x, v, _ = b.state(r)
+            if not (np.array_equal(x, boxes[r][1]) and np.array_equal(v, boxes[r][2])):
+                wrong.append(r)
+
+    threads = [threading.Thread(target=read, args=(r,)) for r in range(len(boxes))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+    b.close()
