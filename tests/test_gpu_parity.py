@@ -907,3 +907,33 @@ def test_window_beyond_16bit_offsets_fails_loudly(tm):
     with pytest.raises(tm.TinyMDError, match="16-bit window range"):
         sim.setup(False, RC, SKIN)
     sim.close()
+
+
+@pytest.mark.parametrize("shift", [False, True])
+@pytest.mark.parametrize("half", [False, True])
+def test_energy_of_two_atoms_at_one_point(tm, half, shift):
+    """The pair energy of a zero distance is infinite, and its virial (f r^2)
+    undefined, as IEEE arithmetic has it: in a thermo, in a batch's, and in the
+    mean energy of a trajectory that brings two atoms to one point."""
+    announce(f"two atoms at one point half={half} shift={shift}")
+    aabb = np.array([0.0, 12.0] * 3)
+    x = np.array([[5.0, 5.0, 5.0], [5.0, 5.0, 5.0], [6.25, 5.0, 5.0], [2.0, 9.0, 9.5]])
+    sim = tm.Simulation(np.ones(4), x, np.zeros_like(x), aabb, RC + SKIN, lj_shift=shift)
+    sim.copy_to_accelerator()
+    sim.setup(half, RC, SKIN)
+    th = sim.thermo(RC)
+    assert th["PE"] == np.inf and np.isnan(th["virial"]) and th["pairs"] == (3 if half else 6)
+    if half:
+        return
+    b = tm.Batch([(aabb, x, np.zeros_like(x))], precision="fp64", lj_shift=shift)
+    th = b.thermo()[0]
+    assert th["PE"] == np.inf and np.isnan(th["virial"]) and th["pairs"] == 6
+    b.close()
+    # 2.75 apart: in the lists, beyond the cutoff; at one point after a step of 0.5
+    for precision in ("fp64", "fp32mixed", "fp32kahan"):
+        x = np.array([[5.0, 5.0, 5.0], [7.75, 5.0, 5.0], [2.0, 9.0, 9.5]])
+        v = np.array([[0.0] * 3, [-5.5, 0.0, 0.0], [0.0] * 3])
+        sim = tm.Simulation(np.ones(3), x, v, aabb, RC + SKIN, lj_shift=shift, precision=precision)
+        sim.copy_to_accelerator()
+        ubar, pbar = sim.traj_loss(1, 20, 0.5)
+        assert ubar == np.inf and np.isnan(pbar)
