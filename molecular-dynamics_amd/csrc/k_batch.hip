@@ -729,7 +729,6 @@ static Batch* find_batch(int h) {
 
 static int scan_scratch(int n) { return div_up(std::max(n, 1), kScanTile) + 1; }
 
-// Descriptors, tables and buffers for the current configuration.
 // Tile of a replica of `n` atoms: of the shapes whose full tile and window
 // leave two blocks a CU (the LDS of all blocks is that of the largest window),
 // the one whose tiles, full and cut off at the far faces, cost least: a tile
@@ -752,41 +751,55 @@ static TileGeom batch_tiles(const Geom& G, int n, double all, int edge) {
     }
     const double rho = (double)n / cells;
     const int T = auto_tile_edge(G, n);
-    TileGeom best = make_tile_geom(G, T, T, T);
-    if (!(rho >= kDenseCell)) return best;
+    int t[3] = {T, T, T};
+    if (!(rho >= kDenseCell)) return make_tile_geom(G, T, T, T);
     const double locals = std::min(kBatchLocals, std::max(2.05 * rho, all / kBatchTiles));
+    // a side cut into tiles of t cells: cells and window of the full tiles [0] and
+    // of the last one [1], and how many of each; the largest tile's
+    struct Side {
+        double own[2], win[2], num[2], most, widest;
+    } side[3][kMaxTile + 1];
+    int top[3];  // longer tiles are the whole side
+    for (int d = 0; d < 3; ++d) {
+        const int nc = (d == 0 ? G.nx : (d == 1 ? G.ny : G.nz)) - 2;
+        top[d] = std::min(kMaxTile, std::max(nc, 1));
+        for (int t = 1; t <= top[d]; ++t) {
+            const int nt = std::max(1, div_up(nc, t)), before = (nt - 1) * t;
+            Side& s = side[d][t];
+            s.num[0] = nt - 1;
+            s.num[1] = 1;
+            s.own[0] = t;
+            s.win[0] = t + 2;
+            s.own[1] = std::min((double)t, std::max(len[d] - before, 0.0));
+            s.win[1] = std::min(t, nc - before) + 2;
+            s.most = s.own[nt > 1 ? 0 : 1];
+            s.widest = s.win[nt > 1 ? 0 : 1];
+        }
+    }
+    // a batch of thousands of small replicas chooses as often: shapes beyond the
+    // bounds are left early (windows grow with t)
     double least = 1e300;
-    for (int z = 1; z <= kMaxTile; ++z)
-        for (int y = 1; y <= kMaxTile; ++y)
-            for (int x = 1; x <= kMaxTile; ++x) {
-                const TileGeom g = make_tile_geom(G, x, y, z);
-                const int t[3] = {x, y, z}, nt[3] = {g.ntx, g.nty, g.ntz}, nc[3] = {G.nx - 2, G.ny - 2, G.nz - 2};
-                double own[3][2], win[3][2], num[3][2];  // cells of the full and the last tile of a side, and their count
-                double most = rho, widest = rho;
-                for (int d = 0; d < 3; ++d) {
-                    const int before = (nt[d] - 1) * t[d];
-                    num[d][0] = nt[d] - 1;
-                    num[d][1] = 1;
-                    own[d][0] = t[d];
-                    win[d][0] = t[d] + 2;
-                    own[d][1] = std::min((double)t[d], std::max(len[d] - before, 0.0));
-                    win[d][1] = std::min(t[d], nc[d] - before) + 2;
-                    most *= nt[d] > 1 ? own[d][0] : own[d][1];
-                    widest *= nt[d] > 1 ? win[d][0] : win[d][1];
-                }
-                if (most > locals || widest > kBatchWindow) continue;
+    for (int z = 1; z <= top[2]; ++z)
+        for (int y = 1; y <= top[1]; ++y)
+            for (int x = 1; x <= top[0]; ++x) {
+                const Side &X = side[0][x], &Y = side[1][y], &Z = side[2][z];
+                if (rho * X.widest * Y.widest * Z.widest > kBatchWindow) break;
+                if (rho * X.most * Y.most * Z.most > locals) continue;
                 double cost = 0.0;
                 for (int k = 0; k < 8; ++k) {
                     const int a = k & 1, b = k >> 1 & 1, c = k >> 2;
-                    const double l = rho * own[0][a] * own[1][b] * own[2][c], w = rho * win[0][a] * win[1][b] * win[2][c];
+                    const double num = X.num[a] * Y.num[b] * Z.num[c];
+                    if (num == 0.0) continue;
+                    const double l = rho * X.own[a] * Y.own[b] * Z.own[c], w = rho * X.win[a] * Y.win[b] * Z.win[c];
                     if (l < 0.5) continue;  // nothing in it
-                    cost += num[0][a] * num[1][b] * num[2][c] * (1.3 + 0.0009 * w + std::ceil(l / kWave));
+                    cost += num * (1.3 + 0.0009 * w + std::ceil(l / kWave));
                 }
-                if (cost < least) { least = cost; best = g; }
+                if (cost < least) { least = cost; t[0] = x; t[1] = y; t[2] = z; }
             }
-    return best;
+    return make_tile_geom(G, t[0], t[1], t[2]);
 }
 
+// Descriptors, tables and buffers for the current configuration.
 static void layout(Batch& B) {
     B.R.assign(B.nrep, RepDesc{});
     const double cut = B.rc + B.skin;

@@ -295,3 +295,23 @@ def test_replicas_read_by_several_threads(tm):
         t.join()
     assert not wrong
     b.close()
+
+
+def test_many_replicas_choose_tiles_quickly(tm):
+    """A restart of 3,072 replicas of 108 and 256 atoms chooses each one's tile;
+    it takes less than 1.2 times as long as with a given tile (35 ms of 127 went
+    into it once, a third again)."""
+    announce("tiles of many replicas")
+    b = tm.Batch(tm.replica_boxes(seed=3, nrep=48, cells=(3, 4)) * 64)
+    best = []
+    for tile in (4, 0):
+        b.configure(tile=tile)
+        times = []
+        for _ in range(5):
+            t = time.perf_counter()
+            b.reset()
+            times.append(time.perf_counter() - t)
+        best.append(min(times))
+    print(best, [i["tile"] for i in b.info()[:8]])
+    assert best[1] < 1.2 * best[0], best
+    b.close()
