@@ -69,6 +69,12 @@ void tmd_set_tile(int tx, int ty, int tz);
  * the fullest tile, 256..768, set at each binning. */
 void tmd_set_tile_threads(int threads);
 
+/* Room for this many ghosts or more makes the step loops and gradients refresh
+ * each step's ghosts in a pass of their own, instead of in the pass that moves
+ * their atoms; the results are the same.  0 (default): 2^26, the most that the
+ * index of that pass can number; less only for tests.  From the next rebuild. */
+void tmd_set_ghost_index_limit(int ghosts);
+
 /* ---- thermo (deterministic device reductions) ------------------------------
  * out = {T, KE, PE, W, P, pairs}: T = sum v^2 / (3N-3) (core/thermo.impala:1-16),
  * PE and the pair virial W = sum r.F over the current list (the reference

@@ -125,7 +125,7 @@ __global__ void __launch_bounds__(G > 1 ? kGroupThreads : kMaxTileThreads) k_tra
             x.y = x.y + v.y * t.dt;
             x.z = x.z + v.z * t.dt;
             t.xnext[kw] = x;
-            each_ghost(t.gh, t.gh.w[w], [&](int e, int kg) { t.xnext[kg] = ghost_image(x, t.gh, e); });
+            each_ghost(t.gh, ghost_entries(t.gh, w), [&](int e, int kg) { t.xnext[kg] = ghost_image(x, t.gh, e); });
         }
         t.vel[kw] = v;
     }
@@ -324,7 +324,7 @@ __global__ void __launch_bounds__(G > 1 ? kGroupThreads : kMaxTileThreads) k_lj_
             t.xb[kw] = xb;
             t.vb[kw] = vb;
             t.fnext[kw] = fb;
-            each_ghost(t.gh, t.gh.w[w], [&](int, int kg) { t.fnext[kg] = fb; });
+            each_ghost(t.gh, ghost_entries(t.gh, w), [&](int, int kg) { t.fnext[kg] = fb; });
         }
     };
     if (staged) atoms(std::true_type{});
@@ -374,7 +374,7 @@ __global__ void k_adj_begin(const int* __restrict__ work, const int* __restrict_
     xb[kw] = xbar[i];
     vb[kw] = b;
     fb[kw] = f;
-    each_ghost(gh, gh.w[w], [&](int, int kg) { fb[kg] = f; });
+    each_ghost(gh, ghost_entries(gh, w), [&](int, int kg) { fb[kg] = f; });
 }
 
 // ---------------------------------------------------------------------------
@@ -401,7 +401,6 @@ static void relist(Sim& s, bool wrap, double cutoff) {
     s.vel_mirror_wanted = 1;
     rebuild_lists(s, wrap, 0, cutoff);
     s.vel_mirror_wanted = 0;
-    if (!has_error() && !s.gh_valid) set_error(__FILE__, __LINE__, "trajectory: too many ghosts for the ghost index");
 }
 
 static int ntiles_of(const Sim& s) { return s.tiles.ntx * s.tiles.nty * s.tiles.ntz; }
@@ -487,6 +486,7 @@ static void traj_step(Sim& s, const TrajSpec& p, const DevBuf& x, TrajStep t, bo
 #undef TMD_TS
     s.timer.end(K_FORCE, s.stream, ev);
     TMD_HIP(hipGetLastError());
+    if (t.adv && !s.gh_valid) ghosts_from_owners(s, t.xnext.p, true);
 }
 
 // The states of the steps t0 .. of a trajectory, mirrors of positions and
@@ -715,6 +715,7 @@ bool traj_adjoint(Sim& s, int steps, int ck, double dt, double rc, double skin, 
                            (const double4*)s.adj_vbar.as<double4>(), (const double4*)s.adj_fbar.as<double4>(), CMir{seg.V(t1)}, cv, h,
                            t1 >= 1 ? 1 : 0, Mir{xb}, Mir{vb}, Mir{fb[0]}, ghost_index(s));
         TMD_HIP(hipGetLastError());
+        if (!s.gh_valid) ghosts_from_owners(s, fb[0], false);
         LJArgs a = make_lj_args(s, rc, eps, sigma);
         a.wcap = std::min(s.max_window + 1, kLdsBudget / kAdjStageBytes);
         const size_t lds = (size_t)a.wcap * kAdjStageBytes;
@@ -758,6 +759,7 @@ bool traj_adjoint(Sim& s, int steps, int ck, double dt, double rc, double skin, 
 #undef TMD_ADJ
             s.timer.end(K_ADJOINT, s.stream, ev);
             TMD_HIP(hipGetLastError());
+            if (!st.end && !s.gh_valid) ghosts_from_owners(s, fb[1], false);
             std::swap(fb[0], fb[1]);
         }
         flush_sums(s, 2, theta);

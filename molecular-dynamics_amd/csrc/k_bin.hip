@@ -575,7 +575,6 @@ bool bin_finish(Sim& s, int nq, bool with_ghosts) {
         if (!mir && s.vel_mirror_wanted) s.vel_mirrored = 1;
     }
     s.inv_valid = 1;
-    s.gsrc_valid = 1;
     s.gh_valid = s.gh_packed;
     s.windows_valid = 0;
     return true;
@@ -645,7 +644,6 @@ void sort_locals(Sim& s) {
     // every atom-indexed table is stale now
     mirror_invalidate(s);
     s.inv_valid = 0;
-    s.gsrc_valid = 0;
     s.gh_valid = s.gh_packed = 0;
     s.windows_valid = 0;
     s.nb_valid = 0;

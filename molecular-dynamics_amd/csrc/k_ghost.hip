@@ -437,32 +437,10 @@ __global__ void k_ghost_step(double4* __restrict__ pos, const int* __restrict__ 
     if (k >= 0) spos[k] = q;
 }
 
-// Mirror indices of each ghost's owner and of the ghost itself, so the
-// step loop's ghost pass reads them in ghost order instead of through inv.
-__global__ void k_ghost_src(const int* __restrict__ g_owner, const int* __restrict__ inv, int n, int ng,
-                            int* __restrict__ g_ko, int* __restrict__ g_kg) {
-    const int g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= ng) return;
-    g_ko[g] = inv[g_owner[g]];
-    g_kg[g] = inv[n + g];
-}
-
-void build_ghost_src(Sim& s) {
-    s.gsrc_valid = 0;
-    if (has_error() || s.ng == 0) return;
-    s.g_ko.reserve(sizeof(int) * (size_t)s.cap_all, false, s.stream);
-    s.g_kg.reserve(sizeof(int) * (size_t)s.cap_all, false, s.stream);
-    if (has_error()) return;
-    const int nt = 256;
-    hipLaunchKernelGGL(k_ghost_src, dim3(div_up(s.ng, nt)), dim3(nt), 0, s.stream, (const int*)s.g_owner.as<int>(),
-                       (const int*)s.cell_inv.as<int>(), s.n, s.ng, s.g_ko.as<int>(), s.g_kg.as<int>());
-    TMD_HIP(hipGetLastError());
-    s.gsrc_valid = 1;
-}
-
-// Ghost refresh inside the fused step loop, mirror only: owner (current in
-// the mirror) + image shift, k_ghost_step's arithmetic.  pos is left for
-// sync_pos_from_mirror.
+// Without a ghost index (room for kGhostIndex ghosts or more) the passes that
+// move the atoms in the mirrors leave the ghosts' entries to these: owner
+// (current in the mirror) + image shift, k_ghost_step's arithmetic.  pos is left
+// for sync_pos_from_mirror.
 __global__ void k_ghost_step_mirror(const int* __restrict__ g_ko, const int* __restrict__ g_kg,
                                     const int* __restrict__ g_code, int ng, double L0, double L1, double L2,
                                     const Mir spos) {
@@ -503,9 +481,29 @@ __global__ void k_ghost_step_mirror_v(const int* __restrict__ g_ko, const int* _
     svel[kg] = svel[ko];
 }
 
+// a vector of each owner copied to its ghosts (the gradients' force adjoints)
+__global__ void k_ghost_copy_mirror(const int* __restrict__ g_ko, const int* __restrict__ g_kg, int ng, const Mir m) {
+    const int g = blockIdx.x * blockDim.x + threadIdx.x;
+    if (g >= ng) return;
+    const int kg = g_kg[g];
+    if (kg >= 0) m[kg] = m[g_ko[g]];
+}
+
+void ghosts_from_owners(Sim& s, double* mirror, bool shift) {
+    if (has_error() || s.ng == 0) return;
+    const int nt = 256;
+    if (shift)
+        hipLaunchKernelGGL(k_ghost_step_mirror, dim3(div_up(s.ng, nt)), dim3(nt), 0, s.stream, (const int*)s.g_ko.as<int>(),
+                           (const int*)s.g_kg.as<int>(), (const int*)s.g_code.as<int>(), s.ng, s.g.len[0], s.g.len[1],
+                           s.g.len[2], Mir{mirror});
+    else
+        hipLaunchKernelGGL(k_ghost_copy_mirror, dim3(div_up(s.ng, nt)), dim3(nt), 0, s.stream, (const int*)s.g_ko.as<int>(),
+                           (const int*)s.g_kg.as<int>(), s.ng, Mir{mirror});
+    TMD_HIP(hipGetLastError());
+}
+
 void dem_ghost_step(Sim& s) {
     if (has_error() || s.ng == 0) return;
-    if (!s.gsrc_valid) build_ghost_src(s);
     const int nt = 256;
     hipLaunchKernelGGL(k_ghost_step_mirror_v, dim3(div_up(s.ng, nt)), dim3(nt), 0, s.stream, (const int*)s.g_ko.as<int>(),
                        (const int*)s.g_kg.as<int>(), (const int*)s.g_code.as<int>(), s.ng, s.g.len[0], s.g.len[1], s.g.len[2],
@@ -571,7 +569,6 @@ void enqueue_ghosts(Sim& s, bool wrap, bool bin) {
     const bool mir = s.pos_stale != 0;
     s.ghost_pos_stale = 0;  // the ghosts are made anew
     s.ng = 0;
-    s.gsrc_valid = 0;
     s.gh_valid = 0;
     if (!mir) {
         s.inv_valid = 0;
@@ -623,8 +620,7 @@ void enqueue_ghosts(Sim& s, bool wrap, bool bin) {
         exclusive_scan_int(counts, s.cls.as<int>() + ncls, ncls, ctr + CT_NGHOST, s);
         counts += ncls;
     }
-    // entry * 32 + count in 31 bits: the index ends where ghosts pass 2^26
-    s.gh_packed = gcap < (1 << 26);
+    s.gh_packed = gcap < (s.gh_limit > 0 ? s.gh_limit : kGhostIndex);
     int* pack = s.gh_packed ? s.gh_pack.as<int>() : nullptr;
 #define TMD_EMIT(M)                                                                                                      \
     hipLaunchKernelGGL(k_ghost_emit<M>, gb, blk, 0, s.stream, s.pos.as<double4>(), s.vel.as<double4>(),                    \
@@ -733,37 +729,31 @@ void rebuild_failed(Sim& s, bool mir, bool binned, int nq) {
     s.pos_stale = 0;
     s.vel_mirrored = 0;
     s.inv_valid = 0;
-    s.gsrc_valid = 0;
     s.gh_valid = 0;
     s.nbinned = 0;
     s.windows_valid = 0;
     s.nb_valid = 0;
 }
 
-// velocities of the locals between atom order (vel) and mirror order (svel)
-__global__ void k_vel_mirror(const int* __restrict__ work, const int* __restrict__ wk, int n, double4* __restrict__ vel,
-                             const Mir svel, int into_mirror) {
+// velocities of the locals from atom order (vel) to mirror order (svel)
+__global__ void k_vel_mirror(const int* __restrict__ work, const int* __restrict__ wk, int n, const double4* __restrict__ vel,
+                             const Mir svel) {
     const int w = blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= n) return;
-    if (into_mirror) svel[wk[w]] = vel[work[w]];
-    else vel[work[w]] = svel[wk[w]];
+    if (w < n) svel[wk[w]] = vel[work[w]];
 }
 
 // The fused step loop keeps the locals' velocities in mirror order (the
 // force pass then reads and writes them with the same coalesced index as the
-// positions); they return to atom order before each rebuild and at loop exit.
-void mirror_velocities(Sim& s, bool into_mirror) {
-    if (has_error() || s.n == 0) return;
-    if (into_mirror == (s.vel_mirrored != 0)) return;
-    if (into_mirror) {
-        s.svel.reserve((size_t)kMirBytes * (size_t)std::max(s.nbinned, 1), false, s.stream);
-        if (has_error()) return;
-    }
+// positions); sync_pos_from_mirror returns them to atom order.
+void mirror_velocities(Sim& s) {
+    if (has_error() || s.n == 0 || s.vel_mirrored) return;
+    s.svel.reserve((size_t)kMirBytes * (size_t)std::max(s.nbinned, 1), false, s.stream);
+    if (has_error()) return;
     const int nt = 256;
     hipLaunchKernelGGL(k_vel_mirror, dim3(div_up(s.n, nt)), dim3(nt), 0, s.stream, (const int*)s.work.as<int>(),
-                       (const int*)s.work_k.as<int>(), s.n, s.vel.as<double4>(), Mir{s.svel.as<double>()}, into_mirror ? 1 : 0);
+                       (const int*)s.work_k.as<int>(), s.n, (const double4*)s.vel.as<double4>(), Mir{s.svel.as<double>()});
     TMD_HIP(hipGetLastError());
-    s.vel_mirrored = into_mirror ? 1 : 0;
+    s.vel_mirrored = 1;
 }
 
 void step_refresh(Sim& s) {
@@ -774,19 +764,11 @@ void step_refresh(Sim& s) {
         return;
     }
     const int nt = 256;
-    if (s.ghost_stale && s.pos_stale && s.gsrc_valid) {
-        // fused step loop: the ghosts in the mirror only (pos at the end)
-        if (s.ng > 0)
-            hipLaunchKernelGGL(k_ghost_step_mirror, dim3(div_up(s.ng, nt)), dim3(nt), 0, s.stream,
-                               (const int*)s.g_ko.as<int>(), (const int*)s.g_kg.as<int>(), (const int*)s.g_code.as<int>(),
-                               s.ng, s.g.len[0], s.g.len[1], s.g.len[2], Mir{s.spos.as<double>()});
+    if (s.ghost_stale && s.pos_stale) {
+        // the last pass moved the locals in the mirror: the ghosts there only
+        // (pos at the end)
+        ghosts_from_owners(s, s.spos.as<double>(), true);
         s.ghost_pos_stale = 1;
-    } else if (s.ghost_stale) {
-        // locals are current in the mirror: rewrite the ghosts only
-        if (s.ng > 0)
-            hipLaunchKernelGGL(k_ghost_step, dim3(div_up(s.ng, nt)), dim3(nt), 0, s.stream, s.pos.as<double4>(),
-                               (const int*)s.g_owner.as<int>(), (const int*)s.g_code.as<int>(), s.n, s.ng, s.g.len[0],
-                               s.g.len[1], s.g.len[2], (const int*)s.cell_inv.as<int>(), Mir{s.spos.as<double>()});
     } else {
         hipLaunchKernelGGL(k_step_refresh, dim3(div_up(s.n + s.ng, nt)), dim3(nt), 0, s.stream, s.pos.as<double4>(),
                            (const int*)s.g_owner.as<int>(), (const int*)s.g_code.as<int>(), s.n, s.ng, s.g.len[0], s.g.len[1],
@@ -815,7 +797,6 @@ static void ensure_atom_capacity(Sim& s, int need) {
     s.cell_inv.reserve(sizeof(int) * (size_t)cap, true, s.stream);
     s.spos.reserve((size_t)kMirBytes * (size_t)cap, true, s.stream);
     s.svel.reserve((size_t)kMirBytes * (size_t)cap, true, s.stream);
-    s.gsrc_valid = 0;
     s.gh_valid = 0;
     if (!has_error()) s.cap_all = cap;  // as in alloc_atoms
 }

@@ -278,7 +278,6 @@ static void reset_state(Sim& s) {
     s.vel_mirror_wanted = 0;
     s.ghost_pos_stale = 0;
     s.dem_mirrored = 0;
-    s.gsrc_valid = 0;
     s.gh_valid = s.gh_packed = 0;
     s.nbinned = 0;
     s.binned_cells = 0;
@@ -896,6 +895,7 @@ void tmd_set_sync(int on) { sim().sync_calls = on ? 1 : 0; }
 void tmd_set_dem_radius(double r) { sim().dem_radius = r; }
 void tmd_set_lj_shift(int on) { sim().lj_shift = on ? 1 : 0; }
 void tmd_set_sort_particles(int on) { sim().sort_particles = on ? 1 : 0; }
+void tmd_set_ghost_index_limit(int ghosts) { sim().gh_limit = std::max(0, std::min(ghosts, kGhostIndex)); }
 void tmd_set_adjoint_precision(int mode) { sim().adj_precision = mode < 0 ? -1 : (mode ? PREC_FP32_MIXED : PREC_FP64); }
 
 void tmd_set_tile_threads(int threads) {
@@ -1121,7 +1121,7 @@ static int run_loop(int steps, int reneigh_every, double dt, bool half, double c
         s.stage_bytes = kPosStageBytes;
         s.stage_budget = kLdsBudget;
         if (steps > 0) initial_integration(s, dt);
-        mirror_velocities(s, true);
+        mirror_velocities(s);
         s.vel_mirror_wanted = 1;  // the rebuild's mirror pass moves them again
         for (int j = 0; j < steps && !has_error(); ++j) {
             if ((j + 1) % reneigh_every == 0) {

@@ -170,7 +170,7 @@ struct Sim {
     int pos_stale = 0;      // local positions in pos lag the mirror (fused step loop; sync_pos_from_mirror)
     int vel_mirrored = 0;   // local velocities live in svel, in mirror order (fused step loop)
     int vel_mirror_wanted = 0;  // fused step loop: refresh_mirror also moves the velocities to svel
-    int gsrc_valid = 0;     // g_ko / g_kg match the ghost table and the binning
+    int gh_limit = 0;       // ghost room from which on there is no ghost index (0: kGhostIndex)
     int gh_packed = 0;      // the ghost index's gh_pack / gh_e match the ghost table
     int gh_valid = 0;       // gh_w / gh_k match the ghost table, binning and work order
     int dem_loop = 0;       // DEM step loop: a rebuild's mirrors hold the ghosts' velocities too
@@ -273,10 +273,10 @@ void refresh_ghosts(Sim& s);
 // fresh ghost positions and the cell-ordered mirror of locals and ghosts in
 // one pass (after positions were advanced inside the force pass)
 void step_refresh(Sim& s);
-void build_ghost_src(Sim& s);  // g_ko / g_kg (binning, after the CSR is built)
 void sync_pos_from_mirror(Sim& s);
 void rebuild_failed(Sim& s, bool mir, bool binned, int nq);
-void mirror_velocities(Sim& s, bool into_mirror);
+void mirror_velocities(Sim& s);
+void ghosts_from_owners(Sim& s, double* mirror, bool shift);
 
 // geometry (core/grid.impala:94-98): world AABB, rank AABB, cell spacing
 void make_geom(Geom& G, const double* aabb, const double* rank_aabb, double cell_spacing);
@@ -347,13 +347,15 @@ __device__ __forceinline__ void img_decode(int c, int& ix, int& iy, int& iz) {
 
 // A local's ghosts in the ghost index: mirror index of each and, when asked,
 // its image shift.
+constexpr int kGhostIndex = 1 << 26;  // entry numbers have 26 bits
 struct GhostIndex {
-    const int* w;  // per work slot: first entry * 32 + number
+    const int* w;  // per work slot: first entry * 32 + number; null: no index, ghosts_from_owners follows
     const int2* k;  // per entry: mirror index (-1: outside the grid), image code
     double L0, L1, L2;
 };
+__device__ __forceinline__ int ghost_entries(const GhostIndex& g, int w) { return g.w ? g.w[w] : 0; }
 template <class F>
-__device__ __forceinline__ void each_ghost(const GhostIndex& g, int pk, F&& f) {  // pk = g.w[work slot]
+__device__ __forceinline__ void each_ghost(const GhostIndex& g, int pk, F&& f) {  // pk = ghost_entries(g, work slot)
     for (int e = pk >> 5, e1 = e + (pk & 31); e < e1; ++e) {
         const int2 k = g.k[e];
         if (k.x >= 0) f(k.y, k.x);
@@ -366,7 +368,7 @@ __device__ __forceinline__ double4 ghost_image(const double4& x, const GhostInde
 }
 
 inline GhostIndex ghost_index(const Sim& s) {
-    return GhostIndex{s.gh_w.as<int>(), s.gh_k.as<int2>(), s.g.len[0], s.g.len[1], s.g.len[2]};
+    return GhostIndex{s.gh_valid ? s.gh_w.as<int>() : nullptr, s.gh_k.as<int2>(), s.g.len[0], s.g.len[1], s.g.len[2]};
 }
 
 __host__ __device__ inline void pbc_wrap(double4& p, const PbcArgs& a) {

@@ -83,6 +83,7 @@ SIGNATURES = {
     "tmd_set_lj_shift": (None, [_i]),
     "tmd_set_tile": (None, [_i, _i, _i]),
     "tmd_set_tile_threads": (None, [_i]),
+    "tmd_set_ghost_index_limit": (None, [_i]),
     "tmd_thermo": (None, [_d, _d, _d, _dp]),
     "tmd_thermo_eshift": (None, [_d, _d, _d, _dp]),
     "tmd_write_vtk": (_i, [ctypes.c_char_p, _i]),

@@ -76,6 +76,7 @@ class Simulation:
             # simulation starts from the automatic ones (set_tile after this)
             L.tmd_set_tile(0, 0, 0)
             L.tmd_set_tile_threads(0)
+            L.tmd_set_ghost_index_limit(0)
             m = np.ascontiguousarray(masses, dtype=np.float64)
             x = np.ascontiguousarray(positions, dtype=np.float64).reshape(-1, 3)
             v = np.ascontiguousarray(velocities, dtype=np.float64).reshape(-1, 3)
@@ -133,6 +134,7 @@ class Simulation:
         L.tmd_set_sort_particles(0)
         L.tmd_set_tile(0, 0, 0)
         L.tmd_set_tile_threads(0)
+        L.tmd_set_ghost_index_limit(0)
         self.n = L.tmd_load_state(os.fsencode(path))
         check()
         self.aabb = None

@@ -305,3 +305,41 @@ def test_atom_lost_in_the_loop(tm, dem, reneigh):
     _, xs, vs, _ = sim.state()
     assert np.array_equal(xs, xr) and np.array_equal(vs, vr)
     sim.close()
+
+
+@pytest.mark.parametrize("shape", [(4, 4, 5), (11, 9, 10), (17, 16, 18)])
+def test_without_a_ghost_index(tm, shape):
+    """With room for more ghosts than the index numbers (2^26; here for any),
+    each step's ghosts follow in a pass of their own: bit for bit the same step
+    loops and gradients."""
+    announce(f"without a ghost index {shape}")
+    out = []
+    for limit in (0, 1):
+        aabb, m, x, v = perturbed_fcc(*shape, amp=0.05, seed=5)
+        res = []
+        for half, precision in ((False, "fp32mixed"), (True, "fp64")):
+            sim = tm.Simulation(m, x, v, aabb, RC + SKIN, precision=precision)
+            tm.load().tmd_set_ghost_index_limit(limit)
+            sim.copy_to_accelerator()
+            sim.setup(half, RC, SKIN)
+            sim.lennard_jones(half, RC)
+            sim.run_lj(25, 10, DT, half)
+            res += list(sim.state()[1:]) + list(sim.ghost_state()[:2])
+        sim = tm.Simulation(m, x, v, aabb, RC + SKIN, lj_shift=True)
+        tm.load().tmd_set_ghost_index_limit(limit)
+        sim.copy_to_accelerator()
+        r = sim.traj_adjoint(13, 5, DT, RC, SKIN, 1.0, 1.0, -4.0, 1.0)
+        res += [r[key] for key in ("ubar", "pbar", "grad_eps", "grad_sigma", "grad_x0", "grad_v0")]
+        m, x, v = tm.generate_granular_gas(shape[0], vmax=2.0)
+        sim = tm.Simulation(m, x, v, np.array([0.0, shape[0] * 1.6796] * 3), 1.3, dem_radius=0.5)
+        tm.load().tmd_set_ghost_index_limit(limit)
+        sim.copy_to_accelerator()
+        sim.setup(True, 1.0, 0.3)
+        sim.dem(True, 1.0)
+        sim.run_dem(25, 10, 0.001, True)
+        res += list(sim.state()[1:]) + list(sim.ghost_state()[:3])
+        out.append(res)
+        sim.close()
+    tm.load().tmd_set_ghost_index_limit(0)
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
