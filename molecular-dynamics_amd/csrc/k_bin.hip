@@ -428,7 +428,11 @@ static void choose_tiles(Sim& s) {
         }
         for (int d = 0; d < 3; ++d) t[d] = s.tile_auto[d];
     }
-    s.tiles = make_tile_geom(s.g, t[0], t[1], t[2]);
+    const TileGeom g = make_tile_geom(s.g, t[0], t[1], t[2]);
+    // sizes of the last tiles tell nothing of larger ones: the rebuild waits for
+    // its own, as the first does (k_nlist of windows that outgrow their room)
+    if (g.tx > s.tiles.tx || g.ty > s.tiles.ty || g.tz > s.tiles.tz) s.max_window = 0;
+    s.tiles = g;
 }
 
 // The automatic choice sees only the mean density.  Where atoms crowd into

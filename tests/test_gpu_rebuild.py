@@ -343,3 +343,32 @@ def test_without_a_ghost_index(tm, shape):
     tm.load().tmd_set_ghost_index_limit(0)
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+def test_larger_tiles_after_smaller_ones(tm):
+    """The first list build with larger tiles does not run with the window sizes
+    of the smaller ones before: it takes less than twice the next one's time
+    (its windows were read from global memory, several times as long)."""
+    announce("larger tiles after smaller ones")
+    aabb, m, x, v = perturbed_fcc(16, amp=0.05, seed=5)
+    sim = tm.Simulation(m, x, v, aabb, RC + SKIN)
+    sim.copy_to_accelerator()
+
+    def build(tile):  # ms of the list build that a run begins with
+        sim.set_tile(tile)
+        sim.profile(True)
+        sim.profile_reset()
+        sim.run_lj(1, 20, 0.0)
+        ms, count = sim.profile_get("neighbor")
+        sim.profile(False)
+        assert count == 1
+        return ms
+
+    first, again = [], []
+    for _ in range(5):
+        build(1)
+        first.append(build(4))
+        again.append(build(4))
+    print(first, again)
+    assert min(first) < 2.0 * min(again), (first, again)
+    sim.close()
