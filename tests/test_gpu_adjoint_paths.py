@@ -108,3 +108,26 @@ def test_lanes_of_an_atom(tm, shape, shift):
     assert r["grad_sigma"] == pytest.approx(q["grad_sigma"], rel=1e-9)
     for key in ("grad_x0", "grad_v0"):
         assert np.linalg.norm(r[key] - q[key]) / np.linalg.norm(q[key]) <= 1e-9, key
+
+
+def test_sheet_leaves_its_room(tm):
+    """The sheet of test_states_no_longer_kept has more ghosts after its rebuild
+    than a simulation made anew has room for, so that test's first gradient
+    recomputes its intervals."""
+    announce("adjoint, room of the sheet")
+    L, ny = 48.0, 43
+    g = np.arange(ny) * (L / ny)
+    z, y, k = np.meshgrid(g, g, np.arange(3), indexing="ij")
+    x = np.stack([4.0 + 1.1 * k.ravel(), y.ravel(), z.ravel()], axis=1)
+    v = np.random.default_rng(3).normal(0.0, 0.3, x.shape)
+    v[:, 0] -= 35.0
+    room = 1.25 * len(x) * ((1 + 2 * (RC + SKIN) / L) ** 3 - 1) + 4096
+    tm.load().md_deallocate_grid()
+    sim = tm.Simulation(np.ones(len(x)), x, v, np.array([0.0, L] * 3), RC + SKIN, lj_shift=True)
+    sim.copy_to_accelerator()
+    sim.setup(False, RC, SKIN)
+    assert sim.nghost < room
+    sim.lennard_jones(False, RC)
+    sim.run_lj(20, 20, DT)
+    assert sim.nghost > room
+    sim.close()

@@ -372,3 +372,40 @@ def test_larger_tiles_after_smaller_ones(tm):
     print(first, again)
     assert min(first) < 2.0 * min(again), (first, again)
     sim.close()
+
+
+def test_ghosts_outgrow_their_room_dem(tm):
+    """The drifting sheet of spheres: the rebuild inside the DEM loop has to grow
+    its arrays and repeat from mirrors that hold the ghosts' velocities too.
+    Contact forces differ from the oracle's by summation rounding only."""
+    announce("ghosts outgrow their room, DEM")
+    L = 76.0
+    g = np.arange(76) + 0.5
+    z, y, k = np.meshgrid(g, g, np.arange(2), indexing="ij")
+    x = np.stack([3.0 + 0.95 * k.ravel(), y.ravel(), z.ravel()], axis=1)
+    v = np.random.default_rng(3).normal(0.0, 0.3, x.shape)
+    v[:, 0] -= 28.0
+    aabb, m = np.array([0.0, L] * 3), np.ones(len(x))
+    room = 1.25 * len(x) * ((1 + 2.6 / L) ** 3 - 1) + 4096
+    tm.load().md_deallocate_grid()
+    sim = tm.Simulation(m, x, v, aabb, 1.3, dem_radius=0.5)
+    sim.copy_to_accelerator()
+    orc = po.OracleSim(m, x, v, aabb, 1.3, threads=4)
+    sim.setup(True, 1.0, 0.3)
+    orc.setup(True, po.HALF_GHOST_FULL, 1.3)
+    assert sim.nghost == orc.ng < room
+    sim.dem(True, 1.0)
+    orc.dem(True, 1.0)
+    sim.run_dem(110, 100, 0.001)
+    orc.run_dem(110, 100, 0.001)
+    assert orc.ng > room
+    gt, go = sim.ghost_table(), orc.ghosts()
+    assert sim.nghost == orc.ng
+    for key in ("owner", "img", "src", "flag"):
+        assert np.array_equal(gt[key], go[key]), key
+    _, xg, vg, _ = sim.state()
+    xo, vo, _ = orc.state()
+    assert np.allclose(xg, xo, rtol=1e-11, atol=1e-11) and np.allclose(vg, vo, rtol=1e-11, atol=1e-11)
+    _, xh, vh, _ = sim.ghost_state()
+    assert np.array_equal(vh, vg[gt["owner"]]) and np.array_equal(xh, xg[gt["owner"]] + gt["img"] * L)
+    sim.close()
