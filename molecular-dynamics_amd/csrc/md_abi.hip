@@ -12,6 +12,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <mutex>
 
 #include "tmd_internal.hpp"
@@ -1025,21 +1026,30 @@ int tmd_get_cells(int* start, int* atoms, int* atom_cell) {
         set_error(__FILE__, __LINE__, "tmd_get_cells: cells not binned (call md_distribute_particles first)");
         return 0;
     }
-    std::vector<int> st(s.binned_cells + 1);
-    TMD_HIP(hipMemcpy(st.data(), s.cell_start.p, sizeof(int) * st.size(), hipMemcpyDeviceToHost));
+    const int nb = s.binned_cells;
+    std::unique_ptr<int[]> own_start, own_parts;  // where the caller's arrays do not hold them
+    if (!start || nc != nb) own_start.reset(new int[(size_t)nb + 1]);
+    int* const st = own_start ? own_start.get() : start;
+    TMD_HIP(hipMemcpy(st, s.cell_start.p, sizeof(int) * ((size_t)nb + 1), hipMemcpyDeviceToHost));
     if (has_error()) return 0;
-    std::vector<int> parts(st.back());
-    if (!parts.empty()) TMD_HIP(hipMemcpy(parts.data(), s.cell_parts.p, sizeof(int) * parts.size(), hipMemcpyDeviceToHost));
-    if (has_error()) return 0;
-    if (start) std::copy(st.begin(), st.begin() + nc + 1, start);
-    if (atoms) std::copy(parts.begin(), parts.begin() + st[nc], atoms);
-    if (atom_cell) {
-        // the ghosts may be others by now, or none
-        const int nall = s.n + s.ng;
-        std::fill(atom_cell, atom_cell + nall, -1);
-        for (int c = 0; c < s.binned_cells; ++c)
-            for (int k = st[c]; k < st[c + 1]; ++k)
-                if (parts[k] < nall) atom_cell[parts[k]] = c;
+    if (start && st != start) std::copy(st, st + nc + 1, start);
+    const int want = atom_cell ? st[nb] : (atoms ? st[nc] : 0);  // entries of the cell order
+    if (want > 0) {
+        if (!atoms || want != st[nc]) own_parts.reset(new int[want]);
+        int* const parts = own_parts ? own_parts.get() : atoms;
+        TMD_HIP(hipMemcpy(parts, s.cell_parts.p, sizeof(int) * (size_t)want, hipMemcpyDeviceToHost));
+        if (has_error()) return 0;
+        if (atoms && parts != atoms) std::copy(parts, parts + st[nc], atoms);
+        if (atom_cell) {
+            // the ghosts may be others by now, or none
+            const int nall = s.n + s.ng;
+            std::fill(atom_cell, atom_cell + nall, -1);
+            for (int c = 0; c < nb; ++c)
+                for (int k = st[c]; k < st[c + 1]; ++k)
+                    if (parts[k] < nall) atom_cell[parts[k]] = c;
+        }
+    } else if (atom_cell) {
+        std::fill(atom_cell, atom_cell + s.n + s.ng, -1);
     }
     return st[nc];
 }
