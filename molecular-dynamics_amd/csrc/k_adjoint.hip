@@ -125,7 +125,7 @@ __global__ void __launch_bounds__(G > 1 ? kGroupThreads : kMaxTileThreads) k_tra
             x.y = x.y + v.y * t.dt;
             x.z = x.z + v.z * t.dt;
             t.xnext[kw] = x;
-            each_ghost(t.gh, ghost_entries(t.gh, w), [&](int e, int kg) { t.xnext[kg] = ghost_image(x, t.gh, e); });
+            each_ghost(t.gh, t.gh.w[w], [&](int e, int kg) { t.xnext[kg] = ghost_image(x, t.gh, e); });
         }
         t.vel[kw] = v;
     }
@@ -324,7 +324,7 @@ __global__ void __launch_bounds__(G > 1 ? kGroupThreads : kMaxTileThreads) k_lj_
             t.xb[kw] = xb;
             t.vb[kw] = vb;
             t.fnext[kw] = fb;
-            each_ghost(t.gh, ghost_entries(t.gh, w), [&](int, int kg) { t.fnext[kg] = fb; });
+            each_ghost(t.gh, t.gh.w[w], [&](int, int kg) { t.fnext[kg] = fb; });
         }
     };
     if (staged) atoms(std::true_type{});
@@ -374,7 +374,7 @@ __global__ void k_adj_begin(const int* __restrict__ work, const int* __restrict_
     xb[kw] = xbar[i];
     vb[kw] = b;
     fb[kw] = f;
-    each_ghost(gh, ghost_entries(gh, w), [&](int, int kg) { fb[kg] = f; });
+    each_ghost(gh, gh.w[w], [&](int, int kg) { fb[kg] = f; });
 }
 
 // ---------------------------------------------------------------------------

@@ -281,7 +281,7 @@ __global__ void __launch_bounds__(256) k_rebuild_finish(FinishArgs a, const int*
         work[w0 + e] = i;
         work_k[w0 + e] = k;  // the atom's mirror index
         work_c[w0 + e] = c;
-        if (gh_pack) gh_w[w0 + e] = gh_pack[i];
+        gh_w[w0 + e] = gh_pack ? gh_pack[i] : 0;
     }
 }
 

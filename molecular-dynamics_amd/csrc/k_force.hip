@@ -93,7 +93,7 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_lj_full(TMD_KERNEL_LIST_PAR
         o.kw = wk[w];
         o.cnt = nbc[w];
         o.cnt2 = PAIR2 ? nbc2[w] : 0;  // half lists: the complementary column continues the same sum
-        o.pk = KICK == 2 ? ghost_entries(gh, w) : 0;
+        o.pk = KICK == 2 && gh.w ? gh.w[w] : 0;
         const size_t col = (size_t)(w >> 6) * (size_t)a.cap * 8 + (w & 63);
         o.head = list_head<PAIR2>(o.cnt, reinterpret_cast<const int4*>(nbl) + col, reinterpret_cast<const int4*>(nbl2) + col);
         o.x = spos[o.kw];
@@ -176,7 +176,7 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_lj_group(const CMir spos, c
         kw = wk[w];
         cnt = nbc[w];
         cnt2 = PAIR2 ? nbc2[w] : 0;
-        pk = ghost_entries(gh, w);
+        pk = gh.w ? gh.w[w] : 0;
         const size_t col = (size_t)(w >> 6) * (size_t)a.cap * 8 + (w & 63);
         lp = reinterpret_cast<const int4*>(nbl) + col;
         lp2 = PAIR2 ? reinterpret_cast<const int4*>(nbl2) + col : nullptr;
@@ -480,7 +480,7 @@ __global__ void __launch_bounds__(kMaxTileThreads, PREC == PREC_FP64 ? 4 : 6) k_
         o.kw = wk[w];
         o.cnt = nbc[w];
         o.cnt2 = PAIR2 ? nbc2[w] : 0;
-        o.pk = ADV ? ghost_entries(gh, w) : 0;
+        o.pk = ADV && gh.w ? gh.w[w] : 0;
         const size_t col = (size_t)(w >> 6) * (size_t)a.cap * 8 + (w & 63);
         o.e0 = ld_stream(reinterpret_cast<const int4*>(nbl) + col);
         if (PAIR2) o.e1 = ld_stream(reinterpret_cast<const int4*>(nbl2) + col);

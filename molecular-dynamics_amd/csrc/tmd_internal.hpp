@@ -349,13 +349,12 @@ __device__ __forceinline__ void img_decode(int c, int& ix, int& iy, int& iz) {
 // its image shift.
 constexpr int kGhostIndex = 1 << 26;  // entry numbers have 26 bits
 struct GhostIndex {
-    const int* w;  // per work slot: first entry * 32 + number; null: no index, ghosts_from_owners follows
+    const int* w;  // per work slot: first entry * 32 + number (0 without an index: ghosts_from_owners follows)
     const int2* k;  // per entry: mirror index (-1: outside the grid), image code
     double L0, L1, L2;
 };
-__device__ __forceinline__ int ghost_entries(const GhostIndex& g, int w) { return g.w ? g.w[w] : 0; }
 template <class F>
-__device__ __forceinline__ void each_ghost(const GhostIndex& g, int pk, F&& f) {  // pk = ghost_entries(g, work slot)
+__device__ __forceinline__ void each_ghost(const GhostIndex& g, int pk, F&& f) {  // pk = g.w[work slot]
     for (int e = pk >> 5, e1 = e + (pk & 31); e < e1; ++e) {
         const int2 k = g.k[e];
         if (k.x >= 0) f(k.y, k.x);
@@ -368,7 +367,7 @@ __device__ __forceinline__ double4 ghost_image(const double4& x, const GhostInde
 }
 
 inline GhostIndex ghost_index(const Sim& s) {
-    return GhostIndex{s.gh_valid ? s.gh_w.as<int>() : nullptr, s.gh_k.as<int2>(), s.g.len[0], s.g.len[1], s.g.len[2]};
+    return GhostIndex{s.gh_w.as<int>(), s.gh_k.as<int2>(), s.g.len[0], s.g.len[1], s.g.len[2]};
 }
 
 __host__ __device__ inline void pbc_wrap(double4& p, const PbcArgs& a) {
