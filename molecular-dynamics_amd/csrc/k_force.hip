@@ -159,7 +159,7 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_lj_group(const CMir spos, c
     constexpr int G = kGroupLanes;
     extern __shared__ __align__(16) double group_lds[];
     const WinStage sp = win_stage(group_lds, a.wcap);
-    double* buf = group_lds + group_buf_at(a.wcap) + threadIdx.x / kWave * (kGroupBufBytes / sizeof(double));
+    double* buf = group_lds + 3 * a.wcap + threadIdx.x / kWave * (kGroupBufBytes / sizeof(double));
     const int tile = block_tile(blockIdx.x, a.g);
     const int w0 = tile_start[tile], nloc = tile_start[tile + 1] - w0;
     if (nloc == 0) return;
@@ -712,7 +712,9 @@ void compute_lj(Sim& s, int half, double rc, double eps, double sigma, double ki
         const int* C2 = s.nb_count2.as<int>();
         const nb_t* L2 = s.nb_list2.as<nb_t>();
         const int gthreads = std::min(kMaxTileThreads, (std::max(s.max_locals, 1) * kGroupLanes + kWave - 1) / kWave * kWave);
-        const size_t glds = group_buf_at(a.wcap) * sizeof(double) + (size_t)gthreads / kWave * kGroupBufBytes;
+        LJArgs ga = a;
+        ga.wcap = group_window(a.wcap);
+        const size_t glds = (size_t)ga.wcap * kPosStageBytes + (size_t)gthreads / kWave * kGroupBufBytes;
         const bool group = kick_dt > 0.0 && advance && VK && s.n <= group_atoms(s.precision) && s.tile_threads_req == 0 &&
                            glds <= (size_t)kLdsBudget;
 #define TMD_LJ_K(P, SH, U, K, H)                                                                                       \
@@ -723,7 +725,7 @@ void compute_lj(Sim& s, int half, double rc, double eps, double sigma, double ki
 #define TMD_LJ_G(P, SH, U, H)                                                                                       \
     hipLaunchKernelGGL((k_lj_group<P, SH, U, H>), dim3(nb), dim3(gthreads), glds, s.stream, CMir{s.spos.as<double>()},  \
                        (const int*)s.cell_start.as<int>(), (const int*)s.tile_start.as<int>(),                            \
-                       (const int*)s.nb_count.as<int>(), (const nb_t*)s.nb_list.as<nb_t>(), a, SV, hdt, kick_dt, WK, SN, C2, L2, GH)
+                       (const int*)s.nb_count.as<int>(), (const nb_t*)s.nb_list.as<nb_t>(), ga, SV, hdt, kick_dt, WK, SN, C2, L2, GH)
 #define TMD_LJ_FULL(P, SH, U)                                                                                          \
     do {                                                                                                               \
         if (group && half) TMD_LJ_G(P, SH, U, true);                                                                   \

@@ -249,13 +249,12 @@ __device__ __forceinline__ double4 lj_full_atom(const double4 pi, int cnt, const
 // through LDS.  Lane c < 3 returns component c.
 constexpr int kGroupLanes = 4;
 constexpr int kGroupBufBytes = 8192 + 1024;  // of a wavefront: 256 entries of up to four doubles, 64 groups of list entries
-// Doubles in front of the first wavefront's buffer: the window's wcap slots, to
-// the next 16 bytes, as the list entries are stored and fetched 16 at a time
-// (3 wcap alone is odd for every other window).
-constexpr __host__ __device__ int group_buf_at(int wcap) { return (3 * wcap + 1) & ~1; }
+// The buffers follow the window, whose slots are then an even number: list
+// entries are stored and fetched 16 bytes at a time.
+constexpr int group_window(int wcap) { return (wcap + 1) & ~1; }
 constexpr bool group_bufs_aligned() {
     for (int wcap = 1; wcap <= 4; ++wcap)
-        if (group_buf_at(wcap) < 3 * wcap || group_buf_at(wcap) * (int)sizeof(double) % (int)alignof(int4) != 0) return false;
+        if (group_window(wcap) < wcap || group_window(wcap) * 3 * (int)sizeof(double) % (int)alignof(int4) != 0) return false;
     return kGroupBufBytes % alignof(int4) == 0 && (kGroupBufBytes - 1024) % alignof(int4) == 0;
 }
 static_assert(group_bufs_aligned(), "list entries are 16-byte accesses");
