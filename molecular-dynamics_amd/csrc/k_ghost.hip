@@ -52,9 +52,8 @@ __device__ __forceinline__ int class_id(int a, int b, int c) {
     const int xy = b == 0 ? a - 1 : 2 + (b - 1) * 3 + a;  // -1: none in x and y
     return c == 0 ? xy : 8 + (c - 1) * 9 + xy + 1;
 }
-constexpr int kGhostItems = 1;                              // locals per thread
-constexpr int kGhostBlock = kScanThreads * kGhostItems;     // locals per block
-constexpr int kGhostSubs = kGhostBlock / kWave;             // wavefront-sized groups of locals per block
+constexpr int kGhostBlock = kScanThreads;  // locals per block, one a thread
+constexpr int kGhostWaves = kGhostBlock / kWave;
 // (class, block) counts that the emitting blocks scan by themselves; more are
 // scanned by launches of their own
 constexpr int kClassFlat = 4096;
@@ -142,23 +141,18 @@ __device__ __forceinline__ void class_digits(int id, int& a, int& b, int& c) {
 // counts[class * nb + block]: members of each class in each block of locals
 __global__ void __launch_bounds__(kScanThreads) k_class_count(const unsigned char* __restrict__ face, int n, int nb,
                                                               int* __restrict__ counts) {
-    __shared__ int wc[kScanThreads / kWave][kClasses];
+    __shared__ int wc[kGhostWaves][kClasses];
     const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
     int ca = 0, cb = 0, cc = 0;
     class_digits(min(lane, kClasses - 1), ca, cb, cc);
-    int sum = 0;
-#pragma unroll
-    for (int it = 0; it < kGhostItems; ++it) {
-        const int i = blockIdx.x * kGhostBlock + it * kScanThreads + (int)threadIdx.x;
-        const FaceBallots f = face_ballots(i < n ? face[i] : 0);
-        if (f.any()) sum += __popcll(f.side(0, ca) & f.side(1, cb) & f.side(2, cc));
-    }
-    if (lane < kClasses) wc[wid][lane] = sum;
+    const int i = blockIdx.x * kGhostBlock + (int)threadIdx.x;
+    const FaceBallots f = face_ballots(i < n ? face[i] : 0);
+    if (lane < kClasses) wc[wid][lane] = f.any() ? __popcll(f.side(0, ca) & f.side(1, cb) & f.side(2, cc)) : 0;
     __syncthreads();
     if (threadIdx.x < kClasses) {
         int t = 0;
 #pragma unroll
-        for (int w = 0; w < kScanThreads / kWave; ++w) t += wc[w][threadIdx.x];
+        for (int w = 0; w < kGhostWaves; ++w) t += wc[w][threadIdx.x];
         counts[threadIdx.x * nb + blockIdx.x] = t;
     }
 }
@@ -185,22 +179,16 @@ __global__ void __launch_bounds__(kScanThreads) k_ghost_emit(double4* __restrict
                                                              int* __restrict__ g_code, int* __restrict__ gh_pack,
                                                              int* __restrict__ gh_e, int* __restrict__ ctr) {
     __shared__ int flat[kClassFlat];
-    __shared__ int sub[kGhostSubs][kClasses];
+    __shared__ int sub[kGhostWaves][kClasses];
     __shared__ int entry0;
     const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
     const int blk = blockIdx.x;
-    int bits[kGhostItems];
-    FaceBallots f[kGhostItems];
     int ca = 0, cb = 0, cc = 0;
     class_digits(min(lane, kClasses - 1), ca, cb, cc);
-#pragma unroll
-    for (int it = 0; it < kGhostItems; ++it) {
-        const int i = blk * kGhostBlock + it * kScanThreads + (int)threadIdx.x;
-        bits[it] = i < a.n ? face[i] : 0;
-        f[it] = face_ballots(bits[it]);
-        if (lane < kClasses)
-            sub[it * (kScanThreads / kWave) + wid][lane] = __popcll(f[it].side(0, ca) & f[it].side(1, cb) & f[it].side(2, cc));
-    }
+    const int i = blk * kGhostBlock + (int)threadIdx.x;
+    const int bt = i < a.n ? face[i] : 0;
+    const FaceBallots F = face_ballots(bt);
+    if (lane < kClasses) sub[wid][lane] = __popcll(F.side(0, ca) & F.side(1, cb) & F.side(2, cc));
     // thread c: ghost number of the block's first member of class c, and of the
     // whole class's first one
     int first = 0, cls0 = 0;
@@ -242,7 +230,7 @@ __global__ void __launch_bounds__(kScanThreads) k_ghost_emit(double4* __restrict
     __syncthreads();
     if (threadIdx.x < kClasses) {
         int run = first;
-        for (int q = 0; q < kGhostSubs; ++q) {
+        for (int q = 0; q < kGhostWaves; ++q) {
             const int t = sub[q][threadIdx.x];
             sub[q][threadIdx.x] = run;
             run += t;
@@ -250,81 +238,73 @@ __global__ void __launch_bounds__(kScanThreads) k_ghost_emit(double4* __restrict
     }
     __syncthreads();
     const unsigned long long below = (1ull << lane) - 1ull;
-    int given = entry0;  // ghost index entries given out so far in the block
-#pragma unroll
-    for (int it = 0; it < kGhostItems; ++it) {
-        const int i = blk * kGhostBlock + it * kScanThreads + (int)threadIdx.x;
-        const FaceBallots& F = f[it];
-        const int* base = sub[it * (kScanThreads / kWave) + wid];
-        const int bt = bits[it];
-        int entry = 0;
-        if (gh_pack) {
-            const int m = (1 + (bt & 1) + ((bt >> 1) & 1)) * (1 + ((bt >> 2) & 1) + ((bt >> 3) & 1)) *
-                              (1 + ((bt >> 4) & 1) + ((bt >> 5) & 1)) - 1;
-            int tot;
-            entry = given + block_exclusive_scan(m, &tot);
-            given += tot;
-            if (i < a.n) gh_pack[i] = m ? entry * 32 + m : 0;
+    const int* base = sub[wid];
+    int entry = 0;
+    if (gh_pack) {
+        const int m = (1 + (bt & 1) + ((bt >> 1) & 1)) * (1 + ((bt >> 2) & 1) + ((bt >> 3) & 1)) *
+                          (1 + ((bt >> 4) & 1) + ((bt >> 5) & 1)) - 1;
+        int tot;
+        entry = entry0 + block_exclusive_scan(m, &tot);
+        if (i < a.n) gh_pack[i] = m ? entry * 32 + m : 0;
+    }
+    if (F.any() == 0) return;  // no border atom in the wavefront
+    double4 p = make_double4(0, 0, 0, 0), v = p;
+    double ms = 0.0;
+    if (bt) {
+        if (MIR) {
+            const int k = inv_src[i];
+            p = spos[k];
+            v = svel[k];
+        } else {
+            p = pos[i];
+            v = vel[i];
         }
-        if (F.any() == 0) continue;  // no border atom in the wavefront
-        double4 p = make_double4(0, 0, 0, 0), v = p;
-        double ms = 0.0;
-        if (bt) {
-            if (MIR) {
-                const int k = inv_src[i];
-                p = spos[k];
-                v = svel[k];
-            } else {
-                p = pos[i];
-                v = vel[i];
-            }
-            ms = mass[i];
-        }
-        const int fl[3][2] = {{p.x > a.whi[0] ? -1 : 0, p.x < a.wlo[0] ? 1 : 0},
-                              {p.y > a.whi[1] ? -1 : 0, p.y < a.wlo[1] ? 1 : 0},
-                              {p.z > a.whi[2] ? -1 : 0, p.z < a.wlo[2] ? 1 : 0}};
-        // every class with members in this wavefront (uniform loops: the
-        // class masks are scalar)
+        ms = mass[i];
+    }
+    const int fl[3][2] = {{p.x > a.whi[0] ? -1 : 0, p.x < a.wlo[0] ? 1 : 0},
+                          {p.y > a.whi[1] ? -1 : 0, p.y < a.wlo[1] ? 1 : 0},
+                          {p.z > a.whi[2] ? -1 : 0, p.z < a.wlo[2] ? 1 : 0}};
+    // every class with members in this wavefront (uniform loops: the
+    // class masks are scalar)
 #pragma unroll 1
-        for (int c = 0; c < 3; ++c) {
-            const unsigned long long mc = F.side(2, c);
+    for (int c = 0; c < 3; ++c) {
+        const unsigned long long mc = F.side(2, c);
 #pragma unroll 1
-            for (int b = 0; b < 3; ++b) {
-                const unsigned long long mb = mc & F.side(1, b);
+        for (int b = 0; b < 3; ++b) {
+            const unsigned long long mb = mc & F.side(1, b);
 #pragma unroll 1
-                for (int s = 0; s < 3; ++s) {
-                    const unsigned long long m = mb & F.side(0, s);
-                    if ((s | b | c) == 0 || m == 0) continue;
-                    const bool has = (m >> lane) & 1ull;
-                    const int id = class_id(s, b, c);
-                    const int g = base[id] + __popcll(m & below);
-                    const int ix = s == 0 ? 0 : (s == 1 ? fl[0][0] : fl[0][1]);
-                    const int iy = b == 0 ? 0 : (b == 1 ? fl[1][0] : fl[1][1]);
-                    const int iz = c == 0 ? 0 : (c == 1 ? fl[2][0] : fl[2][1]);
-                    double4 q;
-                    q.x = p.x + a.len[0] * (double)ix;
-                    q.y = p.y + a.len[1] * (double)iy;
-                    q.z = p.z + a.len[2] * (double)iz;
-                    q.w = p.w;
-                    if (has && g < a.gcap) {
-                        // the immediate source: the class without the last pass
-                        int src = i;
-                        if (c ? (s | b) : (b ? s : 0)) {
-                            const int pc = c ? class_id(s, b, 0) : class_id(s, 0, 0);
-                            const unsigned long long pm = F.side(0, s) & (c ? F.side(1, b) : ~0ull);
-                            src = a.n + base[pc] + __popcll(pm & below);
-                        }
-                        pos[a.n + g] = q;
-                        vel[a.n + g] = v;
-                        mass[a.n + g] = ms;
-                        g_owner[g] = i;
-                        g_src[g] = src;
-                        g_code[g] = img_encode(ix, iy, iz) |
-                                    (img_encode(c || b ? 0 : ix, c ? 0 : (b ? iy : 0), c ? iz : 0) << 8);
-                        if (gh_pack) gh_e[g] = entry;
+            for (int s = 0; s < 3; ++s) {
+                const unsigned long long m = mb & F.side(0, s);
+                if ((s | b | c) == 0 || m == 0) continue;
+                const bool has = (m >> lane) & 1ull;
+                const int id = class_id(s, b, c);
+                const int g = base[id] + __popcll(m & below);
+                const int ix = s == 0 ? 0 : (s == 1 ? fl[0][0] : fl[0][1]);
+                const int iy = b == 0 ? 0 : (b == 1 ? fl[1][0] : fl[1][1]);
+                const int iz = c == 0 ? 0 : (c == 1 ? fl[2][0] : fl[2][1]);
+                double4 q;
+                q.x = p.x + a.len[0] * (double)ix;
+                q.y = p.y + a.len[1] * (double)iy;
+                q.z = p.z + a.len[2] * (double)iz;
+                q.w = p.w;
+                if (has && g < a.gcap) {
+                    // the immediate source: the class without the last pass
+                    int src = i;
+                    if (c ? (s | b) : (b ? s : 0)) {
+                        const int pc = c ? class_id(s, b, 0) : class_id(s, 0, 0);
+                        const unsigned long long pm = F.side(0, s) & (c ? F.side(1, b) : ~0ull);
+                        src = a.n + base[pc] + __popcll(pm & below);
                     }
-                    if (has) ++entry;
+                    pos[a.n + g] = q;
+                    vel[a.n + g] = v;
+                    mass[a.n + g] = ms;
+                    g_owner[g] = i;
+                    g_src[g] = src;
+                    g_code[g] = img_encode(ix, iy, iz) |
+                                (img_encode(c || b ? 0 : ix, c ? 0 : (b ? iy : 0), c ? iz : 0) << 8);
+                    if (gh_pack) gh_e[g] = entry;
                 }
+                if (has) ++entry;
             }
         }
     }
