@@ -30,10 +30,10 @@ double tmd_kahan_sum(const float* x, int n);
  * 2 = as 1 but accumulated in FP32 with Kahan compensation (full lists). */
 void tmd_set_precision(int mode);
 /* Precision of the adjoint kernel alone (tmd_traj_adjoint's reverse pass):
- * -1 (default) follows tmd_set_precision, 0 = FP64, 1 = FP32-mixed (its
- * Hessian-vector product's pair scalars in FP32).  Setting it apart from the
- * forward precision separates the adjoint's own rounding from that of the
- * FP32-mixed forward trajectory. */
+ * -1 (default) follows tmd_set_precision, 0 = FP64, 1 = FP32-mixed (1/r^2
+ * without its last rounding step and r^2 by FMAs, a few 1e-16 apart).  Setting
+ * it apart from the forward precision separates the adjoint's own rounding
+ * from that of the FP32-mixed forward trajectory. */
 void tmd_set_adjoint_precision(int mode);
 /* 1: renumber the local atoms in cell order (index order inside a cell) at
  * every periodic wrap of a rebuild (md_enforce_pbc, and inside tmd_run_*),
@@ -62,7 +62,8 @@ void tmd_set_dem_radius(double radius);
  * (continuous force at rc; used for the differentiable runs). */
 void tmd_set_lj_shift(int on);
 /* Cells per tile of the list/force kernels (one block per tile; 0 0 0 =
- * automatic, about 480 atoms per tile).  Takes effect at the next binning. */
+ * automatic: about 480 atoms per tile in boxes of many tiles, fewer in smaller
+ * ones).  Takes effect at the next binning. */
 void tmd_set_tile(int tx, int ty, int tz);
 /* Threads per tile block of the list-build and pair kernels: a multiple of
  * 64 in 64..1024, or 0 (default) for automatic: one lane per local atom of
@@ -173,11 +174,13 @@ int tmd_generate_granular_gas(int nc, double potential_minimum, unsigned long lo
  * as they were at x0 (full list).  Return 1 on success, 0 on error. */
 int tmd_traj_loss(int steps, int reneigh_every, double dt, double cutoff, double skin, double epsilon, double sigma,
                   double* out2 /* {Ubar, Pbar} */);
-/* Reverse-mode gradient of L: state checkpoints every `reneigh_every` steps,
- * each interval recomputed forward and reversed with the hand-written
- * Hessian-vector-product kernel.  out3 = {L, Ubar, Pbar}; grad_theta2 =
- * {dL/depsilon, dL/dsigma}; grad_x0 / grad_v0 (n entries, may be NULL) =
- * dL/dx0, dL/dv0. */
+/* Reverse-mode gradient of L with the hand-written Hessian-vector-product
+ * kernel.  The states of the forward pass are kept where they take at most
+ * 4 GiB and a quarter of the free device memory; else they are checkpointed
+ * every `reneigh_every` steps and each interval is recomputed.  The memory
+ * stays with the simulation until md_deallocate_grid.  out3 = {L, Ubar, Pbar};
+ * grad_theta2 = {dL/depsilon, dL/dsigma}; grad_x0 / grad_v0 (n entries, may be
+ * NULL) = dL/dx0, dL/dv0. */
 int tmd_traj_adjoint(int steps, int reneigh_every, double dt, double cutoff, double skin, double epsilon, double sigma,
                      double u_target, double p_target, double* out3, double* grad_theta2, struct Vector3D* grad_x0,
                      struct Vector3D* grad_v0);

@@ -19,9 +19,10 @@
 // J_F^T Fbar is a Hessian-vector product over the full neighbour list:
 //   xbar_i += sum_j [f(s) d + 2 f'(s) (r.d) r],  d = Fbar_i - Fbar_owner(j),
 // symmetric in (i, j), so each lane owns its atom (no atomics); ghost
-// adjoints are their owners'.  (x, v) is checkpointed every rebuild interval
-// and each interval is recomputed forward before it is reversed; within an
-// interval the neighbour list and ghost table are fixed, as in the forward.
+// adjoints are their owners'.  Every state of the forward pass is kept where
+// there is room (keep_all); else (x, v) is checkpointed every rebuild interval
+// and each interval is recomputed before it is reversed.  Within an interval
+// the neighbour list and ghost table are fixed, as in the forward.
 #include "tmd_internal.hpp"
 #include "tmd_lj.hpp"
 #include "tmd_pair.hpp"
@@ -38,7 +39,9 @@ struct AdjCoef {
 
 // Both passes give an atom to a group of G lanes (atom_lanes), which share its
 // list by groups of entries and add their sums.
-// 131 registers fit three wavefronts a SIMD; held to four, G > 1 spills.
+// The reverse pass takes up to 130 registers with G > 1: four wavefronts a SIMD
+// in FP64 (128), three in FP32-mixed with the smooth cutoff.  Four more cost
+// FP64 23 -> 31 us a step at 15,028 atoms.
 constexpr int kGroupThreads = 768;  // threads a block with G > 1
 
 // the first list group of the lane in its atom's group of G (clamped: always a

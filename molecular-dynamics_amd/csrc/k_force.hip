@@ -561,7 +561,7 @@ __global__ void __launch_bounds__(kMaxTileThreads, PREC == PREC_FP64 ? 4 : 6) k_
                     return q & ((1u << n) - 1u);
                 };
                 unsigned m = touching(e0, n0) | touching(e1, n1) << 8;
-                // their terms, in list order, the next one's velocity under way
+                // their terms, in list order
                 auto slot = [&](unsigned q) {
                     const int b = __builtin_ctz(q);
                     const bool lo = b < 8;
@@ -674,7 +674,10 @@ void compute_dem_fused(Sim& s, int half, double rc, double gn, double gt, double
 // Boxes up to this many atoms take four lanes an atom: 28,000 and 44,000 of
 // the chip's 65,536 lanes.  us a step, one lane against four: 12^3 cells (6,912
 // atoms) FP32-mixed half lists 19.2 and 17.5, FP64 20.2 and 15.4; 14^3 (10,976)
-// FP32-mixed 18.2 and 19.3, FP64 20.7 and 18.2; 16^3 FP64 20.2 and 21.1.
+// FP32-mixed 18.2 and 19.3, FP64 20.7 and 18.2; 16^3 FP64 20.2 and 21.1.  And
+// only where the fullest tile's buffers (9,216 bytes a wavefront of 16 atoms)
+// fit the LDS share beside the window: at 14^3 up to 96 locals (six wavefronts,
+// 78 of 79 KiB); with a fuller tile the box keeps one lane an atom.
 static int group_atoms(int precision) { return precision == PREC_FP32_MIXED ? 7000 : 11000; }
 
 static size_t lds_bytes(const Sim& s, bool) { return (size_t)window_cap(s) * kStageBytes; }

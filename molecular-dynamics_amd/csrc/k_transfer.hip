@@ -9,7 +9,10 @@
 // 0.88 ms, at 20 KB 19 us instead of 13).  Before, rows were packed by one
 // host thread and copied through pageable memory: 80^3 cells (2,048,000
 // atoms, and 267,000 ghosts on the way out) took 51 ms in and 62 ms out, now 2.1
-// and 3.5; 864 atoms 60 and 160 us, now 20 and 20.
+// and 3.5 where the pinned arrays have been in use before; 864 atoms 60 and 160
+// us, now 20 and 20.  Fresh pinned pages cost the first simulation more: create,
+// upload, read and close at 80^3 together 35 ms, where it was 137 (a process's
+// first: 39 and 198).
 #include <algorithm>
 #include <cstring>
 #include <thread>

@@ -212,9 +212,9 @@ __device__ __forceinline__ int xcd_block(int b, int nblocks) {
     return x * q + min(x, r) + k;
 }
 
-// The same for tiles of uneven work: from kDealFrom blocks on they are dealt
-// to the XCDs in runs of kDealRun, so that thin tiles at a box's far faces do
-// not all come to one XCD.
+// The same for tiles of uneven work (ORDER_DEAL, the batch): dealt to the XCDs
+// in runs of kDealRun, so that thin tiles at a box's far faces do not all come
+// to one XCD; the rest below one run for each XCD in equal ranges.
 constexpr int kDealRun = 16;
 __device__ __forceinline__ int xcd_deal(int b, int nblocks) {
     const int full = nblocks / (kNumXcd * kDealRun) * (kNumXcd * kDealRun);
