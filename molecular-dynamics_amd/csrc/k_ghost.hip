@@ -738,17 +738,16 @@ void mirror_velocities(Sim& s) {
 
 void step_refresh(Sim& s) {
     if (has_error() || s.n + s.ng == 0) return;
-    if (!s.inv_valid || s.ghost_mode != GHOST_FRESH) {
-        s.ghost_stale = 0;
-        refresh_ghosts(s);
-        return;
-    }
     const int nt = 256;
     if (s.ghost_stale && s.pos_stale) {
         // the last pass moved the locals in the mirror: the ghosts there only
         // (pos at the end)
         ghosts_from_owners(s, s.spos.as<double>(), true);
         s.ghost_pos_stale = 1;
+    } else if (!s.inv_valid || s.ghost_mode != GHOST_FRESH) {
+        s.ghost_stale = 0;
+        refresh_ghosts(s);
+        return;
     } else {
         hipLaunchKernelGGL(k_step_refresh, dim3(div_up(s.n + s.ng, nt)), dim3(nt), 0, s.stream, s.pos.as<double4>(),
                            (const int*)s.g_owner.as<int>(), (const int*)s.g_code.as<int>(), s.n, s.ng, s.g.len[0], s.g.len[1],

@@ -149,7 +149,7 @@ static void alloc_atoms(Sim& s, int cap) {
     s.g_code.reserve(sizeof(int) * (size_t)cap, true, s.stream);
     s.cell_parts.reserve(sizeof(int) * (size_t)cap, false, s.stream);
     s.cell_inv.reserve(sizeof(int) * (size_t)cap, false, s.stream);
-    s.inv_valid = 0;
+    if (cap > s.cap_all) s.inv_valid = 0;  // the arrays are new; an upload alone leaves the cells as they are
     s.force.reserve(sizeof(double4) * (size_t)std::max(s.n, 1), false, s.stream);
     // the room that every array has: not raised if one of them could not grow
     if (cap > s.cap_all && !has_error()) s.cap_all = cap;

@@ -138,3 +138,39 @@ def test_cells_of_the_last_binning(tm):
     for c in range(len(st) - 1):
         assert np.all(at[pa[st[c]:st[c + 1]]] == c)
     sim.close()
+
+
+# a drop in the middle of its box has no ghosts; without a ghost index they
+# follow in a pass of their own
+@pytest.mark.parametrize("kind", ["full", "drop", "no_index", "dem"])
+def test_state_put_back_between_runs(tm, kind):
+    """Reading the state and uploading it again between two runs on the same
+    lists changes nothing."""
+    announce(f"state put back between runs, {kind}")
+    out = []
+    for put_back in (False, True):
+        if kind == "dem":
+            m, x, v = tm.generate_granular_gas(9, vmax=2.0)
+            sim = tm.Simulation(m, x, v, np.array([0.0, 9 * 1.6796] * 3), 1.3, dem_radius=0.5)
+        else:
+            aabb, m, x, v = perturbed_fcc(6, 5, 7, amp=0.05, seed=9)
+            if kind == "drop":
+                x, aabb = x + 14.0, np.array([0.0, 40.0] * 3)
+            sim = tm.Simulation(m, x, v, aabb, RC + SKIN)
+            tm.load().tmd_set_ghost_index_limit(1 if kind == "no_index" else 0)
+        sim.copy_to_accelerator()
+        rc = 1.0 if kind == "dem" else RC
+        sim.setup(kind == "dem", rc, SKIN)
+        sim.dem(True, rc) if kind == "dem" else sim.lennard_jones(False, rc)
+        assert (sim.nghost == 0) == (kind == "drop")
+        res = []
+        for steps in (7, 6, 25):
+            sim.run_dem(steps, 20, 0.001) if kind == "dem" else sim.run_lj(steps, 20, 0.005)
+            res += sim.state()[1:]
+            if put_back:
+                sim.copy_to_accelerator()
+        out.append(res)
+        tm.load().tmd_set_ghost_index_limit(0)
+    sim.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
