@@ -332,10 +332,19 @@ __device__ __forceinline__ double lj_group_atom(const double4 pi, int cnt, const
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
-        for (int k = 0; k < E; ++k) {
-            if (PREC == PREC_FP64) F = F + mine[(3 * k + c) * A];
-            else if (PREC == PREC_FP32_MIXED) F = fma(mine[(4 * k + c) * A], mine[(4 * k + 3) * A], F);
-            else kahan_add(fs, fc, minef[(3 * k + c) * A]);
+        for (int k0 = 0; k0 < E; k0 += 4) {
+            if (PREC == PREC_FP32_KAHAN) {
+                // a zero is not nothing to a compensated sum: only the halves of
+                // list groups that lj_full_atom takes
+                const int e = base + k0, g = e >> 3;
+                if ((e & 4) >= ((!PAIR2 || g < ng1) ? cnt - 8 * g : cnt2 - 8 * (g - ng1))) continue;
+            }
+#pragma unroll
+            for (int k = k0; k < k0 + 4; ++k) {
+                if (PREC == PREC_FP64) F = F + mine[(3 * k + c) * A];
+                else if (PREC == PREC_FP32_MIXED) F = fma(mine[(4 * k + c) * A], mine[(4 * k + 3) * A], F);
+                else kahan_add(fs, fc, minef[(3 * k + c) * A]);
+            }
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();

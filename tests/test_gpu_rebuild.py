@@ -409,3 +409,27 @@ def test_ghosts_outgrow_their_room_dem(tm):
     _, xh, vh, _ = sim.ghost_state()
     assert np.array_equal(vh, vg[gt["owner"]]) and np.array_equal(xh, xg[gt["owner"]] + gt["img"] * L)
     sim.close()
+
+
+@pytest.mark.parametrize("shape,seed", [((6, 5, 7), 10), ((8, 7, 6), 44), ((8, 7, 6), 53)])
+def test_lanes_of_an_atom_compensated_half_lists(tm, shape, seed):
+    """Compensated sums over both columns of a half list by four lanes an atom:
+    bit for bit the separate calls' (a zero for each absent entry between the
+    columns moved these boxes' sums by a rounding now and then)."""
+    announce(f"lanes of an atom, compensated {shape} {seed}")
+    rng = np.random.default_rng(seed)
+    m, x, _ = tm.generate_fcc(*shape)
+    L = np.array(shape) * 1.6796
+    aabb = np.stack([0.0 * L, L], axis=1).ravel()
+    x = np.mod(x + rng.uniform(-0.05, 0.05, x.shape), L)
+    v = rng.normal(0.0, 1.2, x.shape)
+    out = []
+    for run in ("run_lj", "run_abi_lj"):
+        sim = tm.Simulation(m, x, v, aabb, RC + SKIN, precision="fp32kahan")
+        sim.copy_to_accelerator()
+        sim.setup(True, RC, SKIN)
+        sim.lennard_jones(True, RC)
+        getattr(sim, run)(60, 20, DT, True)
+        out.append(sim.state()[1:])
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
