@@ -133,7 +133,7 @@ __global__ void __launch_bounds__(G > 1 ? kGroupThreads : kMaxTileThreads) k_tra
         t.vel[kw] = v;
     }
     if (ENERGY) {
-        const double bpe = block_sum_double_any(en.pe);
+        const double bpe = block_sum_double_any(energy_sum(en.pe, a));
         const double bvir = block_sum_double_any(en.vir);
         const double bv2 = block_sum_double_any(v2);
         if (threadIdx.x == 0) {

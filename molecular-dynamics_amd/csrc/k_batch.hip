@@ -612,7 +612,7 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_b_energy(const RepDesc* __r
         if (staged) lj_energy_atom<SHIFT, true>(pos[work[w]], cnt, lp, sp, spos, parts, W, a, 0, D.a0 + D.n, pe, vir, np);
         else lj_energy_atom<SHIFT, false>(pos[work[w]], cnt, lp, sp, spos, parts, W, a, 0, D.a0 + D.n, pe, vir, np);
     }
-    const double bpe = block_sum_double_any(pe);
+    const double bpe = block_sum_double_any(energy_sum(pe, a));
     const double bvir = block_sum_double_any(vir);
     const double bnp = block_sum_double_any(np);
     if (threadIdx.x == 0) {

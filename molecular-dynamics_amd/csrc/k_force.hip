@@ -269,7 +269,7 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_lj_energy(TMD_KERNEL_LIST_P
         if (staged) lj_energy_atom<SHIFT, true>(pos[work[w]], nbc[w], lp, sp, spos, parts, W, a, half, a.n, pe, vir, np);
         else lj_energy_atom<SHIFT, false>(pos[work[w]], nbc[w], lp, sp, spos, parts, W, a, half, a.n, pe, vir, np);
     }
-    const double bpe = block_sum_double_any(pe);
+    const double bpe = block_sum_double_any(energy_sum(pe, a));
     const double bvir = block_sum_double_any(vir);
     const double bnp = block_sum_double_any(np);
     if (threadIdx.x == 0) {

@@ -13,8 +13,9 @@ namespace tmd {
 // (Markstein's final step), as the compiler's division does them, without the
 // scaling and the special-case fix-up around it, which operands of ordinary
 // size do not need (here squared distances, from 2^-1022 to about 1e300).
-// Zero and below give NaN where the division gave infinity: the force of
-// two atoms at one point is NaN either way, their energy takes rcp_near.
+// Zero and below give NaN where the division gave infinity: the force and
+// virial of two atoms at one point are NaN either way, for their energy see
+// energy_sum.
 // Infinity, which the cutoff masks, gives NaN and not zero.  1 / x is 7
 // instructions instead of 11, and quotients by the same x share the first 5.
 __device__ __forceinline__ double rcp_refined(double x) {
@@ -26,8 +27,6 @@ __device__ __forceinline__ double rcp_round(double x) {
     const double y = rcp_refined(x);
     return fma(fma(-x, y, 1.0), y, y);
 }
-// 1 / x of any x >= 0 for the powers of an energy, which are infinite at zero
-__device__ __forceinline__ double rcp_near(double x) { return rcp_round(fmax(x, 0x1p-1022)); }
 __device__ __forceinline__ double div_round(double num, double x, double y) {  // y = rcp_refined(x)
     const double q = num * y;
     return fma(fma(-x, q, num), y, q);
@@ -42,11 +41,10 @@ __device__ __forceinline__ int nb_entry(const int4& q, int u) {
 
 // FP64 pair scalar of the reference closure; UNIT skips the exact
 // multiplications by eps = 1 and sigma^6 = 1 (x * 1.0 == x), so the result
-// is bit-identical either way.  sr6 also serves the energy (ENERGY: infinite
-// at zero distance).
-template <int SHIFT, int UNIT, bool ENERGY = false>
+// is bit-identical either way.  sr6 also serves the energy.
+template <int SHIFT, int UNIT>
 __device__ __forceinline__ double lj_f64u(const LJArgs& a, double rsq, double& sr6) {
-    const double sr2 = ENERGY ? rcp_near(rsq) : rcp_round(rsq);
+    const double sr2 = rcp_round(rsq);
     sr6 = UNIT ? sr2 * sr2 * sr2 : sr2 * sr2 * sr2 * a.sigma6;
     double f = UNIT ? 48.0 * sr6 * (sr6 - 0.5) * sr2 : 48.0 * sr6 * (sr6 - 0.5) * sr2 * a.eps;
     if (SHIFT) f = f - a.fc - (rsq - a.rc2) * a.dfc;
@@ -62,6 +60,12 @@ __device__ __forceinline__ double lj_u64(const LJArgs& a, double rsq, double sr6
         u = u - a.uc + ds * (0.5 * a.fc) + ds * ds * (0.25 * a.dfc);
     }
     return u;
+}
+
+// A lane's energy sum.  A pair at zero distance made it NaN where its energy is
+// infinite, 4 eps sr6^2: set right once, at the end of the sum.
+__device__ __forceinline__ double energy_sum(double pe, const LJArgs& a) {
+    return pe == pe ? pe : 4.0 * a.eps * (__builtin_inf() * a.sigma6);
 }
 
 template <int SHIFT, int UNIT>
@@ -178,7 +182,7 @@ __device__ __forceinline__ double4 lj_full_atom(const double4 pi, int cnt, const
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 double sr6;
-                const double f = lj_f64u<SHIFT, UNIT, true>(a, rs[u], sr6);
+                const double f = lj_f64u<SHIFT, UNIT>(a, rs[u], sr6);
                 en->pe += 0.5 * (ok[u] ? lj_u64<SHIFT>(a, rs[u], sr6) : 0.0);
                 en->vir += 0.5 * (ok[u] ? f * rs[u] : 0.0);
             }
@@ -191,7 +195,7 @@ __device__ __forceinline__ double4 lj_full_atom(const double4 pi, int cnt, const
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 double sr6;
-                const double f = lj_f64u<SHIFT, UNIT, ENERGY>(a, rs[u], sr6);
+                const double f = lj_f64u<SHIFT, UNIT>(a, rs[u], sr6);
                 const double fm = ok[u] ? f : 0.0;
                 if (ENERGY) {
                     en->pe += 0.5 * (ok[u] ? lj_u64<SHIFT>(a, rs[u], sr6) : 0.0);
@@ -390,7 +394,7 @@ __device__ __forceinline__ void lj_energy_atom(const double4 pi, int cnt, const 
             const double dx = pi.x - xj, dy = pi.y - yj, dz = pi.z - zj;
             const double rsq = dx * dx + dy * dy + dz * dz;
             if (rsq < a.rc2) {
-                const double sr2 = rcp_near(rsq);
+                const double sr2 = rcp_round(rsq);
                 const double sr6 = sr2 * sr2 * sr2 * a.sigma6;
                 double f = 48.0 * sr6 * (sr6 - 0.5) * sr2 * a.eps;
                 double uu = 4.0 * a.eps * sr6 * (sr6 - 1.0);
