@@ -736,7 +736,7 @@ static int scan_scratch(int n) { return div_up(std::max(n, 1), kScanTile) + 1; }
 // of 2 and 3 cells.  Ragged cubes of 3 cells in 64 replicas of 864 to 55,296
 // atoms: 200 steps 37.2 ms; windows to 2,000 atoms 39.8, to 2,400 36.4, to
 // 2,700 34.8, to 3,000 34.1 (with the runs of xcd_deal, 1 % of it); the LDS
-// share holds 3,413.  In a batch of `all` atoms a full tile has at most a 200th
+// share holds 3,370.  In a batch of `all` atoms a full tile has at most a 200th
 // of them, down to two cells: fewer tiles leave CUs idle, and the pass lasts
 // as long as its fullest block.  us a step, without and with that bound: 2,728
 // atoms FP64 25.5, 20.2; 11,200 FP32-mixed 24.6, 17.7; 63,396 FP64 45.0, 36.6;
